@@ -61,8 +61,8 @@ constexpr int HDR_VALID = 1;   // entry holds a partial row
 constexpr int HDR_ENDS = 2;    // head entry: the row ends inside this unit
 constexpr int HDR_STARTS = 4;  // tail entry: the row started inside this unit
 
-constexpr int MODE_F32_VEC4 = 0;     // fp32 rows, one 16-byte load per lane
-constexpr int MODE_F32_STRIDED = 1;  // fp32 rows of any width/alignment, dword loads, lane-strided
+constexpr int MODE_F32_VEC4 = 0;     // fp32 rows of 4 columns and more, one 16-byte load per lane, rows on any 4-byte boundary
+constexpr int MODE_F32_STRIDED = 1;  // fp32 rows of 1 to 3 columns, dword loads, one lane per row
 constexpr int MODE_BF16_VEC8 = 2;    // bf16 rows, one 16-byte load (8 values) per lane, fp32 accumulation
 
 struct AggArgs {
@@ -97,6 +97,7 @@ struct AggArgs {
     unsigned win_bytes;       // ... of this many bytes,
     unsigned delta_l, delta_r;// ... the tables starting at these byte offsets;
     int sentinel;             // ... and a row index whose offset falls outside the window (reads as zero)
+    int tail_shift;           // MODE_F32_VEC4: how many columns early the lane with a row's last, partial piece starts its 16 bytes
 };
 
 // Which workgroup descriptor q belongs to.  (An integer division by a run-time value costs some forty instructions; the
@@ -186,6 +187,9 @@ __device__ __forceinline__ int elem_of(int l, int i)
 }
 
 typedef unsigned v4u __attribute__((ext_vector_type(4)));
+// 16-byte accesses to rows that start on any 4-byte boundary (packed rows of 41 floats): one instruction each on gfx950
+typedef unsigned v4u_any __attribute__((ext_vector_type(4), aligned(4)));
+typedef float v4f_any __attribute__((ext_vector_type(4), aligned(4)));
 
 template <int MODE>
 __device__ __forceinline__ void unpack16(float (&v)[ModeTraits<MODE>::NV], const v4u t)
@@ -242,7 +246,7 @@ struct Gather {
                 t.w = *reinterpret_cast<const unsigned *>(p + sofs[3]);
                 return t;
             } else {
-                return *reinterpret_cast<const v4u *>(p);
+                return *reinterpret_cast<const v4u_any *>(p);
             }
         }
     }
@@ -298,8 +302,7 @@ __device__ __forceinline__ void group_softmax(float (&v)[NPL], const bool (&on)[
 // Output rows are written once and not read again by the aggregation: stored with the streaming hint.
 __device__ __forceinline__ void store_row16(float *p, float x, float y, float z, float w)
 {
-    typedef float v4f_s __attribute__((ext_vector_type(4)));
-    __builtin_nontemporal_store((v4f_s){x, y, z, w}, reinterpret_cast<v4f_s *>(p));
+    __builtin_nontemporal_store((v4f_any){x, y, z, w}, reinterpret_cast<v4f_any *>(p));
 }
 
 // Finishes this lane's NV elements of a complete row held in registers.  SMX: the kernel variant that serves calls with
@@ -349,32 +352,19 @@ __device__ __forceinline__ void finish_row(const AggArgs &a, int row, int l, con
     }
     if constexpr (MODE == MODE_F32_VEC4) {
         // the same epilogue as finish_elem on this lane's four contiguous elements, with vector loads and one store
-        if (NV * l < a.dim) {
+        if (NV * l + 3 < a.dim) {
             const float sc = a.rs_out ? a.rs_out[row] : 1.0f;
-            float4 v = make_float4(acc[0] * sc, acc[1] * sc, acc[2] * sc, acc[3] * sc);
-            if (a.flags & MGGX_AGG_GIN) {
-                const float4 s = *reinterpret_cast<const float4 *>(static_cast<const float *>(a.in_l) + (long long)row * a.ld_in + 4 * l);
-                const float k = 1.0f + a.eps;
-                v.x += k * s.x; v.y += k * s.y; v.z += k * s.z; v.w += k * s.w;
-            }
-            float4 *o = reinterpret_cast<float4 *>(a.out + (long long)row * a.ld_out + 4 * l);
-            if (a.flags & MGGX_AGG_ACCUMULATE) {
-                const float4 p = *o;
-                v.x += p.x; v.y += p.y; v.z += p.z; v.w += p.w;
-            }
+            v4f_any v = {acc[0] * sc, acc[1] * sc, acc[2] * sc, acc[3] * sc};
+            if (a.flags & MGGX_AGG_GIN)
+                v += (1.0f + a.eps) * *reinterpret_cast<const v4f_any *>(static_cast<const float *>(a.in_l) + (long long)row * a.ld_in + 4 * l);
+            float *o = a.out + (long long)row * a.ld_out + 4 * l;
+            if (a.flags & MGGX_AGG_ACCUMULATE) v += *reinterpret_cast<const v4f_any *>(o);
             if (a.flags & MGGX_AGG_RELU) {
                 v.x = fmaxf(v.x, 0.f); v.y = fmaxf(v.y, 0.f); v.z = fmaxf(v.z, 0.f); v.w = fmaxf(v.w, 0.f);
             }
-            if (NV * l + 3 < a.dim) {
-                store_row16(reinterpret_cast<float *>(o), v.x, v.y, v.z, v.w);
-            } else {
-                const float t[4] = {v.x, v.y, v.z, v.w};
-#pragma unroll
-                for (int i = 0; i < 4; ++i)
-                    if (4 * l + i < a.dim) reinterpret_cast<float *>(o)[i] = t[i];
-            }
+            store_row16(o, v.x, v.y, v.z, v.w);
+            return;
         }
-        return;
     }
 #pragma unroll
     for (int i = 0; i < NV; ++i) {
@@ -443,6 +433,11 @@ __global__ void __launch_bounds__(1024) MGGX_AGG_OCCUPANCY k_agg(const AggArgs a
     } else {
         cofs = 16u * (unsigned)(NV * l < a.dim ? l : 0);
     }
+    // The lane with a row's last, partial piece (width not a multiple of 4) starts its 16 bytes tail_shift columns early, so
+    // no lane reads past its row whatever the pitch; its sums are moved down by as much where they leave the registers.
+    const bool tail_lane = MODE == MODE_F32_VEC4 && NV * l < a.dim && NV * l + 3 >= a.dim;
+    if constexpr (MODE == MODE_F32_VEC4)
+        if (tail_lane) cofs -= 4u * (unsigned)a.tail_shift;
     if constexpr (BUF) g.rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(a.win_base), 0, a.win_bytes, 0x00020000);
     g.zero = reinterpret_cast<const char *>(g_zero_row) + cofs;
     const int pad_id = BUF ? a.sentinel : -1;  // what a slot holds past the end of its partition
@@ -693,8 +688,17 @@ __global__ void __launch_bounds__(1024) MGGX_AGG_OCCUPANCY k_agg(const AggArgs a
         const bool last_round = (j == a.dist - 1) || (q0 + S >= num_parts);
         bool keep_open = false;
         if (run_last) {
+            float fin[NV];  // the sums by column: acc, moved down by tail_shift in the tail lane
+#pragma unroll
+            for (int i = 0; i < NV; ++i) fin[i] = acc[i];
+            if constexpr (MODE == MODE_F32_VEC4) {
+                if (tail_lane) {
+                    if (a.tail_shift & 1) { fin[0] = fin[1]; fin[1] = fin[2]; fin[2] = fin[3]; }
+                    if (a.tail_shift & 2) { fin[0] = fin[2]; fin[1] = fin[3]; }
+                }
+            }
             if (row_done && has_first) {
-                finish_row<LPR, MODE, SMX>(a, row, l, acc);
+                finish_row<LPR, MODE, SMX>(a, row, l, fin);
             } else if (!row_done && !last_round) {
                 keep_open = true;  // slot S-1 only: continues in the next round
             } else {
@@ -706,7 +710,7 @@ __global__ void __launch_bounds__(1024) MGGX_AGG_OCCUPANCY k_agg(const AggArgs a
 #pragma unroll
                 for (int i = 0; i < NV; ++i) {
                     const int dd = elem_of<LPR, MODE>(l, i);
-                    if (dd < a.dim) dst[dd] = acc[i];
+                    if (dd < a.dim) dst[dd] = fin[i];
                 }
             }
         }
@@ -950,16 +954,20 @@ int pow2_ceil(int x)
     return p;
 }
 
+template <int LPR, int MODE, bool BUF, bool SMX>
+int launch_agg_as(dim3 grid, dim3 block, size_t lds_bytes, hipStream_t stream, const AggArgs &a)
+{
+    if (lds_bytes > (48u << 10))
+        (void)hipFuncSetAttribute(reinterpret_cast<const void *>(&k_agg<LPR, MODE, BUF, SMX>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_bytes);
+    k_agg<LPR, MODE, BUF, SMX><<<grid, block, lds_bytes, stream>>>(a);
+    return MGGX_OK;
+}
+
 template <int MODE, bool BUF, bool SMX>
 int launch_agg(int lpr, dim3 grid, dim3 block, size_t lds_bytes, hipStream_t stream, const AggArgs &a)
 {
     switch (lpr) {
-#define MGGX_CASE(L)                                                      \
-    case L:                                                               \
-        if (lds_bytes > (48u << 10))                                      \
-            (void)hipFuncSetAttribute(reinterpret_cast<const void *>(&k_agg<L, MODE, BUF, SMX>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_bytes); \
-        k_agg<L, MODE, BUF, SMX><<<grid, block, lds_bytes, stream>>>(a);  \
-        break;
+#define MGGX_CASE(L) case L: return launch_agg_as<L, MODE, BUF, SMX>(grid, block, lds_bytes, stream, a);
         MGGX_CASE(1)
         MGGX_CASE(2)
         MGGX_CASE(4)
@@ -971,7 +979,6 @@ int launch_agg(int lpr, dim3 grid, dim3 block, size_t lds_bytes, hipStream_t str
         default:
             return fail(MGGX_EINVAL, "aggregation: no kernel for %d lanes per row", lpr);
     }
-    return MGGX_OK;
 }
 
 // `fixed` != NULL: the carry buffer comes from that block (the static scratch) instead of the library's grow-only
@@ -1021,13 +1028,7 @@ int run_agg(Plan *plan, float *d_out, const void *d_in_l, const void *d_in_r, co
         mode = MODE_BF16_VEC8;
         lpr = pow2_ceil(dim / 8);
     } else if (o.in_dtype == MGGX_F32) {
-        // 16-byte accesses per lane wherever the tables allow them: rows that start on 16-byte boundaries and are at least
-        // ceil(dim/4) pieces long (a width that is not a multiple of 4 reads up to three padding columns of its own row
-        // pitch and never stores them)
-        const long long dim4 = (dim + 3) & ~3;
-        const bool out_ok = blocked || (ld_out % 4 == 0 && ld_out >= dim4 && aligned16(d_out));  // blocked plans write their own partial rows
-        const bool vec = ld_in % 4 == 0 && ld_in >= dim4 && out_ok && aligned16(d_in_l) && (!d_in_r || aligned16(d_in_r));
-        mode = vec ? MODE_F32_VEC4 : MODE_F32_STRIDED;
+        mode = dim >= 4 ? MODE_F32_VEC4 : MODE_F32_STRIDED;
         lpr = pow2_ceil((dim + 3) / 4);
     } else {
         return fail(MGGX_EINVAL, "aggregation: unknown input dtype %d", o.in_dtype);
@@ -1093,6 +1094,9 @@ int run_agg(Plan *plan, float *d_out, const void *d_in_l, const void *d_in_r, co
     a.flags = blocked ? 0u : o.flags;
     a.eps = o.eps;
     a.in_is_bf16 = o.in_dtype == MGGX_BF16;
+    // Rows whose pitch has room for whole pieces are read in aligned pieces (up to three padding columns with them); packed
+    // rows of a width that is not a multiple of 4 never read past their end (see tail_lane in k_agg).
+    a.tail_shift = (dim & 3) && !(ld_in % 4 == 0 && ld_in > dim) ? 4 - (dim & 3) : 0;
 
     // Gather addressing.  Extent of each table: the local one holds the share's rows, the remote one at least the
     // largest remote id.  When both fit one window of < 2 GiB and < 2^24 rows, offsets are 32-bit buffer offsets.
@@ -1159,14 +1163,14 @@ int run_agg(Plan *plan, float *d_out, const void *d_in_l, const void *d_in_r, co
         if (buf) {
             if (mode == MODE_F32_VEC4) rc = smx ? launch_agg<MODE_F32_VEC4, true, true>(lpr, grid, block, lds_bytes, st.stream, a)
                                                 : launch_agg<MODE_F32_VEC4, true, false>(lpr, grid, block, lds_bytes, st.stream, a);
-            else if (mode == MODE_F32_STRIDED) rc = smx ? launch_agg<MODE_F32_STRIDED, true, true>(lpr, grid, block, lds_bytes, st.stream, a)
-                                                        : launch_agg<MODE_F32_STRIDED, true, false>(lpr, grid, block, lds_bytes, st.stream, a);
+            else if (mode == MODE_F32_STRIDED) rc = smx ? launch_agg_as<1, MODE_F32_STRIDED, true, true>(grid, block, lds_bytes, st.stream, a)
+                                                        : launch_agg_as<1, MODE_F32_STRIDED, true, false>(grid, block, lds_bytes, st.stream, a);
             else rc = launch_agg<MODE_BF16_VEC8, true, false>(lpr, grid, block, lds_bytes, st.stream, a);
         } else {
             if (mode == MODE_F32_VEC4) rc = smx ? launch_agg<MODE_F32_VEC4, false, true>(lpr, grid, block, lds_bytes, st.stream, a)
                                                 : launch_agg<MODE_F32_VEC4, false, false>(lpr, grid, block, lds_bytes, st.stream, a);
-            else if (mode == MODE_F32_STRIDED) rc = smx ? launch_agg<MODE_F32_STRIDED, false, true>(lpr, grid, block, lds_bytes, st.stream, a)
-                                                        : launch_agg<MODE_F32_STRIDED, false, false>(lpr, grid, block, lds_bytes, st.stream, a);
+            else if (mode == MODE_F32_STRIDED) rc = smx ? launch_agg_as<1, MODE_F32_STRIDED, false, true>(grid, block, lds_bytes, st.stream, a)
+                                                        : launch_agg_as<1, MODE_F32_STRIDED, false, false>(grid, block, lds_bytes, st.stream, a);
             else rc = launch_agg<MODE_BF16_VEC8, false, false>(lpr, grid, block, lds_bytes, st.stream, a);
         }
         if (rc) return rc;

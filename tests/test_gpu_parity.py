@@ -565,6 +565,23 @@ def test_padded_row_strides(gpu, rmat_graph, dim, ld):
     assert np.all(got[:, dim:] == 7.5), "padding columns of the output must stay untouched"
 
 
+@pytest.mark.parametrize("dim,ld", [(5, 5), (6, 7), (7, 9), (41, 41), (42, 43), (43, 45), (66, 66), (129, 131), (255, 255)])
+def test_rows_off_16_byte_boundaries(gpu, rmat_graph, dim, ld):
+    """Rows that start on any 4-byte boundary: the lane with a row's last, partial piece reads its 16 bytes one to three
+    columns early (a NaN behind every row would show a sum that took in a column too many)."""
+    V, ptr, col = rmat_graph
+    xp = np.full((V, ld), np.nan, np.float32)
+    xp[:, :dim] = gpu.fill_normal((V, dim), seed=300 + dim)
+    sh = share_of(ptr, col, V, 2, 1)
+    x = np.ascontiguousarray(xp[:, :dim])
+    xl = x[sh["lb"]:sh["ub"]]
+    for kw, okw in ((dict(), dict()), (dict(gin=True, eps=0.5), dict(flags=orc.GIN, eps=0.5))):
+        got = run_agg(gpu, sh, to_dev(xp[sh["lb"]:sh["ub"]]), to_dev(xp), dim, 16, 4, 2, ld_in=ld, ld_out=ld, **kw)
+        want, mag = oracle_agg(sh, xl, x, dim, **okw)
+        assert_close_to_oracle(got[:, :dim], want, mag, FP32_TOL, "dim=%d ld=%d %s" % (dim, ld, kw))
+        assert np.all(got[:, dim:] == 7.5), "padding columns of the output must stay untouched"
+
+
 @pytest.mark.parametrize("dim", [16, 41, 64])
 def test_gin_accumulate_relu(gpu, rmat_graph, dim):
     V, ptr, col = rmat_graph
