@@ -1002,6 +1002,11 @@ struct CoreMerge {
     bool merged;
 };
 
+// Rounds of the whole plan from which on a wavefront may take 16 of them (rows of 16 lanes and more); with fewer a wavefront
+// takes at most 4, and never so many that fewer than MIN_WAVEFRONTS wavefronts (3 per SIMD) are left for the chip.
+constexpr long long MANY_ROUNDS = 400000;
+constexpr int MIN_WAVEFRONTS = 3000;
+
 int run_agg(Plan *plan, float *d_out, const void *d_in_l, const void *d_in_r, const int *d_col_l, const int *d_col_r,
             int lb, int dim, int wpb, int dist, const mggx_agg_opts &o_in, const Gate &gate, const FixedScratch *fixed = nullptr, CoreMerge *cm = nullptr)
 {
@@ -1034,29 +1039,34 @@ int run_agg(Plan *plan, float *d_out, const void *d_in_l, const void *d_in_r, co
         return fail(MGGX_EINVAL, "aggregation: unknown input dtype %d", o.in_dtype);
     }
     const int slots = 64 / lpr;
-    // 0 = let the library choose.  Few slots per wavefront (wide rows): 8 wavefronts and 16 rounds, so a workgroup still
-    // covers a few thousand neighbors; column-blocked plans: 4 wavefronts (they share the chip with the dense core's
-    // 4-wavefront workgroups); in row-major order beside a dense core: 8 wavefronts and 4 rounds, 8 rounds where the core
-    // works in wide row groups (width 52 to 64, staged table beyond 12 MB: seven graphs of 0.7 to 3 M nodes at width 64 are
-    // 1.4 - 3.7 % faster with 8 than with 4, one of them by 0.1 %; at width 48, narrow groups, 8 rounds cost 1.1 %); short
-    // rows (under 3 partitions per row): 4 wavefronts.  Many slots (narrow rows): 4 wavefronts, 4 rounds; 8 rounds where a column-blocked
-    // plan is left with short rows (under 8 partitions per row and block); 2 rounds for rows of 84 to 128 bytes (8 slots)
-    // in row-major order beside a dense core -- there a wavefront's share is 16 partitions, as with 4 slots and 4 rounds.
-    // Provenance: wpb x dist sweeps on the three benchmark graphs and the bf16 share (each choice within 1 % of the best
-    // cell there), re-checked on graphs of other generators, sizes, degrees and widths: within 4 % of the best cell on
-    // every one of twenty-four, after two changes they forced -- beside a core in row-major order the first version took
-    // 4 wavefronts, which two 1 M-node graphs at widths 41 and 64 answered with 10 - 17 % over 8 wavefronts; and it took 4
-    // rounds at 8 slots, 4 - 7 % over 2 rounds on two graphs of widths 24 and 32 (then, on three graphs made for the
-    // purpose: widths 24 / 28 / 28 -0.1 / -3.6 / -1.8 % with 2 rounds; two graphs of width 20 were 1.4 and 2.7 % slower with 2,
-    // three of widths 12 to 16 within 0.6 % except one 2.5 % faster: both stay at 4).
+    // 0 = let the library choose.  A wavefront's time is one chain of memory latencies per staged group of rounds, so a plan
+    // is cut into enough wavefronts first and into long ones second:
+    //  - MIN_WAVEFRONTS: 4, then 2, then 1 round per wavefront as the plan gets small (4,096 nodes of mean degree 17, width 41:
+    //    29.6 us with 16 rounds, 14.0 with 4, 10.9 with 1; 20 K nodes of mean degree 7: 31.1 / 14.9 / 13.0 with 2);
+    //  - rows of 16 lanes and more (4 slots and fewer): 4 rounds up to MANY_ROUNDS rounds in all, then 16 (20 K nodes of mean
+    //    degree 130, width 128: 95 us with 8 wavefronts x 16 rounds, 71 with 4 x 4; 300 K nodes, width 64: 157 / 147; but the
+    //    bf16 share of 3.7 M partitions: 957 us with 4 rounds, 942 with 8 or 16);
+    //  - slots of one or two lanes (width up to 8) stage two rounds at a time and take 2 (300 K nodes: 58.5 us with 4, 50.7 with 2).
+    // 4 wavefronts per workgroup, 8 where a large plan has long rows (3 partitions per row and more, MANY_ROUNDS rounds):
+    // 8 wavefronts cost 3 - 20 % on the small graphs above.  Column-blocked plans: 4 wavefronts (they share the chip with the
+    // dense core's 4-wavefront workgroups), 16 rounds at 4 slots and fewer, 8 rounds where such a plan of narrow rows is left
+    // with under 8 partitions per row and block.  In row-major order beside a dense core: 8 wavefronts and 4 rounds, 8 rounds
+    // where the core works in wide row groups (width 52 to 64, staged table beyond 12 MB: seven graphs of 0.7 to 3 M nodes at
+    // width 64 are 1.4 - 3.7 % faster with 8 than with 4, one of them by 0.1 %); 2 rounds for rows of 84 to 128 bytes (8 slots).
+    // Provenance: wpb x dist sweeps over eight graphs of 4 K to 800 K nodes at widths 8 to 128, the shares and the 2.45 M-node
+    // graph: within 6 % of the best cell of {1,2,4,8} x {1,2,4,8,16} on all of them, within 2 % on most.
     const double per_row = (double)plan->num_parts / (double)(plan->rows > 0 ? plan->rows : 1);
+    const long long rounds = (plan->num_parts + slots - 1) / slots;
     const bool beside_core = cm != nullptr;
-    if (wpb == 0) wpb = (beside_core && !blocked && slots <= 4) ? 8 : (blocked || slots > 4 || per_row < 3.0) ? 4 : 8;
+    if (wpb == 0) wpb = (beside_core && !blocked && slots <= 4) ? 8 : (blocked || slots > 4 || per_row < 3.0 || rounds < MANY_ROUNDS) ? 4 : 8;
     if (dist == 0) {
-        if (slots <= 4) dist = (beside_core && !blocked) ? (cm->group_rows == CORE_GROUP_ROWS_WIDE ? 8 : 4) : 16;
+        if (slots <= 4 && beside_core && !blocked) dist = cm->group_rows == CORE_GROUP_ROWS_WIDE ? 8 : 4;
+        else if (slots <= 4) dist = blocked || rounds >= MANY_ROUNDS ? 16 : 4;
         else if (blocked && per_row < 8.0) dist = 8;
         else if (beside_core && !blocked && slots == 8 && dim > 20) dist = 2;
+        else if (slots >= 32) dist = 2;
         else dist = 4;
+        while (dist > 1 && rounds < (long long)MIN_WAVEFRONTS * dist) dist /= 2;
     }
     const long long parts_per_wg = (long long)wpb * slots * dist;
     if (parts_per_wg > 0x3fffffffLL) return fail(MGGX_ELIMIT, "aggregation: wpb*dist too large");
