@@ -62,6 +62,10 @@ constexpr int HDR_ENDS = 2;    // head entry: the row ends inside this unit
 constexpr int HDR_STARTS = 4;  // tail entry: the row started inside this unit
 
 constexpr int MODE_F32_VEC4 = 0;     // fp32 rows of 4 columns and more, one 16-byte load per lane, rows on any 4-byte boundary
+constexpr int MODE_F32_PACKED = 3;   // the same, for rows of a width that is not a multiple of 4 and a pitch without room for the last
+                                     // whole piece (see tail_shift).  A kernel of its own: in one kernel with the rows of whole
+                                     // pieces, the moves of the partial piece cost those 2.5 % (100 K nodes, width 100: 174.5 -> 178.9 us)
+                                     // and 1.6 % (five layers of 2.45 M nodes, width 64: 14.20 -> 14.44 ms)
 constexpr int MODE_F32_STRIDED = 1;  // fp32 rows of 1 to 3 columns, dword loads, one lane per row
 constexpr int MODE_BF16_VEC8 = 2;    // bf16 rows, one 16-byte load (8 values) per lane, fp32 accumulation
 
@@ -97,7 +101,7 @@ struct AggArgs {
     unsigned win_bytes;       // ... of this many bytes,
     unsigned delta_l, delta_r;// ... the tables starting at these byte offsets;
     int sentinel;             // ... and a row index whose offset falls outside the window (reads as zero)
-    int tail_shift;           // MODE_F32_VEC4: how many columns early the lane with a row's last, partial piece starts its 16 bytes
+    int tail_shift;           // MODE_F32_PACKED: how many columns early the lane with a row's last, partial piece starts its 16 bytes
 };
 
 // Which workgroup descriptor q belongs to.  (An integer division by a run-time value costs some forty instructions; the
@@ -177,6 +181,8 @@ template <int MODE>
 struct ModeTraits {
     static constexpr int NV = MODE == MODE_BF16_VEC8 ? 8 : 4;
 };
+template <int MODE>
+constexpr bool F32_PIECES = MODE == MODE_F32_VEC4 || MODE == MODE_F32_PACKED;
 
 // feature index of value i held by lane l of a slot
 template <int LPR, int MODE>
@@ -327,7 +333,7 @@ __device__ __forceinline__ void finish_row(const AggArgs &a, int row, int l, con
             if (on[i]) a.out[(long long)row * a.ld_out + elem_of<LPR, MODE>(l, i)] = v[i];
         return;
     }
-    if constexpr (MODE == MODE_F32_VEC4) {
+    if constexpr (F32_PIECES<MODE>) {
         if (a.flags == 0 && a.rs_out == nullptr) {
             if (NV * l + 3 < a.dim) {
                 store_row16(a.out + (long long)row * a.ld_out + 4 * l, acc[0], acc[1], acc[2], acc[3]);
@@ -350,7 +356,7 @@ __device__ __forceinline__ void finish_row(const AggArgs &a, int row, int l, con
             return;
         }
     }
-    if constexpr (MODE == MODE_F32_VEC4) {
+    if constexpr (F32_PIECES<MODE>) {
         // the same epilogue as finish_elem on this lane's four contiguous elements, with vector loads and one store
         if (NV * l + 3 < a.dim) {
             const float sc = a.rs_out ? a.rs_out[row] : 1.0f;
@@ -435,8 +441,8 @@ __global__ void __launch_bounds__(1024) MGGX_AGG_OCCUPANCY k_agg(const AggArgs a
     }
     // The lane with a row's last, partial piece (width not a multiple of 4) starts its 16 bytes tail_shift columns early, so
     // no lane reads past its row whatever the pitch; its sums are moved down by as much where they leave the registers.
-    const bool tail_lane = MODE == MODE_F32_VEC4 && NV * l < a.dim && NV * l + 3 >= a.dim;
-    if constexpr (MODE == MODE_F32_VEC4)
+    const bool tail_lane = MODE == MODE_F32_PACKED && NV * l < a.dim && NV * l + 3 >= a.dim;
+    if constexpr (MODE == MODE_F32_PACKED)
         if (tail_lane) cofs -= 4u * (unsigned)a.tail_shift;
     if constexpr (BUF) g.rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(a.win_base), 0, a.win_bytes, 0x00020000);
     g.zero = reinterpret_cast<const char *>(g_zero_row) + cofs;
@@ -691,7 +697,7 @@ __global__ void __launch_bounds__(1024) MGGX_AGG_OCCUPANCY k_agg(const AggArgs a
             float fin[NV];  // the sums by column: acc, moved down by tail_shift in the tail lane
 #pragma unroll
             for (int i = 0; i < NV; ++i) fin[i] = acc[i];
-            if constexpr (MODE == MODE_F32_VEC4) {
+            if constexpr (MODE == MODE_F32_PACKED) {
                 if (tail_lane) {
                     if (a.tail_shift & 1) { fin[0] = fin[1]; fin[1] = fin[2]; fin[2] = fin[3]; }
                     if (a.tail_shift & 2) { fin[0] = fin[2]; fin[1] = fin[3]; }
@@ -1033,7 +1039,8 @@ int run_agg(Plan *plan, float *d_out, const void *d_in_l, const void *d_in_r, co
         mode = MODE_BF16_VEC8;
         lpr = pow2_ceil(dim / 8);
     } else if (o.in_dtype == MGGX_F32) {
-        mode = dim >= 4 ? MODE_F32_VEC4 : MODE_F32_STRIDED;
+        // rows whose pitch has room for whole pieces are read in whole pieces, up to three padding columns with them
+        mode = dim < 4 ? MODE_F32_STRIDED : (dim & 3) && !(ld_in % 4 == 0 && ld_in > dim) ? MODE_F32_PACKED : MODE_F32_VEC4;
         lpr = pow2_ceil((dim + 3) / 4);
     } else {
         return fail(MGGX_EINVAL, "aggregation: unknown input dtype %d", o.in_dtype);
@@ -1104,9 +1111,7 @@ int run_agg(Plan *plan, float *d_out, const void *d_in_l, const void *d_in_r, co
     a.flags = blocked ? 0u : o.flags;
     a.eps = o.eps;
     a.in_is_bf16 = o.in_dtype == MGGX_BF16;
-    // Rows whose pitch has room for whole pieces are read in aligned pieces (up to three padding columns with them); packed
-    // rows of a width that is not a multiple of 4 never read past their end (see tail_lane in k_agg).
-    a.tail_shift = (dim & 3) && !(ld_in % 4 == 0 && ld_in > dim) ? 4 - (dim & 3) : 0;
+    a.tail_shift = mode == MODE_F32_PACKED ? 4 - (dim & 3) : 0;
 
     // Gather addressing.  Extent of each table: the local one holds the share's rows, the remote one at least the
     // largest remote id.  When both fit one window of < 2 GiB and < 2^24 rows, offsets are 32-bit buffer offsets.
@@ -1173,12 +1178,16 @@ int run_agg(Plan *plan, float *d_out, const void *d_in_l, const void *d_in_r, co
         if (buf) {
             if (mode == MODE_F32_VEC4) rc = smx ? launch_agg<MODE_F32_VEC4, true, true>(lpr, grid, block, lds_bytes, st.stream, a)
                                                 : launch_agg<MODE_F32_VEC4, true, false>(lpr, grid, block, lds_bytes, st.stream, a);
+            else if (mode == MODE_F32_PACKED) rc = smx ? launch_agg<MODE_F32_PACKED, true, true>(lpr, grid, block, lds_bytes, st.stream, a)
+                                                       : launch_agg<MODE_F32_PACKED, true, false>(lpr, grid, block, lds_bytes, st.stream, a);
             else if (mode == MODE_F32_STRIDED) rc = smx ? launch_agg_as<1, MODE_F32_STRIDED, true, true>(grid, block, lds_bytes, st.stream, a)
                                                         : launch_agg_as<1, MODE_F32_STRIDED, true, false>(grid, block, lds_bytes, st.stream, a);
             else rc = launch_agg<MODE_BF16_VEC8, true, false>(lpr, grid, block, lds_bytes, st.stream, a);
         } else {
             if (mode == MODE_F32_VEC4) rc = smx ? launch_agg<MODE_F32_VEC4, false, true>(lpr, grid, block, lds_bytes, st.stream, a)
                                                 : launch_agg<MODE_F32_VEC4, false, false>(lpr, grid, block, lds_bytes, st.stream, a);
+            else if (mode == MODE_F32_PACKED) rc = smx ? launch_agg<MODE_F32_PACKED, false, true>(lpr, grid, block, lds_bytes, st.stream, a)
+                                                       : launch_agg<MODE_F32_PACKED, false, false>(lpr, grid, block, lds_bytes, st.stream, a);
             else if (mode == MODE_F32_STRIDED) rc = smx ? launch_agg_as<1, MODE_F32_STRIDED, false, true>(grid, block, lds_bytes, st.stream, a)
                                                         : launch_agg_as<1, MODE_F32_STRIDED, false, false>(grid, block, lds_bytes, st.stream, a);
             else rc = launch_agg<MODE_BF16_VEC8, false, false>(lpr, grid, block, lds_bytes, st.stream, a);
