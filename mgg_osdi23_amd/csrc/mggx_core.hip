@@ -1004,6 +1004,14 @@ int core_row_sums(CorePlan *p, int dim, const float4 **sums)
 // 0.55 put the core of a 700 K-node graph of width 64 at 86,016 rows, 4 % slower than 81,920; with 0.62 the four graphs
 // of that width are within 1.3 % of their sweeps' best.
 // The model stops at 98,304 rows.
+// The whole core has to pay too: staging, the second stream, the partial rows and the finishing pass cost 30 to 40 us a call, and
+// a small core keeps k_core_sell busy for as long (a few hundred short workgroups), all of which the bands above do not see.  What the
+// gathers of its edges would take, measured without a core: GATHER ps per edge for rows of up to 4 / 8 / 16 lanes out of the L2s
+// (with the index stream that comes with it), times h + (1 - h) x G_CACHE (G_MEMORY beyond the last-level cache) in row-major order.
+// A core that takes off less than MIN_SAVING_PS does without.  Provenance: 76 graphs and widths (17 K to 1.5 M nodes, mean degrees
+// 20 to 200, widths 16, 32, 41 and 64), with and without the core: 37 of the 54 that had one were slower with it, up to three times
+// (50 K nodes, 2.2 M neighbors, width 64: 103 us with, 41 without; width 16: 70 / 23); the break-even lies at 100 to 150 us of gathers
+// (400 K nodes, 22 M neighbors: width 16 takes off 81 us and loses 7, width 41 198 us and gains 28).
 namespace mggx {
 namespace {
 
@@ -1011,6 +1019,7 @@ constexpr int PROFILE_SLICES = 2048;  // 131072 ranks
 constexpr double ALPHA_PS = 1.40, BETA_PS = 9.0, HALVES = 0.7, HALVES_WIDE = 0.62, F_CACHE = 3.0, F_MEMORY = 4.0;
 constexpr unsigned long long L2_BYTES = 4ull << 20, LAST_LEVEL_CACHE_BYTES = 256ull << 20;
 constexpr int MODEL_STEP = 4096, MODEL_MAX_CORE = 98304;
+constexpr double GATHER_PS[3] = {7.0, 8.0, 14.5}, G_CACHE = 2.5, G_MEMORY = 3.0, MIN_SAVING_PS = 130e6;
 
 __global__ void __launch_bounds__(256) k_degrees(const int *__restrict__ ptr, int rows, int *__restrict__ deg)
 {
@@ -1097,6 +1106,9 @@ int predict_core_rows(GraphInfo &g, int dim, unsigned long long table_bytes, int
     static const PaddingTable padded;
     *core_rows = -1;
     if (g.rows < 2 * MODEL_STEP || g.nnz_l <= 0) return MGGX_OK;
+    const double gather_ps = GATHER_PS[dim <= 16 ? 0 : dim <= 32 ? 1 : 2];
+    const bool cached = table_bytes <= LAST_LEVEL_CACHE_BYTES;
+    if ((double)g.nnz_l * gather_ps * (cached ? G_CACHE : G_MEMORY) < MIN_SAVING_PS) return MGGX_OK;  // not even all of its edges: no look at the degrees
     for (const GraphInfo::Predicted &p : g.predicted)
         if (p.dim == dim && p.block_rows == block_rows && p.table_bytes == table_bytes) {
             *core_rows = p.core_rows;
@@ -1140,7 +1152,7 @@ int predict_core_rows(GraphInfo &g, int dim, unsigned long long table_bytes, int
         const double left = nnz - core_deg * (core_deg / nnz);  // all edges but the core x core block
         return left > 0.0 ? std::min(1.0, hot / left) : 1.0;
     };
-    const double far = table_bytes <= LAST_LEVEL_CACHE_BYTES ? F_CACHE : F_MEMORY;
+    const double far = cached ? F_CACHE : F_MEMORY;
     const double blocks = block_rows > 0 ? std::ceil((double)g.rows / block_rows) : 0.0;
     int best = 0;
     double taken = 0.0;
@@ -1159,7 +1171,10 @@ int predict_core_rows(GraphInfo &g, int dim, unsigned long long table_bytes, int
         best = k;
         taken += useful;
     }
-    if (best >= 2 * MODEL_STEP) *core_rows = best;
+    if (best >= 2 * MODEL_STEP) {
+        const double h = block_rows > 0 ? 1.0 : hot_share(0);
+        if (taken * gather_ps * (h + (1.0 - h) * (cached ? G_CACHE : G_MEMORY)) >= MIN_SAVING_PS) *core_rows = best;
+    }
     g.predicted.push_back({dim, block_rows, table_bytes, *core_rows});
     return MGGX_OK;
 }

@@ -296,6 +296,29 @@ def test_dense_core_from_lds(gpu, rmat_graph, dim, core_rows, flags):
     assert np.array_equal(out.cpu().numpy()[:, :dim], np.repeat(np.diff(ptr).astype(np.float32)[:, None], dim, 1))
 
 
+@pytest.mark.parametrize("dim,V,draws", [(16, 30000, 1_400_000), (64, 30000, 1_400_000), (41, 8192, 300_000)])
+def test_no_dense_core_where_the_whole_call_is_shorter_than_its_overhead(gpu, dim, V, draws):
+    """core_rows = 0 on graphs whose gathers take a few tens of microseconds: the cost model turns the core down (it would
+    have grown one from its bands alone), and the sums are the oracle's, equal to the call with the core switched off."""
+    import torch
+    from mgg_osdi23_amd import host
+    ptr, col = host.gen_rmat(15, V, draws, seed=29)
+    x = gpu.fill_normal((V, dim), seed=303)
+    sh = share_of(ptr, col, V, 1, 0)
+    d_ptr, d_col, d_x = to_dev(ptr), to_dev(col), to_dev(x)
+    z, zc = torch.zeros(V + 1, dtype=torch.int32, device="cuda"), torch.zeros(1, dtype=torch.int32, device="cuda")
+    want, mag = oracle_agg(sh, x, x, dim)
+    outs = []
+    for core in (0, -1):
+        out = torch.full((V, dim), 7.5, device="cuda")
+        gpu.mgg_SAG_np_div(out, d_x, d_ptr, d_col, z, zc, 0, V, dim, V, 0, 0, 0, 0, core_rows=core)
+        gpu.sync()
+        assert "core=" not in gpu.last_agg_kernel()
+        outs.append(out.cpu().numpy())
+    assert_close_to_oracle(outs[0], want, mag, FP32_TOL, "core by the cost model, none expected")
+    assert np.array_equal(outs[0], outs[1])
+
+
 @pytest.mark.parametrize("dim,core_rows", [(16, 12800), (44, 13824)])
 def test_dense_core_with_tile_runs_of_unequal_length(gpu, dim, core_rows):
     """A core of 50 / 54 row groups and as many 256-column tiles, large enough for its workgroups to be cut into runs of
