@@ -639,13 +639,14 @@ struct Scratch {  // device temporaries of one plan build, freed on the way out
     std::vector<void *> ptrs;
     ~Scratch()
     {
-        for (void *q : ptrs) (void)hipFree(q);
+        for (void *q : ptrs) dev_free(q);
     }
     template <typename T>
     int get(T **q, size_t count)
     {
         void *r = nullptr;
-        if (hipMalloc(&r, std::max<size_t>(count, 1) * sizeof(T)) != hipSuccess) return fail(MGGX_ENOMEM, "core plan: %zu bytes of scratch", count * sizeof(T));
+        const int rc = dev_alloc(&r, std::max<size_t>(count, 1) * sizeof(T));
+        if (rc) return rc;
         ptrs.push_back(r);
         *q = static_cast<T *>(r);
         return MGGX_OK;

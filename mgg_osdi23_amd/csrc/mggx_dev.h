@@ -5,6 +5,7 @@
 #include <hip/hip_runtime.h>
 
 #include <list>
+#include <unordered_map>
 #include <vector>
 
 #include "mggx_internal.h"
@@ -219,6 +220,13 @@ struct State {
     bool ws_captured = false, core_ws_captured = false;
     std::vector<void *> retired;
     size_t retired_bytes = 0;
+    // device blocks kept between set-up calls (dev_alloc / dev_free)
+    struct Block { void *p; size_t bytes; int device; };
+    std::vector<Block> pool;                    // free, oldest first
+    std::unordered_map<void *, Block> pool_out; // handed out
+    size_t pool_bytes = 0;
+    bool pool_unordered = false;                // the stream or the device changed since the device was last waited for
+    long long *h_words = nullptr;               // pinned host words (host_words)
     // host-clock time spent on set-up so far (mggx_cache_stats)
     double plan_build_ms = 0.0, core_plan_build_ms = 0.0, search_ms = 0.0;
 };
@@ -227,6 +235,18 @@ State &state();
 int ensure_init();
 // Grow-only scratch owned by the library; valid until the next call that grows it.
 int workspace(size_t bytes, void **p);
+
+// Device memory of plans and of the scratch of set-up calls: dev_free keeps a bounded amount for the next dev_alloc.  Blocks may be
+// given back with kernels that use them still in flight on the library's stream (the next user comes after them there).
+int dev_alloc(void **p, size_t bytes);
+void dev_free(void *p);
+template <typename T>
+int dev_array(T **p, size_t count)
+{
+    return dev_alloc(reinterpret_cast<void **>(p), (count ? count : 1) * sizeof(T));
+}
+constexpr int HOST_WORDS = 64;
+int host_words(long long **w);
 
 // d_out[0..n] = exclusive prefix sum of d_in[0..n) (d_out has n+1 entries); the
 // total is also copied to *total_host when non-NULL (synchronises).

@@ -32,14 +32,33 @@ __device__ __forceinline__ int block_exclusive_scan(int v, int *lds /* 256 ints 
     return incl - v;
 }
 
-__global__ void __launch_bounds__(SCAN_THREADS) k_scan_tile_sums(const int *__restrict__ in, int n, long long *__restrict__ tile_sum)
+// What a scan sums: element i, read (or computed) twice rather than written out in between.
+struct ScanArray {
+    const int *in;
+    __device__ __forceinline__ int operator()(long long i) const { return in[i]; }
+};
+// parts of one CSR side per row: ceil(deg/ps); both sides summed when beg_r != NULL.  Row r spans edges
+// [beg[r], end[r]) (a CSR passes end = ptr + 1).
+struct ScanParts {
+    const int *beg_l, *end_l, *beg_r, *end_r;
+    int ps;
+    __device__ __forceinline__ int operator()(long long r) const
+    {
+        long long c = ((long long)end_l[r] - beg_l[r] + ps - 1) / ps;
+        if (beg_r) c += ((long long)end_r[r] - beg_r[r] + ps - 1) / ps;
+        return (int)c;
+    }
+};
+
+template <typename F>
+__global__ void __launch_bounds__(SCAN_THREADS) k_scan_tile_sums(const F in, int n, long long *__restrict__ tile_sum)
 {
     __shared__ long long red[SCAN_THREADS];
     const long long base = (long long)blockIdx.x * SCAN_TILE;
     long long s = 0;
     for (int i = 0; i < SCAN_ITEMS; ++i) {
         long long idx = base + (long long)threadIdx.x * SCAN_ITEMS + i;
-        if (idx < n) s += in[idx];
+        if (idx < n) s += in(idx);
     }
     red[threadIdx.x] = s;
     __syncthreads();
@@ -78,40 +97,62 @@ __global__ void __launch_bounds__(SCAN_THREADS) k_scan_tile_offsets(long long *_
     if (threadIdx.x == 0) tile_sum[num_tiles] = carry;
 }
 
-__global__ void __launch_bounds__(SCAN_THREADS) k_scan_apply(const int *__restrict__ in, int *__restrict__ out, int n,
-                                                             const long long *__restrict__ tile_off)
+// `tile`: the tiles' exclusive offsets (sums_only = 0), or their sums (sums_only = 1: every workgroup adds up the ones before
+// its own, which for up to SCAN_SUM_TILES tiles is a few KB out of the L2 and saves the launch in between).  The total goes to
+// out[n] and, in 64 bits, to *host_total (pinned host memory, or NULL).
+constexpr int SCAN_SUM_TILES = 1024;
+template <typename F>
+__global__ void __launch_bounds__(SCAN_THREADS) k_scan_apply(const F in, int *__restrict__ out, int n, const long long *__restrict__ tile, int sums_only,
+                                                             long long *host_total)
 {
     __shared__ int lds[SCAN_THREADS];
+    __shared__ long long part[SCAN_THREADS];
     const long long base = (long long)blockIdx.x * SCAN_TILE;
+    long long before = 0;
+    if (sums_only) {
+        for (int i = threadIdx.x; i < (int)blockIdx.x; i += SCAN_THREADS) before += tile[i];
+        part[threadIdx.x] = before;
+        __syncthreads();
+        for (int o = SCAN_THREADS / 2; o > 0; o >>= 1) {
+            if (threadIdx.x < o) part[threadIdx.x] += part[threadIdx.x + o];
+            __syncthreads();
+        }
+        before = part[0];
+    } else {
+        before = tile[blockIdx.x];
+    }
     int v[SCAN_ITEMS];
     int local = 0;
     for (int i = 0; i < SCAN_ITEMS; ++i) {
         long long idx = base + (long long)threadIdx.x * SCAN_ITEMS + i;
-        v[i] = idx < n ? in[idx] : 0;
+        v[i] = idx < n ? in(idx) : 0;
         local += v[i];
     }
     int total;
     int excl = block_exclusive_scan(local, lds, &total);
-    long long run = tile_off[blockIdx.x] + excl;
+    long long run = before + excl;
     for (int i = 0; i < SCAN_ITEMS; ++i) {
         long long idx = base + (long long)threadIdx.x * SCAN_ITEMS + i;
         if (idx < n) out[idx] = (int)run;
         run += v[i];
     }
-    if (blockIdx.x == gridDim.x - 1 && threadIdx.x == SCAN_THREADS - 1) out[n] = (int)run;
+    if (blockIdx.x == gridDim.x - 1 && threadIdx.x == SCAN_THREADS - 1) {
+        out[n] = (int)run;
+        if (host_total) *host_total = run;
+    }
 }
 
-// parts of one CSR side per row: ceil(deg/ps); both sides summed when beg_r != NULL.  Row r spans edges
-// [beg[r], end[r]) (a CSR passes end = ptr + 1).
-__global__ void __launch_bounds__(256) k_count_parts(const int *__restrict__ beg_l, const int *__restrict__ end_l,
-                                                     const int *__restrict__ beg_r, const int *__restrict__ end_r, int rows,
-                                                     int ps, int *__restrict__ cnt)
+// Results of a set-up call for the host: words[0] = the value at a, words[1] at b, words[2] at c (NULL: 0).
+__global__ void k_publish(const int *a, const int *b, const int *c, long long *words)
 {
-    const int r = blockIdx.x * 256 + threadIdx.x;
-    if (r >= rows) return;
-    long long c = ((long long)end_l[r] - beg_l[r] + ps - 1) / ps;
-    if (beg_r) c += ((long long)end_r[r] - beg_r[r] + ps - 1) / ps;
-    cnt[r] = (int)c;
+    words[0] = a ? *a : 0;
+    words[1] = b ? *b : 0;
+    words[2] = c ? *c : 0;
+}
+
+__global__ void k_zero_words(int *w, int n)
+{
+    if ((int)threadIdx.x < n) w[threadIdx.x] = 0;
 }
 
 // largest r in [0, rows) with off[r] <= q (off is non-decreasing, off[rows] > q)
@@ -269,10 +310,11 @@ __global__ void __launch_bounds__(256) k_parts_ref_layout(const int *__restrict_
     part2node[p] = i;
 }
 
-// max over non-negative ints (atomicMax once per block; set-up time only)
-__global__ void __launch_bounds__(256) k_max_i32(const int *__restrict__ v, long long n, int *__restrict__ out)
+// max over non-negative ints (atomicMax once per block; set-up time only); their number is read on the device
+__global__ void __launch_bounds__(256) k_max_i32(const int *__restrict__ v, const int *__restrict__ count, int *__restrict__ out)
 {
     __shared__ int red[256];
+    const long long n = *count;
     int m = 0;
     for (long long i = (long long)blockIdx.x * 256 + threadIdx.x; i < n; i += (long long)gridDim.x * 256) m = max(m, v[i]);
     red[threadIdx.x] = m;
@@ -443,7 +485,7 @@ int guard_arm(Guard &g)
     if (rc) return rc;
     if (!g.d_fp) {
         if (capturing()) return fail(MGGX_EINVAL, "first use of these CSR arrays inside a stream capture: call once outside the capture first");
-        if (hipMalloc((void **)&g.d_fp, 16) != hipSuccess) return fail(MGGX_ENOMEM, "content check: fingerprint");
+        if (const int rc = dev_array(&g.d_fp, 2)) return rc;
     }
     g.id = s.next_guard_id++;
     if (s.next_guard_id > 0x3fffffff) s.next_guard_id = 1;
@@ -483,7 +525,7 @@ void guard_free(Guard &g, bool retire)
 {
     if (g.d_fp) {
         if (retire) retire_block(g.d_fp, 16);
-        else (void)hipFree(g.d_fp);
+        else dev_free(g.d_fp);
     }
     g.d_fp = nullptr;
     g.armed = false;
@@ -518,20 +560,30 @@ size_t scan_tmp_bytes(int n)
     return sizeof(long long) * (tiles + 1);
 }
 
-int exclusive_scan_i32_device(const int *d_in, int *d_out, int n, void *d_tmp)
+// out[0..n] = exclusive prefix sums of in(0..n-1), in 2 or 3 launches; d_tmp: scan_tmp_bytes(n)
+template <typename F>
+static int scan_launch(const F &in, int *d_out, int n, void *d_tmp, long long *host_total)
 {
     State &s = state();
-    if (n <= 0) return fail(MGGX_EINVAL, "exclusive_scan: empty input");
     const int tiles = (n + SCAN_TILE - 1) / SCAN_TILE;
     long long *d_tile = static_cast<long long *>(d_tmp);
-    k_scan_tile_sums<<<tiles, SCAN_THREADS, 0, s.stream>>>(d_in, n, d_tile);
-    k_scan_tile_offsets<<<1, SCAN_THREADS, 0, s.stream>>>(d_tile, tiles);
-    k_scan_apply<<<tiles, SCAN_THREADS, 0, s.stream>>>(d_in, d_out, n, d_tile);
+    const int sums_only = tiles <= SCAN_SUM_TILES;
+    k_scan_tile_sums<F><<<tiles, SCAN_THREADS, 0, s.stream>>>(in, n, d_tile);
+    if (!sums_only) k_scan_tile_offsets<<<1, SCAN_THREADS, 0, s.stream>>>(d_tile, tiles);
+    k_scan_apply<F><<<tiles, SCAN_THREADS, 0, s.stream>>>(in, d_out, n, d_tile, sums_only, host_total);
     MGGX_LAUNCH_CHECK("exclusive scan");
     return MGGX_OK;
 }
 
-int exclusive_scan_i32(const int *d_in, int *d_out, int n, long long *total_host)
+int exclusive_scan_i32_device(const int *d_in, int *d_out, int n, void *d_tmp)
+{
+    if (n <= 0) return fail(MGGX_EINVAL, "exclusive_scan: empty input");
+    return scan_launch(ScanArray{d_in}, d_out, n, d_tmp, nullptr);
+}
+
+// The scan with its total on the host (synchronises).
+template <typename F>
+static int scan_total(const F &in, int *d_out, int n, long long *total_host)
 {
     State &s = state();
     if (n <= 0) {
@@ -539,22 +591,22 @@ int exclusive_scan_i32(const int *d_in, int *d_out, int n, long long *total_host
         if (total_host) *total_host = 0;
         return MGGX_OK;
     }
-    const int tiles = (n + SCAN_TILE - 1) / SCAN_TILE;
-    long long *d_tile = nullptr;
-    MGGX_HIP(hipMalloc((void **)&d_tile, sizeof(long long) * ((size_t)tiles + 1)));
-    k_scan_tile_sums<<<tiles, SCAN_THREADS, 0, s.stream>>>(d_in, n, d_tile);
-    k_scan_tile_offsets<<<1, SCAN_THREADS, 0, s.stream>>>(d_tile, tiles);
-    k_scan_apply<<<tiles, SCAN_THREADS, 0, s.stream>>>(d_in, d_out, n, d_tile);
-    hipError_t e = hipGetLastError();
-    long long total = 0;
-    if (e == hipSuccess) e = hipMemcpyAsync(&total, d_tile + tiles, sizeof(long long), hipMemcpyDeviceToHost, s.stream);
-    if (e == hipSuccess) e = hipStreamSynchronize(s.stream);
-    (void)hipFree(d_tile);
+    void *tmp = nullptr;
+    long long *w = nullptr;
+    int rc = host_words(&w);
+    if (!rc) rc = dev_alloc(&tmp, scan_tmp_bytes(n));
+    if (rc) return rc;
+    rc = scan_launch(in, d_out, n, tmp, w);
+    const hipError_t e = hipStreamSynchronize(s.stream);
+    dev_free(tmp);
+    if (rc) return rc;
     if (e != hipSuccess) return fail(MGGX_EHIP, "exclusive_scan: %s", hipGetErrorString(e));
-    if (total > 0x7fffffffLL) return fail(MGGX_ELIMIT, "exclusive_scan: total %lld exceeds int32", total);
-    if (total_host) *total_host = total;
+    if (w[0] > 0x7fffffffLL) return fail(MGGX_ELIMIT, "exclusive_scan: total %lld exceeds int32", w[0]);
+    if (total_host) *total_host = w[0];
     return MGGX_OK;
 }
+
+int exclusive_scan_i32(const int *d_in, int *d_out, int n, long long *total_host) { return scan_total(ScanArray{d_in}, d_out, n, total_host); }
 
 // A plan that was used inside a stream capture leaves the cache like any other, but a captured graph still holds the
 // addresses of its device arrays: those are retired (freed by mggx_release_cached), not freed.
@@ -566,29 +618,35 @@ void plan_free(Plan *p)
         retire_block(p->d_off, sizeof(int) * ((size_t)p->rows + 1));
         retire_block(p->d_empty_rows, sizeof(int) * (size_t)std::max(p->rows, 1));
     } else {
-        if (p->d_desc) (void)hipFree(p->d_desc);
-        if (p->d_off) (void)hipFree(p->d_off);
-        if (p->d_empty_rows) (void)hipFree(p->d_empty_rows);
+        dev_free(p->d_desc);
+        dev_free(p->d_off);
+        dev_free(p->d_empty_rows);
     }
     guard_free(p->guard, p->pinned);
     delete p;
 }
 
-static int plan_finish(Plan *p)
+// Rows without partitions, and what the host needs to know of a plan, in one wait: words[0] = number of those rows,
+// words[1] = *d_a, words[2] = *d_b (NULL: 0).
+static int plan_finish(Plan *p, const int *d_a, const int *d_b, long long **words)
 {
     State &s = state();
-    // rows without partitions
     int *d_counter = nullptr;
-    MGGX_HIP(hipMalloc((void **)&d_counter, sizeof(int)));
-    MGGX_HIP(hipMemsetAsync(d_counter, 0, sizeof(int), s.stream));
-    MGGX_HIP(hipMalloc((void **)&p->d_empty_rows, sizeof(int) * (size_t)std::max(p->rows, 1)));
-    if (p->rows > 0) {
-        k_collect_empty<<<(p->rows + 255) / 256, 256, 0, s.stream>>>(p->d_off, p->rows, p->d_empty_rows, d_counter);
-        MGGX_LAUNCH_CHECK("k_collect_empty");
+    int rc = host_words(words);
+    if (!rc) rc = dev_array(&d_counter, 1);
+    if (!rc) rc = dev_array(&p->d_empty_rows, (size_t)p->rows);
+    if (rc) {
+        dev_free(d_counter);
+        return rc;
     }
-    MGGX_HIP(hipMemcpyAsync(&p->num_empty, d_counter, sizeof(int), hipMemcpyDeviceToHost, s.stream));
-    MGGX_HIP(hipStreamSynchronize(s.stream));
-    MGGX_HIP(hipFree(d_counter));
+    long long *const w = *words + 1;  // word 0 holds the total of a scan in flight
+    k_zero_words<<<1, 64, 0, s.stream>>>(d_counter, 1);
+    if (p->rows > 0) k_collect_empty<<<(p->rows + 255) / 256, 256, 0, s.stream>>>(p->d_off, p->rows, p->d_empty_rows, d_counter);
+    k_publish<<<1, 1, 0, s.stream>>>(d_counter, d_a, d_b, w);
+    const hipError_t el = hipGetLastError(), e = hipStreamSynchronize(s.stream);
+    dev_free(d_counter);
+    if (el != hipSuccess || e != hipSuccess) return fail(MGGX_EHIP, "plan: %s", hipGetErrorString(el != hipSuccess ? el : e));
+    p->num_empty = (int)w[0];
     return MGGX_OK;
 }
 
@@ -689,66 +747,56 @@ int plan_get(const int *d_ptr_l, const int *d_ptr_r, const int *d_col_r, int row
     p->unit = unit_of(ps);
     const int unit = p->unit;  // neighbors per descriptor: whole partitions of one row and side, at most 16 neighbors (ps < 16)
     int rc = MGGX_OK;
-    int *d_cnt = nullptr;
+    int *d_max = nullptr;
+    void *scan_tmp = nullptr;
     do {
-        if (hipMalloc((void **)&d_cnt, sizeof(int) * (size_t)std::max(rows, 1)) != hipSuccess ||
-            hipMalloc((void **)&p->d_off, sizeof(int) * ((size_t)rows + 1)) != hipSuccess) {
-            rc = fail(MGGX_ENOMEM, "plan: row arrays for %d rows", rows);
-            break;
-        }
-        if (rows > 0)
-            k_count_parts<<<(rows + 255) / 256, 256, 0, s.stream>>>(d_ptr_l, d_ptr_l + 1, d_ptr_r, d_ptr_r ? d_ptr_r + 1 : nullptr, rows, unit,
-                                                                    d_cnt);
-        long long total = 0;
-        rc = exclusive_scan_i32(d_cnt, p->d_off, rows, &total);
-        if (rc) break;
-        p->num_parts = (int)total;
-        int ends[2] = {0, 0};
+        // One wait for everything the host needs: the number of descriptors, the edge counts, the largest remote id, the
+        // number of rows without neighbors.
+        if ((rc = dev_array(&p->d_off, (size_t)rows + 1))) break;
+        const bool remote = d_ptr_r && rows > 0;
         if (rows > 0) {
-            if (hipMemcpy(&ends[0], d_ptr_l + rows, sizeof(int), hipMemcpyDeviceToHost) != hipSuccess ||
-                (d_ptr_r && hipMemcpy(&ends[1], d_ptr_r + rows, sizeof(int), hipMemcpyDeviceToHost) != hipSuccess)) {
-                rc = fail(MGGX_EHIP, "plan: reading edge counts");
-                break;
-            }
-        }
-        p->nnz_l = ends[0];
-        p->nnz_r = ends[1];
-        if (p->nnz_r > 0) {
-            if (!d_col_r) {
-                rc = fail(MGGX_EINVAL, "plan: remote edges but no remote column array");
-                break;
-            }
-            int *d_max = nullptr;
-            if (hipMalloc((void **)&d_max, sizeof(int)) != hipSuccess) {
-                rc = fail(MGGX_ENOMEM, "plan: scratch");
-                break;
-            }
-            (void)hipMemsetAsync(d_max, 0, sizeof(int), s.stream);
-            k_max_i32<<<256, 256, 0, s.stream>>>(d_col_r, p->nnz_r, d_max);
-            hipError_t e = hipMemcpyAsync(&p->max_col_r, d_max, sizeof(int), hipMemcpyDeviceToHost, s.stream);
-            if (e == hipSuccess) e = hipStreamSynchronize(s.stream);
-            (void)hipFree(d_max);
-            if (e != hipSuccess) {
-                rc = fail(MGGX_EHIP, "plan: remote id scan: %s", hipGetErrorString(e));
-                break;
-            }
-        }
-        if (hipMalloc((void **)&p->d_desc, sizeof(int4) * (size_t)std::max(p->num_parts, 1)) != hipSuccess) {
-            rc = fail(MGGX_ENOMEM, "plan: %d descriptors", p->num_parts);
+            if ((rc = dev_alloc(&scan_tmp, scan_tmp_bytes(rows))) || (rc = dev_array(&d_max, 1))) break;
+            long long *w = nullptr;
+            if ((rc = host_words(&w))) break;
+            rc = scan_launch(ScanParts{d_ptr_l, d_ptr_l + 1, d_ptr_r, d_ptr_r ? d_ptr_r + 1 : nullptr, unit}, p->d_off, rows, scan_tmp, w);
+            if (rc) break;
+            k_zero_words<<<1, 64, 0, s.stream>>>(d_max, 1);
+            if (remote && d_col_r) k_max_i32<<<1024, 256, 0, s.stream>>>(d_col_r, d_ptr_r + rows, d_max);
+            k_publish<<<1, 1, 0, s.stream>>>(d_max, d_ptr_r ? d_ptr_r + rows : nullptr, nullptr, w + 8);
+        } else if (hipMemsetAsync(p->d_off, 0, sizeof(int), s.stream) != hipSuccess) {
+            rc = fail(MGGX_EHIP, "plan: row offsets");
             break;
         }
+        long long *w = nullptr;
+        if ((rc = plan_finish(p, rows > 0 ? d_ptr_l + rows : nullptr, nullptr, &w))) break;
+        if (rows > 0) {
+            if (w[0] > 0x7fffffffLL) {
+                rc = fail(MGGX_ELIMIT, "exclusive_scan: total %lld exceeds int32", w[0]);
+                break;
+            }
+            p->num_parts = (int)w[0];
+            p->nnz_l = w[2];
+            p->nnz_r = w[9];
+            if (p->nnz_r > 0) {
+                if (!d_col_r) {
+                    rc = fail(MGGX_EINVAL, "plan: remote edges but no remote column array");
+                    break;
+                }
+                p->max_col_r = (int)w[8];
+            }
+        }
+        if ((rc = dev_array(&p->d_desc, (size_t)p->num_parts))) break;
         if (p->num_parts > 0) {
             k_fill_desc<<<(p->num_parts + 255) / 256, 256, 0, s.stream>>>(p->d_off, d_ptr_l, d_ptr_l + 1, d_ptr_r,
                                                                           d_ptr_r ? d_ptr_r + 1 : nullptr, rows, unit, p->num_parts,
                                                                           p->d_desc);
-            if (hipGetLastError() != hipSuccess) {
-                rc = fail(MGGX_EHIP, "plan: descriptor kernel launch failed");
-                break;
-            }
+            if (hipGetLastError() != hipSuccess) rc = fail(MGGX_EHIP, "plan: descriptor kernel launch failed");
+            // a cached plan may be used on another stream next: it is complete when the call that builds it goes on
+            else if (hipStreamSynchronize(s.stream) != hipSuccess) rc = fail(MGGX_EHIP, "plan: descriptors");
         }
-        rc = plan_finish(p);
     } while (0);
-    if (d_cnt) (void)hipFree(d_cnt);
+    dev_free(scan_tmp);
+    dev_free(d_max);
     if (rc) {
         plan_free(p);
         return rc;
@@ -821,25 +869,17 @@ int plan_get_explicit(const int *d_row_ptr, const int *d_part_ptr, const int *d_
     int *d_tmp = nullptr;
     do {
         long long bound = num_parts;
-        if (hipMalloc((void **)&p->d_off, sizeof(int) * ((size_t)rows + 1)) != hipSuccess ||
-            hipMalloc((void **)&p->d_desc, sizeof(int4) * (size_t)std::max(num_parts, 1)) != hipSuccess ||
-            (p->unit != ps && hipMalloc((void **)&d_tmp, sizeof(int) * explicit_tmp_ints(rows)) != hipSuccess)) {
-            rc = fail(MGGX_ENOMEM, "plan: explicit arrays");
+        if ((rc = dev_array(&p->d_off, (size_t)rows + 1)) || (rc = dev_array(&p->d_desc, (size_t)num_parts)) ||
+            (p->unit != ps && (rc = dev_array(&d_tmp, explicit_tmp_ints(rows)))))
             break;
-        }
         rc = explicit_desc_fill(d_row_ptr, d_part_ptr, d_part2node, rows, num_parts, ps, p->d_desc, p->d_off, d_tmp, &bound);
         if (rc) break;
-        int end = 0, units = num_parts;
-        if (rows > 0 && (hipStreamSynchronize(s.stream) != hipSuccess ||
-                         hipMemcpy(&end, d_row_ptr + rows, sizeof(int), hipMemcpyDeviceToHost) != hipSuccess ||
-                         hipMemcpy(&units, p->d_off + rows, sizeof(int), hipMemcpyDeviceToHost) != hipSuccess)) {
-            rc = fail(MGGX_EHIP, "plan: reading edge count");
-            break;
-        }
-        p->num_parts = rows > 0 ? units : 0;  // several partitions of a row per descriptor when ps < 16 (Plan::unit)
-        p->nnz_l = end;
-        rc = plan_finish(p);
+        long long *w = nullptr;
+        rc = plan_finish(p, rows > 0 ? d_row_ptr + rows : nullptr, rows > 0 ? p->d_off + rows : nullptr, &w);
         if (rc) break;
+        const int end = (int)w[2];
+        p->num_parts = rows > 0 ? (int)w[3] : 0;  // several partitions of a row per descriptor when ps < 16 (Plan::unit)
+        p->nnz_l = end;
         // the descriptors depend on these three arrays (the column array is only read while aggregating)
         p->guard.arr[0] = d_row_ptr;
         p->guard.len[0] = (long long)rows + 1;
@@ -851,7 +891,7 @@ int plan_get_explicit(const int *d_row_ptr, const int *d_part_ptr, const int *d_
         p->guard.want_l = end;
         rc = guard_arm(p->guard);
     } while (0);
-    if (d_tmp) (void)hipFree(d_tmp);
+    dev_free(d_tmp);
     if (rc) {
         plan_free(p);
         return rc;
@@ -889,64 +929,52 @@ int plan_get_blocked(const int *d_ptr_l, const int *d_col_l, int rows, int lb, i
     p->block_rows = block_rows;
     p->block_lb = lb;
     int rc = MGGX_OK;
-    int *d_cnt = nullptr, *d_vbeg = nullptr, *d_flag = nullptr;
+    int *d_vbeg = nullptr, *d_flag = nullptr;
+    void *scan_tmp = nullptr;
+    long long *w = nullptr;
     do {
-        int flag = 0;
-        if (hipMalloc((void **)&d_flag, sizeof(int)) != hipSuccess) {
-            rc = fail(MGGX_ENOMEM, "plan: scratch");
-            break;
-        }
-        (void)hipMemsetAsync(d_flag, 0, sizeof(int), s.stream);
+        if ((rc = host_words(&w)) || (rc = dev_array(&d_flag, 1))) break;
+        k_zero_words<<<1, 64, 0, s.stream>>>(d_flag, 1);
         k_check_sorted<<<(rows + 3) / 4, 256, 0, s.stream>>>(d_ptr_l, d_col_l, rows, d_flag);
-        hipError_t e = hipMemcpyAsync(&flag, d_flag, sizeof(int), hipMemcpyDeviceToHost, s.stream);
-        if (e == hipSuccess) e = hipStreamSynchronize(s.stream);
+        k_publish<<<1, 1, 0, s.stream>>>(d_flag, nullptr, nullptr, w);
+        const hipError_t e = hipStreamSynchronize(s.stream);
         if (e != hipSuccess) {
             rc = fail(MGGX_EHIP, "plan: sortedness check: %s", hipGetErrorString(e));
             break;
         }
-        if (flag) {  // remember the answer; the caller falls back to the plain plan
+        if (w[0]) {  // remember the answer; the caller falls back to the plain plan
             p->unsuitable = true;
             p->rows = rows;
             break;
         }
         p->rows = (int)vrows;
         p->blocks = (int)blocks;
-        if (hipMalloc((void **)&d_vbeg, sizeof(int) * (size_t)(vrows + rows)) != hipSuccess ||
-            hipMalloc((void **)&d_cnt, sizeof(int) * (size_t)vrows) != hipSuccess ||
-            hipMalloc((void **)&p->d_off, sizeof(int) * ((size_t)vrows + 1)) != hipSuccess) {
-            rc = fail(MGGX_ENOMEM, "plan: arrays for %lld virtual rows", vrows);
+        if ((rc = dev_array(&d_vbeg, (size_t)(vrows + rows))) || (rc = dev_array(&p->d_off, (size_t)vrows + 1)) ||
+            (rc = dev_alloc(&scan_tmp, scan_tmp_bytes((int)vrows))))
             break;
-        }
         k_block_bounds<<<(unsigned)((vrows + rows + 255) / 256), 256, 0, s.stream>>>(d_ptr_l, d_col_l, rows, lb, block_rows, (int)blocks,
                                                                                    d_vbeg);
-        k_count_parts<<<(unsigned)((vrows + 255) / 256), 256, 0, s.stream>>>(d_vbeg, d_vbeg + rows, nullptr, nullptr, (int)vrows, unit, d_cnt);
-        long long total = 0;
-        rc = exclusive_scan_i32(d_cnt, p->d_off, (int)vrows, &total);
+        rc = scan_launch(ScanParts{d_vbeg, d_vbeg + rows, nullptr, nullptr, unit}, p->d_off, (int)vrows, scan_tmp, w);
         if (rc) break;
-        p->num_parts = (int)total;
-        int end = 0;
-        if (hipMemcpy(&end, d_ptr_l + rows, sizeof(int), hipMemcpyDeviceToHost) != hipSuccess) {
-            rc = fail(MGGX_EHIP, "plan: reading edge count");
+        if ((rc = plan_finish(p, d_ptr_l + rows, nullptr, &w))) break;
+        if (w[0] > 0x7fffffffLL) {
+            rc = fail(MGGX_ELIMIT, "exclusive_scan: total %lld exceeds int32", w[0]);
             break;
         }
-        p->nnz_l = end;
-        if (hipMalloc((void **)&p->d_desc, sizeof(int4) * (size_t)std::max(p->num_parts, 1)) != hipSuccess) {
-            rc = fail(MGGX_ENOMEM, "plan: %d descriptors", p->num_parts);
-            break;
-        }
+        p->num_parts = (int)w[0];
+        p->nnz_l = w[2];
+        if ((rc = dev_array(&p->d_desc, (size_t)p->num_parts))) break;
         if (p->num_parts > 0) {
             k_fill_desc<<<(p->num_parts + 255) / 256, 256, 0, s.stream>>>(p->d_off, d_vbeg, d_vbeg + rows, nullptr, nullptr, (int)vrows, unit,
                                                                           p->num_parts, p->d_desc);
-            if (hipGetLastError() != hipSuccess) {
-                rc = fail(MGGX_EHIP, "plan: descriptor kernel launch failed");
-                break;
-            }
+            if (hipGetLastError() != hipSuccess) rc = fail(MGGX_EHIP, "plan: descriptor kernel launch failed");
+            // a cached plan may be used on another stream next: it is complete when the call that builds it goes on
+            else if (hipStreamSynchronize(s.stream) != hipSuccess) rc = fail(MGGX_EHIP, "plan: descriptors");
         }
-        rc = plan_finish(p);  // synchronises: d_vbeg is no longer in use afterwards
     } while (0);
-    if (d_cnt) (void)hipFree(d_cnt);
-    if (d_vbeg) (void)hipFree(d_vbeg);
-    if (d_flag) (void)hipFree(d_flag);
+    dev_free(scan_tmp);
+    dev_free(d_vbeg);
+    dev_free(d_flag);
     if (rc) {
         plan_free(p);
         return rc;
@@ -1090,22 +1118,16 @@ MGGX_EXPORT int mggx_build_part_device(const int *d_indptr, int num_nodes, int p
     int rc = mggx::ensure_init();
     if (rc) return rc;
     mggx::State &s = mggx::state();
-    int *d_cnt = nullptr, *d_n2p = d_node2part;
+    int *d_n2p = d_node2part;
     bool own_n2p = false;
-    MGGX_HIP(hipMalloc((void **)&d_cnt, sizeof(int) * (size_t)std::max(num_nodes, 1)));
     if (!d_n2p) {
-        if (hipMalloc((void **)&d_n2p, sizeof(int) * ((size_t)num_nodes + 2)) != hipSuccess) {
-            (void)hipFree(d_cnt);
-            return fail(MGGX_ENOMEM, "build_part_device: node2part");
-        }
+        rc = mggx::dev_array(&d_n2p, (size_t)num_nodes + 2);
+        if (rc) return rc;
         own_n2p = true;
     }
     long long total = 0;
     do {
-        if (num_nodes > 0)
-            mggx::k_count_parts<<<(num_nodes + 255) / 256, 256, 0, s.stream>>>(d_indptr, d_indptr + 1, nullptr, nullptr, num_nodes, part_size,
-                                                                               d_cnt);
-        rc = mggx::exclusive_scan_i32(d_cnt, d_n2p, num_nodes, &total);
+        rc = mggx::scan_total(mggx::ScanParts{d_indptr, d_indptr + 1, nullptr, nullptr, part_size}, d_n2p, num_nodes, &total);
         if (rc) break;
         mggx::k_set_tail<<<1, 1, 0, s.stream>>>(d_n2p, num_nodes);
         *num_parts = (int)total;
@@ -1117,8 +1139,7 @@ MGGX_EXPORT int mggx_build_part_device(const int *d_indptr, int num_nodes, int p
         if (hipGetLastError() != hipSuccess || hipStreamSynchronize(s.stream) != hipSuccess)
             rc = fail(MGGX_EHIP, "build_part_device: kernel failed");
     } while (0);
-    (void)hipFree(d_cnt);
-    if (own_n2p) (void)hipFree(d_n2p);
+    if (own_n2p) mggx::dev_free(d_n2p);
     return rc;
 }
 
@@ -1136,7 +1157,8 @@ MGGX_EXPORT int mggx_split_csr_device(const int *d_ptr, const int *d_col, int lb
     if (!d_local_col || !d_remote_col) {
         // pass 1: per-row counts -> the two pointer arrays and the totals
         int *d_cnt = nullptr;
-        MGGX_HIP(hipMalloc((void **)&d_cnt, sizeof(int) * 2 * (size_t)std::max(rows, 1)));
+        rc = mggx::dev_array(&d_cnt, 2 * (size_t)rows);
+        if (rc) return rc;
         long long tl = 0, tr = 0;
         do {
             if (rows > 0) {
@@ -1147,7 +1169,7 @@ MGGX_EXPORT int mggx_split_csr_device(const int *d_ptr, const int *d_col, int lb
             if (rc) break;
             rc = mggx::exclusive_scan_i32(d_cnt + rows, d_remote_ptr, rows, &tr);
         } while (0);
-        (void)hipFree(d_cnt);
+        mggx::dev_free(d_cnt);
         if (rc) return rc;
         if (n_local) *n_local = tl;
         if (n_remote) *n_remote = tr;

@@ -48,14 +48,14 @@ struct DeviceBuffers {
     std::vector<void *> ptrs;
     ~DeviceBuffers()
     {
-        for (void *p : ptrs) (void)hipFree(p);
+        for (void *p : ptrs) dev_free(p);
     }
     template <typename T>
     int get(T **p, size_t count)
     {
         void *q = nullptr;
-        if (hipMalloc(&q, std::max<size_t>(count, 1) * sizeof(T)) != hipSuccess)
-            return fail(MGGX_ENOMEM, "compact_remote_device: %zu bytes of scratch", count * sizeof(T));
+        const int rc = dev_alloc(&q, std::max<size_t>(count, 1) * sizeof(T));
+        if (rc) return rc;
         ptrs.push_back(q);
         *p = static_cast<T *>(q);
         return MGGX_OK;

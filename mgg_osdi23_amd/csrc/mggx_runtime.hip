@@ -58,6 +58,110 @@ int workspace(size_t bytes, void **p)
     return MGGX_OK;
 }
 
+// ---- device blocks for plans and for the scratch of set-up calls, kept between calls
+//
+// What bounded a set-up on a small graph was hipMalloc and hipFree: 20 to 100 us each, hipFree with a wait for the whole device, a
+// dozen of them per plan (100 K nodes, 2 M neighbors, plan built at every call: 288 -> 167 us; splitting and compacting an
+// eighth of 1 M nodes: 1,830 -> 1,323 us).  A block goes back to this list instead and serves the next request it fits
+// (at most twice the size asked for).  Bounds: blocks beyond POOL_MAX_BLOCK are not kept, at most POOL_MAX_BYTES are, the oldest
+// go first; mggx_release_cached hands all of them back, and so does an allocation that finds no memory.
+// Order: everything the library does with such a block it does on its stream, so the next user on that stream comes after the
+// last one.  Where the stream (or the device) was changed in between, work on the old one may still be in flight: the first
+// request or return after the change waits for the device, as hipFree did every time.
+constexpr size_t POOL_MAX_BLOCK = 64ull << 20, POOL_MAX_BYTES = 256ull << 20;
+
+static void pool_settle()
+{
+    State &s = state();
+    if (!s.pool_unordered) return;
+    (void)hipDeviceSynchronize();
+    s.pool_unordered = false;
+}
+
+static void pool_trim(size_t keep)
+{
+    State &s = state();
+    while (!s.pool.empty() && s.pool_bytes > keep) {
+        (void)hipFree(s.pool.front().p);
+        s.pool_bytes -= s.pool.front().bytes;
+        s.pool.erase(s.pool.begin());
+    }
+}
+
+// sizes in eighths of a power of two, so that a graph that changed a little finds the block of the last one
+static size_t pool_size(size_t bytes)
+{
+    size_t step = 256;
+    while (step * 16 <= bytes) step *= 2;
+    return std::max<size_t>((bytes + step - 1) / step * step, 256);
+}
+
+int dev_alloc(void **p, size_t bytes)
+{
+    State &s = state();
+    *p = nullptr;
+    const size_t want = pool_size(bytes);
+    int dev = -1;
+    if (hipGetDevice(&dev) != hipSuccess) return fail(MGGX_EHIP, "device memory: no current device");
+    size_t best = s.pool.size();
+    for (size_t i = 0; i < s.pool.size(); ++i)
+        if (s.pool[i].device == dev && s.pool[i].bytes >= want && s.pool[i].bytes <= 2 * want && (best == s.pool.size() || s.pool[i].bytes < s.pool[best].bytes)) best = i;
+    if (best < s.pool.size()) {
+        pool_settle();
+        const State::Block b = s.pool[best];
+        s.pool.erase(s.pool.begin() + (long)best);
+        s.pool_bytes -= b.bytes;
+        s.pool_out[b.p] = b;
+        *p = b.p;
+        return MGGX_OK;
+    }
+    void *q = nullptr;
+    hipError_t e = hipMalloc(&q, want);
+    if (e == hipErrorOutOfMemory && !s.pool.empty()) {
+        (void)hipGetLastError();
+        pool_trim(0);
+        e = hipMalloc(&q, want);
+    }
+    if (e != hipSuccess) {
+        (void)hipGetLastError();
+        return fail(MGGX_ENOMEM, "%zu bytes of device memory: %s", want, hipGetErrorString(e));
+    }
+    s.pool_out[q] = State::Block{q, want, dev};
+    *p = q;
+    return MGGX_OK;
+}
+
+void dev_free(void *p)
+{
+    if (!p) return;
+    State &s = state();
+    const auto it = s.pool_out.find(p);
+    const State::Block b = it == s.pool_out.end() ? State::Block{p, 0, -1} : it->second;
+    if (it != s.pool_out.end()) s.pool_out.erase(it);
+    int dev = -1;
+    if (b.bytes == 0 || b.bytes > POOL_MAX_BLOCK || hipGetDevice(&dev) != hipSuccess || dev != b.device) {
+        (void)hipFree(p);
+        return;
+    }
+    pool_settle();
+    pool_trim(POOL_MAX_BYTES - b.bytes);
+    s.pool.push_back(b);
+    s.pool_bytes += b.bytes;
+}
+
+// A few words of pinned host memory that kernels of set-up calls write results to (read after the stream is waited for).
+int host_words(long long **w)
+{
+    State &s = state();
+    if (!s.h_words) {
+        void *q = nullptr;
+        if (hipHostMalloc(&q, HOST_WORDS * sizeof(long long), hipHostMallocMapped) != hipSuccess) return fail(MGGX_ENOMEM, "pinned result words");
+        s.h_words = static_cast<long long *>(q);
+    }
+    *w = s.h_words;
+    return MGGX_OK;
+}
+
 }  // namespace mggx
 
 using mggx::fail;
@@ -75,6 +179,7 @@ MGGX_EXPORT int mggx_init(int device)
     MGGX_HIP(hipGetDeviceProperties(&prop, device));
     if (strncmp(prop.gcnArchName, "gfx950", 6) != 0)
         return fail(MGGX_EHIP, "init: device %d is %s; this library carries gfx950 code only", device, prop.gcnArchName);
+    if (state().device != device) state().pool_unordered = true;
     state().device = device;
     // Set-up of the allocation-free entry point: its array's address on this device is looked up now.  Should the lookup
     // fail, only that entry point is unavailable (mggx_sag_parts_static asks again and reports the error itself).
@@ -96,6 +201,7 @@ MGGX_EXPORT int mggx_device_name(char *buf, size_t len)
 
 MGGX_EXPORT int mggx_set_stream(void *hip_stream)
 {
+    if (state().stream != static_cast<hipStream_t>(hip_stream)) state().pool_unordered = true;
     state().stream = static_cast<hipStream_t>(hip_stream);
     return MGGX_OK;
 }
@@ -251,8 +357,9 @@ MGGX_EXPORT int mggx_release_cached(void)
         s.ws = nullptr;
         s.ws_bytes = 0;
     }
-    for (void *p : s.retired) (void)hipFree(p);
+    for (void *p : s.retired) mggx::dev_free(p);
     s.retired.clear();
+    mggx::pool_trim(0);
     s.retired_bytes = 0;
     s.ws_captured = s.core_ws_captured = false;
     if (s.h_stale) *s.h_stale = 0;

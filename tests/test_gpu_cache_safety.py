@@ -246,6 +246,40 @@ def test_captured_graph_survives_forget(gpu, core_rows):
     assert gpu.cache_stats()["retired_bytes"] == 0
 
 
+@pytest.mark.parametrize("V,dim", [(900, 16), (6000, 41), (70_000, 8)])  # plans of a few hundred bytes, of odd sizes, of several scan tiles
+def test_device_blocks_move_from_plan_to_plan_across_streams(gpu, V, dim):
+    """A plan dropped with mggx_forget leaves its device blocks to the next plan.  Graphs of changing size in one pair of
+    arrays, a new plan each time, every other time on another stream than the last (nothing waited for on the host but what
+    the calls wait for themselves): every sum is the oracle's, and mggx_release_cached lets go of everything."""
+    import torch
+    x = gpu.fill_normal((V, dim), seed=71)
+    d_x = to_dev(x)
+    graphs = [gpu.gen_rmat(17, V, V * d, seed=72 + d) for d in (4, 9, 3, 9, 6, 1)]
+    room = max(len(c) for _, c in graphs)
+    d_ptr, d_col = torch.zeros(V + 1, dtype=torch.int32, device="cuda"), torch.zeros(room, dtype=torch.int32, device="cuda")
+    dev = [(to_dev(p), to_dev(c)) for p, c in graphs]
+    outs = []
+    streams = [torch.cuda.current_stream(), torch.cuda.Stream()]
+    for i, (p, c) in enumerate(dev):
+        st = streams[i % 2]
+        st.wait_stream(streams[(i + 1) % 2])
+        with torch.cuda.stream(st):
+            gpu.use_torch_stream()
+            gpu.forget(d_ptr)
+            d_ptr.copy_(p)
+            d_col[: c.numel()].copy_(c)
+            out = torch.full((V, dim), 7.5, device="cuda")
+            _agg(gpu, out, d_x, d_ptr, d_col, V, dim, ps=(16, 4)[i % 2], wpb=0, dist=0)
+            outs.append(out)
+    torch.cuda.synchronize()
+    gpu.use_torch_stream()
+    for out, (ptr, col) in zip(outs, graphs):
+        want, mag = _want(x, ptr, col, V, dim)
+        assert_close_to_oracle(out.cpu().numpy(), want, mag, FP32_TOL, "graph of %d neighbors" % len(col))
+    gpu.release_cached()
+    assert gpu.cache_stats()["plans"] == 0
+
+
 def test_plans_go_with_their_graph_record(gpu):
     """The content check lives with the graph record (32 cached).  A dense-core plan must not outlive the record it was
     built under: after 33 other CSR sets have passed through, the first set's arrays are rewritten in place with another
