@@ -137,8 +137,8 @@ def compact_remote_device(d_remote_col, n_remote: int):
     import torch
     nu = C.c_int64()
     _check(lib().mggx_compact_remote_device(_dptr(d_remote_col), C.c_int64(n_remote), None, None, C.byref(nu)))
-    out = torch.zeros(max(n_remote, 1), dtype=torch.int32, device=d_remote_col.device)
-    ids = torch.zeros(max(nu.value, 1), dtype=torch.int32, device=d_remote_col.device)
+    out = torch.empty(max(n_remote, 1), dtype=torch.int32, device=d_remote_col.device)
+    ids = torch.empty(max(nu.value, 1), dtype=torch.int32, device=d_remote_col.device)
     _check(lib().mggx_compact_remote_device(_dptr(d_remote_col), C.c_int64(n_remote), _dptr(out), _dptr(ids), C.byref(nu)))
     return out[:n_remote], ids[: nu.value]
 
@@ -203,13 +203,13 @@ def split_CSR_device(d_ptr, d_col, lb: int, ub: int):
     """split_CSR on the GPU -> (local_ptr, remote_ptr, local_col_idx, remote_col_idx) as device tensors."""
     import torch
     rows = ub - lb
-    lp = torch.zeros(rows + 1, dtype=torch.int32, device=d_ptr.device)
-    rp = torch.zeros(rows + 1, dtype=torch.int32, device=d_ptr.device)
+    lp = torch.empty(rows + 1, dtype=torch.int32, device=d_ptr.device)
+    rp = torch.empty(rows + 1, dtype=torch.int32, device=d_ptr.device)
     nl, nr = C.c_int64(), C.c_int64()
     _check(lib().mggx_split_csr_device(_dptr(d_ptr), _dptr(d_col), lb, ub, _dptr(lp), _dptr(rp), None, None,
                                        C.byref(nl), C.byref(nr)))
-    lc = torch.zeros(max(nl.value, 1), dtype=torch.int32, device=d_ptr.device)
-    rc = torch.zeros(max(nr.value, 1), dtype=torch.int32, device=d_ptr.device)
+    lc = torch.empty(max(nl.value, 1), dtype=torch.int32, device=d_ptr.device)
+    rc = torch.empty(max(nr.value, 1), dtype=torch.int32, device=d_ptr.device)
     _check(lib().mggx_split_csr_device(_dptr(d_ptr), _dptr(d_col), lb, ub, _dptr(lp), _dptr(rp), _dptr(lc), _dptr(rc),
                                        C.byref(nl), C.byref(nr)))
     sync()
@@ -347,9 +347,9 @@ def build_part_device(d_indptr, num_nodes: int, part_size: int, compat: bool = T
     import torch
     n = C.c_int()
     _check(lib().mggx_build_part_device(_dptr(d_indptr), num_nodes, part_size, int(compat), None, None, None, C.byref(n)))
-    pp = torch.zeros(n.value + 1, dtype=torch.int32, device=d_indptr.device)
-    p2n = torch.zeros(max(n.value, 1), dtype=torch.int32, device=d_indptr.device)[: n.value]
-    n2p = torch.zeros(num_nodes + 2, dtype=torch.int32, device=d_indptr.device)
+    pp = torch.empty(n.value + 1, dtype=torch.int32, device=d_indptr.device)
+    p2n = torch.empty(max(n.value, 1), dtype=torch.int32, device=d_indptr.device)[: n.value]
+    n2p = torch.empty(num_nodes + 2, dtype=torch.int32, device=d_indptr.device)
     _check(lib().mggx_build_part_device(_dptr(d_indptr), num_nodes, part_size, int(compat), _dptr(pp),
                                         C.c_void_p(p2n.data_ptr()) if n.value else C.c_void_p(pp.data_ptr()),
                                         _dptr(n2p), C.byref(n)))

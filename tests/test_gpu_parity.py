@@ -1101,3 +1101,40 @@ def test_softmax_epilogue_on_every_path(gpu, rmat_graph, dim, ld, path):
             assert np.all(got[:, dim:] == 7.5)  # padding columns are not touched
         assert np.allclose(got[5, :dim], 1.0 / dim, atol=1e-7)  # a row without neighbors: uniform
     gpu.forget(d_ptr)
+
+
+@pytest.mark.parametrize("n,largest", [(1, 0), (1, 2**20 - 1), (1, 2**20), (300, 2**20 - 1), (300, 2**20), (300, 2**31 - 2), (300, 2**31 - 1),
+                                       (70_001, 15), (70_001, 70_000), (400_000, 1_599_999), (400_000, 1_600_000)])
+def test_compact_remote_device_dense_and_sparse_ids(gpu, n, largest):
+    """Both ways the device makes the staging order -- a table with an entry per id, and sorting where ids are too sparse for
+    one -- against the host version, bit for bit, at the largest ids where one changes into the other (2^20, four per edge);
+    one id that most edges ask for, so counts of many digits and of one are among them."""
+    rng = np.random.default_rng(n + largest)
+    col = rng.integers(0, largest + 1, n).astype(np.int32)
+    col[rng.random(n) < 0.6] = largest // 3
+    col[n // 2] = largest
+    want, want_ids = gpu.compact_remote(col)
+    got, got_ids = gpu.compact_remote_device(to_dev(col), n)
+    assert np.array_equal(got.cpu().numpy(), want) and np.array_equal(got_ids.cpu().numpy(), want_ids)
+    col[0] = -2
+    with pytest.raises(Exception, match="negative neighbor id -2"):
+        gpu.compact_remote_device(to_dev(col), n)
+
+
+@pytest.mark.parametrize("lens", [[64, 65, 127, 128, 129, 0, 1], [511, 512, 513, 640, 641], [20_000, 3, 700, 0, 191]])
+def test_split_csr_device_rows_of_many_chunks(gpu, lens):
+    """Rows around the number of neighbors a wavefront takes at a time, and one of thousands: the device split is the host's."""
+    from mgg_osdi23_amd import host
+    rng = np.random.default_rng(sum(lens))
+    V, lb = 50_000, 100
+    ptr = np.zeros(V + 1, np.int32)
+    ptr[lb + 1: lb + 1 + len(lens)] = lens
+    ptr = np.cumsum(ptr).astype(np.int32)
+    ub = lb + len(lens)
+    col = rng.integers(0, V, ptr[-1]).astype(np.int32)
+    near = rng.random(len(col)) < 0.4
+    col[near] = rng.integers(lb, ub, int(near.sum()))
+    want = host.split_CSR(ptr, col, lb, ub)
+    got = gpu.split_CSR_device(to_dev(ptr), to_dev(col), lb, ub)
+    for g, w in zip(got, want):
+        assert np.array_equal(g.cpu().numpy(), w)
