@@ -658,6 +658,40 @@ __device__ __forceinline__ void split8(const float (&x)[8], v8bf &hi, v8bf &mid,
 // position in a staged row of Wb^T of the K index k (see above): step k / 32, lane group (k / 4) % 4, slot 4 ((k / 16) % 2) + k % 4
 __device__ __forceinline__ int split_k_slot(int k) { return 32 * (k >> 5) + 8 * ((k >> 2) & 3) + 4 * ((k >> 4) & 1) + (k & 3); }
 
+// 64 values of K of a weight matrix (NB * 16 columns) as three bf16 parts in LDS, [part][column][SPLIT_KP], by the 8 wavefronts of
+// a workgroup, in two steps so that the loads can fly meanwhile: thread -> column 16 (unit % NB) + i and K pair 4 (unit / NB) + kb
+// of the group, unit = 8 u + wavefront, so that a wavefront writes two K values of 16 columns x 4 pairs per instruction, 4 bytes
+// to each of the 64 banks.  k_of(r): K index of row r of the group, or -1 for a zero row; slot(kp): where in a staged column pair
+// kp goes.
+template <int NB, typename K>
+__device__ __forceinline__ void split_load_w(float (&v)[2 * NB], const float *w, int d2, int c0, int wave, int i, int kb, K k_of)
+{
+#pragma unroll
+    for (int u = 0; u < NB; ++u) {
+        const int unit = u * (RES_THREADS / 64) + wave, c = min(c0 + 16 * (unit % NB) + i, d2 - 1), r = 2 * (4 * (unit / NB) + kb);
+        v[2 * u] = w[(long long)max(k_of(r), 0) * d2 + c];
+        v[2 * u + 1] = w[(long long)max(k_of(r + 1), 0) * d2 + c];
+    }
+}
+template <int NB, typename K, typename SLOT, typename SEEN>
+__device__ __forceinline__ void split_put_w(unsigned short *dst, const float (&v)[2 * NB], int d2, int c0, int wave, int i, int kb, K k_of, SLOT slot, SEEN seen)
+{
+    constexpr int PART = NB * 16 * SPLIT_KP;
+#pragma unroll
+    for (int u = 0; u < NB; ++u) {
+        const int unit = u * (RES_THREADS / 64) + wave, c = 16 * (unit % NB) + i, kp = 4 * (unit / NB) + kb;
+        const bool on = c0 + c < d2;
+        const float v0 = on && k_of(2 * kp) >= 0 ? v[2 * u] : 0.f, v1 = on && k_of(2 * kp + 1) >= 0 ? v[2 * u + 1] : 0.f;
+        seen(v0, v1);
+        unsigned h, m, l;
+        split_pair(v0, v1, h, m, l);
+        unsigned *q = reinterpret_cast<unsigned *>(dst + c * SPLIT_KP + slot(kp));
+        q[0] = h;
+        q[PART / 2] = m;
+        q[PART] = l;
+    }
+}
+
 template <int NB2>
 __global__ void __launch_bounds__(RES_THREADS, 4) k_mlp2_split(const MlpArgs a)
 {
@@ -673,30 +707,9 @@ __global__ void __launch_bounds__(RES_THREADS, 4) k_mlp2_split(const MlpArgs a)
     // buys nothing.  Whole rows through LDS (16 wavefronts, one workgroup per CU) were measured as well: 0.304 against
     // 0.308 ms at 64 columns out, 0.394 against 0.374 at 47 -- memory is not what holds this kernel; per 16-row tile it
     // issues 96 matrix-core instructions, 48 16-byte LDS reads of weights and some 260 vector instructions of splitting.
-    for (int idx = (int)threadIdx.x; idx < 64 * 64; idx += RES_THREADS) {
-        const int k = idx >> 6, c = idx & 63;
-        unsigned h, m, l;
-        split_pair(a.wa[(long long)k * 64 + c], 0.f, h, m, l);
-        wa[c * KP + k] = (unsigned short)h;
-        wa[PART_A + c * KP + k] = (unsigned short)m;
-        wa[2 * PART_A + c * KP + k] = (unsigned short)l;
-    }
-    for (int idx = (int)threadIdx.x; idx < 64 * NB2 * 16; idx += RES_THREADS) {
-        const int k = idx / (NB2 * 16), c = idx % (NB2 * 16);
-        unsigned h, m, l;
-        split_pair(c < a.d3 ? a.wb[(long long)k * a.d3 + c] : 0.f, 0.f, h, m, l);
-        const int at = c * KP + split_k_slot(k);
-        wb[at] = (unsigned short)h;
-        wb[PART_B + at] = (unsigned short)m;
-        wb[2 * PART_B + at] = (unsigned short)l;
-    }
-    __syncthreads();
-    const __bf16 *wab = reinterpret_cast<const __bf16 *>(wa), *wbb = reinterpret_cast<const __bf16 *>(wb);
-
     const long long tiles = (a.n + 15) / 16;
     const long long stride = (long long)gridDim.x * WAVES;
     long long tile = (long long)blockIdx.x * WAVES + wave;
-    if (tile >= tiles) return;
     typedef float v4f_x __attribute__((ext_vector_type(4), aligned(16)));
     v4f_x xn[4];  // the lane's 8 floats of K step 0 and of K step 1
     const auto issue = [&](long long t) {
@@ -707,8 +720,24 @@ __global__ void __launch_bounds__(RES_THREADS, 4) k_mlp2_split(const MlpArgs a)
             xn[2 * ks + 1] = *reinterpret_cast<const v4f_x *>(xrow + 32 * ks + 4);
         }
     };
-    issue(tile);
+    issue(tile);  // the first rows are on their way while the weights are split (on a few tiles per wavefront that is the kernel's time:
+                  // 50,000 rows, one tile of 16 per wavefront: 15.4 -> 13 us, five layers of GIN 321 -> 303)
     float scale = a.rs ? a.rs[min(tile * 16 + i, a.n - 1)] : 1.0f;
+    __builtin_amdgcn_sched_barrier(0);
+    {
+        float va[2 * NB1], vb[2 * NB2];
+        const auto k_of = [](int r) { return r; };
+        const auto seen = [](float, float) {};
+        split_load_w<NB1>(va, a.wa, 64, 0, wave, i, kb, k_of);
+        split_load_w<NB2>(vb, a.wb, a.d3, 0, wave, i, kb, k_of);
+        __builtin_amdgcn_sched_barrier(0);
+        split_put_w<NB1>(wa, va, 64, 0, wave, i, kb, k_of, [](int kp) { return 2 * kp; }, seen);
+        split_put_w<NB2>(wb, vb, a.d3, 0, wave, i, kb, k_of, [](int kp) { return split_k_slot(2 * kp); }, seen);
+    }
+    __syncthreads();
+    const __bf16 *wab = reinterpret_cast<const __bf16 *>(wa), *wbb = reinterpret_cast<const __bf16 *>(wb);
+
+    if (tile >= tiles) return;
     asm volatile("" : "+v"(xn[0]), "+v"(xn[1]), "+v"(xn[2]), "+v"(xn[3]), "+v"(scale));  // waited for here, not at the head of the loop (see its end)
     const float floor_mid = a.relu_mid ? 0.f : -3.4e38f;  // ReLU between the layers as one max per value
     // acc += the six products of a split operand pair, smallest first
