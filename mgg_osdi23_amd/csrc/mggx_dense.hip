@@ -33,6 +33,7 @@ struct DenseArgs {
                   // bit 1: and they are whole 128-byte lines written once: streaming stores;
                   // bit 2: bf16 rows may be written 8 elements (16 bytes) at a time
     int stream_x; // rows of X are whole 128-byte lines per K group (d1 % 64 == 0, aligned base and pitch)
+    int w_whole;         // k_dense_xw_split: W is kept in LDS whole
     int tiles_per_wave;  // k_dense_xw_bf16_lines: rounds of consecutive tiles per workgroup
 };
 
@@ -828,6 +829,185 @@ __global__ void __launch_bounds__(RES_THREADS, 4) k_mlp2_split(const MlpArgs a)
     }
 }
 
+// Wide updates (more than 16 columns, 64 values of K and more) on the bf16 matrix cores with fp32 results: X and W split into
+// three bf16 parts each and multiplied as in k_mlp2_split, six products where the fp32 matrix cores need eight at sixteen times
+// the cycles.  Bound: reading X where W is small (170 K rows, 128 -> 128: 75 -> 42.5 us, 4.1 TB/s; 128 -> 40: 34.8 -> 24.0, 4.8 TB/s),
+// else the matrix cores and the LDS (100 K rows, 602 -> 128: 295 -> 142 us; 400 -> 128: 197 -> 102; 602 -> 50: 122 -> 95; 20 K rows,
+// 602 -> 64: 71 -> 40).  Error against 64 bits: 1.5e-7 of the result (2-norm) at K = 128, 3.7e-7 at 602; the fp32 matrix cores: 2.0e-7
+// and 4.4e-7.
+// A wavefront forms 32 rows x NB * 16 columns, so that a part of W read from LDS serves two row tiles (with one, the LDS would
+// be as busy as the matrix cores); the workgroup's threads split W themselves while they stage it.
+//   RES    W stays in LDS whole, workgroups walk over the rows
+//   !RES   a workgroup takes 256 rows through all of K; W comes in groups of 64 values of K into two buffers in turn, the loads
+//          of a group and the rows' next values in flight while the group before is multiplied
+// Values that bf16 rounds to infinity (infinities, NaN, the last 1/512 below the largest float) have no three parts: the tiles
+// (of X) or the workgroups (of W) that meet one go through the fp32 matrix cores instead.
+constexpr unsigned SPLIT_LIMIT = 0x7F7F8000u;
+constexpr size_t SPLIT_RESIDENT_LIMIT = 112 * 1024;  // W stays in LDS whole up to this size
+__device__ __forceinline__ bool beyond_split(float v) { return (__float_as_uint(v) & 0x7FFFFFFFu) >= SPLIT_LIMIT; }
+
+__host__ __device__ constexpr size_t split_group_bytes(int nb) { return (size_t)3 * nb * 16 * SPLIT_KP * sizeof(unsigned short); }
+
+template <int NB, bool RES>
+__global__ void __launch_bounds__(RES_THREADS, 2) k_dense_xw_split(const DenseArgs a)
+{
+    constexpr int KP = SPLIT_KP, PART = NB * 16 * KP, GROUP = 3 * PART, WAVES = RES_THREADS / 64;
+    extern __shared__ __align__(16) float lds_raw[];
+    __shared__ int w_beyond;
+    unsigned short *wl = reinterpret_cast<unsigned short *>(lds_raw);
+    const int lane = (int)(threadIdx.x & 63u), wave = (int)(threadIdx.x >> 6);
+    const int i = lane & 15, kb = lane >> 4;
+    const int c0 = (int)blockIdx.y * (NB * 16);
+    const int ngroups = (a.d1 + 63) >> 6;
+    const float *w = static_cast<const float *>(a.w), *x = static_cast<const float *>(a.x);
+    if (threadIdx.x == 0) w_beyond = 0;
+
+    bool wbad = false;
+    const auto load_w = [&](float (&v)[2 * NB], int g) {
+        split_load_w<NB>(v, w, a.d2, c0, wave, i, kb, [&](int r) { return lds_row_k<true>(64 * g + r, ngroups, a.d1); });
+    };
+    const auto put_w = [&](const float (&v)[2 * NB], int g, int buf) {
+        split_put_w<NB>(wl + buf * GROUP, v, a.d2, c0, wave, i, kb, [&](int r) { return lds_row_k<true>(64 * g + r, ngroups, a.d1); },
+                        [](int kp) { return 2 * kp; }, [&](float v0, float v1) { wbad |= beyond_split(v0) || beyond_split(v1); });
+    };
+
+    // 32 rows per wavefront and step
+    const long long steps = (a.n + 31) / 32, stride = (long long)gridDim.x * WAVES;
+    long long step = (long long)blockIdx.x * WAVES + wave;
+    typedef float v4f_any __attribute__((ext_vector_type(4), aligned(4)));
+    v4f xn[2][4];  // the next group's values of the wavefront's two row tiles: lane (i, kb): 8 floats of K step 0, 8 of K step 1
+    float scale[2] = {1.f, 1.f}, scale_next[2] = {1.f, 1.f};
+    const auto issue = [&](long long st, int g) {
+        const int k = (g == ngroups - 1 ? a.d1 - 64 : 64 * g) + 8 * kb;
+#pragma unroll
+        for (int t = 0; t < 2; ++t) {
+            const long long row = min(st * 32 + 16 * t + i, a.n - 1);
+            const float *xrow = x + row * a.ld_x + k;
+#pragma unroll
+            for (int j = 0; j < 4; ++j) xn[t][j] = *reinterpret_cast<const v4f_any *>(xrow + 32 * (j >> 1) + 4 * (j & 1));
+            if (g == 0 && a.rs) scale_next[t] = a.rs[row];
+        }
+    };
+    issue(step, 0);
+    __builtin_amdgcn_sched_barrier(0);
+    {
+        float v[2 * NB];
+        for (int g = 0; g < (RES ? ngroups : 1); ++g) {
+            load_w(v, g);
+            put_w(v, g, g);
+        }
+    }
+    const auto settle = [&]() {  // what is staged so far is there for everybody, and so is the word about its values
+        if (wbad) w_beyond = 1;
+        __syncthreads();
+    };
+    __syncthreads();  // w_beyond is zero before anybody sets it
+    settle();
+    if (RES && step >= steps) return;
+
+    const __bf16 *wlb = reinterpret_cast<const __bf16 *>(wl);
+    const auto six = [](v4f acc, const v8bf (&wp)[3], const v8bf (&xp)[3]) {
+        acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wp[2], xp[0], acc, 0, 0, 0);
+        acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wp[1], xp[1], acc, 0, 0, 0);
+        acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wp[0], xp[2], acc, 0, 0, 0);
+        acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wp[1], xp[0], acc, 0, 0, 0);
+        acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wp[0], xp[1], acc, 0, 0, 0);
+        acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wp[0], xp[0], acc, 0, 0, 0);
+        return acc;
+    };
+    v4f acc[2][NB];
+    bool xbad = false;
+    int g = 0;
+    asm volatile("" : "+v"(xn[0][0]), "+v"(xn[0][1]), "+v"(xn[0][2]), "+v"(xn[0][3]), "+v"(xn[1][0]), "+v"(xn[1][1]), "+v"(xn[1][2]), "+v"(xn[1][3]),
+                 "+v"(scale_next[0]), "+v"(scale_next[1]));
+    for (;;) {
+        if (g == 0) {
+#pragma unroll
+            for (int t = 0; t < 2; ++t) {
+                scale[t] = scale_next[t];
+#pragma unroll
+                for (int nb = 0; nb < NB; ++nb) acc[t][nb] = (v4f){0.f, 0.f, 0.f, 0.f};
+            }
+            xbad = false;
+        }
+        v4f xc[2][4];
+#pragma unroll
+        for (int t = 0; t < 2; ++t)
+#pragma unroll
+            for (int j = 0; j < 4; ++j) xc[t][j] = xn[t][j];
+        const bool last = g + 1 == ngroups;
+        const long long nstep = last ? step + stride : step;
+        const int ng = last ? 0 : g + 1;
+        const bool more = RES ? nstep < steps : !last;
+        float v[2 * NB];
+        if (more) {
+            issue(nstep, ng);
+            if constexpr (!RES) load_w(v, ng);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        const __bf16 *wg = wlb + (RES ? g : g & 1) * GROUP;
+#pragma unroll
+        for (int ks = 0; ks < 2; ++ks) {
+            v8bf xs[2][3];
+#pragma unroll
+            for (int t = 0; t < 2; ++t) {
+                const float x8[8] = {xc[t][2 * ks][0], xc[t][2 * ks][1], xc[t][2 * ks][2], xc[t][2 * ks][3],
+                                     xc[t][2 * ks + 1][0], xc[t][2 * ks + 1][1], xc[t][2 * ks + 1][2], xc[t][2 * ks + 1][3]};
+                unsigned top = 0;
+#pragma unroll
+                for (int e = 0; e < 8; ++e) top = max(top, __float_as_uint(x8[e]) & 0x7FFFFFFFu);
+                xbad |= top >= SPLIT_LIMIT;
+                split8(x8, xs[t][0], xs[t][1], xs[t][2]);
+            }
+#pragma unroll
+            for (int nb = 0; nb < NB; ++nb) {
+                v8bf w3[3];
+#pragma unroll
+                for (int p = 0; p < 3; ++p) w3[p] = *reinterpret_cast<const v8bf *>(wg + p * PART + (16 * nb + i) * KP + 32 * ks + 8 * kb);
+                acc[0][nb] = six(acc[0][nb], w3, xs[0]);
+                acc[1][nb] = six(acc[1][nb], w3, xs[1]);
+            }
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        // the next values are waited for here, before this step's stores are issued (see `arrived`)
+        asm volatile("" : "+v"(xn[0][0]), "+v"(xn[0][1]), "+v"(xn[0][2]), "+v"(xn[0][3]), "+v"(xn[1][0]), "+v"(xn[1][1]), "+v"(xn[1][2]), "+v"(xn[1][3]),
+                     "+v"(scale_next[0]), "+v"(scale_next[1]));
+        if constexpr (!RES) {
+            if (more) {
+                put_w(v, ng, ng & 1);  // the buffer of the group before this one: every wavefront is past it since the last barrier
+                settle();
+            }
+        }
+        if (last) {
+            if (__any(xbad) || w_beyond) {
+#pragma unroll
+                for (int t = 0; t < 2; ++t) {
+                    const float *xrow = x + min(step * 32 + 16 * t + i, a.n - 1) * a.ld_x;
+#pragma unroll
+                    for (int nb = 0; nb < NB; ++nb) {
+                        v4f s = (v4f){0.f, 0.f, 0.f, 0.f};
+                        const int c = min(c0 + 16 * nb + i, a.d2 - 1);
+                        for (int k = kb; k < a.d1 + kb; k += 4) {
+                            const bool in = k < a.d1;
+                            const float xv = xrow[min(k, a.d1 - 1)], wv = w[(long long)min(k, a.d1 - 1) * a.d2 + c];
+                            s = __builtin_amdgcn_mfma_f32_16x16x4f32(in ? wv : 0.f, in ? xv : 0.f, s, 0, 0, 0);
+                        }
+                        acc[t][nb] = s;
+                    }
+                }
+            }
+#pragma unroll
+            for (int t = 0; t < 2; ++t) {
+                const long long row = step * 32 + 16 * t + i;
+                store_rows<NB, false>(a.out, a.ld_out, a.d2, scale[t], a.relu, a.vec_out, acc[t], row, row < a.n, c0, kb);
+            }
+        }
+        if (!more) break;
+        step = nstep;
+        g = ng;
+    }
+}
+
 // W staged in K chunks (any d1): fallback when W does not fit in LDS.
 template <int NB>
 __global__ void __launch_bounds__(256) k_dense_xw(const DenseArgs a)
@@ -1266,6 +1446,19 @@ struct LaunchResident {
     }
 };
 template <int NB>
+struct LaunchSplit {
+    static void run(dim3 grid, size_t lds, hipStream_t s, const DenseArgs &a)
+    {
+        if (a.w_whole) {
+            allow_lds(k_dense_xw_split<NB, true>, lds);
+            k_dense_xw_split<NB, true><<<grid, dim3(RES_THREADS), lds, s>>>(a);
+        } else {
+            allow_lds(k_dense_xw_split<NB, false>, lds);
+            k_dense_xw_split<NB, false><<<grid, dim3(RES_THREADS), lds, s>>>(a);
+        }
+    }
+};
+template <int NB>
 struct LaunchChunked {
     static void run(dim3 grid, size_t, hipStream_t s, const DenseArgs &a) { k_dense_xw<NB><<<grid, dim3(256), 0, s>>>(a); }
 };
@@ -1351,6 +1544,20 @@ MGGX_EXPORT int mggx_dense_xw(float *d_out, const float *d_x, const float *d_w, 
     const int nb = mggx::pick_nb(d2);
     const int gy = ((d2 + 15) / 16 + nb - 1) / nb;
     const size_t lds = (size_t)((d1 + 63) & ~63) * (nb * 16 + 4) * sizeof(float);
+    // The split kernel where the fp32 matrix cores or the LDS would hold the update: more than 32 columns, or a W that does not fit
+    // in LDS at all (1 M rows, 101 -> 20: 110 us either way; 50 K rows, 64 -> 32: 7.1 / 6.8), from 8,192 rows on (128 -> 64: 10.6 /
+    // 10.3; below, every wavefront has one step and the time is W's).
+    if (d1 >= 64 && n >= 8192 && (d2 > 32 || (d2 > 16 && lds > mggx::LDS_RESIDENT_LIMIT))) {
+        const size_t group = mggx::split_group_bytes(nb), whole = group * (size_t)((d1 + 63) / 64);
+        const long long blocks = (n + 255) / 256;
+        if (blocks > 0x7fffffffLL) return fail(MGGX_ELIMIT, "dense_xw: too many rows");
+        a.w_whole = whole <= mggx::SPLIT_RESIDENT_LIMIT;
+        const long long room = 256 * std::max<long long>(1, std::min<long long>(2, (long long)(mggx::SPLIT_RESIDENT_LIMIT / whole)));  // workgroups the chip holds
+        const dim3 grid((unsigned)(a.w_whole ? std::min(blocks, room) : blocks), (unsigned)gy);
+        mggx::dispatch_nb<mggx::LaunchSplit>(nb, grid, a.w_whole ? whole : 2 * group, stream, a);
+        MGGX_LAUNCH_CHECK("k_dense_xw_split");
+        return MGGX_OK;
+    }
     if (lds <= mggx::LDS_RESIDENT_LIMIT) {
         const dim3 grid(mggx::persistent_blocks(n), (unsigned)gy);
         mggx::dispatch_nb<mggx::LaunchResident>(nb, grid, lds, stream, a);

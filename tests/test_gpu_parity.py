@@ -1138,3 +1138,60 @@ def test_split_csr_device_rows_of_many_chunks(gpu, lens):
     got = gpu.split_CSR_device(to_dev(ptr), to_dev(col), lb, ub)
     for g, w in zip(got, want):
         assert np.array_equal(g.cpu().numpy(), w)
+
+
+@pytest.mark.parametrize("n,d1,d2", [(8192, 64, 17), (8193, 65, 33), (8207, 100, 47), (8224, 127, 64), (8192, 128, 128), (8300, 129, 96), (9001, 128, 130),
+                                     (8450, 320, 40), (8200, 300, 64), (8223, 602, 50), (8199, 700, 128), (8192, 1500, 20), (200_003, 64, 41)])
+def test_wide_dense_update_of_many_rows(gpu, n, d1, d2):
+    """The update on split operands: K of one group, several, a last group that overlaps the one before it; columns of every
+    number of 16-column blocks, more than one pass over them; W kept in LDS whole and in groups; the last rows of a step
+    missing; rows at a pitch that leaves them off any 16-byte boundary; scale and ReLU.  The tolerance is that of the other
+    fp32 updates: what the three parts of an operand leave out is below 2^-24 of it."""
+    import torch
+    x = gpu.fill_normal((n, d1), seed=420)
+    w = gpu.glorot(d1, d2, seed=421)
+    s = gpu.fill_uniform((n,), 0.5, 2.0, seed=422)
+    idx = np.unique(np.concatenate([np.arange(0, n, max(1, n // 1500)), np.arange(n - 70, n)]))
+    want = orc.dense(x[idx], w, f64=True)
+    mag = np.abs(x[idx]).astype(np.float64) @ np.abs(w).astype(np.float64)
+    out = torch.full((n, d2), 3.0, device="cuda")
+    gpu.dense_forward(out, to_dev(x), to_dev(w), n, d1, d2)
+    gpu.sync()
+    assert_close_to_oracle(out.cpu().numpy()[idx], want, mag, FP32_TOL, "dense %dx%dx%d" % (n, d1, d2))
+    xp = np.full((n, d1 + 3), np.nan, np.float32)
+    xp[:, :d1] = x
+    out = torch.full((n, d2 + 1), 3.0, device="cuda")
+    gpu.dense_forward(out, to_dev(xp), to_dev(w), n, d1, d2, ld_x=d1 + 3, ld_out=d2 + 1, row_scale=to_dev(s), relu=True)
+    gpu.sync()
+    got = out.cpu().numpy()
+    assert np.all(got[:, d2] == 3.0)
+    assert_close_to_oracle(got[idx, :d2], np.maximum(want * s[idx][:, None], 0), mag * s[idx][:, None], FP32_TOL, "dense, strided, scaled, ReLU")
+
+
+@pytest.mark.parametrize("d1,d2", [(128, 64), (300, 128)])
+def test_wide_dense_update_with_values_that_have_no_bf16_parts(gpu, d1, d2):
+    """Infinities, NaN and the largest floats in X or in W: what plain fp32 arithmetic gives -- an infinity times a weight that
+    bf16 holds exactly is an infinity, not a NaN -- and rows without such a value stay as they are."""
+    import torch
+    n = 8200
+    x = gpu.fill_normal((n, d1), seed=430)
+    w = gpu.glorot(d1, d2, seed=431)
+    w[5] = 1.0
+    big = np.float32(3.4028235e38)
+    x[3, 5], x[40, 5], x[41, 5], x[70, 7], x[8199, 5] = np.inf, -np.inf, big, np.nan, np.inf
+    xd, wd = to_dev(x), to_dev(w)
+    out = torch.empty(n, d2, device="cuda")
+    gpu.dense_forward(out, xd, wd, n, d1, d2)
+    gpu.sync()
+    got = out.cpu().numpy()
+    assert np.all(got[[3, 8199]] == np.inf) and np.all(got[40] == -np.inf) and np.all(np.isnan(got[70]))
+    np.testing.assert_allclose(got[41], big, rtol=1e-6)
+    ok = np.setdiff1d(np.arange(n), [3, 40, 41, 70, 8199])[:2000]
+    want = orc.dense(x[ok], w, f64=True)
+    assert_close_to_oracle(got[ok], want, np.abs(x[ok]).astype(np.float64) @ np.abs(w).astype(np.float64), FP32_TOL, "rows beside them")
+    w[9, 2] = np.inf
+    x = np.abs(gpu.fill_normal((n, d1), seed=432)) + np.float32(0.1)
+    gpu.dense_forward(out, to_dev(x), to_dev(w), n, d1, d2)
+    gpu.sync()
+    got = out.cpu().numpy()
+    assert np.all(got[:, 2] == np.inf) and np.isfinite(np.delete(got, 2, 1)).all()
