@@ -848,6 +848,7 @@ __global__ void __launch_bounds__(RES_THREADS, 4) k_mlp2_split(const MlpArgs a)
 // (of X) or the workgroups (of W) that meet one go through the fp32 matrix cores instead.
 constexpr unsigned SPLIT_LIMIT = 0x7F7F8000u;
 constexpr size_t SPLIT_RESIDENT_LIMIT = 112 * 1024;  // W stays in LDS whole up to this size
+constexpr long long SPLIT_WORKGROUPS = 150, SPLIT_MIN_ROWS = 1024;
 __device__ __forceinline__ bool beyond_split(float v) { return (__float_as_uint(v) & 0x7FFFFFFFu) >= SPLIT_LIMIT; }
 
 __host__ __device__ constexpr size_t split_group_bytes(int nb) { return (size_t)3 * nb * 16 * SPLIT_KP * sizeof(unsigned short); }
@@ -1549,16 +1550,22 @@ MGGX_EXPORT int mggx_dense_xw(float *d_out, const float *d_x, const float *d_w, 
     const int gy = ((d2 + 15) / 16 + nb - 1) / nb;
     const size_t lds = (size_t)((d1 + 63) & ~63) * (nb * 16 + 4) * sizeof(float);
     // The split kernel where the fp32 matrix cores or the LDS would hold the update: more than 32 columns, or a W that does not fit
-    // in LDS at all (1 M rows, 101 -> 20: 110 us either way; 50 K rows, 64 -> 32: 7.1 / 6.8), from 8,192 rows on (128 -> 64: 10.6 /
-    // 10.3; below, every wavefront has one step and the time is W's).
-    if (d1 >= 64 && n >= 8192 && (d2 > 32 || (d2 > 16 && lds > mggx::LDS_RESIDENT_LIMIT))) {
-        const size_t group = mggx::split_group_bytes(nb), whole = group * (size_t)((d1 + 63) / 64);
+    // in LDS at all (1 M rows, 101 -> 20: 110 us either way; 50 K rows, 64 -> 32: 7.1 / 6.8), from SPLIT_MIN_ROWS rows on
+    // (1,024 rows, 64 -> 41: 6.3 / 5.7; 128 -> 128: 18.0 / 7.3; 300 -> 64: 22.4 / 10.6).
+    if (d1 >= 64 && n >= mggx::SPLIT_MIN_ROWS && (d2 > 32 || (d2 > 16 && lds > mggx::LDS_RESIDENT_LIMIT))) {
         const long long blocks = (n + 255) / 256;
         if (blocks > 0x7fffffffLL) return fail(MGGX_ELIMIT, "dense_xw: too many rows");
+        // Few rows: fewer columns per workgroup until the chip has something to do.  A workgroup's time is its chain of K groups, which
+        // costs more the more columns of W it splits (8,000 rows, 602 -> 128: 64.6 us with 32 workgroups of 128 columns, 29.3 with
+        // 128 of 32, 21.5 with 256 of 16; 20 K rows, 602 -> 64: 41.6 / 31.8 with 158 of 32 / 44.6 with 316 of 16, X read four times).
+        int sb = nb;
+        const auto passes = [&](int b) { return ((d2 + 15) / 16 + b - 1) / b; };
+        while (sb > 1 && blocks * passes(sb) < mggx::SPLIT_WORKGROUPS) sb = (sb + 1) / 2;
+        const size_t group = mggx::split_group_bytes(sb), whole = group * (size_t)((d1 + 63) / 64);
         a.w_whole = whole <= mggx::SPLIT_RESIDENT_LIMIT;
         const long long room = 256 * std::max<long long>(1, std::min<long long>(2, (long long)(mggx::SPLIT_RESIDENT_LIMIT / whole)));  // workgroups the chip holds
-        const dim3 grid((unsigned)(a.w_whole ? std::min(blocks, room) : blocks), (unsigned)gy);
-        mggx::dispatch_nb<mggx::LaunchSplit>(nb, grid, a.w_whole ? whole : 2 * group, stream, a);
+        const dim3 grid((unsigned)(a.w_whole ? std::min(blocks, room) : blocks), (unsigned)passes(sb));
+        mggx::dispatch_nb<mggx::LaunchSplit>(sb, grid, a.w_whole ? whole : 2 * group, stream, a);
         MGGX_LAUNCH_CHECK("k_dense_xw_split");
         return MGGX_OK;
     }

@@ -1141,7 +1141,8 @@ def test_split_csr_device_rows_of_many_chunks(gpu, lens):
 
 
 @pytest.mark.parametrize("n,d1,d2", [(8192, 64, 17), (8193, 65, 33), (8207, 100, 47), (8224, 127, 64), (8192, 128, 128), (8300, 129, 96), (9001, 128, 130),
-                                     (8450, 320, 40), (8200, 300, 64), (8223, 602, 50), (8199, 700, 128), (8192, 1500, 20), (200_003, 64, 41)])
+                                     (8450, 320, 40), (8200, 300, 64), (8223, 602, 50), (8199, 700, 128), (8192, 1500, 20), (200_003, 64, 41),
+                                     (1024, 64, 33), (1500, 602, 128), (4099, 300, 50), (20_011, 130, 64), (2000, 700, 20)])
 def test_wide_dense_update_of_many_rows(gpu, n, d1, d2):
     """The update on split operands: K of one group, several, a last group that overlaps the one before it; columns of every
     number of 16-column blocks, more than one pass over them; W kept in LDS whole and in groups; the last rows of a step
