@@ -419,7 +419,10 @@ __global__ void __launch_bounds__(RES_THREADS, 4) k_dense_xw_resident(const Dens
 // 38 KB of L2 reads).
 constexpr int FLAT_WAVES = 8;
 constexpr int FLAT_THREADS = FLAT_WAVES * 64;
-constexpr int FLAT_TILES = 4;  // consecutive tiles per workgroup
+constexpr int FLAT_TILES = 4;  // consecutive tiles per workgroup ...
+constexpr int FLAT_FEW = 4096; // ... half as many where the array has fewer tiles than this: 1,024 workgroups of 4 are little more
+                               // than one per place the chip has for one (602 -> 16, us, 4 / 2 / 1 tiles: 8,000 rows 8.7 / 5.6 / 5.7;
+                               // 20 K rows 13.9 / 11.8 / 11.4; 50 K rows 25.3 / 24.3 / 25.7; 100 K rows 44.1 / 45.3 / 50.1)
 // LDS floats of the tile: the 16 rows and what the last wavefront's K slice reads past them (masked), and never less than
 // the whole rounds of 16-byte pieces the workgroup lays down
 inline __host__ __device__ int flat_tile_floats(int d1, int sw)
@@ -1539,8 +1542,8 @@ MGGX_EXPORT int mggx_dense_xw(float *d_out, const float *d_x, const float *d_w, 
         (reinterpret_cast<uintptr_t>(d_x) & 15u) == 0) {
         const int sw = ((d1 + 31) / 32 + 3) & ~3;  // K steps per wavefront, in whole rounds of loads
         const size_t lds_flat = ((size_t)mggx::flat_tile_floats(d1, sw) + mggx::FLAT_WAVES * 256) * sizeof(float);
-        a.tiles_per_wave = mggx::FLAT_TILES;
         const long long tiles = (n + 15) / 16;
+        a.tiles_per_wave = tiles < mggx::FLAT_FEW ? mggx::FLAT_TILES / 2 : mggx::FLAT_TILES;
         const dim3 grid((unsigned)((tiles + a.tiles_per_wave - 1) / a.tiles_per_wave));
         mggx::launch_flat(sw, grid, lds_flat, stream, a);
         MGGX_LAUNCH_CHECK("k_dense_xw_flat");
