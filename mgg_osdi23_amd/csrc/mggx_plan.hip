@@ -153,7 +153,7 @@ __global__ void k_publish(const int *a, const int *b, const int *c, long long *w
 
 __global__ void k_zero_words(int *w, int n)
 {
-    if ((int)threadIdx.x < n) w[threadIdx.x] = 0;
+    for (int i = threadIdx.x; i < n; i += blockDim.x) w[i] = 0;
 }
 
 // largest r in [0, rows) with off[r] <= q (off is non-decreasing, off[rows] > q)
@@ -644,10 +644,12 @@ void plan_free(Plan *p)
         retire_block(p->d_desc, sizeof(int4) * (size_t)std::max(p->num_parts, 1));
         retire_block(p->d_off, sizeof(int) * ((size_t)p->rows + 1));
         retire_block(p->d_empty_rows, sizeof(int) * (size_t)std::max(p->rows, 1));
+        retire_block(p->d_chain, sizeof(int) * FUSE_MAX_WORKGROUPS);
     } else {
         dev_free(p->d_desc);
         dev_free(p->d_off);
         dev_free(p->d_empty_rows);
+        dev_free(p->d_chain);
     }
     guard_free(p->guard, p->pinned);
     delete p;
@@ -662,6 +664,10 @@ static int plan_finish(Plan *p, const int *d_a, const int *d_b, long long **word
     int rc = host_words(words);
     if (!rc) rc = dev_array(&d_counter, 1);
     if (!rc) rc = dev_array(&p->d_empty_rows, (size_t)p->rows);
+    if (!rc && p->blocks == 1 && !p->d_part_ptr) {  // (the caller's partition arrays may list a row's partitions apart)
+        rc = dev_array(&p->d_chain, FUSE_MAX_WORKGROUPS);
+        if (!rc) k_zero_words<<<1, 1024, 0, s.stream>>>(p->d_chain, FUSE_MAX_WORKGROUPS);
+    }
     if (rc) {
         dev_free(d_counter);
         return rc;

@@ -1196,3 +1196,53 @@ def test_wide_dense_update_with_values_that_have_no_bf16_parts(gpu, d1, d2):
     gpu.sync()
     got = out.cpu().numpy()
     assert np.all(got[:, 2] == np.inf) and np.isfinite(np.delete(got, 2, 1)).all()
+
+
+@pytest.mark.parametrize("dim,kw", [(16, {}), (13, {"relu": True}), (32, {}), (41, {"softmax": True}), (64, {"relu": True}), (100, {}), (128, {"accumulate": True})])
+def test_rows_across_workgroups_finished_in_the_same_launch(gpu, dim, kw):
+    """Rows that cross workgroups in plans of up to 4,096 of them: one row over hundreds of workgroups, one over two, one that
+    ends where a workgroup ends, a workgroup with the end of one and the start of another.  Several calls on one plan with
+    other workgroup sizes in between (what counts the parts has to be back at zero): bit for bit the same each time, equal to the
+    call in 64-bit addressing (which finishes such rows in a launch of its own), and the oracle's sums."""
+    import torch
+    rng = np.random.default_rng(dim)
+    V = 3000
+    deg = rng.integers(1, 40, V)
+    deg[[0, 700, 701, 1500, 2999]] = [20_000, 900, 64 * 16, 5000, 300]
+    ptr = np.zeros(V + 1, np.int32)
+    ptr[1:] = np.cumsum(deg)
+    col = rng.integers(0, V, ptr[-1]).astype(np.int32)
+    x = gpu.fill_normal((V, dim), seed=440)
+    base = gpu.fill_normal((V, dim), seed=441)
+    sh = share_of(ptr, col, V, 1, 0)
+    want, mag = oracle_agg(sh, x, x, dim)
+    if "accumulate" in kw:
+        want, mag = want + base, mag + np.abs(base)
+    if "relu" in kw:
+        want = np.maximum(want, 0)
+    d_ptr, d_col, d_x, d_base = to_dev(ptr), to_dev(col), to_dev(x), to_dev(base)
+    z, zc = torch.zeros(V + 1, dtype=torch.int32, device="cuda"), torch.zeros(1, dtype=torch.int32, device="cuda")
+
+    def run(wpb, dist):
+        out = d_base.clone()
+        gpu.mgg_SAG_np_div(out, d_x, d_ptr, d_col, z, zc, 0, V, dim, V, 0, 16, wpb, dist, **kw)
+        gpu.sync()
+        return out.cpu().numpy()
+
+    first = {}
+    for wpb, dist in ((1, 1), (4, 1), (0, 0), (1, 1), (4, 2), (1, 1), (4, 1), (4, 2)):
+        got = run(wpb, dist)
+        if "softmax" in kw:
+            e = np.exp(want - want.max(1, keepdims=True))
+            assert np.abs(got - e / e.sum(1, keepdims=True)).max() < 2e-4  # exp of logits of up to 600 in magnitude, 1e-7 each
+        else:
+            assert_close_to_oracle(got, want, mag, FP32_TOL, "wpb=%d dist=%d" % (wpb, dist))
+        assert np.array_equal(first.setdefault((wpb, dist), got), got)
+    gpu.set_gather_addressing(1)
+    try:
+        if "softmax" in kw:  # the same logits; the row's exponentials are added in another order: 41 terms, below 41 x 2^-24 of the sum
+            np.testing.assert_allclose(run(4, 1), first[(4, 1)], rtol=4e-6, atol=1e-37)
+        else:
+            assert np.array_equal(run(4, 1), first[(4, 1)])
+    finally:
+        gpu.set_gather_addressing(0)
