@@ -851,7 +851,7 @@ __global__ void __launch_bounds__(RES_THREADS, 4) k_mlp2_split(const MlpArgs a)
 // (of X) or the workgroups (of W) that meet one go through the fp32 matrix cores instead.
 constexpr unsigned SPLIT_LIMIT = 0x7F7F8000u;
 constexpr size_t SPLIT_RESIDENT_LIMIT = 112 * 1024;  // W stays in LDS whole up to this size
-constexpr long long SPLIT_WORKGROUPS = 150, SPLIT_MIN_ROWS = 1024;
+constexpr long long SPLIT_WORKGROUPS = 150, SPLIT_MIN_ROWS = 1024, SPLIT_MANY_ROWS = 500000;
 __device__ __forceinline__ bool beyond_split(float v) { return (__float_as_uint(v) & 0x7FFFFFFFu) >= SPLIT_LIMIT; }
 
 __host__ __device__ constexpr size_t split_group_bytes(int nb) { return (size_t)3 * nb * 16 * SPLIT_KP * sizeof(unsigned short); }
@@ -1555,7 +1555,11 @@ MGGX_EXPORT int mggx_dense_xw(float *d_out, const float *d_x, const float *d_w, 
     // The split kernel where the fp32 matrix cores or the LDS would hold the update: more than 32 columns, or a W that does not fit
     // in LDS at all (1 M rows, 101 -> 20: 110 us either way; 50 K rows, 64 -> 32: 7.1 / 6.8), from SPLIT_MIN_ROWS rows on
     // (1,024 rows, 64 -> 41: 6.3 / 5.7; 128 -> 128: 18.0 / 7.3; 300 -> 64: 22.4 / 10.6).
-    if (d1 >= 64 && n >= mggx::SPLIT_MIN_ROWS && (d2 > 32 || (d2 > 16 && lds > mggx::LDS_RESIDENT_LIMIT))) {
+    // Half a million rows and more with a W of up to 64 columns that fits in LDS stay on the fp32 matrix cores: memory holds both (1 M
+    // rows, 100 -> 64: 166 us / 158 split; 64 -> 48: 91 / 89), and the other rounding of the first update, carried through the five
+    // layers of sums of a 2.45 M-node graph, moved single results by 6e-5 of their size.
+    const bool wide = d2 > 32 && (n < mggx::SPLIT_MANY_ROWS || d2 > 64);
+    if (d1 >= 64 && n >= mggx::SPLIT_MIN_ROWS && (wide || (d2 > 16 && lds > mggx::LDS_RESIDENT_LIMIT))) {
         const long long blocks = (n + 255) / 256;
         if (blocks > 0x7fffffffLL) return fail(MGGX_ELIMIT, "dense_xw: too many rows");
         // Few rows: fewer columns per workgroup until the chip has something to do.  A workgroup's time is its chain of K groups, which
