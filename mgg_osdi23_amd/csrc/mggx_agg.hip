@@ -17,7 +17,8 @@
 //   wavefronts a row that crosses wavefronts is finished through LDS
 //   workgroups a row that crosses workgroups leaves two partial rows in a
 //              carry buffer; a small second kernel sums them in a fixed order
-// No atomics anywhere; the summation order depends only on (ps, wpb, dist, dim).
+// No value is added atomically; the summation order depends only on (ps, wpb, dist, dim).  (Small plans count, with an atomic, which
+// workgroups of a row have left their part: FUSE below.)
 // Index stream: a wavefront fetches the descriptors and the first ids of its next few rounds together into its own
 // piece of LDS (two HBM latencies per four rounds instead of per round, with no feature row in flight meanwhile) and
 // the rounds read them from there; the 16 lanes or so of a slot read the same words.
