@@ -91,7 +91,8 @@ int mggx_timer_start(void *timer);
 int mggx_timer_stop(void *timer);
 int mggx_timer_elapsed_ms(void *timer, float *ms); /* synchronises on the stop event */
 int mggx_timer_destroy(void *timer);
-/* Frees the workspace and every cached plan (also what captured graphs may still point at: destroy those first). */
+/* Frees the workspace, every cached plan (also what captured graphs may still point at: destroy those first) and the
+ * device blocks kept for the plans and set-up calls to come (at most 256 MB of them). */
 int mggx_release_cached(void);
 /* Drops what the library remembers about the CSR array at this device address (cached partition plans, search
  * results): call it before freeing or rewriting an index array that aggregation calls have seen, when the memory is
