@@ -63,8 +63,8 @@ constexpr int HDR_ENDS = 2;    // head entry: the row ends inside this unit
 constexpr int HDR_STARTS = 4;  // tail entry: the row started inside this unit
 
 constexpr int MODE_F32_VEC4 = 0;     // fp32 rows of 4 columns and more, one 16-byte load per lane, rows on any 4-byte boundary
-constexpr int MODE_F32_PACKED = 3;   // the same, for rows of a width that is not a multiple of 4 and a pitch without room for the last
-                                     // whole piece (see tail_shift).  A kernel of its own: in one kernel with the rows of whole
+constexpr int MODE_F32_PACKED = 3;   // the same, for rows of a width that is not a multiple of 4 whose last whole piece could lie past the
+                                     // row's pitch (see tail_shift).  A kernel of its own: in one kernel with the rows of whole
                                      // pieces, the moves of the partial piece cost those 2.5 % (100 K nodes, width 100: 174.5 -> 178.9 us)
                                      // and 1.6 % (five layers of 2.45 M nodes, width 64: 14.20 -> 14.44 ms)
 constexpr int MODE_F32_STRIDED = 1;  // fp32 rows of 1 to 3 columns, dword loads, one lane per row
@@ -1109,8 +1109,12 @@ int run_agg(Plan *plan, float *d_out, const void *d_in_l, const void *d_in_r, co
         mode = MODE_BF16_VEC8;
         lpr = pow2_ceil(dim / 8);
     } else if (o.in_dtype == MGGX_F32) {
-        // rows whose pitch has room for whole pieces are read in whole pieces, up to three padding columns with them
-        mode = dim < 4 ? MODE_F32_STRIDED : (dim & 3) && !(ld_in % 4 == 0 && ld_in > dim) ? MODE_F32_PACKED : MODE_F32_VEC4;
+        // A width that is not a multiple of 4 is read in whole pieces, up to three padding columns with them, only where a piece
+        // cannot leave the row: the pitch is a multiple of 4 beyond the width and the rows start on 16-byte boundaries.  In a column
+        // window of a wider table that starts anywhere else, the last piece may lie past the pitch (columns 7 to 47 of 48: it would be
+        // columns 47 to 50), for the last row past the table.
+        const bool whole_pieces = ld_in % 4 == 0 && ld_in > dim && aligned16(d_in_l) && (plan->nnz_r == 0 || aligned16(d_in_r));
+        mode = dim < 4 ? MODE_F32_STRIDED : (dim & 3) && !whole_pieces ? MODE_F32_PACKED : MODE_F32_VEC4;
         lpr = pow2_ceil((dim + 3) / 4);
     } else {
         return fail(MGGX_EINVAL, "aggregation: unknown input dtype %d", o.in_dtype);

@@ -605,6 +605,28 @@ def test_rows_off_16_byte_boundaries(gpu, rmat_graph, dim, ld):
         assert np.all(got[:, dim:] == 7.5), "padding columns of the output must stay untouched"
 
 
+@pytest.mark.parametrize("addressing", [0, 1])
+@pytest.mark.parametrize("left", [1, 2, 3, 4, 5, 7])
+def test_column_window_of_a_wider_table(gpu, rmat_graph, left, addressing):
+    """41 columns from column `left` on of tables with a pitch of 48, NaN in every other column: the sums are those of the
+    window, and from a column off 16 bytes the last piece starts early (mode 3) instead of reaching past the pitch."""
+    V, ptr, col = rmat_graph
+    dim, ld = 41, 48
+    xp = np.full((V, ld), np.nan, np.float32)
+    xp[:, left:left + dim] = gpu.fill_normal((V, dim), seed=320)
+    x = np.ascontiguousarray(xp[:, left:left + dim])
+    sh = share_of(ptr, col, V, 2, 1)
+    want, mag = oracle_agg(sh, x[sh["lb"]:sh["ub"]], x, dim, flags=orc.GIN, eps=0.5)
+    dl, dr = to_dev(xp[sh["lb"]:sh["ub"]]), to_dev(xp)
+    gpu.set_gather_addressing(addressing)
+    try:
+        got = run_agg(gpu, sh, dl.view(-1)[left:], dr.view(-1)[left:], dim, 16, 4, 2, ld_in=ld, gin=True, eps=0.5)
+        assert ",%d," % (3 if left % 4 else 0) in gpu.last_agg_kernel()
+    finally:
+        gpu.set_gather_addressing(0)
+    assert_close_to_oracle(got, want, mag, FP32_TOL, "window at column %d" % left)
+
+
 @pytest.mark.parametrize("dim", [16, 41, 64])
 def test_gin_accumulate_relu(gpu, rmat_graph, dim):
     V, ptr, col = rmat_graph
