@@ -629,7 +629,8 @@ __global__ void __launch_bounds__(RES_THREADS, 4) k_mlp2_resident(const MlpArgs 
 // split exactly into three bf16 parts, x = x1 + x2 + x3 (x1 = bf16(x), x2 = bf16(x - x1), x3 = bf16(x - x1 - x2): 24
 // mantissa bits, the subtractions are exact), and a product x w becomes the six bf16 products that matter,
 // x1 w1 + (x1 w2 + x2 w1) + (x1 w3 + x2 w2 + x3 w1) -- each exact in the fp32 accumulator, what is dropped is below
-// 2^-24 of |x w|.  Six v_mfma_f32_16x16x32_bf16 do the work of eight v_mfma_f32_16x16x4_f32 at a sixteenth of the
+// 2^-24 of |x w|.  (That holds for values from 2^-110 up, and for intermediate ones: bf16 ends at 2^-133, so smaller values keep
+// fewer of their bits -- none under 2^-134 -- and an infinity becomes a NaN.)  Six v_mfma_f32_16x16x32_bf16 do the work of eight v_mfma_f32_16x16x4_f32 at a sixteenth of the
 // cycles each, so the kernel that the fp32 matrix cores held at 68 % busy becomes bound by memory.
 // Layout as in k_mlp2_resident (transposed products; lane (i, kb) = (L % 16, L / 16)): the first product leaves the lane
 // with T[row i][16 nb + 4 kb + r], r = 0..3; the second wants eight K values per lane and step, and takes for step s the
@@ -670,7 +671,7 @@ __device__ __forceinline__ int split_k_slot(int k) { return 32 * (k >> 5) + 8 * 
 // a workgroup, in two steps so that the loads can fly meanwhile: thread -> column 16 (unit % NB) + i and K pair 4 (unit / NB) + kb
 // of the group, unit = 8 u + wavefront, so that a wavefront writes two K values of 16 columns x 4 pairs per instruction, 4 bytes
 // to each of the 64 banks.  k_of(r): K index of row r of the group, or -1 for a zero row; slot(kp): where in a staged column pair
-// kp goes.
+// kp goes; up: a power of two the values are multiplied by first.
 template <int NB, typename K>
 __device__ __forceinline__ void split_load_w(float (&v)[2 * NB], const float *w, int d2, int c0, int wave, int i, int kb, K k_of)
 {
@@ -681,16 +682,15 @@ __device__ __forceinline__ void split_load_w(float (&v)[2 * NB], const float *w,
         v[2 * u + 1] = w[(long long)max(k_of(r + 1), 0) * d2 + c];
     }
 }
-template <int NB, typename K, typename SLOT, typename SEEN>
-__device__ __forceinline__ void split_put_w(unsigned short *dst, const float (&v)[2 * NB], int d2, int c0, int wave, int i, int kb, K k_of, SLOT slot, SEEN seen)
+template <int NB, typename K, typename SLOT>
+__device__ __forceinline__ void split_put_w(unsigned short *dst, const float (&v)[2 * NB], int d2, int c0, int wave, int i, int kb, float up, K k_of, SLOT slot)
 {
     constexpr int PART = NB * 16 * SPLIT_KP;
 #pragma unroll
     for (int u = 0; u < NB; ++u) {
         const int unit = u * (RES_THREADS / 64) + wave, c = 16 * (unit % NB) + i, kp = 4 * (unit / NB) + kb;
         const bool on = c0 + c < d2;
-        const float v0 = on && k_of(2 * kp) >= 0 ? v[2 * u] : 0.f, v1 = on && k_of(2 * kp + 1) >= 0 ? v[2 * u + 1] : 0.f;
-        seen(v0, v1);
+        const float v0 = on && k_of(2 * kp) >= 0 ? v[2 * u] * up : 0.f, v1 = on && k_of(2 * kp + 1) >= 0 ? v[2 * u + 1] * up : 0.f;
         unsigned h, m, l;
         split_pair(v0, v1, h, m, l);
         unsigned *q = reinterpret_cast<unsigned *>(dst + c * SPLIT_KP + slot(kp));
@@ -735,12 +735,11 @@ __global__ void __launch_bounds__(RES_THREADS, 4) k_mlp2_split(const MlpArgs a)
     {
         float va[2 * NB1], vb[2 * NB2];
         const auto k_of = [](int r) { return r; };
-        const auto seen = [](float, float) {};
         split_load_w<NB1>(va, a.wa, 64, 0, wave, i, kb, k_of);
         split_load_w<NB2>(vb, a.wb, a.d3, 0, wave, i, kb, k_of);
         __builtin_amdgcn_sched_barrier(0);
-        split_put_w<NB1>(wa, va, 64, 0, wave, i, kb, k_of, [](int kp) { return 2 * kp; }, seen);
-        split_put_w<NB2>(wb, vb, a.d3, 0, wave, i, kb, k_of, [](int kp) { return split_k_slot(2 * kp); }, seen);
+        split_put_w<NB1>(wa, va, 64, 0, wave, i, kb, 1.0f, k_of, [](int kp) { return 2 * kp; });
+        split_put_w<NB2>(wb, vb, a.d3, 0, wave, i, kb, 1.0f, k_of, [](int kp) { return split_k_slot(2 * kp); });
     }
     __syncthreads();
     const __bf16 *wab = reinterpret_cast<const __bf16 *>(wa), *wbb = reinterpret_cast<const __bf16 *>(wb);
@@ -838,21 +837,29 @@ __global__ void __launch_bounds__(RES_THREADS, 4) k_mlp2_split(const MlpArgs a)
 
 // Wide updates (more than 16 columns, 64 values of K and more) on the bf16 matrix cores with fp32 results: X and W split into
 // three bf16 parts each and multiplied as in k_mlp2_split, six products where the fp32 matrix cores need eight at sixteen times
-// the cycles.  Bound: reading X where W is small (170 K rows, 128 -> 128: 75 -> 42.5 us, 4.1 TB/s; 128 -> 40: 34.8 -> 24.0, 4.8 TB/s),
-// else the matrix cores and the LDS (100 K rows, 602 -> 128: 295 -> 142 us; 400 -> 128: 197 -> 102; 602 -> 50: 122 -> 95; 20 K rows,
-// 602 -> 64: 71 -> 40).  Error against 64 bits: 1.5e-7 of the result (2-norm) at K = 128, 3.7e-7 at 602; the fp32 matrix cores: 2.0e-7
+// the cycles.  Bound: reading X where W is small (170 K rows, 128 -> 128: 75 -> 45 us, 3.9 TB/s; 128 -> 40: 34.8 -> 25, 4.6 TB/s),
+// else the matrix cores and the LDS (100 K rows, 602 -> 128: 295 -> 139 us; 400 -> 128: 197 -> 99; 602 -> 50: 122 -> 81; 20 K rows,
+// 602 -> 64: 71 -> 30).  Error against 64 bits: 1.5e-7 of the result (2-norm) at K = 128, 3.7e-7 at 602; the fp32 matrix cores: 2.0e-7
 // and 4.4e-7.
 // A wavefront forms 32 rows x NB * 16 columns, so that a part of W read from LDS serves two row tiles (with one, the LDS would
 // be as busy as the matrix cores); the workgroup's threads split W themselves while they stage it.
 //   RES    W stays in LDS whole, workgroups walk over the rows
 //   !RES   a workgroup takes 256 rows through all of K; W comes in groups of 64 values of K into two buffers in turn, the loads
 //          of a group and the rows' next values in flight while the group before is multiplied
-// Values that bf16 rounds to infinity (infinities, NaN, the last 1/512 below the largest float) have no three parts: the tiles
-// (of X) or the workgroups (of W) that meet one go through the fp32 matrix cores instead.
-constexpr unsigned SPLIT_LIMIT = 0x7F7F8000u;
+// Range: bf16 has fp32's exponents but 16 bits less below its leading one, so the third part of a value under 2^-110 and the second
+// of one under 2^-118 would fall below the smallest bf16.  Both operands are therefore multiplied by 2^24 first, which puts every bit
+// of every fp32 value, subnormals included, where three bf16 parts (none of them subnormal) hold it, and the sums by 2^-48 (with the
+// row's scale) last.
+// (Without the scale the error grew from 2e-7 of the result at inputs of 1e-34 to 2.5e-5 at 1e-36.)
+// At the other end: a value that bf16 rounds to infinity after the scale (2^103 = 1e31 and more, infinities, NaN) has an infinity or
+// a NaN for its first part and makes every sum it enters one too (times zero as well), and so does a sum beyond 2^80 = 1.2e24 that
+// does not fit once scaled.  Row tiles with a sum that is not finite (or a row scale under 2^-78) go through the fp32
+// matrix cores instead.  (The scale costs an instruction per value of X and the look at the sums half a one per sum; a look at every
+// value of X and W, which it replaces, cost two: 233 K rows, 602 -> 64: 199 -> 194 us; 100 K rows, 602 -> 50: 85 -> 81; 170 K rows,
+// 128 -> 128: 44.4 / 45.4; 1 M rows: 244 / 247.)
+constexpr float SPLIT_UP = 0x1p24f, SPLIT_DOWN = 0x1p-48f;
 constexpr size_t SPLIT_RESIDENT_LIMIT = 112 * 1024;  // W stays in LDS whole up to this size
 constexpr long long SPLIT_WORKGROUPS = 150, SPLIT_MIN_ROWS = 1024, SPLIT_MANY_ROWS = 500000;
-__device__ __forceinline__ bool beyond_split(float v) { return (__float_as_uint(v) & 0x7FFFFFFFu) >= SPLIT_LIMIT; }
 
 __host__ __device__ constexpr size_t split_group_bytes(int nb) { return (size_t)3 * nb * 16 * SPLIT_KP * sizeof(unsigned short); }
 
@@ -861,22 +868,18 @@ __global__ void __launch_bounds__(RES_THREADS, 2) k_dense_xw_split(const DenseAr
 {
     constexpr int KP = SPLIT_KP, PART = NB * 16 * KP, GROUP = 3 * PART, WAVES = RES_THREADS / 64;
     extern __shared__ __align__(16) float lds_raw[];
-    __shared__ int w_beyond;
     unsigned short *wl = reinterpret_cast<unsigned short *>(lds_raw);
     const int lane = (int)(threadIdx.x & 63u), wave = (int)(threadIdx.x >> 6);
     const int i = lane & 15, kb = lane >> 4;
     const int c0 = (int)blockIdx.y * (NB * 16);
     const int ngroups = (a.d1 + 63) >> 6;
     const float *w = static_cast<const float *>(a.w), *x = static_cast<const float *>(a.x);
-    if (threadIdx.x == 0) w_beyond = 0;
-
-    bool wbad = false;
     const auto load_w = [&](float (&v)[2 * NB], int g) {
         split_load_w<NB>(v, w, a.d2, c0, wave, i, kb, [&](int r) { return lds_row_k<true>(64 * g + r, ngroups, a.d1); });
     };
     const auto put_w = [&](const float (&v)[2 * NB], int g, int buf) {
-        split_put_w<NB>(wl + buf * GROUP, v, a.d2, c0, wave, i, kb, [&](int r) { return lds_row_k<true>(64 * g + r, ngroups, a.d1); },
-                        [](int kp) { return 2 * kp; }, [&](float v0, float v1) { wbad |= beyond_split(v0) || beyond_split(v1); });
+        split_put_w<NB>(wl + buf * GROUP, v, a.d2, c0, wave, i, kb, SPLIT_UP, [&](int r) { return lds_row_k<true>(64 * g + r, ngroups, a.d1); },
+                        [](int kp) { return 2 * kp; });
     };
 
     // 32 rows per wavefront and step
@@ -905,12 +908,7 @@ __global__ void __launch_bounds__(RES_THREADS, 2) k_dense_xw_split(const DenseAr
             put_w(v, g, g);
         }
     }
-    const auto settle = [&]() {  // what is staged so far is there for everybody, and so is the word about its values
-        if (wbad) w_beyond = 1;
-        __syncthreads();
-    };
-    __syncthreads();  // w_beyond is zero before anybody sets it
-    settle();
+    __syncthreads();
     if (RES && step >= steps) return;
 
     const __bf16 *wlb = reinterpret_cast<const __bf16 *>(wl);
@@ -924,7 +922,6 @@ __global__ void __launch_bounds__(RES_THREADS, 2) k_dense_xw_split(const DenseAr
         return acc;
     };
     v4f acc[2][NB];
-    bool xbad = false;
     int g = 0;
     asm volatile("" : "+v"(xn[0][0]), "+v"(xn[0][1]), "+v"(xn[0][2]), "+v"(xn[0][3]), "+v"(xn[1][0]), "+v"(xn[1][1]), "+v"(xn[1][2]), "+v"(xn[1][3]),
                  "+v"(scale_next[0]), "+v"(scale_next[1]));
@@ -936,7 +933,6 @@ __global__ void __launch_bounds__(RES_THREADS, 2) k_dense_xw_split(const DenseAr
 #pragma unroll
                 for (int nb = 0; nb < NB; ++nb) acc[t][nb] = (v4f){0.f, 0.f, 0.f, 0.f};
             }
-            xbad = false;
         }
         v4f xc[2][4];
 #pragma unroll
@@ -959,12 +955,9 @@ __global__ void __launch_bounds__(RES_THREADS, 2) k_dense_xw_split(const DenseAr
             v8bf xs[2][3];
 #pragma unroll
             for (int t = 0; t < 2; ++t) {
-                const float x8[8] = {xc[t][2 * ks][0], xc[t][2 * ks][1], xc[t][2 * ks][2], xc[t][2 * ks][3],
-                                     xc[t][2 * ks + 1][0], xc[t][2 * ks + 1][1], xc[t][2 * ks + 1][2], xc[t][2 * ks + 1][3]};
-                unsigned top = 0;
+                float x8[8];
 #pragma unroll
-                for (int e = 0; e < 8; ++e) top = max(top, __float_as_uint(x8[e]) & 0x7FFFFFFFu);
-                xbad |= top >= SPLIT_LIMIT;
+                for (int e = 0; e < 8; ++e) x8[e] = xc[t][2 * ks + (e >> 2)][e & 3] * SPLIT_UP;
                 split8(x8, xs[t][0], xs[t][1], xs[t][2]);
             }
 #pragma unroll
@@ -976,6 +969,20 @@ __global__ void __launch_bounds__(RES_THREADS, 2) k_dense_xw_split(const DenseAr
                 acc[1][nb] = six(acc[1][nb], w3, xs[1]);
             }
         }
+        float top[2] = {0.f, 0.f}, down[2];  // largest size of a sum, NaN if there is one (one instruction for two sums on gfx950)
+        bool small_scale = false;
+        if (last) {
+#pragma unroll
+            for (int t = 0; t < 2; ++t) {
+#pragma unroll
+                for (int nb = 0; nb < NB; ++nb)
+#pragma unroll
+                    for (int r = 0; r < 4; r += 2)
+                        top[t] = __builtin_elementwise_maximum(__builtin_elementwise_maximum(fabsf(acc[t][nb][r]), fabsf(acc[t][nb][r + 1])), top[t]);
+                down[t] = scale[t] * SPLIT_DOWN;
+                small_scale |= scale[t] != 0.f && fabsf(scale[t]) < 0x1p-78f;  // the product with 2^-48 may be subnormal
+            }
+        }
         __builtin_amdgcn_sched_barrier(0);
         // the next values are waited for here, before this step's stores are issued (see `arrived`)
         asm volatile("" : "+v"(xn[0][0]), "+v"(xn[0][1]), "+v"(xn[0][2]), "+v"(xn[0][3]), "+v"(xn[1][0]), "+v"(xn[1][1]), "+v"(xn[1][2]), "+v"(xn[1][3]),
@@ -983,14 +990,15 @@ __global__ void __launch_bounds__(RES_THREADS, 2) k_dense_xw_split(const DenseAr
         if constexpr (!RES) {
             if (more) {
                 put_w(v, ng, ng & 1);  // the buffer of the group before this one: every wavefront is past it since the last barrier
-                settle();
+                __syncthreads();
             }
         }
         if (last) {
-            if (__any(xbad) || w_beyond) {
+            if (__any(!(top[0] < INFINITY && top[1] < INFINITY) || small_scale)) {
 #pragma unroll
                 for (int t = 0; t < 2; ++t) {
                     const float *xrow = x + min(step * 32 + 16 * t + i, a.n - 1) * a.ld_x;
+                    down[t] = scale[t];
 #pragma unroll
                     for (int nb = 0; nb < NB; ++nb) {
                         v4f s = (v4f){0.f, 0.f, 0.f, 0.f};
@@ -1007,7 +1015,7 @@ __global__ void __launch_bounds__(RES_THREADS, 2) k_dense_xw_split(const DenseAr
 #pragma unroll
             for (int t = 0; t < 2; ++t) {
                 const long long row = step * 32 + 16 * t + i;
-                store_rows<NB, false>(a.out, a.ld_out, a.d2, scale[t], a.relu, a.vec_out, acc[t], row, row < a.n, c0, kb);
+                store_rows<NB, false>(a.out, a.ld_out, a.d2, down[t], a.relu, a.vec_out, acc[t], row, row < a.n, c0, kb);
             }
         }
         if (!more) break;

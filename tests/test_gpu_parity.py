@@ -1220,6 +1220,31 @@ def test_wide_dense_update_with_values_that_have_no_bf16_parts(gpu, d1, d2):
     assert np.all(got[:, 2] == np.inf) and np.isfinite(np.delete(got, 2, 1)).all()
 
 
+@pytest.mark.parametrize("d1,d2", [(128, 128), (602, 50)])
+@pytest.mark.parametrize("sx,sw", [(-113, 100), (-118, 100), (-126, 110), (-140, 120), (0, -118), (20, -140), (-60, -57), (90, -100), (70, 10), (50, 60), (70, 50), (104, -104)])
+def test_wide_dense_update_of_small_and_large_values(gpu, d1, d2, sx, sw):
+    """X and W times powers of two that keep every result a normal number: inputs whose lower bf16 parts would fall below the
+    smallest bf16, subnormal ones, sums beyond 2^80 (which leave the split operands).  The error against 64 bits stays what it is at
+    magnitude 1: sums of K fp32 products in sequence, about sqrt(K) 2^-24 of the result (2-norm), three times that allowed."""
+    import torch
+    n = 2100
+    with np.errstate(under="ignore"):
+        x = (gpu.fill_normal((n, d1), seed=440).astype(np.float64) * 2.0 ** sx).astype(np.float32)
+        w = (gpu.glorot(d1, d2, seed=441).astype(np.float64) * 2.0 ** sw).astype(np.float32)
+    out = torch.empty(n, d2, device="cuda")
+    gpu.dense_forward(out, to_dev(x), to_dev(w), n, d1, d2)
+    gpu.sync()
+    want = x.astype(np.float64) @ w.astype(np.float64)
+    want /= 2.0 ** (sx + sw)
+    err = np.linalg.norm(out.cpu().numpy() / 2.0 ** (sx + sw) - want) / np.linalg.norm(want)
+    assert err < 3 * np.sqrt(d1) * 2.0 ** -24, err
+    scale = np.full(n, 2.0 ** -(sx + sw), np.float32)  # row scales from 2^-120 to 2^120
+    gpu.dense_forward(out, to_dev(x), to_dev(w), n, d1, d2, row_scale=to_dev(scale))
+    gpu.sync()
+    err = np.linalg.norm(out.cpu().numpy() - want) / np.linalg.norm(want)
+    assert err < 3 * np.sqrt(d1) * 2.0 ** -24, err
+
+
 @pytest.mark.parametrize("dim,kw", [(16, {}), (13, {"relu": True}), (32, {}), (41, {"softmax": True}), (64, {"relu": True}), (100, {}), (128, {"accumulate": True})])
 def test_rows_across_workgroups_finished_in_the_same_launch(gpu, dim, kw):
     """Rows that cross workgroups in plans of up to 4,096 of them: one row over hundreds of workgroups, one over two, one that
