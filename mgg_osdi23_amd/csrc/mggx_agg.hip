@@ -1083,6 +1083,25 @@ struct CoreMerge {
 constexpr long long MANY_ROUNDS = 400000;
 constexpr int MIN_WAVEFRONTS = 3000;
 
+// Parts of the static scratch in a call of mggx_sag_parts_static: descriptors | first descriptor of each row | [scratch of the
+// unit builder, ps < 16] | carry buffer.
+struct StaticLayout {
+    size_t desc, off, tmp;
+    StaticLayout(int rows, int num_parts, int ps)
+    {
+        const auto pad = [](size_t b) { return (b + 255) & ~(size_t)255; };
+        desc = pad(sizeof(int4) * (size_t)num_parts);
+        off = pad(sizeof(int) * ((size_t)rows + 1));
+        tmp = unit_of(ps) != ps ? pad(sizeof(int) * explicit_tmp_ints(rows)) : 0;
+    }
+    size_t used() const { return desc + off + tmp; }
+    size_t carry_room() const { return used() < MGGX_STATIC_SCRATCH_BYTES ? MGGX_STATIC_SCRATCH_BYTES - used() : 0; }
+};
+
+// Carry buffer of num_wg workgroups: a head and a tail entry each, and behind them their partial rows of cpad floats.
+size_t carry_hdr_bytes(long long num_wg) { return ((size_t)num_wg * 2 * sizeof(int2) + 255) & ~(size_t)255; }
+size_t carry_buffer_bytes(long long num_wg, int cpad) { return (carry_hdr_bytes(num_wg) + (size_t)num_wg * 2 * cpad * sizeof(float) + 255) & ~(size_t)255; }
+
 int run_agg(Plan *plan, float *d_out, const void *d_in_l, const void *d_in_r, const int *d_col_l, const int *d_col_r,
             int lb, int dim, int wpb, int dist, const mggx_agg_opts &o_in, const Gate &gate, const FixedScratch *fixed = nullptr, CoreMerge *cm = nullptr)
 {
@@ -1136,9 +1155,16 @@ int run_agg(Plan *plan, float *d_out, const void *d_in_l, const void *d_in_r, co
     // width 64 are 1.4 - 3.7 % faster with 8 than with 4, one of them by 0.1 %); 2 rounds for rows of 84 to 128 bytes (8 slots).
     // Provenance: wpb x dist sweeps over eight graphs of 4 K to 800 K nodes at widths 8 to 128, the shares and the 2.45 M-node
     // graph: within 6 % of the best cell of {1,2,4,8} x {1,2,4,8,16} on all of them, within 2 % on most.
-    const double per_row = (double)plan->num_parts / (double)(plan->rows > 0 ? plan->rows : 1);
-    const long long rounds = (plan->num_parts + slots - 1) / slots;
-    const bool beside_core = cm != nullptr;
+    // Explicit partitions: the rule looks at the sizes the caller states, since mggx_sag_parts_static never learns how many
+    // descriptors they make and has to choose as mggx_sag_parts does; and its carry buffer has to fit what the static scratch leaves,
+    // so both take longer wavefronts where it would not, up to the 16 rounds (4 with more than 4 slots) and 8 wavefronts of a large
+    // plan (width 256, ps 4, 1.15 M partitions of 100 K rows: 24,219 workgroups of 4 x 4 rounds would need 50 MB beside 18 MB of
+    // descriptors; 12,110 of 4 x 8 need 25).
+    const long long stated = plan->d_part_ptr ? explicit_units_bound(plan->rows, plan->caller_parts, plan->ps) : plan->num_parts;
+    const int cpad = (dim + 3) & ~3;
+    const double per_row = (double)stated / (double)(plan->rows > 0 ? plan->rows : 1);
+    const long long rounds = (stated + slots - 1) / slots;
+    const bool beside_core = cm != nullptr, wpb_free = wpb == 0, dist_free = dist == 0;
     if (wpb == 0) wpb = (beside_core && !blocked && slots <= 4) ? 8 : (blocked || slots > 4 || per_row < 3.0 || rounds < MANY_ROUNDS) ? 4 : 8;
     if (dist == 0) {
         if (slots <= 4 && beside_core && !blocked) dist = cm->group_rows == CORE_GROUP_ROWS_WIDE ? 8 : 4;
@@ -1149,11 +1175,19 @@ int run_agg(Plan *plan, float *d_out, const void *d_in_l, const void *d_in_r, co
         else dist = 4;
         while (dist > 1 && rounds < (long long)MIN_WAVEFRONTS * dist) dist /= 2;
     }
+    if (plan->d_part_ptr && (wpb_free || dist_free)) {
+        const size_t room = StaticLayout(plan->rows, plan->caller_parts, plan->ps).carry_room();
+        const auto fits = [&]() {
+            const long long per_wg = (long long)wpb * slots * dist;
+            return room == 0 || carry_buffer_bytes((stated + per_wg - 1) / per_wg, cpad) <= room;  // (room 0: not a call for the static scratch)
+        };
+        while (!fits() && dist_free && dist < (slots <= 4 ? 16 : 4)) dist *= 2;
+        if (!fits() && wpb_free && slots <= 4 && per_row >= 3.0) wpb = 8;
+    }
     const long long parts_per_wg = (long long)wpb * slots * dist;
     if (parts_per_wg > 0x3fffffffLL) return fail(MGGX_ELIMIT, "aggregation: wpb*dist too large");
     const long long num_wg = (plan->num_parts + parts_per_wg - 1) / parts_per_wg;
     if (num_wg > 0x7fffffffLL) return fail(MGGX_ELIMIT, "aggregation: too many workgroups");
-    const int cpad = (dim + 3) & ~3;
 
     AggArgs a{};
     const int ldp = (dim + 3) & ~3;  // row stride of the per-block partial sums of a column-blocked plan
@@ -1222,10 +1256,9 @@ int run_agg(Plan *plan, float *d_out, const void *d_in_l, const void *d_in_r, co
     a.chain = fuse ? plan->d_chain : nullptr;
 
     if (num_wg > 0) {
-        const size_t hdr_bytes = (size_t)num_wg * 2 * sizeof(int2);
-        const size_t hdr_pad = (hdr_bytes + 255) & ~(size_t)255;
+        const size_t hdr_pad = carry_hdr_bytes(num_wg);
         void *ws = nullptr;
-        const size_t carry_bytes = (hdr_pad + (size_t)num_wg * 2 * cpad * sizeof(float) + 255) & ~(size_t)255;
+        const size_t carry_bytes = carry_buffer_bytes(num_wg, cpad);
         const size_t part_bytes = blocked ? (size_t)plan->rows * ldp * sizeof(float) : 0;
         int rc = MGGX_OK;
         if (fixed) {
@@ -1686,15 +1719,11 @@ MGGX_EXPORT int mggx_sag_parts_static(float *d_out, const float *d_in, const int
     unsigned char *base = nullptr;
     rc = mggx::static_scratch_ptr(&base);
     if (rc) return rc;
-    // layout of the scratch: descriptors | first descriptor of each row | [scratch of the unit builder, ps < 16] | carry
-    // buffer (sized by run_agg)
-    const auto pad = [](size_t b) { return (b + 255) & ~(size_t)255; };
+    const mggx::StaticLayout at(num_nodes, num_parts, ps);
     const bool grouped = mggx::unit_of(ps) != ps;
-    const size_t desc_bytes = pad(sizeof(int4) * (size_t)num_parts), off_bytes = pad(sizeof(int) * ((size_t)num_nodes + 1));
-    const size_t tmp_bytes = grouped ? pad(sizeof(int) * mggx::explicit_tmp_ints(num_nodes)) : 0;
-    if (desc_bytes + off_bytes + tmp_bytes >= (size_t)MGGX_STATIC_SCRATCH_BYTES)
+    if (at.carry_room() == 0)
         return fail(MGGX_ELIMIT, "sag_parts_static: %d partitions over %d rows need %zu bytes of descriptors; the static scratch holds %zu",
-                    num_parts, num_nodes, desc_bytes + off_bytes + tmp_bytes, (size_t)MGGX_STATIC_SCRATCH_BYTES);
+                    num_parts, num_nodes, at.used(), (size_t)MGGX_STATIC_SCRATCH_BYTES);
     mggx::Plan plan;  // lives for this call only; its arrays are views into the scratch
     plan.d_ptr_l = d_row_ptr;
     plan.d_part_ptr = d_part_ptr;
@@ -1704,16 +1733,15 @@ MGGX_EXPORT int mggx_sag_parts_static(float *d_out, const float *d_in, const int
     plan.unit = mggx::unit_of(ps);
     plan.caller_parts = num_parts;
     plan.d_desc = reinterpret_cast<int4 *>(base);
-    plan.d_off = reinterpret_cast<int *>(base + desc_bytes);
+    plan.d_off = reinterpret_cast<int *>(base + at.desc);
     plan.nnz_l = 1;  // "has local edges"; the kernels read the count itself from d_row_ptr[num_nodes]
     long long bound = num_parts;
     rc = mggx::explicit_desc_fill(d_row_ptr, d_part_ptr, d_part2node, num_nodes, num_parts, ps, plan.d_desc, plan.d_off,
-                                  reinterpret_cast<int *>(base + desc_bytes + off_bytes), &bound);
+                                  reinterpret_cast<int *>(base + at.desc + at.off), &bound);
     if (rc) return rc;
     // ps < 16: several partitions per descriptor; their number stays on the device (d_off[rows]) and the grid is sized by a bound
     plan.num_parts = (int)bound;
-    const size_t used = desc_bytes + off_bytes + tmp_bytes;
-    const mggx::FixedScratch fx{base + used, (size_t)MGGX_STATIC_SCRATCH_BYTES - used, d_row_ptr + num_nodes, grouped ? plan.d_off + num_nodes : nullptr};
+    const mggx::FixedScratch fx{base + at.used(), at.carry_room(), d_row_ptr + num_nodes, grouped ? plan.d_off + num_nodes : nullptr};
     mggx_agg_opts o{};
     o.flags = MGGX_AGG_ACCUMULATE;
     return mggx::run_agg(&plan, d_out, d_in, nullptr, d_col, nullptr, lowbound, dim, wpb, dist, o, mggx::Gate{}, &fx);

@@ -281,6 +281,14 @@ int plan_get_explicit(const int *d_row_ptr, const int *d_part_ptr, const int *d_
                       int num_parts, int ps, Plan **out);
 // Neighbors per kernel slot for a partition size (see Plan::unit).
 inline int unit_of(int ps) { return ps >= 16 ? ps : ps * (16 / ps); }
+// Units of explicit partitions, at most: every row with partitions has up to (its partitions / g) + 1, and at most `rows` rows have any.
+inline long long explicit_units_bound(int rows, int num_parts, int ps)
+{
+    const int g = unit_of(ps) / ps;
+    if (g <= 1 || rows <= 0 || num_parts <= 0) return num_parts;
+    const long long bound = (long long)num_parts / g + (rows < num_parts ? rows : num_parts);
+    return bound < num_parts ? bound : num_parts;
+}
 // Explicit partition arrays -> unit descriptors and the first unit of each row, into caller-provided device arrays, with
 // kernels on the library's stream only.  Partitions per unit g = unit_of(ps) / ps.  g == 1: one descriptor per partition,
 // d_tmp unused.  g > 1: d_tmp holds explicit_tmp_ints(rows) ints of scratch; the number of units stays on the device

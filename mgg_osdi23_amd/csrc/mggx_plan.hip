@@ -867,8 +867,7 @@ int explicit_desc_fill(const int *d_row_ptr, const int *d_part_ptr, const int *d
     k_units_per_row<<<(rows + 255) / 256, 256, 0, s.stream>>>(off_p, rows, g, cnt);
     const int rc = exclusive_scan_i32_device(cnt, d_off, rows, scan_tmp);
     if (rc) return rc;
-    // every row with partitions has at most (its partitions / g) + 1 units, and at most `rows` rows have any
-    const long long bound = std::min<long long>(num_parts, (long long)num_parts / g + std::min(rows, num_parts));
+    const long long bound = explicit_units_bound(rows, num_parts, ps);
     k_desc_from_units<<<(unsigned)((bound + 255) / 256), 256, 0, s.stream>>>(d_row_ptr, d_part_ptr, off_p, d_off, rows, ps, g, d_desc);
     if (hipGetLastError() != hipSuccess) return fail(MGGX_EHIP, "plan: explicit unit kernel launch failed");
     if (units_bound) *units_bound = bound;

@@ -61,3 +61,48 @@ for dim in (41, 40):
 ''')
     got = {tuple(map(int, l.split()[:2])): int(l.split()[2]) for l in out.splitlines()}
     assert got == {(d, c): (3 if d == 41 and c % 4 else 0) for d in (41, 40) for c in range(8)}
+
+
+def test_static_entry_point_takes_what_longer_wavefronts_fit(without_device):
+    """mggx_sag_parts_static with wpb and dist left at 0: its carry buffer (two partial rows per workgroup) shares the 64 MiB of
+    the static scratch with 16 bytes per partition and 4 per row.  A call is taken exactly if it fits with the longest wavefronts of
+    the rule (16 rounds, 4 with more than 4 slots; 8 of them per workgroup for rows of 3 partitions and more, 4 slots and fewer),
+    and mggx_sag_parts chooses the same ones, which is what makes the two bit-identical."""
+    out = without_device(r'''
+import random
+rng = random.Random(5)
+SCRATCH = 64 << 20
+sizes = [(100_000, 1_150_000, 4, 256), (100_000, 1_150_000, 16, 256), (13_000_000, 200_000, 16, 64), (12_000_000, 300_000, 16, 256)]
+for _ in range(300):  # the arrays take 60 to 100 % of the scratch, so that the carry buffer decides
+    dim = rng.choice([3, 5, 16, 41, 64, 100, 128, 200, 256])
+    fill, share = rng.uniform(.6, 1.0) * SCRATCH, rng.random() ** 2
+    sizes.append((max(int(fill * (1 - share) / 4), 1), max(int(fill * share / 16), 1), rng.choice([16, 32, 5, 4, 1]), dim))
+p = malloc(1 << 20)
+def pad(b): return (b + 255) & ~255
+for rows, parts, ps, dim in sizes:
+    for wpb0, dist0 in ((0, 0), (4, 0), (0, 1)):
+        fake.fake_clear()
+        args = (at(p), at(p), at(p), at(p), at(p), at(p), 0, rows, parts, ps, dim, wpb0, dist0)
+        rc = lib.mggx_sag_parts_static(*args)
+        took = re.search(r"wpb=\d+ dist=\d+", host.last_agg_kernel()).group(0) if rc == 0 else None
+        g = max(16 // ps, 1)
+        units = min(parts, parts // g + min(rows, parts)) if g > 1 else parts
+        lanes = 1
+        while lanes * 4 < dim: lanes *= 2
+        slots = 64 // lanes
+        wpb = wpb0 or (8 if slots <= 4 and units >= 3 * rows else 4)
+        dist = dist0 or (16 if slots <= 4 else 4)
+        tiles = (rows + 1023) // 1024
+        used = pad(16 * parts) + pad(4 * (rows + 1)) + (pad(4 * (2 * (rows + 1) + 2 * (tiles + 1) + 2)) if g > 1 else 0)
+        wgs = -(-units // (wpb * slots * dist))
+        carry = pad(pad(16 * wgs) + 8 * wgs * ((dim + 3) & ~3))
+        assert (rc == 0) == (used < SCRATCH and used + carry <= SCRATCH), (rows, parts, ps, dim, wpb0, dist0, rc, used, carry)
+        if rc == 0:
+            assert lib.mggx_sag_parts(*args) == 0, lib.mggx_last_error()
+            assert took in host.last_agg_kernel(), (took, host.last_agg_kernel())
+            lib.mggx_forget(at(p))
+        else:
+            assert rc == -6 and b"static scratch" in lib.mggx_last_error()
+        print(rc == 0, took)
+''').split("\n")
+    assert sum(l.startswith("True") for l in out) > 100 and sum(l.startswith("False") for l in out) > 100
