@@ -1022,14 +1022,16 @@ void launch_agg_kernel(dim3 grid, dim3 block, size_t lds_bytes, hipStream_t stre
     k_agg<LPR, MODE, BUF, SMX, FUSE><<<grid, block, lds_bytes, stream>>>(a);
 }
 
-// Which kernels have a variant that finishes rows crossing workgroups by itself (AggArgs::chain).
-template <int MODE, bool BUF>
-constexpr bool has_fused(int lpr) { return BUF && F32_PIECES<MODE> && lpr >= 4 && lpr <= 32; }
+// Which kernels have a variant that finishes rows crossing workgroups by itself (AggArgs::chain): what decides on the host whether a
+// call takes it and leaves k_agg_tail out is this function, too.  fp32 rows of 9 to 128 columns with both tables in one window,
+// which is what the forwards of small graphs aggregate; every further row class, element type or addressing mode is two to four
+// kernels more in the library (16 now) and has not been measured: those calls keep the second launch.
+constexpr bool has_fused(int mode, bool buf, int lpr) { return buf && (mode == MODE_F32_VEC4 || mode == MODE_F32_PACKED) && lpr >= 4 && lpr <= 32; }
 
 template <int LPR, int MODE, bool BUF, bool SMX>
 int launch_agg_as(dim3 grid, dim3 block, size_t lds_bytes, hipStream_t stream, const AggArgs &a)
 {
-    if constexpr (has_fused<MODE, BUF>(LPR)) {
+    if constexpr (has_fused(MODE, BUF, LPR)) {
         if (a.chain) {
             launch_agg_kernel<LPR, MODE, BUF, SMX, true>(grid, block, lds_bytes, stream, a);
             return MGGX_OK;
@@ -1251,8 +1253,8 @@ int run_agg(Plan *plan, float *d_out, const void *d_in_l, const void *d_in_r, co
     // rows without neighbors are written by k_agg_tail
     const bool touch_empty = !(o.flags & MGGX_AGG_ACCUMULATE) || (o.flags & (MGGX_AGG_GIN | MGGX_AGG_RELU | MGGX_AGG_SOFTMAX));
     const int n_empty = touch_empty ? plan->num_empty : 0;
-    const bool fuse = !blocked && !beside_core && !fixed && plan->d_chain && n_empty == 0 && num_wg > 1 && num_wg <= FUSE_MAX_WORKGROUPS && buf &&
-                      (mode == MODE_F32_VEC4 || mode == MODE_F32_PACKED) && lpr >= 4 && lpr <= 32;
+    // (a call with rows without neighbors launches k_agg_tail for them, which finishes the crossing rows on the way)
+    const bool fuse = !blocked && !beside_core && !fixed && plan->d_chain && n_empty == 0 && num_wg > 1 && num_wg <= FUSE_MAX_WORKGROUPS && has_fused(mode, buf, lpr);
     a.chain = fuse ? plan->d_chain : nullptr;
 
     if (num_wg > 0) {
@@ -1348,8 +1350,8 @@ int run_agg(Plan *plan, float *d_out, const void *d_in_l, const void *d_in_r, co
             MGGX_LAUNCH_CHECK("k_agg_tail");
         }
     }
-    snprintf(st.last_kernel, sizeof(st.last_kernel), "k_agg<%d,%d,%d> grid=%lld block=%d parts=%d blocks=%d ps=%d wpb=%d dist=%d addr=%s", lpr, mode, (int)buf,
-             num_wg, 64 * wpb, plan->num_parts, plan->blocks, plan->ps, wpb, dist, buf ? "buffer32" : "flat64");
+    snprintf(st.last_kernel, sizeof(st.last_kernel), "k_agg<%d,%d,%d> grid=%lld block=%d parts=%d blocks=%d ps=%d wpb=%d dist=%d addr=%s fused=%d", lpr, mode, (int)buf,
+             num_wg, 64 * wpb, plan->num_parts, plan->blocks, plan->ps, wpb, dist, buf ? "buffer32" : "flat64", (int)fuse);
     return MGGX_OK;
 }
 

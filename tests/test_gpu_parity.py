@@ -605,9 +605,8 @@ def test_rows_off_16_byte_boundaries(gpu, rmat_graph, dim, ld):
         assert np.all(got[:, dim:] == 7.5), "padding columns of the output must stay untouched"
 
 
-@pytest.mark.parametrize("addressing", [0, 1])
 @pytest.mark.parametrize("left", [1, 2, 3, 4, 5, 7])
-def test_column_window_of_a_wider_table(gpu, rmat_graph, left, addressing):
+def test_column_window_of_a_wider_table(gpu, rmat_graph, left):
     """41 columns from column `left` on of tables with a pitch of 48, NaN in every other column: the sums are those of the
     window, and from a column off 16 bytes the last piece starts early (mode 3) instead of reaching past the pitch."""
     V, ptr, col = rmat_graph
@@ -618,12 +617,8 @@ def test_column_window_of_a_wider_table(gpu, rmat_graph, left, addressing):
     sh = share_of(ptr, col, V, 2, 1)
     want, mag = oracle_agg(sh, x[sh["lb"]:sh["ub"]], x, dim, flags=orc.GIN, eps=0.5)
     dl, dr = to_dev(xp[sh["lb"]:sh["ub"]]), to_dev(xp)
-    gpu.set_gather_addressing(addressing)
-    try:
-        got = run_agg(gpu, sh, dl.view(-1)[left:], dr.view(-1)[left:], dim, 16, 4, 2, ld_in=ld, gin=True, eps=0.5)
-        assert ",%d," % (3 if left % 4 else 0) in gpu.last_agg_kernel()
-    finally:
-        gpu.set_gather_addressing(0)
+    got = run_agg(gpu, sh, dl.view(-1)[left:], dr.view(-1)[left:], dim, 16, 4, 2, ld_in=ld, gin=True, eps=0.5)
+    assert ",%d," % (3 if left % 4 else 0) in gpu.last_agg_kernel()
     assert_close_to_oracle(got, want, mag, FP32_TOL, "window at column %d" % left)
 
 
@@ -1274,6 +1269,7 @@ def test_rows_across_workgroups_finished_in_the_same_launch(gpu, dim, kw):
         out = d_base.clone()
         gpu.mgg_SAG_np_div(out, d_x, d_ptr, d_col, z, zc, 0, V, dim, V, 0, 16, wpb, dist, **kw)
         gpu.sync()
+        assert "fused=%d" % ("addr=buffer32" in gpu.last_agg_kernel()) in gpu.last_agg_kernel()
         return out.cpu().numpy()
 
     first = {}
@@ -1293,3 +1289,28 @@ def test_rows_across_workgroups_finished_in_the_same_launch(gpu, dim, kw):
             assert np.array_equal(run(4, 1), first[(4, 1)])
     finally:
         gpu.set_gather_addressing(0)
+
+
+@pytest.mark.parametrize("dim,parts,empty,fused", [(128, 8191, 0, 1), (128, 8192, 0, 1), (128, 8193, 0, 0), (128, 8192, 1, 0), (100, 8192, 0, 1), (9, 600, 0, 1),
+                                                   (8, 600, 0, 0), (129, 600, 0, 0)])
+def test_where_crossing_rows_take_a_launch_of_their_own(gpu, addressing, dim, parts, empty, fused):
+    """Both sides of the rule: 4,096 workgroups and 4,097 (two partitions each at width 128), a row without neighbors, the
+    narrowest and widest rows of the one-launch kernels and the next ones, 64-bit addresses.  Rows of three partitions cross workgroups everywhere."""
+    import torch
+    rows = parts // 3
+    deg = np.full(rows, 40)
+    deg[-1] -= {0: 0, 2: -32, 1: -16}[parts % 3]
+    deg = np.concatenate([deg, np.zeros(empty, np.int64)])
+    V = len(deg)
+    ptr = np.zeros(V + 1, np.int32)
+    ptr[1:] = np.cumsum(deg)
+    col = np.random.default_rng(parts).integers(0, V, ptr[-1]).astype(np.int32)
+    x = gpu.fill_normal((V, dim), seed=460)
+    sh = share_of(ptr, col, V, 1, 0)
+    want, mag = oracle_agg(sh, x, x, dim)
+    out = torch.full((V, dim), 7.5, device="cuda")
+    z, zc = torch.zeros(V + 1, dtype=torch.int32, device="cuda"), torch.zeros(1, dtype=torch.int32, device="cuda")
+    gpu.mgg_SAG_np_div(out, to_dev(x), to_dev(ptr), to_dev(col), z, zc, 0, V, dim, V, 0, 16, 1, 1)
+    gpu.sync()
+    assert "parts=%d " % parts in gpu.last_agg_kernel() and "fused=%d" % (fused and addressing == "auto") in gpu.last_agg_kernel(), gpu.last_agg_kernel()
+    assert_close_to_oracle(out.cpu().numpy(), want, mag, FP32_TOL, "dim %d, %d partitions" % (dim, parts))
