@@ -69,6 +69,10 @@ const char *mggx_version(void);
  *      of the reference mains, e.g. src/mgg_np_div_kernel.cu:86,116-153,223-228) ---- */
 int mggx_init(int device);
 int mggx_device_name(char *buf, size_t len);
+/* Calls on one stream follow one another.  Aggregation calls use one scratch of the library's (rows that cross workgroups,
+ * partial rows of column blocks and of the dense core), whatever graph they are on: calls that could run at the same time --
+ * on two streams, or a replay of a captured graph beside a live call or another replay -- have to be put in order by the
+ * caller (events, or a wait), or they spoil each other's results.  Calls made after them are not affected. */
 int mggx_set_stream(void *hip_stream);
 int mggx_sync(void);
 int mggx_malloc(void **d_ptr, size_t bytes);

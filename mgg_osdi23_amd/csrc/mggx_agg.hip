@@ -82,7 +82,9 @@ struct AggArgs {
     Gate gate;      // closed = the plan is stale (the caller's CSR arrays changed): every kernel returns at once
     int2 *c_hdr;   // [2 * workgroups]: head, tail
     float *c_val;  // [2 * workgroups][cpad]
-    int *chain;    // FUSE: [workgroups] how many workgroups of the row that starts in this one have left their part (zero between calls)
+    unsigned long long *chain;  // FUSE: [workgroups] call number << 16 | how many workgroups of the row that starts in this one have left
+                                // their part in that call
+    unsigned long long call;    // FUSE: number of this call << 16; later calls have larger ones
     long long ld_in, ld_out;
     int num_parts;
     const int *num_parts_dev; // when set: the descriptor count is read from here (it was made on the device and never copied back;
@@ -387,7 +389,11 @@ __device__ __forceinline__ void finish_row(const AggArgs &a, int row, int l, con
 // microseconds are a good part of theirs.  Every workgroup of such a row leaves its partial row in the carry buffer and
 // then counts itself in; the one that finds the others there adds the parts, in the same order as k_agg_tail.  The XCDs' L2s
 // are not coherent with each other for plain accesses, so parts and counters go with device-scope accesses, and a workgroup
-// waits until its part has arrived before it counts.  GCN forward, 4,096 nodes: 35.4 -> 32.7 us; GIN forward, 50 K nodes: 299 -> 288.
+// waits until its part has arrived before it counts.  GCN forward, 4,096 nodes: 35.4 -> 33.3 us; GIN forward, 50 K nodes: 299 -> 289.
+// Counters carry the number of the call, and the first workgroup of a call to come by starts them anew (a maximum with the call's
+// number, then the addition, to one address in order), so nothing depends on how an earlier call left them: calls that overlapped by
+// mistake spoil each other, not the ones that follow.  (With a counter that the last workgroup sets back to zero: 32.9 and 288.5 us.
+// The maximum issued ahead of the wait for the part, or only where the count turns out to be an earlier call's: 34 and 291.)
 template <int LPR, int MODE, bool BUF, bool SMX, bool FUSE>
 __global__ void __launch_bounds__(1024) MGGX_AGG_OCCUPANCY k_agg(const AggArgs a)
 {
@@ -819,43 +825,62 @@ __global__ void __launch_bounds__(1024) MGGX_AGG_OCCUPANCY k_agg(const AggArgs a
     }
     if (open) emit(false);
     if constexpr (FUSE) {
-        int first[2], others[2];  // where each row's chain starts, and how many workgroups follow
-#pragma unroll
-        for (int j = 0; j < 2; ++j) {
-            first[j] = others[j] = 0;
-            if (chain_row[j] < 0) continue;
-            first[j] = wg_of_part(a, a.off[chain_row[j]]);
-            others[j] = wg_of_part(a, a.off[chain_row[j] + 1] - 1) - first[j];
+        // lane 0: the row of the head entry, lane 1: that of the tail entry; where its chain starts, and how many workgroups follow
+        const int mine = lane == 0 ? chain_row[0] : lane == 1 ? chain_row[1] : -1;
+        int first = 0, others = 0;
+        if (mine >= 0) {
+            first = wg_of_part(a, a.off[mine]);
+            others = wg_of_part(a, a.off[mine + 1] - 1) - first;
         }
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the parts have arrived
+        bool complete = false;
+        if (mine >= 0) {
+            (void)__hip_atomic_fetch_max(a.chain + first, a.call, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            complete = __hip_atomic_fetch_add(a.chain + first, 1ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) - a.call == (unsigned long long)others;
+        }
+        const unsigned long long to_finish = __ballot(complete);
+        asm volatile("" ::: "memory");
 #pragma unroll
         for (int j = 0; j < 2; ++j) {
-            if (chain_row[j] < 0) continue;
-            int before = 0;
-            if (lane == 0) before = __hip_atomic_fetch_add(a.chain + first[j], 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            if (__builtin_amdgcn_readfirstlane(before) != others[j]) continue;
-            asm volatile("" ::: "memory");
-            if (lane == 0) __hip_atomic_store(a.chain + first[j], 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            if (!(to_finish >> j & 1)) continue;
+            const int row = chain_row[j], n = __builtin_amdgcn_readlane(others, j), start = __builtin_amdgcn_readlane(first, j);
             float t[4];
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
                 t[i] = 0.f;
                 const int dd = lane + 64 * i;
                 if (dd >= a.dim) continue;
-                const float *src = a.c_val + (size_t)(2 * first[j]) * a.cpad + dd;  // head entries are two rows apart, the tail entry is the next row
+                const float *src = a.c_val + (size_t)(2 * start) * a.cpad + dd;  // head entries are two rows apart, the tail entry is the next row
                 const auto part = [&](int k) { return __hip_atomic_load(src + (size_t)(2 * k) * a.cpad, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); };
                 t[i] = __hip_atomic_load(src + a.cpad, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
                 int k = 1;
-                for (; k + 7 <= others[j]; k += 8) {
+                for (; k + 7 <= n; k += 8) {
                     float v[8];
 #pragma unroll
                     for (int q = 0; q < 8; ++q) v[q] = part(k + q);
 #pragma unroll
                     for (int q = 0; q < 8; ++q) t[i] += v[q];
                 }
-                for (; k <= others[j]; ++k) t[i] += part(k);
+                for (; k <= n; ++k) t[i] += part(k);
             }
-            finish(chain_row[j], t);
+            if constexpr (SMX) {
+                // the columns as k_agg_tail holds them, four to a lane, so that the row's exponentials are added in the same order there
+                float v[4];
+                bool on[4];
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    const int c = 4 * (lane % LPR) + i;
+                    const float lo = lane_read(t[0], c & 63), hi = lane_read(t[1], c & 63);  // (at most 128 columns)
+                    on[i] = c < a.dim;
+                    v[i] = on[i] ? epilogue_value(a, row, c, c < 64 ? lo : hi) : 0.f;
+                }
+                group_softmax<4>(v, on, LPR);
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+                    if (lane < LPR && on[i]) a.out[(long long)row * a.ld_out + 4 * lane + i] = v[i];
+            } else {
+                finish(row, t);
+            }
         }
     }
 }
@@ -1253,9 +1278,13 @@ int run_agg(Plan *plan, float *d_out, const void *d_in_l, const void *d_in_r, co
     // rows without neighbors are written by k_agg_tail
     const bool touch_empty = !(o.flags & MGGX_AGG_ACCUMULATE) || (o.flags & (MGGX_AGG_GIN | MGGX_AGG_RELU | MGGX_AGG_SOFTMAX));
     const int n_empty = touch_empty ? plan->num_empty : 0;
-    // (a call with rows without neighbors launches k_agg_tail for them, which finishes the crossing rows on the way)
-    const bool fuse = !blocked && !beside_core && !fixed && plan->d_chain && n_empty == 0 && num_wg > 1 && num_wg <= FUSE_MAX_WORKGROUPS && has_fused(mode, buf, lpr);
+    // (a call with rows without neighbors launches k_agg_tail for them, which finishes the crossing rows on the way; a captured call
+    // would have one number for all of its replays, so a plan used in a capture takes the second launch from then on)
+    const bool fuse = !blocked && !beside_core && !fixed && plan->d_chain && n_empty == 0 && num_wg > 1 && num_wg <= FUSE_MAX_WORKGROUPS && has_fused(mode, buf, lpr) &&
+                      !plan->pinned;
+    static_assert(FUSE_MAX_WORKGROUPS < 1 << 16, "the count of a chain lies below the call number");
     a.chain = fuse ? plan->d_chain : nullptr;
+    a.call = fuse ? ++st.fused_calls << 16 : 0;
 
     if (num_wg > 0) {
         const size_t hdr_pad = carry_hdr_bytes(num_wg);

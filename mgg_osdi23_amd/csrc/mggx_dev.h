@@ -109,7 +109,7 @@ struct Plan {
     int4 *d_desc = nullptr;      // [num_parts] one per unit
     int *d_off = nullptr;        // [rows+1] first descriptor of each row
     int *d_empty_rows = nullptr; // rows without any partition
-    int *d_chain = nullptr;      // [FUSE_MAX_WORKGROUPS] zero between calls: workgroups that have left their part of a row (k_agg, FUSE)
+    unsigned long long *d_chain = nullptr;  // [FUSE_MAX_WORKGROUPS] workgroups that have left their part of a row, with the call's number (k_agg, FUSE)
     int num_parts = 0;
     int num_empty = 0;
     int64_t nnz_l = 0, nnz_r = 0;
@@ -216,6 +216,7 @@ struct State {
     hipStream_t side_stream = nullptr;  // the core block runs here, beside the rest of the CSR on `stream`
     hipEvent_t side_fork = nullptr, side_join = nullptr;
     size_t core_ws_bytes = 0;
+    unsigned long long fused_calls = 0;  // numbers of the calls that count the workgroups of crossing rows (k_agg, FUSE)
     char last_kernel[224] = "";
     int gather_addressing = 0;  // 0 = choose per call, 1 = always 64-bit addresses
     // content checks of cached records (Guard)

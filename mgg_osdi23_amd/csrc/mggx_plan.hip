@@ -645,13 +645,12 @@ void plan_free(Plan *p)
         retire_block(p->d_desc, sizeof(int4) * (size_t)std::max(p->num_parts, 1));
         retire_block(p->d_off, sizeof(int) * ((size_t)p->rows + 1));
         retire_block(p->d_empty_rows, sizeof(int) * (size_t)std::max(p->rows, 1));
-        retire_block(p->d_chain, sizeof(int) * FUSE_MAX_WORKGROUPS);
     } else {
         dev_free(p->d_desc);
         dev_free(p->d_off);
         dev_free(p->d_empty_rows);
-        dev_free(p->d_chain);
     }
+    dev_free(p->d_chain);  // (captured calls do not use it)
     guard_free(p->guard, p->pinned);
     delete p;
 }
@@ -667,7 +666,7 @@ static int plan_finish(Plan *p, const int *d_a, const int *d_b, long long **word
     if (!rc) rc = dev_array(&p->d_empty_rows, (size_t)p->rows);
     if (!rc && p->blocks == 1 && !p->d_part_ptr) {  // (the caller's partition arrays may list a row's partitions apart)
         rc = dev_array(&p->d_chain, FUSE_MAX_WORKGROUPS);
-        if (!rc) k_zero_words<<<1, 1024, 0, s.stream>>>(p->d_chain, FUSE_MAX_WORKGROUPS);
+        if (!rc) k_zero_words<<<1, 1024, 0, s.stream>>>(reinterpret_cast<int *>(p->d_chain), 2 * FUSE_MAX_WORKGROUPS);
     }
     if (rc) {
         dev_free(d_counter);

@@ -280,6 +280,65 @@ def test_device_blocks_move_from_plan_to_plan_across_streams(gpu, V, dim):
     assert gpu.cache_stats()["plans"] == 0
 
 
+@pytest.mark.parametrize("softmax", [False, True])
+def test_calls_that_overlapped_spoil_no_later_call(gpu, softmax):
+    """Rows over hundreds of workgroups, finished by whichever workgroup leaves its part last (fused=1).  Calls on one plan issued
+    on two streams with nothing to order them may spoil each other, but no call after them: what counts the parts starts anew
+    with every call.  A captured call takes the second launch instead, and its replays give the eager call's result bit for bit."""
+    import torch
+    V, dim = 3000, 41
+    rng = np.random.default_rng(9)
+    deg = rng.integers(1, 40, V)
+    deg[[0, 700, 701, 1500, 2999]] = [20_000, 900, 1024, 5000, 300]
+    ptr = np.concatenate([[0], np.cumsum(deg)]).astype(np.int32)
+    col = rng.integers(0, V, ptr[-1]).astype(np.int32)
+    d_ptr, d_col, d_x = to_dev(ptr), to_dev(col), to_dev(gpu.fill_normal((V, dim), seed=81))
+    z, zc = torch.zeros(V + 1, dtype=torch.int32, device="cuda"), torch.zeros(1, dtype=torch.int32, device="cuda")
+    outs = [torch.empty(V, dim, device="cuda") for _ in range(3)]
+    call = lambda i: gpu.mgg_SAG_np_div(outs[i], d_x, d_ptr, d_col, z, zc, 0, V, dim, V, 0, 16, 1, 1, softmax=softmax)
+    streams = [torch.cuda.Stream(), torch.cuda.Stream()]
+    try:
+        call(2)
+        assert "fused=1" in gpu.last_agg_kernel()
+        torch.cuda.synchronize()
+        want = outs[2].clone()
+        for _ in range(4):
+            for st in streams:
+                with torch.cuda.stream(st):
+                    torch.cuda._sleep(2_000_000)  # both queues fill up behind it
+            for k in range(40):
+                with torch.cuda.stream(streams[k % 2]):
+                    gpu.use_torch_stream()
+                    call(k % 2)
+            torch.cuda.synchronize()
+            gpu.use_torch_stream()
+            for _ in range(2):
+                outs[2].fill_(-1.0)
+                call(2)
+                torch.cuda.synchronize()
+                assert torch.equal(outs[2], want)
+        with torch.cuda.stream(streams[0]):
+            graph = torch.cuda.CUDAGraph()
+            with torch.cuda.graph(graph, stream=streams[0]):
+                gpu.use_torch_stream()
+                call(2)
+                assert "fused=0" in gpu.last_agg_kernel()
+            gpu.use_torch_stream()
+            for i in range(3):
+                outs[2].fill_(-1.0)
+                graph.replay()
+                streams[0].synchronize()
+                assert torch.equal(outs[2], want), "replay %d" % i
+                outs[2].fill_(-1.0)
+                call(2)
+                streams[0].synchronize()
+                assert torch.equal(outs[2], want)
+    finally:
+        torch.cuda.synchronize()
+        gpu.use_torch_stream()
+        gpu.release_cached()
+
+
 def test_plans_go_with_their_graph_record(gpu):
     """The content check lives with the graph record (32 cached).  A dense-core plan must not outlive the record it was
     built under: after 33 other CSR sets have passed through, the first set's arrays are rewritten in place with another
