@@ -96,7 +96,8 @@ int mggx_timer_stop(void *timer);
 int mggx_timer_elapsed_ms(void *timer, float *ms); /* synchronises on the stop event */
 int mggx_timer_destroy(void *timer);
 /* Frees the workspace, every cached plan (also what captured graphs may still point at: destroy those first) and the
- * device blocks kept for the plans and set-up calls to come (at most 256 MB of them). */
+ * device blocks kept for the plans and set-up calls to come (at most 256 MB of them; an allocation of the library's that
+ * finds no memory frees those by itself). */
 int mggx_release_cached(void);
 /* Drops what the library remembers about the CSR array at this device address (cached partition plans, search
  * results): call it before freeing or rewriting an index array that aggregation calls have seen, when the memory is
@@ -114,7 +115,8 @@ int mggx_release_cached(void);
 int mggx_forget(const void *d_ptr);
 int mggx_set_plan_check(int level);
 
-/* What the library holds and what its set-up has cost so far (host clock, milliseconds, since the process started). */
+/* What the library holds and what its set-up has cost so far (host clock, milliseconds, since the process started).  Bytes are
+ * what was asked for; not counted are a counter array of 32 KB per plan and the kept blocks of mggx_release_cached. */
 typedef struct mggx_cache_stats_t {
     int64_t plans, plan_bytes;             /* cached partition plans (descriptors, row offsets) and their device bytes */
     int64_t core_plans, core_plan_bytes;   /* dense-core plans (ranking, index lists, remaining CSR) */

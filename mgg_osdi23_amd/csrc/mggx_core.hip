@@ -656,7 +656,7 @@ struct Scratch {  // device temporaries of one plan build, freed on the way out
 template <typename T>
 int device_array(T **q, size_t count)
 {
-    if (hipMalloc((void **)q, std::max<size_t>(count, 1) * sizeof(T)) != hipSuccess) return fail(MGGX_ENOMEM, "core plan: %zu bytes of device memory", count * sizeof(T));
+    if (device_malloc((void **)q, std::max<size_t>(count, 1) * sizeof(T)) != hipSuccess) return fail(MGGX_ENOMEM, "core plan: %zu bytes of device memory", count * sizeof(T));
     return MGGX_OK;
 }
 
@@ -892,7 +892,7 @@ static int core_scratch(CorePlan *p, int n4, v4f **tab, v4f **partial, const Cor
         }
         s.core_ws = nullptr;
         s.core_ws_bytes = 0;
-        if (hipMalloc(&s.core_ws, tab_bytes + part_bytes) != hipSuccess) return fail(MGGX_ENOMEM, "core: %zu bytes of scratch", tab_bytes + part_bytes);
+        if (device_malloc(&s.core_ws, tab_bytes + part_bytes) != hipSuccess) return fail(MGGX_ENOMEM, "core: %zu bytes of scratch", tab_bytes + part_bytes);
         s.core_ws_bytes = tab_bytes + part_bytes;
     }
     if (!s.core_ws_captured && capturing()) s.core_ws_captured = true;

@@ -247,6 +247,8 @@ int workspace(size_t bytes, void **p);
 // Device memory of plans and of the scratch of set-up calls: dev_free keeps a bounded amount for the next dev_alloc.  Blocks may be
 // given back with kernels that use them still in flight on the library's stream (the next user comes after them there).
 int dev_alloc(void **p, size_t bytes);
+// hipMalloc for everything else: hands the kept blocks back and asks again where there is no memory.
+hipError_t device_malloc(void **p, size_t bytes);
 void dev_free(void *p);
 template <typename T>
 int dev_array(T **p, size_t count)

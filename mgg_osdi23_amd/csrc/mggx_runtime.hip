@@ -46,7 +46,7 @@ int workspace(size_t bytes, void **p)
             s.ws_bytes = 0;
         }
         size_t want = bytes + bytes / 4 + 4096;
-        hipError_t e = hipMalloc(&s.ws, want);
+        hipError_t e = device_malloc(&s.ws, want);
         if (e != hipSuccess) {
             s.ws = nullptr;
             return fail(MGGX_ENOMEM, "workspace of %zu bytes: %s", want, hipGetErrorString(e));
@@ -64,7 +64,7 @@ int workspace(size_t bytes, void **p)
 // dozen of them per plan (100 K nodes, 2 M neighbors, plan built at every call: 288 -> 167 us; splitting and compacting an
 // eighth of 1 M nodes: 1,830 -> 1,323 us).  A block goes back to this list instead and serves the next request it fits
 // (at most twice the size asked for).  Bounds: blocks beyond POOL_MAX_BLOCK are not kept, at most POOL_MAX_BYTES are, the oldest
-// go first; mggx_release_cached hands all of them back, and so does an allocation that finds no memory.
+// go first; mggx_release_cached hands all of them back, and so does any allocation of the library's that finds no memory.
 // Order: everything the library does with such a block it does on its stream, so the next user on that stream comes after the
 // last one.  Where the stream (or the device) was changed in between, work on the old one may still be in flight: the first
 // request or return after the change waits for the device, as hipFree did every time.
@@ -86,6 +86,22 @@ static void pool_trim(size_t keep)
         s.pool_bytes -= s.pool.front().bytes;
         s.pool.erase(s.pool.begin());
     }
+}
+
+// Every allocation of the library's goes through here: one that finds no memory gets the kept blocks back first.
+hipError_t device_malloc(void **p, size_t bytes)
+{
+    hipError_t e = hipMalloc(p, bytes);
+    if (e == hipErrorOutOfMemory && !state().pool.empty()) {
+        (void)hipGetLastError();
+        pool_trim(0);
+        e = hipMalloc(p, bytes);
+    }
+    if (e != hipSuccess) {
+        (void)hipGetLastError();  // reported by the caller, not by the next launch check
+        *p = nullptr;
+    }
+    return e;
 }
 
 // sizes in eighths of a power of two, so that a graph that changed a little finds the block of the last one
@@ -116,16 +132,8 @@ int dev_alloc(void **p, size_t bytes)
         return MGGX_OK;
     }
     void *q = nullptr;
-    hipError_t e = hipMalloc(&q, want);
-    if (e == hipErrorOutOfMemory && !s.pool.empty()) {
-        (void)hipGetLastError();
-        pool_trim(0);
-        e = hipMalloc(&q, want);
-    }
-    if (e != hipSuccess) {
-        (void)hipGetLastError();
-        return fail(MGGX_ENOMEM, "%zu bytes of device memory: %s", want, hipGetErrorString(e));
-    }
+    const hipError_t e = device_malloc(&q, want);
+    if (e != hipSuccess) return fail(MGGX_ENOMEM, "%zu bytes of device memory: %s", want, hipGetErrorString(e));
     s.pool_out[q] = State::Block{q, want, dev};
     *p = q;
     return MGGX_OK;
@@ -218,7 +226,7 @@ MGGX_EXPORT int mggx_malloc(void **d_ptr, size_t bytes)
     int rc = mggx::ensure_init();
     if (rc) return rc;
     *d_ptr = nullptr;
-    hipError_t e = hipMalloc(d_ptr, bytes ? bytes : 1);
+    hipError_t e = mggx::device_malloc(d_ptr, bytes ? bytes : 1);
     if (e != hipSuccess) return fail(MGGX_ENOMEM, "malloc of %zu bytes: %s", bytes, hipGetErrorString(e));
     return MGGX_OK;
 }
@@ -231,7 +239,7 @@ MGGX_EXPORT int mggx_malloc_tables(void **d_local, size_t local_bytes, void **d_
     *d_local = *d_remote = nullptr;
     const size_t first = (std::max<size_t>(local_bytes, 1) + 255) & ~(size_t)255;
     void *p = nullptr;
-    hipError_t e = hipMalloc(&p, first + std::max<size_t>(remote_bytes, 1));
+    hipError_t e = mggx::device_malloc(&p, first + std::max<size_t>(remote_bytes, 1));
     if (e != hipSuccess) return fail(MGGX_ENOMEM, "malloc_tables of %zu + %zu bytes: %s", local_bytes, remote_bytes, hipGetErrorString(e));
     *d_local = p;
     *d_remote = static_cast<char *>(p) + first;

@@ -25,6 +25,7 @@ std::string &launch_log()
     static std::string s;
     return s;
 }
+long long *g_words;  // the pinned words that the library's set-up kernels leave their results in: here the test does
 hipError_t g_last = hipSuccess;
 hipError_t result(hipError_t e)
 {
@@ -40,6 +41,7 @@ FAKE void fake_budget(size_t bytes) { g_budget = bytes; }
 FAKE size_t fake_used() { return g_used; }
 FAKE void fake_capturing(int on) { g_capturing = on != 0; }
 FAKE const char *fake_launches() { return launch_log().c_str(); }
+FAKE void fake_word(int i, long long v) { g_words[i] = v; }
 FAKE void fake_clear() { launch_log().clear(); }
 
 FAKE void **__hipRegisterFatBinary(const void *)
@@ -117,6 +119,7 @@ FAKE hipError_t hipFree(void *p)
 FAKE hipError_t hipHostMalloc(void **p, size_t bytes, unsigned)
 {
     *p = calloc(1, bytes);
+    if (bytes == 512) g_words = static_cast<long long *>(*p);
     return hipSuccess;
 }
 FAKE hipError_t hipMemcpy(void *d, const void *s, size_t n, hipMemcpyKind)
