@@ -835,9 +835,9 @@ __global__ void __launch_bounds__(RES_THREADS, 4) k_mlp2_split(const MlpArgs a)
     }
 }
 
-// Wide updates (more than 16 columns, 64 values of K and more) on the bf16 matrix cores with fp32 results: X and W split into
+// Wide updates (more than 64 columns, or a W beyond the LDS; 64 values of K and more) on the bf16 matrix cores with fp32 results: X and W split into
 // three bf16 parts each and multiplied as in k_mlp2_split, six products where the fp32 matrix cores need eight at sixteen times
-// the cycles.  Bound: reading X where W is small (170 K rows, 128 -> 128: 75 -> 45 us, 3.9 TB/s; 128 -> 40: 34.8 -> 25, 4.6 TB/s),
+// the cycles.  Bound: reading X where W is small (170 K rows, 128 -> 128: 75 -> 45 us, 3.9 TB/s),
 // else the matrix cores and the LDS (100 K rows, 602 -> 128: 295 -> 139 us; 400 -> 128: 197 -> 99; 602 -> 50: 122 -> 81; 20 K rows,
 // 602 -> 64: 71 -> 30).  Error against 64 bits: 1.5e-7 of the result (2-norm) at K = 128, 3.7e-7 at 602; the fp32 matrix cores: 2.0e-7
 // and 4.4e-7.
@@ -859,7 +859,7 @@ __global__ void __launch_bounds__(RES_THREADS, 4) k_mlp2_split(const MlpArgs a)
 // 128 -> 128: 44.4 / 45.4; 1 M rows: 244 / 247.)
 constexpr float SPLIT_UP = 0x1p24f, SPLIT_DOWN = 0x1p-48f;
 constexpr size_t SPLIT_RESIDENT_LIMIT = 112 * 1024;  // W stays in LDS whole up to this size
-constexpr long long SPLIT_WORKGROUPS = 150, SPLIT_MIN_ROWS = 1024, SPLIT_MANY_ROWS = 500000;
+constexpr long long SPLIT_WORKGROUPS = 150, SPLIT_MIN_ROWS = 1024;
 
 __host__ __device__ constexpr size_t split_group_bytes(int nb) { return (size_t)3 * nb * 16 * SPLIT_KP * sizeof(unsigned short); }
 
@@ -1560,14 +1560,16 @@ MGGX_EXPORT int mggx_dense_xw(float *d_out, const float *d_x, const float *d_w, 
     const int nb = mggx::pick_nb(d2);
     const int gy = ((d2 + 15) / 16 + nb - 1) / nb;
     const size_t lds = (size_t)((d1 + 63) & ~63) * (nb * 16 + 4) * sizeof(float);
-    // The split kernel where the fp32 matrix cores or the LDS would hold the update: more than 32 columns, or a W that does not fit
-    // in LDS at all (1 M rows, 101 -> 20: 110 us either way; 50 K rows, 64 -> 32: 7.1 / 6.8), from SPLIT_MIN_ROWS rows on
-    // (1,024 rows, 64 -> 41: 6.3 / 5.7; 128 -> 128: 18.0 / 7.3; 300 -> 64: 22.4 / 10.6).
-    // Half a million rows and more with a W of up to 64 columns that fits in LDS stay on the fp32 matrix cores: memory holds both (1 M
-    // rows, 100 -> 64: 166 us / 158 split; 64 -> 48: 91 / 89), and the other rounding of the first update, carried through the five
-    // layers of sums of a 2.45 M-node graph, moved single results by 6e-5 of their size.
-    const bool wide = d2 > 32 && (n < mggx::SPLIT_MANY_ROWS || d2 > 64);
-    if (d1 >= 64 && n >= mggx::SPLIT_MIN_ROWS && (wide || (d2 > 16 && lds > mggx::LDS_RESIDENT_LIMIT))) {
+    // The split kernel where the fp32 matrix cores or the LDS would hold the update longest: more than 64 columns, or a W that does not
+    // fit in LDS at all, from SPLIT_MIN_ROWS rows on (us, fp32 matrix cores / split: 1,024 rows, 128 -> 128: 18.0 / 7.2; 300 -> 64:
+    // 22.4 / 10.6; 170 K rows, 128 -> 128: 75 / 45; 20 K rows, 602 -> 64: 71 / 30).
+    // Up to 32 columns it gains nothing (1 M rows, 101 -> 20: 110 us either way; 50 K rows, 64 -> 32: 7.1 / 6.8).  From 33 to 64 with a W
+    // that fits it would (1,024 rows, 64 -> 41: 6.3 / 5.4; 50 K rows, 100 -> 64: 15.6 / 10.3; 170 K rows, 128 -> 40: 35 / 25; 1 M rows,
+    // 100 -> 64: 160 / 158; 2.45 M: 393 / 372), but these are the first updates of a GIN's layers: the other rounding, no larger
+    // by itself, comes out of five layers of sums as single values that differ by up to 4e-5 of their size at 490 K nodes and 8e-5 at
+    // 2.45 M, more than results may move from one build to the next.  They keep the fp32 matrix cores at every number of
+    // rows, so that the rows of a share round as the whole matrix does.
+    if (d1 >= 64 && n >= mggx::SPLIT_MIN_ROWS && (d2 > 64 || (d2 > 16 && lds > mggx::LDS_RESIDENT_LIMIT))) {
         const long long blocks = (n + 255) / 256;
         if (blocks > 0x7fffffffLL) return fail(MGGX_ELIMIT, "dense_xw: too many rows");
         // Few rows: fewer columns per workgroup until the chip has something to do.  A workgroup's time is its chain of K groups, which

@@ -1159,11 +1159,13 @@ def test_split_csr_device_rows_of_many_chunks(gpu, lens):
 
 @pytest.mark.parametrize("n,d1,d2", [(8192, 64, 17), (8193, 65, 33), (8207, 100, 47), (8224, 127, 64), (8192, 128, 128), (8300, 129, 96), (9001, 128, 130),
                                      (8450, 320, 40), (8200, 300, 64), (8223, 602, 50), (8199, 700, 128), (8192, 1500, 20), (200_003, 64, 41),
-                                     (1024, 64, 33), (1500, 602, 128), (4099, 300, 50), (20_011, 130, 64), (2000, 700, 20)])
+                                     (1024, 64, 33), (1500, 602, 128), (4099, 300, 50), (20_011, 130, 64), (2000, 700, 20),
+                                     (1024, 64, 65), (20_011, 130, 128), (30_001, 130, 96), (40_001, 129, 96), (40_001, 128, 128), (40_001, 400, 40),
+                                     (40_001, 300, 64), (40_001, 400, 96), (40_001, 400, 128)])
 def test_wide_dense_update_of_many_rows(gpu, n, d1, d2):
-    """The update on split operands: K of one group, several, a last group that overlaps the one before it; columns of every
-    number of 16-column blocks, more than one pass over them; W kept in LDS whole and in groups; the last rows of a step
-    missing; rows at a pitch that leaves them off any 16-byte boundary; scale and ReLU.  The tolerance is that of the other
+    """The update on split operands (more than 64 columns, or a W beyond the LDS) and its neighbors on the fp32 matrix cores: K of
+    one group, several, a last group that overlaps the one before it; columns of every number of 16-column blocks, in workgroups
+    of all of them and of fewer, more than one pass over them; W kept in LDS whole and in groups; the last rows of a step missing; rows at a pitch that leaves them off any 16-byte boundary; scale and ReLU.  The tolerance is that of the other
     fp32 updates: what the three parts of an operand leave out is below 2^-24 of it."""
     import torch
     x = gpu.fill_normal((n, d1), seed=420)
@@ -1186,7 +1188,7 @@ def test_wide_dense_update_of_many_rows(gpu, n, d1, d2):
     assert_close_to_oracle(got[idx, :d2], np.maximum(want * s[idx][:, None], 0), mag * s[idx][:, None], FP32_TOL, "dense, strided, scaled, ReLU")
 
 
-@pytest.mark.parametrize("d1,d2", [(128, 64), (300, 128)])
+@pytest.mark.parametrize("d1,d2", [(128, 64), (128, 128), (300, 128)])
 def test_wide_dense_update_with_values_that_have_no_bf16_parts(gpu, d1, d2):
     """Infinities, NaN and the largest floats in X or in W: what plain fp32 arithmetic gives -- an infinity times a weight that
     bf16 holds exactly is an infinity, not a NaN -- and rows without such a value stay as they are."""
