@@ -1180,8 +1180,9 @@ int run_agg(Plan *plan, float *d_out, const void *d_in_l, const void *d_in_r, co
     // with under 8 partitions per row and block.  In row-major order beside a dense core: 8 wavefronts and 4 rounds, 8 rounds
     // where the core works in wide row groups (width 52 to 64, staged table beyond 12 MB: seven graphs of 0.7 to 3 M nodes at
     // width 64 are 1.4 - 3.7 % faster with 8 than with 4, one of them by 0.1 %); 2 rounds for rows of 84 to 128 bytes (8 slots).
-    // Provenance: wpb x dist sweeps over eight graphs of 4 K to 800 K nodes at widths 8 to 128, the shares and the 2.45 M-node
-    // graph: within 6 % of the best cell of {1,2,4,8} x {1,2,4,8,16} on all of them, within 2 % on most.
+    // Provenance: wpb x dist sweeps over eight graphs of 4 K to 800 K nodes at widths 8 to 128 (profiles/dse_ps_wpb_dist.md): of the
+    // forty, 17 are within 2 % of the best cell of {1,2,4,8} x {1,2,4,8,16}, 35 within 6 %, the worst 11 % over it (calls of 8 to
+    // 11 us, which one wavefront per workgroup would make a microsecond shorter, and 170 K nodes at width 8: 29.2 against 26.3 us).
     // Explicit partitions: the rule looks at the sizes the caller states, since mggx_sag_parts_static never learns how many
     // descriptors they make and has to choose as mggx_sag_parts does; and its carry buffer has to fit what the static scratch leaves,
     // so both take longer wavefronts where it would not, up to the 16 rounds (4 with more than 4 slots) and 8 wavefronts of a large

@@ -1010,9 +1010,10 @@ int core_row_sums(CorePlan *p, int dim, const float4 **sums)
 // gathers of its edges would take, measured without a core: GATHER ps per edge for rows of up to 4 / 8 / 16 lanes out of the L2s
 // (with the index stream that comes with it), times h + (1 - h) x G_CACHE (G_MEMORY beyond the last-level cache) in row-major order.
 // A core that takes off less than MIN_SAVING_PS does without.  Provenance: 76 graphs and widths (17 K to 1.5 M nodes, mean degrees
-// 20 to 200, widths 16, 32, 41 and 64), with and without the core: 37 of the 54 that had one were slower with it, up to three times
-// (50 K nodes, 2.2 M neighbors, width 64: 103 us with, 41 without; width 16: 70 / 23); the break-even lies at 100 to 150 us of gathers
-// (400 K nodes, 22 M neighbors: width 16 takes off 81 us and loses 7, width 41 198 us and gains 28).
+// 20 to 200, widths 16, 32, 41 and 64; profiles/core_size_model.md), with and without the core: 36 of the 54 for which the bands grow
+// one are slower with it, up to three times (50 K nodes, 2.2 M neighbors, width 64: 103 us with, 39 without; width 16: 70 / 22); the
+// break-even lies at 100 to 150 us of gathers (400 K nodes, 22 M neighbors: width 16 154 us with, 150 without; width 41 368 / 397).
+// Of the 54 the rule takes the slower side twice, by 2 and 6 %.
 namespace mggx {
 namespace {
 
