@@ -67,15 +67,15 @@ int workspace(size_t bytes, void **p)
 // go first; mggx_release_cached hands all of them back, and so does any allocation of the library's that finds no memory.
 // Order: everything the library does with such a block it does on its stream, so the next user on that stream comes after the
 // last one.  Where the stream (or the device) was changed in between, work on the old one may still be in flight: the first
-// request or return after the change waits for the device, as hipFree did every time.
+// request after the change waits for the device, as hipFree did every time, and takes no kept block if it could not.
 constexpr size_t POOL_MAX_BLOCK = 64ull << 20, POOL_MAX_BYTES = 256ull << 20;
 
-static void pool_settle()
+static bool pool_settle()
 {
     State &s = state();
-    if (!s.pool_unordered) return;
-    (void)hipDeviceSynchronize();
-    s.pool_unordered = false;
+    if (s.pool_unordered && hipDeviceSynchronize() == hipSuccess) s.pool_unordered = false;
+    if (s.pool_unordered) (void)hipGetLastError();  // (another thread is capturing, say): the kept blocks stay where they are
+    return !s.pool_unordered;
 }
 
 static void pool_trim(size_t keep)
@@ -122,8 +122,7 @@ int dev_alloc(void **p, size_t bytes)
     size_t best = s.pool.size();
     for (size_t i = 0; i < s.pool.size(); ++i)
         if (s.pool[i].device == dev && s.pool[i].bytes >= want && s.pool[i].bytes <= 2 * want && (best == s.pool.size() || s.pool[i].bytes < s.pool[best].bytes)) best = i;
-    if (best < s.pool.size()) {
-        pool_settle();
+    if (best < s.pool.size() && pool_settle()) {
         const State::Block b = s.pool[best];
         s.pool.erase(s.pool.begin() + (long)best);
         s.pool_bytes -= b.bytes;
@@ -151,7 +150,6 @@ void dev_free(void *p)
         (void)hipFree(p);
         return;
     }
-    pool_settle();
     pool_trim(POOL_MAX_BYTES - b.bytes);
     s.pool.push_back(b);
     s.pool_bytes += b.bytes;

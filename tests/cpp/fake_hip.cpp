@@ -12,7 +12,7 @@
 
 namespace {
 size_t g_budget = (size_t)1 << 40, g_used = 0;
-bool g_capturing = false;
+bool g_capturing = false, g_sync_fails = false;
 std::map<void *, size_t> g_blocks;
 // (function statics: the library registers its kernels before this file's globals are made)
 std::map<const void *, std::string> &names()
@@ -40,6 +40,7 @@ hipStream_t g_stream;
 FAKE void fake_budget(size_t bytes) { g_budget = bytes; }
 FAKE size_t fake_used() { return g_used; }
 FAKE void fake_capturing(int on) { g_capturing = on != 0; }
+FAKE void fake_sync_fails(int on) { g_sync_fails = on != 0; }
 FAKE const char *fake_launches() { return launch_log().c_str(); }
 FAKE void fake_word(int i, long long v) { g_words[i] = v; }
 FAKE void fake_clear() { launch_log().clear(); }
@@ -154,7 +155,7 @@ FAKE hipError_t hipGetLastError()
     g_last = hipSuccess;
     return e;
 }
-FAKE hipError_t hipDeviceSynchronize() { return hipSuccess; }
+FAKE hipError_t hipDeviceSynchronize() { return g_sync_fails ? result(hipErrorStreamCaptureUnsupported) : hipSuccess; }
 FAKE hipError_t hipStreamSynchronize(hipStream_t) { return hipSuccess; }
 FAKE hipError_t hipStreamWaitEvent(hipStream_t, hipEvent_t, unsigned) { return hipSuccess; }
 FAKE hipError_t hipEventRecord(hipEvent_t, hipStream_t) { return hipSuccess; }

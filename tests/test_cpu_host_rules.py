@@ -149,6 +149,29 @@ print(fake.fake_used() - before)
     assert out.strip() == "0"
 
 
+def test_kept_blocks_wait_for_the_stream_they_were_used_on(without_device):
+    """After a change of stream a kept block may still be in use on the old one.  Where the wait for the device fails, the blocks
+    are left alone (new ones are made) until it succeeds."""
+    out = without_device(r'''
+held = malloc(1 << 20)
+n = C.c_int()
+def call():
+    assert lib.mggx_build_part_device(at(held), 1 << 20, 16, 1, None, None, None, C.byref(n)) == 0, lib.mggx_last_error()
+    return fake.fake_used()
+first = call()
+assert call() == first
+lib.mggx_set_stream(C.c_void_p(64))
+fake.fake_sync_fails(1)
+second = call()
+assert second > first, "a block that may be in use was handed out"
+fake.fake_sync_fails(0)
+assert call() == second
+lib.mggx_release_cached()
+print(fake.fake_used())
+''')
+    assert out.strip() == str(1 << 20)
+
+
 def test_no_allocation_passes_the_kept_blocks_by():
     """hipMalloc is called in one place, the helper that frees the kept blocks and asks again."""
     import glob
