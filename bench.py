@@ -148,12 +148,13 @@ def fail_on_parity(res, checks):
         sys.exit(4)
 
 
-def gather_ceiling(torch, host, ld_bytes, row_bytes, table_rows, edges, ms, core_edges=0):
+def gather_ceiling(torch, host, ld_bytes, row_bytes, table_rows, edges, ms, core_edges=0, cell_edges=0):
     """Where the feature table is cache resident the HBM peak does not bound the kernel; the L2 and, for the dense core,
     the LDS do.  Measured live with the library's yardsticks (random row reads of the kernel's geometry, no index
     stream, no reduction): from a 3 MB table (every load hits the L2), from a table of the kernel's size, and from an
     LDS tile.  The ceiling of a call is the longer of its two halves at those rates -- the core block's edges at the LDS
-    rate, the remaining edges at the all-hit L2 rate -- because the two kernels run side by side on different units."""
+    rate, the remaining edges at the all-hit L2 rate -- because the two kernels run side by side on different units.  Edges in
+    dense cells are not gathered at all: that kernel's own time is not part of this ceiling."""
     sink = torch.empty(262144, device="cuda")
     small = max(1, (3 << 20) // ld_bytes)
     table = torch.zeros(max(small, table_rows) * ld_bytes, dtype=torch.uint8, device="cuda")
@@ -173,9 +174,10 @@ def gather_ceiling(torch, host, ld_bytes, row_bytes, table_rows, edges, ms, core
         out[key + "_G_rows_per_s"] = round(rate(lambda sd: host.gather_probe(sink, table, rows, ld_bytes, row_bytes, 100_000_000, seed=sd)), 1)
     out["lds_G_rows_per_s"] = round(rate(lambda sd: host.lds_probe(sink, (row_bytes + 15) // 16 * 16, 400_000_000, seed=sd)), 1)
     out["kernel_G_rows_per_s"] = round(edges / (ms * 1e-3) / 1e9, 1)
-    t_l2 = (edges - core_edges) / (out["all_l2_hits_G_rows_per_s"] * 1e9) * 1e3
+    t_l2 = (edges - core_edges - cell_edges) / (out["all_l2_hits_G_rows_per_s"] * 1e9) * 1e3
     t_lds = core_edges / (out["lds_G_rows_per_s"] * 1e9) * 1e3
-    out["edges_from_lds"], out["edges_through_l2"] = int(core_edges), int(edges - core_edges)
+    out["edges_from_lds"], out["edges_through_l2"] = int(core_edges), int(edges - core_edges - cell_edges)
+    out["edges_in_dense_cells"] = int(cell_edges)
     out["ceiling_ms"] = round(max(t_l2, t_lds), 4)
     out["ceiling_is"] = "max(edges through the L2 / all-hit rate = %.4f ms, edges from LDS / LDS rate = %.4f ms)" % (t_l2, t_lds)
     out["frac_of_gather_ceiling"] = round(max(t_l2, t_lds) / ms, 3)
@@ -224,6 +226,7 @@ class Knobs:
 
     def __init__(self, args, search=None):
         self.ps, self.wpb, self.dist, self.blk, self.core = args.ps, args.wpb, args.dist, args.col_block_rows, args.core_rows
+        self.cells = 0  # dense cells the library chose (their plan has no size to pass: core_rows stays 0)
         self.searched_ms = None
         if search is not None:
             k, ms = search(args.ps, args.col_block_rows, args.core_rows)
@@ -242,8 +245,10 @@ class Knobs:
         if self.blk == 0:
             self.blk = 49152 if m and int(m.group(1)) > 1 else -1
         if self.core == 0:
+            m = re.search(r"cells=(\d+)", k)
+            self.cells = int(m.group(1)) if m else 0
             m = re.search(r"core=(\d+)", k)
-            self.core = int(m.group(1)) if m else -1
+            self.core = 0 if self.cells else int(m.group(1)) if m else -1
         m = re.search(r"wpb=(\d+) dist=(\d+)", k)
         if m:
             self.wpb, self.dist = (self.wpb or int(m.group(1))), (self.dist or int(m.group(2)))
@@ -253,7 +258,8 @@ class Knobs:
         return "ps=%d wpb=%d dist=%d %s%s" % (self.ps, self.wpb, self.dist,
                                               "column blocks of %d ids" % self.blk if self.blk > 0 else
                                               ("plain order" if self.blk < 0 else "order by rule"),
-                                              ", dense core of %d rows from LDS" % self.core if self.core > 0 else "")
+                                              ", dense core of %d rows from LDS" % self.core if self.core > 0 else
+                                              ", %d dense cells on the matrix cores" % self.cells if self.cells else "")
 
 
 def bench_gcn2(args, torch, host):
@@ -382,20 +388,21 @@ def bench_gcn2(args, torch, host):
     # The GCN graph's feature tables (15 / 45 MB) live in cache: algorithmic bytes / time exceeds the HBM peak and
     # bounds nothing.  What the aggregation must move through HBM at least (index lists and ids actually streamed, the
     # table once, the output once) and what the L2 / LDS sustain for its gathers are the ceilings it can be below.
-    agg2 = {"kernel": "%sk_agg (agg2 with the softmax epilogue, dim %d)" % ("k_core_sell + " if k2.core > 0 else "", out_dim), "knobs": str(k2),
+    agg2 = {"kernel": "%sk_agg (agg2 with the softmax epilogue, dim %d)" % ("k_core_sell + " if k2.core > 0 else "k_cells + " if k2.cells else "", out_dim), "knobs": str(k2),
             "avg_launch_ms": round(avg["agg2"], 4), "median_launch_ms": round(med["agg2"], 4),
             "algorithmic_bytes": b2, "algorithmic_gbps": round(b2 / (avg["agg2"] * 1e-3) / 1e9, 1),
             "algorithmic_gbps_over_hbm_peak": round(b2 / (avg["agg2"] * 1e-3) / 1e9 / HBM_PEAK_GBPS, 3),
-            **load_traffic("gcn2_agg2", args, k2.blk, k2.core)}
-    comp = agg2_core_plan_bytes if k2.core > 0 else nnz * 4        # lists + remaining ids, or the plain id stream
+            **({"traffic": None} if k2.cells else load_traffic("gcn2_agg2", args, k2.blk, k2.core))}
+    comp = agg2_core_plan_bytes if k2.core > 0 or k2.cells else nnz * 4   # lists or cells + remaining ids, or the plain id stream
     comp += V * pitch * 4 + V * out_dim * 4 + (V + 1) * 4           # the table once, the output once, the row pointers
     agg2["compulsory_hbm_bytes"] = int(comp)
     agg2["frac_compulsory"] = round(comp / (avg["agg2"] * 1e-3) / 1e9 / HBM_PEAK_GBPS, 4)
     if agg2.get("traffic"):
         agg2["frac_traffic"] = round(agg2["traffic"] / (avg["agg2"] * 1e-3) / 1e9 / HBM_PEAK_GBPS, 4)
-    agg2["gather_ceiling"] = gather_ceiling(torch, host, pitch * 4, ldo * 4, V, nnz, avg["agg2"], core_edges if k2.core > 0 else 0)
+    agg2["gather_ceiling"] = gather_ceiling(torch, host, pitch * 4, ldo * 4, V, nnz, avg["agg2"], core_edges if k2.core > 0 else 0,
+                                            core_edges if k2.cells else 0)
     extra["launches_per_forward"] = ("dense 1 + aggregation %d + dense 1 + aggregation %d (softmax inside)" %
-                                     ((5, 5) if k2.core > 0 and k2.blk > 0 else ((6, 6) if k2.core > 0 else (2, 2))))
+                                     ((5, 5) if (k2.core > 0 or k2.cells) and k2.blk > 0 else ((6, 6) if k2.core > 0 or k2.cells else (2, 2))))
     extra["agg2_cache_resident"] = agg2
     extra.update({
         "stage_ms": {k: round(v, 4) for k, v in med.items()},

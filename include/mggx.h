@@ -119,7 +119,7 @@ int mggx_set_plan_check(int level);
  * what was asked for; not counted are a counter array of 32 KB per plan and the kept blocks of mggx_release_cached. */
 typedef struct mggx_cache_stats_t {
     int64_t plans, plan_bytes;             /* cached partition plans (descriptors, row offsets) and their device bytes */
-    int64_t core_plans, core_plan_bytes;   /* dense-core plans (ranking, index lists, remaining CSR) */
+    int64_t core_plans, core_plan_bytes;   /* dense-core plans (ranking, index lists or cells, remaining CSR) */
     int64_t workspace_bytes;               /* carry buffer and per-block partial rows */
     int64_t core_scratch_bytes;            /* staged core table and the partial rows of the core kernel's workgroups */
     int64_t retired_bytes;                 /* outgrown blocks kept because a captured graph may point at them */
@@ -250,13 +250,13 @@ typedef struct mggx_agg_opts {
     const float *d_row_scale_out;/* [ub-lb] multiplies each finished sum (NULL = 1) */
     int in_dtype;                /* MGGX_F32 or MGGX_BF16 (out is always fp32) */
     int col_block_rows;          /* column-blocked order: 0 = library decides, -1 = off, > 0 = neighbor ids per block */
-    int core_rows;               /* dense core served from LDS: 0 = library decides, -1 = off, > 0 = rows in the core */
+    int core_rows;               /* dense core: 0 = library decides (from LDS, or dense cells on the matrix cores), -1 = off, > 0 = rows in the core, from LDS */
 } mggx_agg_opts;
 
 typedef struct mggx_agg_knobs {
     int ps, wpb, dist;           /* partSize / warpPerBlock / interleaved_dist */
     int col_block_rows;          /* > 0: column-blocked with that many ids per block; -1: plain order */
-    int core_rows;               /* > 0: dense core of that many rows; -1: none */
+    int core_rows;               /* > 0: dense core of that many rows; -1: none; 0 (from a search): what the library chooses, dense cells */
 } mggx_agg_knobs;
 
 /* mgg_SAG_np_div / mgg_GIN_np_div (include/neighbor_utils.cuh:787-841, 902-958;
@@ -283,6 +283,11 @@ typedef struct mggx_agg_knobs {
  * caller's stream by events inside the call (LDS-bound work beside cache-bound work).  Same result up to summation order.
  * With core_rows = 0 the library picks the size itself (possibly none) from the degree histogram: it grows the core
  * while the predicted padding of the added rows' index lists costs less than the gathers they remove.
+ * Dense cells: with core_rows = 0, where such a core would pay and most edges lie in cells of 512 rows x 192 columns (by degree rank) that
+ * hold 1,000 (rows of up to 16 columns) or 1,400 edges and more, those cells are summed on the matrix cores instead, as products of 0/1 rows
+ * with features split exactly into three bf16 parts (fp32 sums; infinities and NaN as in plain sums), on the caller's stream.
+ * mggx_last_agg_kernel reports cells=<number> and as core the side of a square of the area they cover.  A CSR that lists an edge twice
+ * among the ranked rows keeps the core from LDS.  mggx_cells_prepare builds such a plan at any size.
  * MGGX_AGG_SOFTMAX (fp32 tables): the finished rows leave as their row softmax, on every path above.
  * The partition plan of (d_ptr_l, d_ptr_r, d_col_r, rows, ps) -- and d_col_l for the column-blocked order -- is built on
  * first use and cached by pointer identity.  The arrays stay the caller's: what happens when they are rewritten in
@@ -309,6 +314,14 @@ int mggx_sag_np_div_tune(float *d_out, const void *d_in_local, const void *d_in_
                          const int *d_ptr_l, const int *d_col_l, const int *d_ptr_r, const int *d_col_r,
                          int lb, int ub, int dim, int nodes_per_pe, int ps, const mggx_agg_opts *opts,
                          mggx_agg_knobs *best, float *ms_best);
+
+/* Dense cells by request (see mggx_sag_np_div): builds (or finds) the plan of dense cells of this local-only CSR for fp32 rows of dim
+ * columns (1..64), of all cells with at least least_edges edges, and has later mggx_sag_np_div calls on the same arrays and dim that
+ * leave core_rows = 0 use it, whatever the rule says.  The arrays are those of mggx_sag_np_div.  *num_cells, *num_edges (may be
+ * NULL): cells kept and edges in them; 0 where there is none, or where the CSR lists an edge twice among its 122,880 rows of highest
+ * degree.  Synchronises; not for a first use inside a stream capture. */
+int mggx_cells_prepare(const int *d_ptr_l, const int *d_col_l, const int *d_ptr_r, const int *d_col_r, int lb, int ub, int dim,
+                       int least_edges, int64_t *num_cells, int64_t *num_edges);
 
 /* SAG_host / SAG_cuda_kernel (include/neighbor_utils.cuh:463-506, 2373-2447) and
  * the local half of SAG_host_fused_interleaved (:593-676, 2598-2688): explicit

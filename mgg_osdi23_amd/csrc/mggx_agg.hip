@@ -24,6 +24,7 @@
 // the rounds read them from there; the 16 lanes or so of a slot read the same words.
 #include <algorithm>
 #include <chrono>
+#include <cmath>
 #include <cstring>
 #include <type_traits>
 
@@ -1101,7 +1102,7 @@ struct CoreMerge {
     const float4 *sums;
     const int *rank;
     int group_rows;  // of the core beside this call (the rules look at it)
-    hipEvent_t join;
+    hipEvent_t join;  // NULL: the sums were made on the call's own stream
     bool merged;
 };
 
@@ -1192,7 +1193,7 @@ int run_agg(Plan *plan, float *d_out, const void *d_in_l, const void *d_in_r, co
     const int cpad = (dim + 3) & ~3;
     const double per_row = (double)stated / (double)(plan->rows > 0 ? plan->rows : 1);
     const long long rounds = (stated + slots - 1) / slots;
-    const bool beside_core = cm != nullptr, wpb_free = wpb == 0, dist_free = dist == 0;
+    const bool beside_core = cm && cm->join, wpb_free = wpb == 0, dist_free = dist == 0;
     if (wpb == 0) wpb = (beside_core && !blocked && slots <= 4) ? 8 : (blocked || slots > 4 || per_row < 3.0 || rounds < MANY_ROUNDS) ? 4 : 8;
     if (dist == 0) {
         if (slots <= 4 && beside_core && !blocked) dist = cm->group_rows == CORE_GROUP_ROWS_WIDE ? 8 : 4;
@@ -1352,7 +1353,7 @@ int run_agg(Plan *plan, float *d_out, const void *d_in_l, const void *d_in_r, co
         r.flags = o.flags;
         CoreMergeArgs cma{nullptr, nullptr};
         if (cm) {
-            MGGX_HIP(hipStreamWaitEvent(st.stream, cm->join, 0));
+            if (cm->join) MGGX_HIP(hipStreamWaitEvent(st.stream, cm->join, 0));
             cma = CoreMergeArgs{cm->sums, cm->rank};
             cm->merged = true;
         }
@@ -1397,17 +1398,33 @@ constexpr int DEFAULT_BLOCK_ROWS = 48 * 1024;  // neighbor ids per column block 
 
 // A column-blocked plan re-reads and re-writes a partial output row per block: it pays off when rows are long.
 constexpr int MIN_NEIGHBORS_PER_ROW_AND_BLOCK = 20;
-bool blocking_eligible(const GraphInfo &g, int block_rows)
+// (Beside dense cells, rows of more than 16 columns: 233 K nodes, 52 M neighbors, 15 M of them left, 13 per row and block: width 41 493 us in
+// this order, 546 in plain order; at width 16 208 and 187.)
+constexpr int MIN_NEIGHBORS_BESIDE_CELLS = 10;
+bool blocking_eligible(const GraphInfo &g, int block_rows, int least = MIN_NEIGHBORS_PER_ROW_AND_BLOCK)
 {
     if (g.nnz_r > 0 || g.rows < 2 * (long long)block_rows) return false;
     const long long blocks = ((long long)g.rows + block_rows - 1) / block_rows;
-    return g.nnz_l >= MIN_NEIGHBORS_PER_ROW_AND_BLOCK * blocks * (long long)g.rows;
+    return g.nnz_l >= least * blocks * (long long)g.rows;
 }
 
 struct Knobs {
     int ps, wpb, dist, block_rows;  // block_rows: > 0 column-blocked, -1 plain
     int core_rows;                  // > 0: that many highest-degree rows form a dense core served from LDS, -1: none
+    int cells = 0;                  // > 0: cells of at least that many edges on the matrix cores ...
+    double cells_share = 0.0;       // ... where they hold this share of the edges
 };
+
+// Dense cells (mggx_cells.hip) where a core from LDS would pay and they hold most of the edges.  Least edges of a cell: what it costs
+// over what an edge costs the gather kernel beside it (233 K nodes, 228 M neighbors: 5.1 ns and 7.3 ps at width 16, 14.4 and 18 at 41; the
+// optimum is flat: 700 to 1,400 edges at width 16 and 700 to 2,000 at 41 and 64 are within 2 %).  Least share: graphs of 50 to 233 K nodes
+// and mean degrees of 220 to 970 have 69 to 92 % of their edges in such cells and gain 5 to 35 % over the core from LDS at widths 16, 41
+// and 64 (100 K nodes, 51 M neighbors: 172 -> 124, 403 -> 276, 445 -> 328 us); 500 K to 1.5 M nodes of mean degree 57 to 168 have 38
+// to 66 % and lose up to 17 % (1 M nodes, 168 M neighbors, width 64: 2,459 -> 2,797), 233 K nodes of a flatter RMAT (a = 0.45) have 42 to 53 %,
+// gain 4 % at width 16 and lose 3 % at 64.  The degrees alone say which graphs to count the cells of.
+constexpr int CELLS_LEAST_NARROW = 1000, CELLS_LEAST = 1400;
+constexpr double CELLS_SHARE = 0.67, CELLS_SHARE_BY_DEGREES = 0.5;
+int cells_least_edges(int dim) { return dim <= 16 ? CELLS_LEAST_NARROW : CELLS_LEAST; }
 
 // The dense-core path pays for a plan and partial rows: worth considering on a local-only fp32 CSR with many rows
 // beyond the core and a mean degree of 16 or more (on a power-law graph of mean degree 50 the 32 Ki highest-degree rows
@@ -1428,7 +1445,7 @@ int resolve_knobs(GraphInfo &g, int dim, int dtype, int ps, int wpb, int dist, i
         if (e.dim == dim && e.dtype == dtype) t = &e;
     Knobs k{ps, wpb, dist, block_rows, core_rows};
     if (t && (ps == 0 || ps == t->ps) && wpb == 0 && dist == 0 && block_rows == 0 && core_rows == 0) {
-        *out = Knobs{t->ps, t->wpb, t->dist, t->block_rows, t->core_rows};
+        *out = Knobs{t->ps, t->wpb, t->dist, t->block_rows, t->core_rows, t->cells, t->cells ? CELLS_SHARE : 0.0};
         return MGGX_OK;
     }
     if (k.ps == 0) k.ps = 16;
@@ -1439,6 +1456,15 @@ int resolve_knobs(GraphInfo &g, int dim, int dtype, int ps, int wpb, int dist, i
             const int rc = predict_core_rows(g, dim, table_bytes, k.block_rows, MIN_NEIGHBORS_PER_ROW_AND_BLOCK, &k.core_rows);
             if (rc) return rc;
         }
+        if (k.core_rows > 0 && predicted_cells_share(g, cells_least_edges(dim)) >= CELLS_SHARE_BY_DEGREES) {
+            k.cells = cells_least_edges(dim);
+            k.cells_share = CELLS_SHARE;
+        }
+        for (const GraphInfo::CellsAsked &c : g.cells_asked)
+            if (c.dim == dim && dtype == MGGX_F32) {
+                k.cells = c.least;
+                k.cells_share = 0.0;
+            }
     }
     *out = k;
     return MGGX_OK;
@@ -1450,57 +1476,76 @@ int run_knobs(const GraphInfo &g, const Knobs &k, float *d_out, const void *d_in
 {
     Plan *plan = nullptr;
     int rc;
-    if (k.core_rows > 0 && ub - lb >= 1024 && g.nnz_r == 0 && g.nnz_l > 0 && d_col_l && o.in_dtype == MGGX_F32 && dim >= 1 && dim <= 64 && d_out &&
-        d_in_local) {
-        CorePlan *cp = nullptr;
+    const bool core_call = g.nnz_r == 0 && g.nnz_l > 0 && d_col_l && o.in_dtype == MGGX_F32 && dim >= 1 && dim <= 64 && d_out && d_in_local;
+    CorePlan *cp = nullptr;
+    if (k.cells > 0 && core_call) {
+        rc = cells_plan_get(d_ptr_l, d_col_l, ub - lb, lb, dim, k.cells, g.nnz_l, k.cells_share, g.serial, &cp);
+        if (rc) return rc;
+        if (cp->unsuitable) cp = nullptr;  // the core from LDS, if one was asked for as well
+    }
+    if (!cp && k.core_rows > 0 && core_call && ub - lb >= 1024) {
         rc = core_plan_get(d_ptr_l, d_col_l, ub - lb, lb, k.core_rows, core_group_rows((dim + 3) / 4, std::min(k.core_rows, ub - lb)), g.serial, &cp);
         if (rc) return rc;
-        if (!cp->unsuitable) {
-            // The core block is bound by the LDS, the rest of the CSR by the caches: they run side by side.  The core's sums
-            // go to partial rows on a second stream while the rest of the CSR runs here.  Where that rest ends in the finish
-            // kernel of a column-blocked plan, the same kernel joins the side stream, adds the core's partial rows and
-            // applies the caller's epilogue; otherwise the rest runs with the epilogue except its post-operations (ReLU,
-            // softmax), and k_core_finish adds the partial rows (times the row scale) and applies those last.
-            const long long ld_in = o.ld_in ? o.ld_in : dim, ld_out = o.ld_out ? o.ld_out : dim;
-            if (ld_in < dim || ld_out < dim) return fail(MGGX_EINVAL, "aggregation: row stride smaller than dim");
-            State &st0 = state();
-            hipStream_t side;
-            hipEvent_t fork, join;
+        if (cp->unsuitable) cp = nullptr;
+    }
+    if (cp) {
+        // Index lists: the core block is bound by the LDS, the rest of the CSR by the caches, and they run side by side, the core's
+        // sums on a second stream.  Dense cells: they hold the chip's registers, so they run first, on this stream (side by side
+        // with the rest: 405 us instead of 385 at width 16, 950 instead of 967 at width 41, 233 K nodes).
+        // Where the rest ends in the finish kernel of a column-blocked plan, the same kernel joins the side stream, adds the core's
+        // sums and applies the caller's epilogue; otherwise the rest runs with the epilogue except its post-operations (ReLU,
+        // softmax), and k_core_finish adds the sums (times the row scale) and applies those last.
+        const long long ld_in = o.ld_in ? o.ld_in : dim, ld_out = o.ld_out ? o.ld_out : dim;
+        if (ld_in < dim || ld_out < dim) return fail(MGGX_EINVAL, "aggregation: row stride smaller than dim");
+        State &st = state();
+        const float *table = static_cast<const float *>(d_in_local);
+        hipStream_t side = st.stream;
+        hipEvent_t fork = nullptr, join = nullptr;
+        const float4 *sums = nullptr;
+        hipError_t er = hipSuccess;
+        if (cp->cells) {
+            rc = cells_sums(cp, table, dim, ld_in, gate, st.stream, &sums);
+            if (rc) return rc;
+        } else {
             rc = core_side_stream(&side, &fork, &join);
             if (rc) return rc;
-            rc = run_core_stage(cp, static_cast<const float *>(d_in_local), dim, ld_in, gate, st0.stream);
+            rc = run_core_stage(cp, table, dim, ld_in, gate, st.stream);
             if (rc) return rc;
-            MGGX_HIP(hipEventRecord(fork, st0.stream));
+            MGGX_HIP(hipEventRecord(fork, st.stream));
             MGGX_HIP(hipStreamWaitEvent(side, fork, 0));
             rc = run_core_sums(cp, dim, gate, side);
-            const hipError_t er = hipEventRecord(join, side);
-            int rc2 = MGGX_OK;
-            GraphInfo *gr = nullptr;
-            CoreMerge cm{nullptr, cp->d_rank, cp->group_rows, join, false};
-            if (!rc) rc2 = core_row_sums(cp, dim, &cm.sums);
-            if (!rc && !rc2) rc2 = graph_info(cp->d_rem_ptr, nullptr, cp->d_rem_col, nullptr, ub - lb, true, &gr);
-            if (!rc && !rc2 && er == hipSuccess) {
-                Knobs k2 = k;
-                k2.core_rows = -1;
-                if (k2.block_rows > 0 && !blocking_eligible(*gr, k2.block_rows)) k2.block_rows = -1;
-                rc2 = run_knobs(*gr, k2, d_out, d_in_local, nullptr, cp->d_rem_ptr, cp->d_rem_col, nullptr, nullptr, lb, ub, dim, o, gate, &cm);
-            }
-            // the caller's stream takes the side stream back in whatever happened, so no work of this call outlives it unordered
-            const hipError_t ew = er == hipSuccess ? (cm.merged ? hipSuccess : hipStreamWaitEvent(st0.stream, join, 0)) : er;
-            if (rc) return rc;
-            if (rc2) return rc2;
-            if (ew != hipSuccess) return fail(MGGX_EHIP, "aggregation: joining the side stream: %s", hipGetErrorString(ew));
-            if (!cm.merged) {
-                rc = run_core_finish(cp, d_out, dim, ld_out, o.d_row_scale_out, (o.flags & MGGX_AGG_RELU) ? 1 : 0, (o.flags & MGGX_AGG_SOFTMAX) ? 1 : 0, gate,
-                                     st0.stream);
-                if (rc) return rc;
-            }
-            State &st = state();
-            const size_t n = strlen(st.last_kernel);
-            snprintf(st.last_kernel + n, sizeof(st.last_kernel) - n, " core=%d core_nnz=%lld rem_nnz=%lld%s", cp->core, (long long)cp->core_nnz,
-                     (long long)cp->rem_nnz, cm.merged ? " merged_finish" : "");
-            return MGGX_OK;
+            er = hipEventRecord(join, side);
         }
+        int rc2 = MGGX_OK;
+        GraphInfo *gr = nullptr;
+        if (!rc && !cp->cells) rc2 = core_row_sums(cp, dim, &sums);
+        CoreMerge cm{sums, cp->d_rank, cp->group_rows, join, false};
+        if (!rc && !rc2) rc2 = graph_info(cp->d_rem_ptr, nullptr, cp->d_rem_col, nullptr, ub - lb, true, &gr);
+        if (!rc && !rc2 && er == hipSuccess) {
+            Knobs k2 = k;
+            k2.core_rows = -1;
+            k2.cells = 0;
+            if (k2.block_rows > 0 && !blocking_eligible(*gr, k2.block_rows, cp->cells > 1 ? MIN_NEIGHBORS_BESIDE_CELLS : MIN_NEIGHBORS_PER_ROW_AND_BLOCK)) k2.block_rows = -1;
+            rc2 = run_knobs(*gr, k2, d_out, d_in_local, nullptr, cp->d_rem_ptr, cp->d_rem_col, nullptr, nullptr, lb, ub, dim, o, gate, &cm);
+        }
+        // the caller's stream takes the side stream back in whatever happened, so no work of this call outlives it unordered
+        const hipError_t ew = er == hipSuccess && join ? (cm.merged ? hipSuccess : hipStreamWaitEvent(st.stream, join, 0)) : er;
+        if (rc) return rc;
+        if (rc2) return rc2;
+        if (ew != hipSuccess) return fail(MGGX_EHIP, "aggregation: joining the side stream: %s", hipGetErrorString(ew));
+        if (!cm.merged) {
+            rc = run_core_finish(cp, sums, d_out, dim, ld_out, o.d_row_scale_out, (o.flags & MGGX_AGG_RELU) ? 1 : 0, (o.flags & MGGX_AGG_SOFTMAX) ? 1 : 0, gate,
+                                 st.stream);
+            if (rc) return rc;
+        }
+        const size_t n = strlen(st.last_kernel);
+        snprintf(st.last_kernel + n, sizeof(st.last_kernel) - n, " core=%d core_nnz=%lld rem_nnz=%lld%s", cp->cells ? cp->side : cp->core, (long long)cp->core_nnz,
+                 (long long)cp->rem_nnz, cm.merged ? " merged_finish" : "");
+        if (cp->cells) {
+            const size_t m = strlen(st.last_kernel);
+            snprintf(st.last_kernel + m, sizeof(st.last_kernel) - m, " cells=%d", cp->ncells);
+        }
+        return MGGX_OK;
     }
     if (k.block_rows > 0 && g.nnz_r == 0 && d_col_l && ub - lb >= 2 * (long long)k.block_rows) {
         rc = plan_get_blocked(d_ptr_l, d_col_l, ub - lb, lb, k.ps, k.block_rows, g.serial, &plan);
@@ -1551,6 +1596,33 @@ MGGX_EXPORT int mggx_sag_np_div(float *d_out, const void *d_in_local, const void
                              (unsigned long long)(ub - lb) * (unsigned long long)(o.ld_in ? o.ld_in : dim) * (o.in_dtype == MGGX_BF16 ? 2 : 4), &k);
     if (rc) return rc;
     return mggx::run_knobs(*g, k, d_out, d_in_local, d_in_remote, d_ptr_l, d_col_l, d_ptr_r, d_col_r, lb, ub, dim, o, gate);
+}
+
+MGGX_EXPORT int mggx_cells_prepare(const int *d_ptr_l, const int *d_col_l, const int *d_ptr_r, const int *d_col_r, int lb, int ub, int dim, int least_edges,
+                                   int64_t *num_cells, int64_t *num_edges)
+{
+    int rc = mggx::ensure_init();
+    if (rc) return rc;
+    if (!d_ptr_l || !d_col_l || ub <= lb || dim < 1 || dim > 64 || least_edges < 1)
+        return fail(MGGX_EINVAL, "cells_prepare: NULL CSR, rows [%d,%d), dim %d outside 1..64 or least_edges %d", lb, ub, dim, least_edges);
+    rc = mggx::stale_poll();
+    if (rc) return rc;
+    mggx::GraphInfo *g = nullptr;
+    rc = mggx::graph_info(d_ptr_l, d_ptr_r, d_col_l, d_col_r, ub - lb, false, &g);
+    if (rc) return rc;
+    if (g->nnz_r > 0 || g->nnz_l < 1) return fail(MGGX_EINVAL, "cells_prepare: %lld local and %lld remote edges (local only)", (long long)g->nnz_l, (long long)g->nnz_r);
+    mggx::CorePlan *p = nullptr;
+    rc = mggx::cells_plan_get(d_ptr_l, d_col_l, ub - lb, lb, dim, least_edges, g->nnz_l, 0.0, g->serial, &p);
+    if (rc) return rc;
+    if (num_cells) *num_cells = p->unsuitable ? 0 : p->ncells;
+    if (num_edges) *num_edges = p->unsuitable ? 0 : p->core_nnz;
+    for (mggx::GraphInfo::CellsAsked &c : g->cells_asked)
+        if (c.dim == dim) {
+            c.least = least_edges;
+            return MGGX_OK;
+        }
+    g->cells_asked.push_back({dim, least_edges});
+    return MGGX_OK;
 }
 
 MGGX_EXPORT int mggx_sag_np_div_tune(float *d_out, const void *d_in_local, const void *d_in_remote, const int *d_ptr_l,
@@ -1686,9 +1758,9 @@ MGGX_EXPORT int mggx_sag_np_div_tune(float *d_out, const void *d_in_local, const
                     (st.plan_build_ms + st.core_plan_build_ms - build_ms0);
     bool found = false;
     for (mggx::GraphInfo::Tuned &t : g->tuned)
-        if (t.dim == dim && t.dtype == o.in_dtype) { t.ps = bk.ps; t.wpb = bk.wpb; t.dist = bk.dist; t.block_rows = bk.block_rows; t.core_rows = bk.core_rows; found = true; }
-    if (!found) g->tuned.push_back({dim, o.in_dtype, bk.ps, bk.wpb, bk.dist, bk.block_rows, bk.core_rows});
-    if (best_out) { best_out->ps = bk.ps; best_out->wpb = bk.wpb; best_out->dist = bk.dist; best_out->col_block_rows = bk.block_rows; best_out->core_rows = bk.core_rows; }
+        if (t.dim == dim && t.dtype == o.in_dtype) { t.ps = bk.ps; t.wpb = bk.wpb; t.dist = bk.dist; t.block_rows = bk.block_rows; t.core_rows = bk.core_rows; t.cells = bk.cells; found = true; }
+    if (!found) g->tuned.push_back({dim, o.in_dtype, bk.ps, bk.wpb, bk.dist, bk.block_rows, bk.core_rows, bk.cells});
+    if (best_out) { best_out->ps = bk.ps; best_out->wpb = bk.wpb; best_out->dist = bk.dist; best_out->col_block_rows = bk.block_rows; best_out->core_rows = bk.cells ? 0 : bk.core_rows; }
     if (ms_best) *ms_best = best;
     return MGGX_OK;
 }

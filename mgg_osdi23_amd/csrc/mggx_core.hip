@@ -589,9 +589,11 @@ void core_plan_free_arrays(CorePlan *p)
             retire_block(q, left);
             left = 0;
         } else {
-            (void)hipFree(q);
+            dev_free(q);
         }
     };
+    drop(p->d_words);
+    drop(p->d_cell_tile);
     drop(p->d_order);
     drop(p->d_rank);
     drop(p->d_blk_off);
@@ -605,6 +607,8 @@ void core_plan_free_arrays(CorePlan *p)
     p->d_order = p->d_rank = p->d_rem_ptr = p->d_rem_col = nullptr;
     p->d_blk_off = nullptr;
     p->d_idx = nullptr;
+    p->d_words = nullptr;
+    p->d_cell_tile = nullptr;
     p->cuts.clear();
 }
 
@@ -750,14 +754,16 @@ static int core_plan_build_device(CorePlan *p, int tc)
     return MGGX_OK;
 }
 
-int core_plan_get(const int *d_ptr_l, const int *d_col_l, int rows, int lb, int core, int group_rows, int graph_serial, CorePlan **out)
+static int find_or_build(const int *d_ptr_l, const int *d_col_l, int rows, int lb, int core, int group_rows, int cells, int dim, long long nnz, double least_share,
+                         int graph_serial, CorePlan **out)
 {
     State &s = state();
     for (size_t i = 0; i < s.cores.size(); ++i) {
         CorePlan *p = s.cores[i];
         // a plan belongs to the graph record it was built under (see drop_plans_of_record): it carries its own copy of that
         // graph's remaining CSR and index lists, and a later record of the same addresses may stand for another graph
-        if (p->d_ptr_l == d_ptr_l && p->d_col_l == d_col_l && p->rows == rows && p->lb == lb && p->asked == core && p->group_rows == group_rows && p->graph_serial == graph_serial) {
+        if (p->d_ptr_l == d_ptr_l && p->d_col_l == d_col_l && p->rows == rows && p->lb == lb && p->asked == core && p->group_rows == group_rows &&
+            p->cells == cells && p->graph_serial == graph_serial) {
             if (i + 1 != s.cores.size()) {  // most recently used last
                 s.cores.erase(s.cores.begin() + (long)i);
                 s.cores.push_back(p);
@@ -779,8 +785,13 @@ int core_plan_get(const int *d_ptr_l, const int *d_col_l, int rows, int lb, int 
     p->lb = lb;
     p->asked = core;
     p->group_rows = group_rows;
+    p->cells = cells;
     p->graph_serial = graph_serial;
-    int rc = core_plan_build_device(p, CORE_TC);
+    int rc = cells ? cells_plan_build(p, dim, nnz, least_share) : core_plan_build_device(p, CORE_TC);
+    if (!rc && p->unsuitable) {  // what was built on the way is not needed to remember that
+        (void)hipStreamSynchronize(s.stream);
+        core_plan_free_arrays(p);
+    }
     if (rc) {
         core_plan_free_arrays(p);
         delete p;
@@ -799,6 +810,16 @@ int core_plan_get(const int *d_ptr_l, const int *d_col_l, int rows, int lb, int 
     s.core_plan_build_ms += std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count();
     *out = p;
     return MGGX_OK;
+}
+
+int core_plan_get(const int *d_ptr_l, const int *d_col_l, int rows, int lb, int core, int group_rows, int graph_serial, CorePlan **out)
+{
+    return find_or_build(d_ptr_l, d_col_l, rows, lb, core, group_rows, 0, 0, 0, 0.0, graph_serial, out);
+}
+
+int cells_plan_get(const int *d_ptr_l, const int *d_col_l, int rows, int lb, int dim, int least, long long nnz, double least_share, int graph_serial, CorePlan **out)
+{
+    return find_or_build(d_ptr_l, d_col_l, rows, lb, least, CORE_GROUP_ROWS, (dim + 15) / 16, dim, nnz, least_share, graph_serial, out);
 }
 
 // The workgroups of the LDS kernel for rows of n4 16-byte pieces: every row group's tiles cut into runs of about
@@ -868,17 +889,10 @@ static int core_cut(CorePlan *p, int n4, const CorePlan::Cut **out)
     return MGGX_OK;
 }
 
-// Scratch of the dense-core path: the staged core table, then one partial row per workgroup of the LDS kernel and row of its group.
-static int core_scratch(CorePlan *p, int n4, v4f **tab, v4f **partial, const CorePlan::Cut **cut_out = nullptr)
+int core_workspace(size_t bytes, void **p)
 {
     State &s = state();
-    const CorePlan::Cut *cut = nullptr;
-    const int rc_cut = core_cut(p, n4, &cut);
-    if (rc_cut) return rc_cut;
-    if (cut_out) *cut_out = cut;
-    const size_t tab_bytes = (tab_stride(p->core) * n4 * sizeof(v4f) + 255) & ~(size_t)255;
-    const size_t part_bytes = (size_t)cut->nwg * p->group_rows * n4 * sizeof(v4f);
-    if (tab_bytes + part_bytes > s.core_ws_bytes) {
+    if (bytes > s.core_ws_bytes) {
         if (capturing()) return fail(MGGX_EINVAL, "core: the scratch block would have to grow inside a stream capture; run the largest call once outside it first");
         MGGX_HIP(hipDeviceSynchronize());  // both streams may still use the old block
         if (s.core_ws) {
@@ -892,12 +906,28 @@ static int core_scratch(CorePlan *p, int n4, v4f **tab, v4f **partial, const Cor
         }
         s.core_ws = nullptr;
         s.core_ws_bytes = 0;
-        if (device_malloc(&s.core_ws, tab_bytes + part_bytes) != hipSuccess) return fail(MGGX_ENOMEM, "core: %zu bytes of scratch", tab_bytes + part_bytes);
-        s.core_ws_bytes = tab_bytes + part_bytes;
+        if (device_malloc(&s.core_ws, bytes) != hipSuccess) return fail(MGGX_ENOMEM, "core: %zu bytes of scratch", bytes);
+        s.core_ws_bytes = bytes;
     }
     if (!s.core_ws_captured && capturing()) s.core_ws_captured = true;
-    *tab = static_cast<v4f *>(s.core_ws);
-    *partial = reinterpret_cast<v4f *>(static_cast<char *>(s.core_ws) + tab_bytes);
+    *p = s.core_ws;
+    return MGGX_OK;
+}
+
+// Scratch of the dense-core path: the staged core table, then one partial row per workgroup of the LDS kernel and row of its group.
+static int core_scratch(CorePlan *p, int n4, v4f **tab, v4f **partial, const CorePlan::Cut **cut_out = nullptr)
+{
+    void *ws = nullptr;
+    const CorePlan::Cut *cut = nullptr;
+    const int rc_cut = core_cut(p, n4, &cut);
+    if (rc_cut) return rc_cut;
+    if (cut_out) *cut_out = cut;
+    const size_t tab_bytes = (tab_stride(p->core) * n4 * sizeof(v4f) + 255) & ~(size_t)255;
+    const size_t part_bytes = (size_t)cut->nwg * p->group_rows * n4 * sizeof(v4f);
+    const int rc = core_workspace(tab_bytes + part_bytes, &ws);
+    if (rc) return rc;
+    *tab = static_cast<v4f *>(ws);
+    *partial = reinterpret_cast<v4f *>(static_cast<char *>(ws) + tab_bytes);
     return MGGX_OK;
 }
 
@@ -943,20 +973,16 @@ int run_core_sums(CorePlan *p, int dim, const Gate &gate, hipStream_t stream)
 }
 
 // out += scale * (the core block's sum of the row, as k_core_reduce left it), then the ReLU and / or the row softmax if asked for, on `stream`.
-int run_core_finish(CorePlan *p, float *d_out, int dim, long long ld_out, const float *d_row_scale, int relu, int softmax, const Gate &gate,
+int run_core_finish(CorePlan *p, const float4 *sums, float *d_out, int dim, long long ld_out, const float *d_row_scale, int relu, int softmax, const Gate &gate,
                     hipStream_t stream)
 {
     const int n4 = (dim + 3) / 4;
-    v4f *tab = nullptr, *partial = nullptr;
-    const CorePlan::Cut *cut = nullptr;
-    int rc = core_scratch(p, n4, &tab, &partial, &cut);  // sized by run_core_sums already: only hands the pointers out
-    if (rc) return rc;
     const int all_rows = (relu || softmax) ? 1 : 0;
     int g_shift = 0;
     while ((1 << g_shift) < n4) ++g_shift;
     const long long n = (long long)(all_rows ? p->rows : p->core) << g_shift;
     const int vec_out = ld_out % 4 == 0 && (reinterpret_cast<uintptr_t>(d_out) & 15u) == 0;
-    k_core_finish<<<dim3((unsigned)((n + 255) / 256)), dim3(256), 0, stream>>>(d_out, tab, p->d_rank, p->d_order, d_row_scale, p->rows, dim, ld_out,
+    k_core_finish<<<dim3((unsigned)((n + 255) / 256)), dim3(256), 0, stream>>>(d_out, reinterpret_cast<const v4f *>(sums), p->d_rank, p->d_order, d_row_scale, p->rows, dim, ld_out,
                                                                                 p->core, g_shift, relu, softmax, all_rows, vec_out, gate);
     MGGX_LAUNCH_CHECK("k_core_finish");
     return MGGX_OK;
@@ -1179,6 +1205,27 @@ int predict_core_rows(GraphInfo &g, int dim, unsigned long long table_bytes, int
     }
     g.predicted.push_back({dim, block_rows, table_bytes, *core_rows});
     return MGGX_OK;
+}
+
+double predicted_cells_share(const GraphInfo &g, int least)
+{
+    if (!g.have_profile || g.nnz_l <= 0) return 0.0;
+    const size_t slices = std::min<size_t>(g.slice_deg.size(), 1920);
+    std::vector<double> group, tile;  // degree sums of 512 rows and of 192 columns
+    for (size_t s = 0; s < slices; ++s) {
+        if (s % 8 == 0) group.push_back(0.0);
+        if (s % 3 == 0) tile.push_back(0.0);
+        group.back() += g.slice_deg[s];
+        tile.back() += g.slice_deg[s];
+    }
+    double in_cells = 0.0;
+    for (const double dg : group)
+        for (const double dt : tile) {
+            const double edges = std::min(dg * dt / (double)g.nnz_l, 512.0 * 192.0);
+            if (edges < least) break;  // the tiles are in falling order
+            in_cells += edges;
+        }
+    return in_cells / (double)g.nnz_l;
 }
 
 }  // namespace mggx

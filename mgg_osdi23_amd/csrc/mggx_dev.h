@@ -169,12 +169,20 @@ struct CorePlan {
     struct Cut {
         int target = 0;            // workgroups asked for
         int nwg = 0;               // workgroups made
+        int slots = 0;             // plans of cells: slots of partial rows
         int4 *d_wgs = nullptr;     // [nwg] {row group, first tile, end tile, slot of the partial rows}, in launch order
         int *d_wg_base = nullptr;  // [core / CORE_GROUP_ROWS + 1] first slot of every row group
     };
     std::vector<Cut> cuts;
     std::vector<int> work;    // [core / CORE_GROUP_ROWS][ntiles] list chunks of a row group in a tile (host copy)
     long long total_chunks = 0;
+    // Plans of dense cells (mggx_cells.hip) instead of index lists: cells > 0 is their row width in groups of 16 columns (part of the
+    // key; asked = least edges of a cell); core = ranked rows that have cells, ntiles = column tiles that have, one cut.
+    int cells = 0;
+    int ncells = 0;
+    int side = 0;                 // of a square as large as the part of the (row, column) plane the cells cover
+    unsigned *d_words = nullptr;  // [ncells][4096]
+    int *d_cell_tile = nullptr;   // [ncells], row group by row group
     bool unsuitable = false;  // no core of whole units fits, or the ids do not allow it
     bool pinned = false;      // used inside a stream capture: its device blocks outlive the cache entry (retired, not freed)
     int graph_serial = 0;     // as Plan::graph_serial
@@ -194,13 +202,15 @@ struct GraphInfo {
     bool have_profile = false;
     struct Predicted { int dim; int block_rows; unsigned long long table_bytes; int core_rows; };
     std::vector<Predicted> predicted;  // what the cost model said for a row width (evaluated once, a millisecond of host time)
+    struct CellsAsked { int dim; int least; };
+    std::vector<CellsAsked> cells_asked;  // mggx_cells_prepare
     bool internal = false;  // arrays owned by the library (the remainder CSR of a dense-core plan): no content check
     bool pinned = false;    // used inside a stream capture: never evicted
     int serial = 0;         // unique per record: plans remember the record they were built under
     Guard guard;
     int64_t nnz_l = 0, nnz_r = 0;
     // knobs measured best by mggx_sag_np_div_tune for a row width and element type; used where a call passes 0
-    struct Tuned { int dim, dtype, ps, wpb, dist, block_rows, core_rows; };
+    struct Tuned { int dim, dtype, ps, wpb, dist, block_rows, core_rows, cells; };
     std::vector<Tuned> tuned;
 };
 
@@ -318,11 +328,21 @@ int predict_core_rows(GraphInfo &g, int dim, unsigned long long table_bytes, int
 void core_plan_free(CorePlan *p);
 int run_core_stage(CorePlan *p, const float *d_in, int dim, long long ld_in, const Gate &gate, hipStream_t stream);
 int run_core_sums(CorePlan *p, int dim, const Gate &gate, hipStream_t stream);
-int run_core_finish(CorePlan *p, float *d_out, int dim, long long ld_out, const float *d_row_scale, int relu, int softmax, const Gate &gate,
+int run_core_finish(CorePlan *p, const float4 *sums, float *d_out, int dim, long long ld_out, const float *d_row_scale, int relu, int softmax, const Gate &gate,
                     hipStream_t stream);
 // Where run_core_sums leaves the core block's sums: [slot][row in its group][ceil(dim/4)] float4, and the first slot of
 // every row group (CorePlan::Cut::d_wg_base of the cut used for this width).
 int core_row_sums(CorePlan *p, int dim, const float4 **sums);
+// Grow-only scratch of the dense-core paths (both streams of a call use it).
+int core_workspace(size_t bytes, void **p);
+// Dense cells on the matrix cores (mggx_cells.hip): the plan of a row width (found in or added to the list of core plans), and the sums
+// of its cells by rank, on `stream`, for run_core_finish or the finishing kernel of a column-blocked plan to add.
+int cells_plan_get(const int *d_ptr_l, const int *d_col_l, int rows, int lb, int dim, int least, long long nnz, double least_share, int graph_serial, CorePlan **out);
+int cells_plan_build(CorePlan *p, int dim, long long nnz, double least_share);
+int cells_sums(const CorePlan *p, const float *d_in, int dim, long long ld_in, const Gate &gate, hipStream_t stream, const float4 **d_sums);
+// What the degrees alone say of the share of a CSR's edges that lies in cells of at least `least` edges (after predict_core_rows, which
+// fetches the degree profile).
+double predicted_cells_share(const GraphInfo &g, int least);
 // Second stream of the dense-core path (created on first use, default priority) and the two events that fork and join it.
 int core_side_stream(hipStream_t *stream, hipEvent_t *fork, hipEvent_t *join);
 

@@ -126,7 +126,7 @@ def held_out_table(args):
         host.forget(w["ptr_l"])
         import re
         m = re.search(r"core=(\d+)", rule_kernel)
-        predicted = int(m.group(1)) if m else -1
+        predicted = int(m.group(1)) if m and "cells=" not in rule_kernel else -1  # (cells have no size to pass)
         best_core = (rule if predicted < 0 else 1e30, -1)
         if not len(w["host"]["col_r"]):
             for K in (-1, 8192, 16384, 24576, 32768, 40960, 49152, 65536, 81920, 98304):

@@ -61,7 +61,7 @@ EXPORTS = [
     "mggx_timer_create", "mggx_timer_start", "mggx_timer_stop", "mggx_timer_elapsed_ms", "mggx_timer_destroy",
     "mggx_release_cached", "mggx_forget", "mggx_set_plan_check", "mggx_cache_stats", "mggx_range_partition", "mggx_split_csr", "mggx_compact_remote", "mggx_build_part", "mggx_core_layout_build", "mggx_core_layout_fetch", "mggx_core_layout_device", "mggx_convert_probe", "mggx_graph_read",
     "mggx_graph_write", "mggx_mtx_read", "mggx_gen_rmat", "mggx_gen_er", "mggx_gen_fetch", "mggx_fill_normal",
-    "mggx_fill_uniform", "mggx_build_part_device", "mggx_split_csr_device", "mggx_compact_remote_device", "mggx_edgelist_to_bin", "mggx_sag_np_div", "mggx_sag_np_div_tune", "mggx_sag_parts", "mggx_sag_parts_static", "mggx_mlp2_xw", "mggx_spmm",
+    "mggx_fill_uniform", "mggx_build_part_device", "mggx_split_csr_device", "mggx_compact_remote_device", "mggx_edgelist_to_bin", "mggx_sag_np_div", "mggx_sag_np_div_tune", "mggx_cells_prepare", "mggx_sag_parts", "mggx_sag_parts_static", "mggx_mlp2_xw", "mggx_spmm",
     "mggx_dense_xw", "mggx_dense_xw_bf16", "mggx_softmax_rows", "mggx_cast_f32_to_bf16", "mggx_copy_bytes", "mggx_copy_bytes_nt", "mggx_gather_probe", "mggx_lds_probe", "mggx_gather_rows", "mggx_last_agg_kernel", "mggx_set_gather_addressing",
 ]
 
@@ -547,3 +547,11 @@ def core_layout_device(d_ptr, d_col, rows: int, lb: int, core_rows: int):
                                          blk_off.ctypes.data_as(C.c_void_p), idx.ctypes.data_as(C.c_void_p), _iptr(rem_ptr), _iptr(rem_col)))
     return dict(core=core, ntiles=core // 256, core_nnz=int(sizes[4]), order=order, rank=rank, blk_off=blk_off, idx=idx,
                 rem_ptr=rem_ptr, rem_col=rem_col)
+
+
+def cells_prepare(d_ptr_l, d_col_l, d_ptr_r, d_col_r, lb: int, ub: int, dim: int, least_edges: int):
+    """Plan of dense cells for later aggregations of this width (device tensors) -> (cells, edges in them)."""
+    cells, edges = C.c_int64(), C.c_int64()
+    _pin(d_ptr_l, d_col_l, d_ptr_r, d_col_r)
+    _check(lib().mggx_cells_prepare(_dptr(d_ptr_l), _dptr(d_col_l), _dptr(d_ptr_r), _dptr(d_col_r), lb, ub, dim, least_edges, C.byref(cells), C.byref(edges)))
+    return cells.value, edges.value
