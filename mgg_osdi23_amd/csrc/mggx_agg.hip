@@ -17,7 +17,8 @@
 //   wavefronts a row that crosses wavefronts is finished through LDS
 //   workgroups a row that crosses workgroups leaves two partial rows in a
 //              carry buffer; a small second kernel sums them in a fixed order
-// No value is added atomically; the summation order depends only on (ps, wpb, dist, dim).  (Small plans count, with an atomic, which
+// No value is added atomically; the summation order depends only on (ps, wpb, dist, dim) and the size of the tables (slices of
+// columns below).  (Small plans count, with an atomic, which
 // workgroups of a row have left their part: FUSE below.)
 // Index stream: a wavefront fetches the descriptors and the first ids of its next few rounds together into its own
 // piece of LDS (two HBM latencies per four rounds instead of per round, with no feature row in flight meanwhile) and
@@ -106,6 +107,8 @@ struct AggArgs {
     unsigned win_bytes;       // ... of this many bytes,
     unsigned delta_l, delta_r;// ... the tables starting at these byte offsets;
     int sentinel;             // ... and a row index whose offset falls outside the window (reads as zero)
+    int slices, slice_cols;   // rows cut into this many slices of columns, a multiple of 4 each (the last one may be narrower), each XCD working on one
+    int num_wg;               // workgroups of a slice
     int tail_shift;           // MODE_F32_PACKED: how many columns early the lane with a row's last, partial piece starts its 16 bytes
 };
 
@@ -396,7 +399,7 @@ __device__ __forceinline__ void finish_row(const AggArgs &a, int row, int l, con
 // mistake spoil each other, not the ones that follow.  (With a counter that the last workgroup sets back to zero: 32.9 and 288.5 us.
 // The maximum issued ahead of the wait for the part, or only where the count turns out to be an earlier call's: 34 and 291.)
 template <int LPR, int MODE, bool BUF, bool SMX, bool FUSE>
-__global__ void __launch_bounds__(1024) MGGX_AGG_OCCUPANCY k_agg(const AggArgs a)
+__global__ void __launch_bounds__(1024) MGGX_AGG_OCCUPANCY k_agg(AggArgs a)
 {
     constexpr int NV = ModeTraits<MODE>::NV;
     constexpr int S = 64 / LPR;
@@ -421,6 +424,24 @@ __global__ void __launch_bounds__(1024) MGGX_AGG_OCCUPANCY k_agg(const AggArgs a
     extern __shared__ __align__(16) float lds[];
     if (gate_closed(a.gate)) return;
     const int num_parts = a.num_parts_dev ? *a.num_parts_dev : a.num_parts;
+    int wg = (int)blockIdx.x;
+    int slice = 0;
+    if (a.slices > 1) {
+        // workgroups go to the eight XCDs in turn: XCD x works on slice x % slices (run_agg says when)
+        const int xcd = wg & 7;
+        slice = xcd & (a.slices - 1);
+        wg = (wg >> 3) * (8 / a.slices) + xcd / a.slices;
+        if (wg >= a.num_wg) return;
+        const int c0 = slice * a.slice_cols;
+        a.dim = min(a.slice_cols, a.dim - c0);
+        a.out += c0;
+        a.in_l = static_cast<const float *>(a.in_l) + c0;
+        a.in_r = static_cast<const float *>(a.in_r) + c0;
+        a.delta_l += 4u * (unsigned)c0;
+        a.delta_r += 4u * (unsigned)c0;
+        a.c_val += c0;
+        if (FUSE) a.chain += (size_t)slice * a.num_wg;
+    }
 
     const int lane = lane_id();
     const int wave = (int)(threadIdx.x >> 6);
@@ -436,7 +457,7 @@ __global__ void __launch_bounds__(1024) MGGX_AGG_OCCUPANCY k_agg(const AggArgs a
         hdr[2 * wave + 1] = make_int2(-1, 0);
     }
 
-    const long long q_wave = ((long long)blockIdx.x * wpb + wave) * ((long long)S * a.dist);
+    const long long q_wave = ((long long)wg * wpb + wave) * ((long long)S * a.dist);
 
     // this lane's place inside a feature row
     Gather<LPR, MODE, BUF> g;
@@ -742,8 +763,7 @@ __global__ void __launch_bounds__(1024) MGGX_AGG_OCCUPANCY k_agg(const AggArgs a
     if (wave != 0) return;
 
     // ---- combine the wavefronts of this workgroup (wavefront 0; lane = feature index mod 64) ----
-    const int wg = (int)blockIdx.x;
-    if (!FUSE && lane == 0) {
+    if (!FUSE && lane == 0 && slice == 0) {
         a.c_hdr[2 * wg] = make_int2(-1, 0);
         a.c_hdr[2 * wg + 1] = make_int2(-1, 0);
     }
@@ -778,7 +798,7 @@ __global__ void __launch_bounds__(1024) MGGX_AGG_OCCUPANCY k_agg(const AggArgs a
         } else {
             const int e = started ? 2 * wg + 1 : 2 * wg;
             if constexpr (FUSE) chain_row[started ? 1 : 0] = orow;
-            else if (lane == 0) a.c_hdr[e] = make_int2(orow, HDR_VALID | (started ? HDR_STARTS : 0) | (ends ? HDR_ENDS : 0));
+            else if (lane == 0 && slice == 0) a.c_hdr[e] = make_int2(orow, HDR_VALID | (started ? HDR_STARTS : 0) | (ends ? HDR_ENDS : 0));
             float *dst = a.c_val + (size_t)e * a.cpad;
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
@@ -1166,6 +1186,29 @@ int run_agg(Plan *plan, float *d_out, const void *d_in_l, const void *d_in_r, co
     } else {
         return fail(MGGX_EINVAL, "aggregation: unknown input dtype %d", o.in_dtype);
     }
+    // Rows of several cache lines out of a table beyond the L2s: each XCD gathers one slice of the columns, whole lines, so that its L2
+    // holds its slice of twice (four times) as many rows; every slice reads the index stream for itself.  Only where rows start on line
+    // boundaries (slices of 40, 41 or 100 packed columns share their lines: 25 to 50 % slower), fp32, without the softmax, which needs
+    // the whole row, and not beside the LDS kernel, which takes the CUs the smaller hit latency would free (1 M nodes, 47 M neighbors, width
+    // 64: 950 -> 1,113 us).  Table sizes (us whole / 2 / 4 slices): 256-byte rows: 13 MB 41.0 / 42.5, 26 MB 42.7 / 44.5, 84.6 / 85.7 and 43.7 / 41.1,
+    // 44 MB 99.7 / 89.5, 77 MB 144 / 117; 512-byte rows: 15 MB 39.9 / 38.2 / 46.0, 31 MB 92 / 81 / 89, 51 MB 180 / 155 / 172, 87 MB 232 / 171 / 180 and
+    // 205 / 174 / 151, 154 MB 203 / 171 / 161 and 886 / 651 / 576, 512 MB 3,517 / 2,770 / 2,671; 1,024-byte rows: 31 MB 73 / 67 / 67, 61 MB 244 / 167 / 152,
+    // 102 MB 600 / 431 / 325, 307 MB 1,952 / 1,549 / 1,220 (eight slices: 362 at 102 MB, 1,236 at 307).
+    int slices = 1, slice_cols = dim;
+    {
+        const auto on_line = [](const void *p) { return (reinterpret_cast<uintptr_t>(p) & 127u) == 0; };
+        const int lines = (dim + 31) / 32;
+        const unsigned long long table_mb = ((unsigned long long)plan->real_rows + (plan->nnz_r > 0 ? (unsigned long long)plan->max_col_r + 1 : 0)) * (unsigned long long)ld_in * 4 >> 20;
+        if (mode == MODE_F32_VEC4 && lines > 1 && ld_in % 32 == 0 && on_line(d_in_l) && (plan->nnz_r == 0 || on_line(d_in_r)) &&
+            (blocked || !(o.flags & MGGX_AGG_SOFTMAX)) && !(cm && cm->join)) {
+            if (lines % 2 == 0 && table_mb >= (lines == 2 ? 32u : 12u)) slices = 2;
+            if (lines % 4 == 0 && table_mb >= (lines == 4 ? 80u : 31u)) slices = 4;
+            if (slices > 1) {
+                slice_cols = 32 * lines / slices;
+                lpr = pow2_ceil(slice_cols / 4);
+            }
+        }
+    }
     const int slots = 64 / lpr;
     // 0 = let the library choose.  A wavefront's time is one chain of memory latencies per staged group of rounds, so a plan
     // is cut into enough wavefronts first and into long ones second:
@@ -1192,7 +1235,7 @@ int run_agg(Plan *plan, float *d_out, const void *d_in_l, const void *d_in_r, co
     const long long stated = plan->d_part_ptr ? explicit_units_bound(plan->rows, plan->caller_parts, plan->ps) : plan->num_parts;
     const int cpad = (dim + 3) & ~3;
     const double per_row = (double)stated / (double)(plan->rows > 0 ? plan->rows : 1);
-    const long long rounds = (stated + slots - 1) / slots;
+    const long long rounds = (stated + slots - 1) / slots * slices;
     const bool beside_core = cm && cm->join, wpb_free = wpb == 0, dist_free = dist == 0;
     if (wpb == 0) wpb = (beside_core && !blocked && slots <= 4) ? 8 : (blocked || slots > 4 || per_row < 3.0 || rounds < MANY_ROUNDS) ? 4 : 8;
     if (dist == 0) {
@@ -1249,6 +1292,9 @@ int run_agg(Plan *plan, float *d_out, const void *d_in_l, const void *d_in_r, co
     a.eps = o.eps;
     a.in_is_bf16 = o.in_dtype == MGGX_BF16;
     a.tail_shift = mode == MODE_F32_PACKED ? 4 - (dim & 3) : 0;
+    a.slices = slices;
+    a.slice_cols = slice_cols;
+    a.num_wg = (int)num_wg;
 
     // Gather addressing.  Extent of each table: the local one holds the share's rows, the remote one at least the
     // largest remote id.  When both fit one window of < 2 GiB and < 2^24 rows, offsets are 32-bit buffer offsets.
@@ -1282,7 +1328,7 @@ int run_agg(Plan *plan, float *d_out, const void *d_in_l, const void *d_in_r, co
     const int n_empty = touch_empty ? plan->num_empty : 0;
     // (a call with rows without neighbors launches k_agg_tail for them, which finishes the crossing rows on the way; a captured call
     // would have one number for all of its replays, so a plan used in a capture takes the second launch from then on)
-    const bool fuse = !blocked && !beside_core && !fixed && plan->d_chain && n_empty == 0 && num_wg > 1 && num_wg <= FUSE_MAX_WORKGROUPS && has_fused(mode, buf, lpr) &&
+    const bool fuse = !blocked && !beside_core && !fixed && plan->d_chain && n_empty == 0 && num_wg > 1 && num_wg * slices <= FUSE_MAX_WORKGROUPS && has_fused(mode, buf, lpr) &&
                       !plan->pinned;
     static_assert(FUSE_MAX_WORKGROUPS < 1 << 16, "the count of a chain lies below the call number");
     a.chain = fuse ? plan->d_chain : nullptr;
@@ -1320,7 +1366,7 @@ int run_agg(Plan *plan, float *d_out, const void *d_in_l, const void *d_in_r, co
         a.stage_rounds = stage;
         const size_t lds_bytes = carry_lds + (size_t)wpb * stage * round_bytes + (size_t)MGGX_AGG_LDS_PAD;
         if (lds_bytes > (160u << 10)) return fail(MGGX_ELIMIT, "aggregation: %zu bytes of LDS per workgroup (wpb %d, dim %d)", lds_bytes, wpb, dim);
-        const dim3 grid((unsigned)num_wg), block((unsigned)(64 * wpb));
+        const dim3 grid((unsigned)(slices > 1 ? 8 * ((num_wg * slices + 7) / 8) : num_wg)), block((unsigned)(64 * wpb));
         const bool smx = (a.flags & MGGX_AGG_SOFTMAX) != 0;  // fp32 tables only (checked above)
         if (buf) {
             if (mode == MODE_F32_VEC4) rc = smx ? launch_agg<MODE_F32_VEC4, true, true>(lpr, grid, block, lds_bytes, st.stream, a)
@@ -1381,8 +1427,8 @@ int run_agg(Plan *plan, float *d_out, const void *d_in_l, const void *d_in_r, co
             MGGX_LAUNCH_CHECK("k_agg_tail");
         }
     }
-    snprintf(st.last_kernel, sizeof(st.last_kernel), "k_agg<%d,%d,%d> grid=%lld block=%d parts=%d blocks=%d ps=%d wpb=%d dist=%d addr=%s fused=%d", lpr, mode, (int)buf,
-             num_wg, 64 * wpb, plan->num_parts, plan->blocks, plan->ps, wpb, dist, buf ? "buffer32" : "flat64", (int)fuse);
+    snprintf(st.last_kernel, sizeof(st.last_kernel), "k_agg<%d,%d,%d> grid=%lld block=%d parts=%d blocks=%d ps=%d wpb=%d dist=%d addr=%s fused=%d slices=%d", lpr, mode, (int)buf,
+             num_wg, 64 * wpb, plan->num_parts, plan->blocks, plan->ps, wpb, dist, buf ? "buffer32" : "flat64", (int)fuse, slices);
     return MGGX_OK;
 }
 
