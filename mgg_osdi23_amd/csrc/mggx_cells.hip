@@ -409,34 +409,44 @@ __global__ void __launch_bounds__(256, WAVES) k_cells(const CellArgs a)
             __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
             for (int rb = 0; rb < 8; ++rb) acc[rb] = (v4f){0.f, 0.f, 0.f, 0.f};
-            // the smallest parts of the whole cell first: what is added at the size of the sum is four products
+            // The smallest parts of the whole cell first: what is added at the size of the sum is four products.  An operand is read from
+            // the LDS while the products of the one before are on their way (left to the compiler, it is read right before its use).
+            v4u x[2][2];
+            const auto read = [&](int k) {  // k = 4 (2 - part) + step
+                const int at = ((k & 3) * 6 + 2 * (2 - (k >> 2))) * 64 + lane;
+                x[k & 1][0] = buf[b][at];
+                x[k & 1][1] = buf[b][at + 64];
+            };
+            read(0);
 #pragma unroll
-            for (int p = 2; p >= 0; --p)
-#pragma unroll
-                for (int st = 0; st < STEPS; ++st) {
-                    if (p == 1 && st == STEPS / 2) {
-                        __builtin_amdgcn_sched_barrier(0);
-                        put(b ^ 1, 0);
-                        ask(src, 1);
-                        __builtin_amdgcn_sched_barrier(0);
-                    }
-                    const v4u lo = buf[b][(st * 6 + 2 * p) * 64 + lane], hi = buf[b][(st * 6 + 2 * p + 1) * 64 + lane];
-                    const unsigned t[8] = {lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
-                    v16bf x;
-                    __builtin_memcpy(&x, t, 32);
-#pragma unroll
-                    for (int rb = 0; rb < 8; ++rb) {
-                        const int index = (int)m[2 * rb + (st >> 1)];
-                        acc[rb] = (st & 1) ? __builtin_amdgcn_smfmac_f32_16x16x64_bf16(one, x, acc[rb], index, 0, 1)
-                                           : __builtin_amdgcn_smfmac_f32_16x16x64_bf16(one, x, acc[rb], index, 0, 0);
-                    }
+            for (int k = 0; k < 3 * STEPS; ++k) {
+                const int st = k & 3;
+                if (k == 6) {
+                    put(b ^ 1, 0);
+                    ask(src, 1);
                 }
+                if (k + 1 < 3 * STEPS) read(k + 1);
+                __builtin_amdgcn_sched_barrier(0);
+                v16bf xk;
+                const unsigned t[8] = {x[k & 1][0].x, x[k & 1][0].y, x[k & 1][0].z, x[k & 1][0].w, x[k & 1][1].x, x[k & 1][1].y, x[k & 1][1].z, x[k & 1][1].w};
+                __builtin_memcpy(&xk, t, 32);
+#pragma unroll
+                for (int rb = 0; rb < 8; ++rb) {
+                    const int index = (int)m[2 * rb + (st >> 1)];
+                    acc[rb] = (st & 1) ? __builtin_amdgcn_smfmac_f32_16x16x64_bf16(one, xk, acc[rb], index, 0, 1)
+                                       : __builtin_amdgcn_smfmac_f32_16x16x64_bf16(one, xk, acc[rb], index, 0, 0);
+                }
+                __builtin_amdgcn_sched_barrier(0);
+            }
             __builtin_amdgcn_sched_barrier(0);
             asm volatile("" ::"v"(touched));
             if (f + 1 == FG && !last) ask_words(cell + 1);
             put(b ^ 1, 1);
 #pragma unroll
-            for (int rb = 0; rb < 8; ++rb) sum[f][rb] += acc[rb];
+            for (int rb = 0; rb < 8; ++rb) {
+                sum[f][rb] += acc[rb];
+                asm volatile("" : "+v"(sum[f][rb]));  // here, not after the next products: these 32 registers are theirs
+            }
             b ^= 1;
             __syncthreads();
         }
@@ -717,7 +727,7 @@ int cells_sums(const CorePlan *p, const float *d_in, int dim, long long ld_in, c
         case 1: k_cells<1, 3><<<(unsigned)cut.nwg, 256, 0, stream>>>(a); break;
         case 2: k_cells<2, 2><<<(unsigned)cut.nwg, 256, 0, stream>>>(a); break;
         case 3: k_cells<3, 2><<<(unsigned)cut.nwg, 256, 0, stream>>>(a); break;
-        case 4: k_cells<2, 2><<<dim3((unsigned)cut.nwg, 2), 256, 0, stream>>>(a); break;
+        case 4: k_cells<4, 2><<<(unsigned)cut.nwg, 256, 0, stream>>>(a); break;
         default: return fail(MGGX_ELIMIT, "dense cells: dim %d outside 1..64", dim);
     }
     MGGX_LAUNCH_CHECK("k_cells");
