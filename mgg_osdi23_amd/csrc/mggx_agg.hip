@@ -72,6 +72,11 @@ constexpr int MODE_F32_PACKED = 3;   // the same, for rows of a width that is no
 constexpr int MODE_F32_STRIDED = 1;  // fp32 rows of 1 to 3 columns, dword loads, one lane per row
 constexpr int MODE_BF16_VEC8 = 2;    // bf16 rows, one 16-byte load (8 values) per lane, fp32 accumulation
 
+// How rows that lie across the workgroups' shares of the descriptors are finished (k_agg).
+constexpr int FORM_PLAIN = 0;  // k_agg_tail adds their parts
+constexpr int FORM_FUSE = 1;   // the last workgroup to leave a part adds them
+constexpr int FORM_WHOLE = 2;  // there are none: a workgroup takes the whole of every row that starts in its share
+
 struct AggArgs {
     float *out;
     const void *in_l;
@@ -109,6 +114,7 @@ struct AggArgs {
     int sentinel;             // ... and a row index whose offset falls outside the window (reads as zero)
     int slices, slice_cols;   // rows cut into this many slices of columns, a multiple of 4 each (the last one may be narrower), each XCD working on one
     int num_wg;               // workgroups of a slice
+    int whole;                // FORM_WHOLE (no row crosses workgroups)
     int tail_shift;           // MODE_F32_PACKED: how many columns early the lane with a row's last, partial piece starts its 16 bytes
 };
 
@@ -393,14 +399,22 @@ __device__ __forceinline__ void finish_row(const AggArgs &a, int row, int l, con
 // microseconds are a good part of theirs.  Every workgroup of such a row leaves its partial row in the carry buffer and
 // then counts itself in; the one that finds the others there adds the parts, in the same order as k_agg_tail.  The XCDs' L2s
 // are not coherent with each other for plain accesses, so parts and counters go with device-scope accesses, and a workgroup
-// waits until its part has arrived before it counts.  GCN forward, 4,096 nodes: 35.4 -> 33.3 us; GIN forward, 50 K nodes: 299 -> 289.
+// waits until its part has arrived before it counts.  GIN forward, 50 K nodes: 299 -> 289 us.
 // Counters carry the number of the call, and the first workgroup of a call to come by starts them anew (a maximum with the call's
 // number, then the addition, to one address in order), so nothing depends on how an earlier call left them: calls that overlapped by
 // mistake spoil each other, not the ones that follow.  (With a counter that the last workgroup sets back to zero: 32.9 and 288.5 us.
 // The maximum issued ahead of the wait for the part, or only where the count turns out to be an earlier call's: 34 and 291.)
-template <int LPR, int MODE, bool BUF, bool SMX, bool FUSE>
+// WHOLE: where no row has more than a few descriptors, a workgroup takes whole rows: every row whose first descriptor lies in its
+// share of parts_per_wg descriptors, which is longest - 1 smaller than what its wavefronts hold, so that the row at the end of the
+// share fits as a whole; slots that hold a piece of a neighbor's row stay empty.  Nothing is left for others to finish: no part
+// goes through memory, nobody counts or waits (a chain of four memory latencies at the end of a workgroup's life, 2 to 4.5 us), and
+// the next launch is never needed, under capture either.  The first descriptor of a row comes from the plan's row offsets, asked
+// for together with the neighbor ids.  4,096 nodes of mean degree 17: 8.8 -> 7.0 us at width 16, 13.5 -> 8.8 at 41 with the softmax,
+// 9.6 -> 6.6 at 64; GCN forward 33.1 -> 26.4; 20 K nodes of degree 40, width 64: 20.2 -> 17.6; 100 K nodes of degree 16: 63.6 -> 60.1.
+template <int LPR, int MODE, bool BUF, bool SMX, int FORM>
 __global__ void __launch_bounds__(1024) MGGX_AGG_OCCUPANCY k_agg(AggArgs a)
 {
+    constexpr bool FUSE = FORM == FORM_FUSE, WHOLE = FORM == FORM_WHOLE;
     constexpr int NV = ModeTraits<MODE>::NV;
     constexpr int S = 64 / LPR;
     constexpr int CH = LPR > 16 ? LPR : 16;  // neighbor ids fetched per slot per chunk
@@ -422,7 +436,8 @@ __global__ void __launch_bounds__(1024) MGGX_AGG_OCCUPANCY k_agg(AggArgs a)
     // at width 32: 1.59 -> 1.77 ms) and the same without it.
     constexpr bool OFF_CROSSBAR = LPR == 4 || LPR == 16 || LPR == 32;
     extern __shared__ __align__(16) float lds[];
-    if (gate_closed(a.gate)) return;
+    const GateSeen seen = gate_read(a.gate);
+    if (FORM == FORM_PLAIN && gate_closed(a.gate, seen)) return;
     const int num_parts = a.num_parts_dev ? *a.num_parts_dev : a.num_parts;
     int wg = (int)blockIdx.x;
     int slice = 0;
@@ -457,7 +472,7 @@ __global__ void __launch_bounds__(1024) MGGX_AGG_OCCUPANCY k_agg(AggArgs a)
         hdr[2 * wave + 1] = make_int2(-1, 0);
     }
 
-    const long long q_wave = ((long long)wg * wpb + wave) * ((long long)S * a.dist);
+    const long long q_wave = WHOLE ? (long long)wg * a.parts_per_wg + wave * (S * a.dist) : ((long long)wg * wpb + wave) * ((long long)S * a.dist);
 
     // this lane's place inside a feature row
     Gather<LPR, MODE, BUF> g;
@@ -590,10 +605,20 @@ __global__ void __launch_bounds__(1024) MGGX_AGG_OCCUPANCY k_agg(AggArgs a)
             int idv[STAGE][IPL];
 #pragma unroll
             for (int u = 0; u < STAGE; ++u) dd[u] = load_desc(q_wave + (long long)(j0 + u) * S + slot, u < nst && j0 + u < a.dist);
+            if (FORM != FORM_PLAIN && j0 == 0 && gate_closed(a.gate, seen)) break;  // (small plans: asked once the first descriptors are on their way)
+            int first[STAGE];  // WHOLE: first descriptor of the row
 #pragma unroll
             for (int u = 0; u < STAGE; ++u) {
                 issue_ids(dd[u], 0, idv[u]);
-                if (u < nst && l == 0) st_desc[u * S + slot] = dd[u];
+                if constexpr (WHOLE) first[u] = a.off[dd[u].y >= 0 ? dd[u].y : 0];
+                else if (u < nst && l == 0) st_desc[u * S + slot] = dd[u];
+            }
+            if constexpr (WHOLE) {
+#pragma unroll
+                for (int u = 0; u < STAGE; ++u) {
+                    if ((unsigned)(first[u] - wg * a.parts_per_wg) >= (unsigned)a.parts_per_wg) dd[u] = make_int4(0, -1, 0, 0);  // another workgroup's row
+                    if (u < nst && l == 0) st_desc[u * S + slot] = dd[u];
+                }
             }
 #pragma unroll
             for (int u = 0; u < STAGE; ++u) {
@@ -725,7 +750,7 @@ __global__ void __launch_bounds__(1024) MGGX_AGG_OCCUPANCY k_agg(AggArgs a)
         // The last slot of each run now holds the run's sum.  A run ends where its row ends (the descriptor of a row's last
         // partition says so: the next descriptor, if any, belongs to another row) and at the last slot of the round.
         const bool row_done = ((unsigned)d.z & DESC_LAST) != 0;
-        const bool run_last = pv && (row_done || slot == S - 1);
+        const bool run_last = (WHOLE ? row >= 0 : pv) && (row_done || slot == S - 1);
         const bool last_round = (j == a.dist - 1) || (q0 + S >= num_parts);
         bool keep_open = false;
         if (run_last) {
@@ -763,7 +788,7 @@ __global__ void __launch_bounds__(1024) MGGX_AGG_OCCUPANCY k_agg(AggArgs a)
     if (wave != 0) return;
 
     // ---- combine the wavefronts of this workgroup (wavefront 0; lane = feature index mod 64) ----
-    if (!FUSE && lane == 0 && slice == 0) {
+    if (FORM == FORM_PLAIN && lane == 0 && slice == 0) {
         a.c_hdr[2 * wg] = make_int2(-1, 0);
         a.c_hdr[2 * wg + 1] = make_int2(-1, 0);
     }
@@ -795,7 +820,7 @@ __global__ void __launch_bounds__(1024) MGGX_AGG_OCCUPANCY k_agg(AggArgs a)
     auto emit = [&](bool ends) {
         if (started && ends) {
             finish(orow, s);
-        } else {
+        } else if constexpr (!WHOLE) {
             const int e = started ? 2 * wg + 1 : 2 * wg;
             if constexpr (FUSE) chain_row[started ? 1 : 0] = orow;
             else if (lane == 0 && slice == 0) a.c_hdr[e] = make_int2(orow, HDR_VALID | (started ? HDR_STARTS : 0) | (ends ? HDR_ENDS : 0));
@@ -1060,12 +1085,12 @@ int pow2_ceil(int x)
     return p;
 }
 
-template <int LPR, int MODE, bool BUF, bool SMX, bool FUSE>
+template <int LPR, int MODE, bool BUF, bool SMX, int FORM>
 void launch_agg_kernel(dim3 grid, dim3 block, size_t lds_bytes, hipStream_t stream, const AggArgs &a)
 {
     if (lds_bytes > (48u << 10))
-        (void)hipFuncSetAttribute(reinterpret_cast<const void *>(&k_agg<LPR, MODE, BUF, SMX, FUSE>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_bytes);
-    k_agg<LPR, MODE, BUF, SMX, FUSE><<<grid, block, lds_bytes, stream>>>(a);
+        (void)hipFuncSetAttribute(reinterpret_cast<const void *>(&k_agg<LPR, MODE, BUF, SMX, FORM>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_bytes);
+    k_agg<LPR, MODE, BUF, SMX, FORM><<<grid, block, lds_bytes, stream>>>(a);
 }
 
 // Which kernels have a variant that finishes rows crossing workgroups by itself (AggArgs::chain): what decides on the host whether a
@@ -1078,12 +1103,16 @@ template <int LPR, int MODE, bool BUF, bool SMX>
 int launch_agg_as(dim3 grid, dim3 block, size_t lds_bytes, hipStream_t stream, const AggArgs &a)
 {
     if constexpr (has_fused(MODE, BUF, LPR)) {
+        if (a.whole) {
+            launch_agg_kernel<LPR, MODE, BUF, SMX, FORM_WHOLE>(grid, block, lds_bytes, stream, a);
+            return MGGX_OK;
+        }
         if (a.chain) {
-            launch_agg_kernel<LPR, MODE, BUF, SMX, true>(grid, block, lds_bytes, stream, a);
+            launch_agg_kernel<LPR, MODE, BUF, SMX, FORM_FUSE>(grid, block, lds_bytes, stream, a);
             return MGGX_OK;
         }
     }
-    launch_agg_kernel<LPR, MODE, BUF, SMX, false>(grid, block, lds_bytes, stream, a);
+    launch_agg_kernel<LPR, MODE, BUF, SMX, FORM_PLAIN>(grid, block, lds_bytes, stream, a);
     return MGGX_OK;
 }
 
@@ -1130,6 +1159,13 @@ struct CoreMerge {
 // takes at most 4, and never so many that fewer than MIN_WAVEFRONTS wavefronts (3 per SIMD) are left for the chip.
 constexpr long long MANY_ROUNDS = 400000;
 constexpr int MIN_WAVEFRONTS = 3000;
+
+// A workgroup may hold back up to a fifth of its slots to take whole rows (k_agg, FORM_WHOLE), in wavefronts of up to WHOLE_ROUNDS rounds
+// (with 16 rounds the chain at the end is nothing: 300 K nodes of degree 40, width 128: 865 -> 882 us), and only where enough
+// rows cross: a sixteenth or more of the slots held back has to be paid for by rows of more than one descriptor (20 K nodes of degree
+// 8, 1.6 % such rows, width 41: 11.9 us, 12.1 with one slot in sixteen held back).
+constexpr long long WHOLE_SLACK = 5;
+constexpr int WHOLE_ROUNDS = 4;
 
 // Parts of the static scratch in a call of mggx_sag_parts_static: descriptors | first descriptor of each row | [scratch of the
 // unit builder, ps < 16] | carry buffer.
@@ -1193,7 +1229,11 @@ int run_agg(Plan *plan, float *d_out, const void *d_in_l, const void *d_in_r, co
     // 64: 950 -> 1,113 us).  Table sizes (us whole / 2 / 4 slices): 256-byte rows: 13 MB 41.0 / 42.5, 26 MB 42.7 / 44.5, 84.6 / 85.7 and 43.7 / 41.1,
     // 44 MB 99.7 / 89.5, 77 MB 144 / 117; 512-byte rows: 15 MB 39.9 / 38.2 / 46.0, 31 MB 92 / 81 / 89, 51 MB 180 / 155 / 172, 87 MB 232 / 171 / 180 and
     // 205 / 174 / 151, 154 MB 203 / 171 / 161 and 886 / 651 / 576, 512 MB 3,517 / 2,770 / 2,671; 1,024-byte rows: 31 MB 73 / 67 / 67, 61 MB 244 / 167 / 152,
-    // 102 MB 600 / 431 / 325, 307 MB 1,952 / 1,549 / 1,220 (eight slices: 362 at 102 MB, 1,236 at 307).
+    // 102 MB 600 / 431 / 325, 307 MB 1,952 / 1,549 / 1,220 (eight slices: 362 at 102 MB, 1,236 at 307).  Single lines of 512-byte rows from beyond
+    // the memory-side cache cost more than pairs of them (1 M nodes, 512 MB: 813 whole, 696 in pairs, 743 in fours).  Graphs without hubs
+    // (the longest row less than 16 mean ones; not known of a caller's own partitions) re-use too little of a large slice: above 32 MB of it they stay whole (uniform
+    // neighbors, 43 MB 95 / 92, 87 MB 198 / - / 182, but 77 MB, 40 per row, 428 / 436, 256 MB 428 / 454, 512 MB 855 / - / 917); column blocks of 12 MB and
+    // more gain without hubs, too (150 K nodes, 150 per row, 256- / 512- / 1,024-byte rows: 631 -> 445, 1,435 -> 1,241, 3,153 -> 2,569).
     int slices = 1, slice_cols = dim;
     {
         const auto on_line = [](const void *p) { return (reinterpret_cast<uintptr_t>(p) & 127u) == 0; };
@@ -1201,8 +1241,10 @@ int run_agg(Plan *plan, float *d_out, const void *d_in_l, const void *d_in_r, co
         const unsigned long long table_mb = ((unsigned long long)plan->real_rows + (plan->nnz_r > 0 ? (unsigned long long)plan->max_col_r + 1 : 0)) * (unsigned long long)ld_in * 4 >> 20;
         if (mode == MODE_F32_VEC4 && lines > 1 && ld_in % 32 == 0 && on_line(d_in_l) && (plan->nnz_r == 0 || on_line(d_in_r)) &&
             (blocked || !(o.flags & MGGX_AGG_SOFTMAX)) && !(cm && cm->join)) {
+            const bool hubs = blocked || (plan->longest > 0 && (double)plan->longest * plan->rows > 16.0 * plan->num_parts);
             if (lines % 2 == 0 && table_mb >= (lines == 2 ? 32u : 12u)) slices = 2;
-            if (lines % 4 == 0 && table_mb >= (lines == 4 ? 80u : 31u)) slices = 4;
+            if (lines % 4 == 0 && table_mb >= (lines == 4 ? 80u : 31u) && (lines > 4 || table_mb <= 256u)) slices = 4;
+            if (!hubs && table_mb > 32u * (unsigned)slices) slices = 1;
             if (slices > 1) {
                 slice_cols = 32 * lines / slices;
                 lpr = pow2_ceil(slice_cols / 4);
@@ -1258,7 +1300,7 @@ int run_agg(Plan *plan, float *d_out, const void *d_in_l, const void *d_in_r, co
     }
     const long long parts_per_wg = (long long)wpb * slots * dist;
     if (parts_per_wg > 0x3fffffffLL) return fail(MGGX_ELIMIT, "aggregation: wpb*dist too large");
-    const long long num_wg = (plan->num_parts + parts_per_wg - 1) / parts_per_wg;
+    long long num_wg = (plan->num_parts + parts_per_wg - 1) / parts_per_wg;
     if (num_wg > 0x7fffffffLL) return fail(MGGX_ELIMIT, "aggregation: too many workgroups");
 
     AggArgs a{};
@@ -1326,9 +1368,20 @@ int run_agg(Plan *plan, float *d_out, const void *d_in_l, const void *d_in_r, co
     // rows without neighbors are written by k_agg_tail
     const bool touch_empty = !(o.flags & MGGX_AGG_ACCUMULATE) || (o.flags & (MGGX_AGG_GIN | MGGX_AGG_RELU | MGGX_AGG_SOFTMAX));
     const int n_empty = touch_empty ? plan->num_empty : 0;
+    const long long held_back = plan->longest - 1;
+    const bool whole = wpb_free && dist_free && dist <= WHOLE_ROUNDS && !blocked && !beside_core && !fixed && plan->longest > 0 && n_empty == 0 && num_wg > 1 &&
+                       has_fused(mode, buf, lpr) && held_back * WHOLE_SLACK <= parts_per_wg &&
+                       (held_back * 16 < parts_per_wg || (long long)plan->num_parts * 10 >= (long long)plan->rows * 11);
+    if (whole) {
+        a.parts_per_wg = (int)(parts_per_wg - held_back);
+        a.ppw_shift = -1;
+        num_wg = (plan->num_parts + a.parts_per_wg - 1) / a.parts_per_wg;
+        a.num_wg = (int)num_wg;
+        a.whole = 1;
+    }
     // (a call with rows without neighbors launches k_agg_tail for them, which finishes the crossing rows on the way; a captured call
     // would have one number for all of its replays, so a plan used in a capture takes the second launch from then on)
-    const bool fuse = !blocked && !beside_core && !fixed && plan->d_chain && n_empty == 0 && num_wg > 1 && num_wg * slices <= FUSE_MAX_WORKGROUPS && has_fused(mode, buf, lpr) &&
+    const bool fuse = !whole && !blocked && !beside_core && !fixed && plan->d_chain && n_empty == 0 && num_wg > 1 && num_wg * slices <= FUSE_MAX_WORKGROUPS && has_fused(mode, buf, lpr) &&
                       !plan->pinned;
     static_assert(FUSE_MAX_WORKGROUPS < 1 << 16, "the count of a chain lies below the call number");
     a.chain = fuse ? plan->d_chain : nullptr;
@@ -1415,7 +1468,7 @@ int run_agg(Plan *plan, float *d_out, const void *d_in_l, const void *d_in_r, co
             default: k_agg_finish_blocked<4><<<fgrid, dim3(256), 0, st.stream>>>(r, part, plan->real_rows, plan->blocks, ldp, g_shift, cma);
         }
         MGGX_LAUNCH_CHECK("k_agg_finish_blocked");
-    } else if (!fuse) {
+    } else if (!fuse && !whole) {
         // rows that cross workgroups and rows without neighbors, in one launch
         const int G = pow2_ceil((dim + 3) / 4);
         const long long per_block = 4 * (64 / G);
@@ -1427,8 +1480,8 @@ int run_agg(Plan *plan, float *d_out, const void *d_in_l, const void *d_in_r, co
             MGGX_LAUNCH_CHECK("k_agg_tail");
         }
     }
-    snprintf(st.last_kernel, sizeof(st.last_kernel), "k_agg<%d,%d,%d> grid=%lld block=%d parts=%d blocks=%d ps=%d wpb=%d dist=%d addr=%s fused=%d slices=%d", lpr, mode, (int)buf,
-             num_wg, 64 * wpb, plan->num_parts, plan->blocks, plan->ps, wpb, dist, buf ? "buffer32" : "flat64", (int)fuse, slices);
+    snprintf(st.last_kernel, sizeof(st.last_kernel), "k_agg<%d,%d,%d> grid=%lld block=%d parts=%d blocks=%d ps=%d wpb=%d dist=%d addr=%s fused=%d whole=%d slices=%d", lpr, mode, (int)buf,
+             num_wg, 64 * wpb, plan->num_parts, plan->blocks, plan->ps, wpb, dist, buf ? "buffer32" : "flat64", (int)(fuse || whole), (int)whole, slices);
     return MGGX_OK;
 }
 

@@ -60,18 +60,32 @@ struct Gate {
     int tag = 0;
 };
 
-__device__ __forceinline__ bool gate_closed(const Gate &g)
+// What the words of a gate hold.  All of them are asked for before the first is looked at (one memory latency, not one after the
+// other), and a kernel may issue loads of its own plan between the two steps.
+struct GateSeen {
+    int ok, cnt_l, cnt_r;
+};
+
+__device__ __forceinline__ GateSeen gate_read(const Gate &g)
 {
-    if (g.ok && *g.ok == 0) return true;
-    if (g.cnt_l) {
-        const bool bad = *g.cnt_l != g.want_l || (g.cnt_r && *g.cnt_r != g.want_r);
-        if (bad) {
-            *g.flag = g.tag;
-            return true;
-        }
+    GateSeen s{1, 0, 0};
+    if (g.ok) s.ok = *g.ok;
+    if (g.cnt_l) s.cnt_l = *g.cnt_l;
+    if (g.cnt_l && g.cnt_r) s.cnt_r = *g.cnt_r;
+    return s;
+}
+
+__device__ __forceinline__ bool gate_closed(const Gate &g, const GateSeen &s)
+{
+    if (s.ok == 0) return true;
+    if (g.cnt_l && (s.cnt_l != g.want_l || (g.cnt_r && s.cnt_r != g.want_r))) {
+        *g.flag = g.tag;
+        return true;
     }
     return false;
 }
+
+__device__ __forceinline__ bool gate_closed(const Gate &g) { return gate_closed(g, gate_read(g)); }
 
 struct Guard {
     const int *arr[4] = {nullptr, nullptr, nullptr, nullptr};  // fingerprinted arrays ...
@@ -112,6 +126,7 @@ struct Plan {
     unsigned long long *d_chain = nullptr;  // [FUSE_MAX_WORKGROUPS] workgroups that have left their part of a row, with the call's number (k_agg, FUSE)
     int num_parts = 0;
     int num_empty = 0;
+    int longest = 0;           // most descriptors of one row; 0: not known (explicit partitions, column blocks)
     int64_t nnz_l = 0, nnz_r = 0;
     int max_col_r = -1;        // largest remote neighbor id (bounds the remote table)
     // Column-blocked plans: the neighbor ids [lb, lb + real_rows) are cut into `blocks` ranges of `block_rows` ids and

@@ -286,12 +286,20 @@ __global__ void __launch_bounds__(256) k_off_from_parts(const int *__restrict__ 
     off[r] = lo;
 }
 
+// Rows without any descriptor (counter[0] of them), and the most descriptors that one row has (counter[1]).
 __global__ void __launch_bounds__(256) k_collect_empty(const int *__restrict__ off, int rows, int *__restrict__ list,
                                                        int *__restrict__ counter)
 {
     const int r = blockIdx.x * 256 + threadIdx.x;
-    if (r >= rows) return;
-    if (off[r + 1] == off[r]) list[atomicAdd(counter, 1)] = r;
+    int n = -1;
+    if (r < rows) n = off[r + 1] - off[r];
+    if (n == 0) list[atomicAdd(counter, 1)] = r;
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) n = max(n, __shfl_xor(n, o));
+    __shared__ int most[4];
+    if ((threadIdx.x & 63u) == 0) most[threadIdx.x >> 6] = n;
+    __syncthreads();
+    if (threadIdx.x == 0) atomicMax(counter + 1, max(max(most[0], most[1]), max(most[2], most[3])));
 }
 
 // reference-layout arrays
@@ -662,9 +670,10 @@ static int plan_finish(Plan *p, const int *d_a, const int *d_b, long long **word
     State &s = state();
     int *d_counter = nullptr;
     int rc = host_words(words);
-    if (!rc) rc = dev_array(&d_counter, 1);
+    if (!rc) rc = dev_array(&d_counter, 2);
     if (!rc) rc = dev_array(&p->d_empty_rows, (size_t)p->rows);
-    if (!rc && p->blocks == 1 && !p->d_part_ptr) {  // (the caller's partition arrays may list a row's partitions apart)
+    const bool plain = p->blocks == 1 && !p->d_part_ptr;
+    if (!rc && plain) {  // (the caller's partition arrays may list a row's partitions apart)
         rc = dev_array(&p->d_chain, FUSE_MAX_WORKGROUPS);
         if (!rc) k_zero_words<<<1, 1024, 0, s.stream>>>(reinterpret_cast<int *>(p->d_chain), 2 * FUSE_MAX_WORKGROUPS);
     }
@@ -673,13 +682,14 @@ static int plan_finish(Plan *p, const int *d_a, const int *d_b, long long **word
         return rc;
     }
     long long *const w = *words + 1;  // word 0 holds the total of a scan in flight
-    k_zero_words<<<1, 64, 0, s.stream>>>(d_counter, 1);
+    k_zero_words<<<1, 64, 0, s.stream>>>(d_counter, 2);
     if (p->rows > 0) k_collect_empty<<<(p->rows + 255) / 256, 256, 0, s.stream>>>(p->d_off, p->rows, p->d_empty_rows, d_counter);
-    k_publish<<<1, 1, 0, s.stream>>>(d_counter, d_a, d_b, w);
+    k_publish<<<1, 1, 0, s.stream>>>(d_counter, d_a, plain ? d_counter + 1 : d_b, w);
     const hipError_t el = hipGetLastError(), e = hipStreamSynchronize(s.stream);
     dev_free(d_counter);
     if (el != hipSuccess || e != hipSuccess) return fail(MGGX_EHIP, "plan: %s", hipGetErrorString(el != hipSuccess ? el : e));
     p->num_empty = (int)w[0];
+    if (plain) p->longest = (int)w[2];
     return MGGX_OK;
 }
 
