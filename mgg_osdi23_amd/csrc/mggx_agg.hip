@@ -1225,13 +1225,13 @@ int run_agg(Plan *plan, float *d_out, const void *d_in_l, const void *d_in_r, co
     // Rows of several cache lines out of a table beyond the L2s: each XCD gathers one slice of the columns, whole lines, so that its L2
     // holds its slice of twice (four times) as many rows; every slice reads the index stream for itself.  Only where rows start on line
     // boundaries (slices of 40, 41 or 100 packed columns share their lines: 25 to 50 % slower), fp32, without the softmax, which needs
-    // the whole row, and not beside the LDS kernel, which takes the CUs the smaller hit latency would free (1 M nodes, 47 M neighbors, width
+    // the whole row, not with a caller's own partitions (the static scratch takes what it took: its carry buffer depends on the slots), and not beside the LDS kernel, which takes the CUs the smaller hit latency would free (1 M nodes, 47 M neighbors, width
     // 64: 950 -> 1,113 us).  Table sizes (us whole / 2 / 4 slices): 256-byte rows: 13 MB 41.0 / 42.5, 26 MB 42.7 / 44.5, 84.6 / 85.7 and 43.7 / 41.1,
     // 44 MB 99.7 / 89.5, 77 MB 144 / 117; 512-byte rows: 15 MB 39.9 / 38.2 / 46.0, 31 MB 92 / 81 / 89, 51 MB 180 / 155 / 172, 87 MB 232 / 171 / 180 and
     // 205 / 174 / 151, 154 MB 203 / 171 / 161 and 886 / 651 / 576, 512 MB 3,517 / 2,770 / 2,671; 1,024-byte rows: 31 MB 73 / 67 / 67, 61 MB 244 / 167 / 152,
     // 102 MB 600 / 431 / 325, 307 MB 1,952 / 1,549 / 1,220 (eight slices: 362 at 102 MB, 1,236 at 307).  Single lines of 512-byte rows from beyond
     // the memory-side cache cost more than pairs of them (1 M nodes, 512 MB: 813 whole, 696 in pairs, 743 in fours).  Graphs without hubs
-    // (the longest row less than 16 mean ones; not known of a caller's own partitions) re-use too little of a large slice: above 32 MB of it they stay whole (uniform
+    // (the longest row less than 16 mean ones) re-use too little of a large slice: above 32 MB of it they stay whole (uniform
     // neighbors, 43 MB 95 / 92, 87 MB 198 / - / 182, but 77 MB, 40 per row, 428 / 436, 256 MB 428 / 454, 512 MB 855 / - / 917); column blocks of 12 MB and
     // more gain without hubs, too (150 K nodes, 150 per row, 256- / 512- / 1,024-byte rows: 631 -> 445, 1,435 -> 1,241, 3,153 -> 2,569).
     int slices = 1, slice_cols = dim;
@@ -1240,7 +1240,7 @@ int run_agg(Plan *plan, float *d_out, const void *d_in_l, const void *d_in_r, co
         const int lines = (dim + 31) / 32;
         const unsigned long long table_mb = ((unsigned long long)plan->real_rows + (plan->nnz_r > 0 ? (unsigned long long)plan->max_col_r + 1 : 0)) * (unsigned long long)ld_in * 4 >> 20;
         if (mode == MODE_F32_VEC4 && lines > 1 && ld_in % 32 == 0 && on_line(d_in_l) && (plan->nnz_r == 0 || on_line(d_in_r)) &&
-            (blocked || !(o.flags & MGGX_AGG_SOFTMAX)) && !(cm && cm->join)) {
+            (blocked || !(o.flags & MGGX_AGG_SOFTMAX)) && !(cm && cm->join) && !plan->d_part_ptr) {
             const bool hubs = blocked || (plan->longest > 0 && (double)plan->longest * plan->rows > 16.0 * plan->num_parts);
             if (lines % 2 == 0 && table_mb >= (lines == 2 ? 32u : 12u)) slices = 2;
             if (lines % 4 == 0 && table_mb >= (lines == 4 ? 80u : 31u) && (lines > 4 || table_mb <= 256u)) slices = 4;

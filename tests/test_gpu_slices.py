@@ -103,7 +103,7 @@ def test_slices_on_a_share_and_in_column_blocks_and_small_workgroups(gpu):
     gpu.forget(d_ptr)
 
 
-def test_slices_of_explicit_partitions_are_bit_identical_in_the_static_form(gpu):
+def test_explicit_partitions_stay_whole_and_bit_identical_in_the_static_form(gpu):
     import torch
     V, dim = 30_000, 128
     ptr, col = csr(V, 2)
@@ -115,7 +115,7 @@ def test_slices_of_explicit_partitions_are_bit_identical_in_the_static_form(gpu)
         out = torch.zeros(V, dim, device="cuda")
         call(out, d_x, d_ptr, d_col, pp, p2n, 0, V, p2n.numel(), 16, dim, 16, 4, 2)
         gpu.sync()
-        assert "slices=2" in gpu.last_agg_kernel()
+        assert "slices=1" in gpu.last_agg_kernel()
         outs.append(out.cpu().numpy())
     assert np.array_equal(outs[0], outs[1])
     want, mag = oracle_agg(share_of(ptr, col, V, 1, 0), x, x, dim)
