@@ -103,7 +103,7 @@ __global__ void __launch_bounds__(SCAN_THREADS) k_scan_tile_offsets(long long *_
 // out[n] and, in 64 bits, to *host_total (pinned host memory, or NULL).
 constexpr int SCAN_SUM_TILES = 1024;
 template <typename F>
-__global__ void __launch_bounds__(SCAN_THREADS) k_scan_apply(const F in, int *__restrict__ out, int n, const long long *__restrict__ tile, int sums_only,
+__global__ void __launch_bounds__(SCAN_THREADS) k_scan_apply(const F in, int *__restrict__ out, int n, long long *__restrict__ tile, int sums_only,
                                                              long long *host_total)
 {
     __shared__ int lds[SCAN_THREADS];
@@ -139,6 +139,7 @@ __global__ void __launch_bounds__(SCAN_THREADS) k_scan_apply(const F in, int *__
     }
     if (blockIdx.x == gridDim.x - 1 && threadIdx.x == SCAN_THREADS - 1) {
         out[n] = (int)run;
+        tile[gridDim.x] = run;
         if (host_total) *host_total = run;
     }
 }
@@ -302,21 +303,24 @@ __global__ void __launch_bounds__(256) k_collect_empty(const int *__restrict__ o
     if (threadIdx.x == 0) atomicMax(counter + 1, max(max(most[0], most[1]), max(most[2], most[3])));
 }
 
-// reference-layout arrays
-__global__ void __launch_bounds__(256) k_parts_ref_layout(const int *__restrict__ indptr, const int *__restrict__ node2part,
-                                                          int num_nodes, int ps, int num_parts, int compat,
-                                                          int *__restrict__ part_ptr, int *__restrict__ part2node)
+// Reference-layout arrays, launched behind the scan that makes node2part, without the host: *d_total is the number of partitions as
+// the scan left it (a total that is no count of 32 bits writes nothing; the host refuses it afterwards).
+__global__ void __launch_bounds__(256) k_parts_ref_layout(const int *__restrict__ indptr, int *__restrict__ node2part, const long long *__restrict__ d_total,
+                                                          int num_nodes, int ps, int compat, int *__restrict__ part_ptr, int *__restrict__ part2node)
 {
-    const int p = blockIdx.x * 256 + threadIdx.x;
-    if (p > num_parts) return;
-    if (p == num_parts) {
+    const long long total = *d_total;
+    if (total < 0 || total > 0x7ffffffeLL) return;
+    const int num_parts = (int)total;
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        node2part[num_nodes + 1] = num_parts;
         const bool last_has = num_nodes > 0 && indptr[num_nodes] > indptr[num_nodes - 1];
-        part_ptr[p] = (compat && !last_has) ? 0 : (num_nodes > 0 ? indptr[num_nodes] : 0);
-        return;
+        part_ptr[num_parts] = (compat && !last_has) ? 0 : (num_nodes > 0 ? indptr[num_nodes] : 0);
     }
-    const int i = row_of_part(node2part, num_nodes, p);
-    part_ptr[p] = indptr[i] + (p - node2part[i]) * ps;
-    part2node[p] = i;
+    for (long long q = (long long)blockIdx.x * 256 + threadIdx.x; q < num_parts; q += (long long)gridDim.x * 256) {
+        const int p = (int)q, i = row_of_part(node2part, num_nodes, p);
+        part_ptr[p] = indptr[i] + (p - node2part[i]) * ps;
+        part2node[p] = i;
+    }
 }
 
 // max over non-negative ints into a word that holds 0; their number is read on the device.  One atomicMax per workgroup that saw
@@ -1167,20 +1171,36 @@ MGGX_EXPORT int mggx_build_part_device(const int *d_indptr, int num_nodes, int p
         if (rc) return rc;
         own_n2p = true;
     }
-    long long total = 0;
+    // One wait for the whole call: the arrays are laid out behind the scan, which leaves the number of partitions on the device.  (Asked
+    // for by the host first, two of a share's set-up's nine waits, 12 to 20 us each with the launch after it.)
+    const bool layout = d_part_ptr && d_part2node;
+    void *tmp = nullptr;
+    long long *w = nullptr;
     do {
-        rc = mggx::scan_total(mggx::ScanParts{d_indptr, d_indptr + 1, nullptr, nullptr, part_size}, d_n2p, num_nodes, &total);
-        if (rc) break;
-        mggx::k_set_tail<<<1, 1, 0, s.stream>>>(d_n2p, num_nodes);
-        *num_parts = (int)total;
-        if (d_part_ptr && d_part2node) {
-            const int n = (int)total + 1;
-            mggx::k_parts_ref_layout<<<(n + 255) / 256, 256, 0, s.stream>>>(d_indptr, d_n2p, num_nodes, part_size, (int)total,
-                                                                            compat, d_part_ptr, d_part2node);
+        if ((rc = mggx::host_words(&w)) || (rc = mggx::dev_alloc(&tmp, mggx::scan_tmp_bytes(num_nodes)))) break;
+        if (num_nodes > 0) {
+            rc = mggx::scan_launch(mggx::ScanParts{d_indptr, d_indptr + 1, nullptr, nullptr, part_size}, d_n2p, num_nodes, tmp, w);
+            if (rc) break;
+        } else {
+            mggx::k_zero_words<<<1, 64, 0, s.stream>>>(d_n2p, 1);
+            mggx::k_zero_words<<<1, 64, 0, s.stream>>>(static_cast<int *>(tmp), 2);
         }
-        if (hipGetLastError() != hipSuccess || hipStreamSynchronize(s.stream) != hipSuccess)
+        if (layout) {
+            const long long *d_total = static_cast<long long *>(tmp) + (num_nodes + mggx::SCAN_TILE - 1) / mggx::SCAN_TILE;
+            mggx::k_parts_ref_layout<<<1024, 256, 0, s.stream>>>(d_indptr, d_n2p, d_total, num_nodes, part_size, compat, d_part_ptr, d_part2node);
+        } else if (!own_n2p) {
+            mggx::k_set_tail<<<1, 1, 0, s.stream>>>(d_n2p, num_nodes);
+        }
+        if (hipGetLastError() != hipSuccess || hipStreamSynchronize(s.stream) != hipSuccess) {
             rc = fail(MGGX_EHIP, "build_part_device: kernel failed");
+            break;
+        }
+        const long long total = num_nodes > 0 ? w[0] : 0;
+        if (total > 0x7fffffffLL) rc = fail(MGGX_ELIMIT, "exclusive_scan: total %lld exceeds int32", total);
+        else if (layout && (total < 0 || total > 0x7ffffffeLL)) rc = fail(MGGX_EHIP, "build_part_device: %lld partitions", total);
+        else *num_parts = (int)total;
     } while (0);
+    mggx::dev_free(tmp);
     if (own_n2p) mggx::dev_free(d_n2p);
     return rc;
 }
@@ -1202,15 +1222,32 @@ MGGX_EXPORT int mggx_split_csr_device(const int *d_ptr, const int *d_col, int lb
         rc = mggx::dev_array(&d_cnt, 2 * (size_t)rows);
         if (rc) return rc;
         long long tl = 0, tr = 0;
+        void *tmp = nullptr;
         do {
             if (rows > 0) {
                 if (!d_col) { rc = fail(MGGX_EINVAL, "split_csr_device: NULL column array"); break; }
                 mggx::k_split_count<<<blocks, 256, 0, s.stream>>>(d_ptr, d_col, lb, ub, d_cnt, d_cnt + rows);
             }
-            rc = mggx::exclusive_scan_i32(d_cnt, d_local_ptr, rows, &tl);
-            if (rc) break;
-            rc = mggx::exclusive_scan_i32(d_cnt + rows, d_remote_ptr, rows, &tr);
+            if (rows == 0) {
+                mggx::k_zero_words<<<1, 64, 0, s.stream>>>(d_local_ptr, 1);
+                mggx::k_zero_words<<<1, 64, 0, s.stream>>>(d_remote_ptr, 1);
+                if (hipGetLastError() != hipSuccess) rc = fail(MGGX_EHIP, "split_csr_device: launch failed");
+                break;
+            }
+            // both scans, one wait
+            long long *w = nullptr;
+            const size_t scan_bytes = mggx::scan_tmp_bytes(rows);
+            if ((rc = mggx::host_words(&w)) || (rc = mggx::dev_alloc(&tmp, 2 * scan_bytes))) break;
+            if ((rc = mggx::scan_launch(mggx::ScanArray{d_cnt}, d_local_ptr, rows, tmp, w)) ||
+                (rc = mggx::scan_launch(mggx::ScanArray{d_cnt + rows}, d_remote_ptr, rows, static_cast<char *>(tmp) + scan_bytes, w + 1)))
+                break;
+            const hipError_t e = hipStreamSynchronize(s.stream);
+            if (e != hipSuccess) rc = fail(MGGX_EHIP, "exclusive_scan: %s", hipGetErrorString(e));
+            else if (std::max(w[0], w[1]) > 0x7fffffffLL) rc = fail(MGGX_ELIMIT, "exclusive_scan: total %lld exceeds int32", std::max(w[0], w[1]));
+            tl = w[0];
+            tr = w[1];
         } while (0);
+        mggx::dev_free(tmp);
         mggx::dev_free(d_cnt);
         if (rc) return rc;
         if (n_local) *n_local = tl;
