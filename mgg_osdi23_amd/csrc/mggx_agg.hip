@@ -17,9 +17,9 @@
 //   wavefronts a row that crosses wavefronts is finished through LDS
 //   workgroups a row that crosses workgroups leaves two partial rows in a
 //              carry buffer; a small second kernel sums them in a fixed order
-// No value is added atomically; the summation order depends only on (ps, wpb, dist, dim) and the size of the tables (slices of
-// columns below).  (Small plans count, with an atomic, which
-// workgroups of a row have left their part: FUSE below.)
+// No value is added atomically; the summation order depends only on (ps, wpb, dist, dim), the size of the tables (slices of columns
+// below) and whether no row is long (whole rows below).  (Small plans count, with an atomic, which workgroups of a row have left their
+// part: FUSE below.)
 // Index stream: a wavefront fetches the descriptors and the first ids of its next few rounds together into its own
 // piece of LDS (two HBM latencies per four rounds instead of per round, with no feature row in flight meanwhile) and
 // the rounds read them from there; the 16 lanes or so of a slot read the same words.
@@ -1515,8 +1515,8 @@ struct Knobs {
 };
 
 // Dense cells (mggx_cells.hip) where a core from LDS would pay and they hold most of the edges.  Least edges of a cell: what it costs
-// over what an edge costs the gather kernel beside it (233 K nodes, 228 M neighbors: 5.1 ns and 7.3 ps at width 16, 14.4 and 18 at 41; the
-// optimum is flat: 700 to 1,400 edges at width 16 and 700 to 2,000 at 41 and 64 are within 2 %).  Least share: graphs of 50 to 233 K nodes
+// over what an edge costs the gather kernel beside it (233 K nodes, 228 M neighbors: 4.9 ns and 7.2 ps at width 16, 13.1 and 18 at 41; the
+// optimum is flat: 850 to 1,700 edges at widths 16, 41 and 64 are within 2 %).  Least share: graphs of 50 to 233 K nodes
 // and mean degrees of 220 to 970 have 69 to 92 % of their edges in such cells and gain 5 to 35 % over the core from LDS at widths 16, 41
 // and 64 (100 K nodes, 51 M neighbors: 172 -> 124, 403 -> 276, 445 -> 328 us); 500 K to 1.5 M nodes of mean degree 57 to 168 have 38
 // to 66 % and lose up to 17 % (1 M nodes, 168 M neighbors, width 64: 2,459 -> 2,797), 233 K nodes of a flatter RMAT (a = 0.45) have 42 to 53 %,

@@ -18,7 +18,7 @@
 //
 // Before this, the core of such a graph came from the LDS, index list by index list, beside the gather kernel (mggx_core.hip, still the
 // faster one where less of a graph lies in cells): GCN on the 233 K-node graph, width 16: 529 -> 381 us per aggregation, width 41:
-// 1,313 -> 965; first use 26 -> 12 ms; error against 64 bits 3.1e-7 -> 1.6e-7 of the result.
+// 1,313 -> 935; first use 26 -> 12 ms; error against 64 bits 3.1e-7 -> 1.6e-7 of the result.
 #include <algorithm>
 #include <chrono>
 #include <cmath>
@@ -329,7 +329,7 @@ struct CellArgs {
     const int *huge;   // [units] of the splitting kernel
     int units;
     float *partial;    // [slot][512][4 n4]
-    int n4, fg;
+    int n4;
     const float *in;   // for sums the matrix cores cannot give (see below)
     const int *order;
     long long ld_in;
@@ -348,9 +348,10 @@ constexpr int PIECES = STEPS * 6 * 64;  // 16-byte pieces of a tile's 16 feature
 // a wavefront of 128 rows reads them at half the LDS's rate.  A cell's products are summed on their own, smallest parts first, before
 // they join the row's sums: four additions at the size of the sum and one, instead of a chain of hundreds (233 K nodes, width 16: one
 // chain 3.5e-7 of the result, this way 1.6e-7).
-// Bound: at width 41 the matrix cores are busy 57 % of the time (330 us for 22,900 cells), the rest goes to the end of the launch, where
-// some shares finish up to a fifth earlier than others, and to waits for the LDS; 1.55 of 2.9 GB come from beyond the L2s.  At width 16
-// 116 us, 375 MB of indexes out of memory among them.  (Shares of about two per place instead of one: 3 - 5 % slower; tiles not in blocks:
+// Bound: at width 41 the matrix cores are busy 61 % of the time (299 us for 22,900 cells, 13.1 ns each; 330 us with an operand read right before
+// its use and the sums kept to the end of the cell), the rest goes to the end of the launch, where some shares finish up to a fifth
+// earlier than others, and to waits for the LDS; 1.55 of 2.9 GB come from beyond the L2s.  At width 16 113 us, 5.5 TB/s from beyond the
+// L2s, 375 MB of indexes out of memory among them.  (Shares of about two per place instead of one: 3 - 5 % slower; tiles not in blocks:
 // 40 % more misses, 3 % slower at width 16.)
 template <int FG, int WAVES>
 __global__ void __launch_bounds__(256, WAVES) k_cells(const CellArgs a)
@@ -360,7 +361,6 @@ __global__ void __launch_bounds__(256, WAVES) k_cells(const CellArgs a)
     if (gate_closed(a.gate)) return;
     const int4 wg = a.wgs[blockIdx.x];  // {first segment, first cell, end cell, -}
     const int lane = (int)(threadIdx.x & 63u), wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
-    const int f0 = FG * (int)blockIdx.y;  // groups of 16 features f0 .. f0 + FG - 1 of a.fg
     int seg = wg.x;
     int4 part = a.segs[seg];            // {row group, first cell, end cell, slot}
     v4f acc[8], sum[FG][8];
@@ -393,7 +393,7 @@ __global__ void __launch_bounds__(256, WAVES) k_cells(const CellArgs a)
     ask_words(wg.y);
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
-        ask(a.tab + ((size_t)tile * a.fg + f0) * PIECES, h);
+        ask(a.tab + (size_t)tile * FG * PIECES, h);
         put(0, h);
     }
     __syncthreads();
@@ -402,7 +402,7 @@ __global__ void __launch_bounds__(256, WAVES) k_cells(const CellArgs a)
         const int next_tile = last ? tile : a.cell_tile[cell + 1];
 #pragma unroll
         for (int f = 0; f < FG; ++f) {
-            const v4u *src = a.tab + ((size_t)(f + 1 < FG ? tile : next_tile) * a.fg + f0 + (f + 1) % FG) * PIECES;  // (after the last cell: not used)
+            const v4u *src = a.tab + ((size_t)(f + 1 < FG ? tile : next_tile) * FG + (f + 1) % FG) * PIECES;  // (after the last cell: not used)
             ask(src, 0);
             unsigned touched = 0;  // brings the next cell's words into the L2
             if (f == 0 && lane < LANE_WORDS * 2) touched = a.words[(size_t)(last ? cell : cell + 1) * CELL_WORDS + wave * (LANE_WORDS * 64) + lane * 32];
@@ -464,12 +464,12 @@ __global__ void __launch_bounds__(256, WAVES) k_cells(const CellArgs a)
             for (int rb = 0; rb < 8; ++rb)
 #pragma unroll
                 for (int t = 0; t < 4; ++t) check += 0.f * sum[f][rb][t];
-            if (16 * (f0 + f) + (lane & 15) < w4) {
+            if (16 * f + (lane & 15) < w4) {
 #pragma unroll
                 for (int rb = 0; rb < 8; ++rb)
 #pragma unroll
                     for (int t = 0; t < 4; ++t) {
-                        (out + 16 * (f0 + f) + (16 * rb + t) * w4)[first] = sum[f][rb][t] * DOWN;
+                        (out + 16 * f + (16 * rb + t) * w4)[first] = sum[f][rb][t] * DOWN;
                         __builtin_amdgcn_sched_barrier(0);
                     }
             }
@@ -484,7 +484,7 @@ __global__ void __launch_bounds__(256, WAVES) k_cells(const CellArgs a)
         }
         if (again) {
             asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // what follows writes the same rows again, other lanes their columns
-            const int d = 16 * f0 + lane;
+            const int d = lane;
             const bool on = lane < 16 * FG && d < a.dim;
             for (int r = 0; r < 128; ++r) {
                 float s = 0.f;
@@ -722,7 +722,7 @@ int cells_sums(const CorePlan *p, const float *d_in, int dim, long long ld_in, c
     k_cells_stage<<<(unsigned)((units + 3) / 4), 256, 0, stream>>>(tab, huge, d_in, p->d_order, fg, dim, ld_in, units, gate);
     MGGX_LAUNCH_CHECK("k_cells_stage");
     const CorePlan::Cut &cut = p->cuts[0];
-    const CellArgs a{p->d_words, p->d_cell_tile, cut.d_wgs, cut.d_wgs + cut.nwg, tab, huge, units, reinterpret_cast<float *>(partial), n4, fg, d_in, p->d_order, ld_in, dim, gate};
+    const CellArgs a{p->d_words, p->d_cell_tile, cut.d_wgs, cut.d_wgs + cut.nwg, tab, huge, units, reinterpret_cast<float *>(partial), n4, d_in, p->d_order, ld_in, dim, gate};
     switch (fg) {
         case 1: k_cells<1, 3><<<(unsigned)cut.nwg, 256, 0, stream>>>(a); break;
         case 2: k_cells<2, 2><<<(unsigned)cut.nwg, 256, 0, stream>>>(a); break;

@@ -144,6 +144,83 @@ __global__ void __launch_bounds__(256) k_look_up(const int *__restrict__ col, lo
     }
 }
 
+// ---- ids by falling count
+//
+// Stable counting passes over COUNT_BITS bits of the counts at a time: how often each digit occurs in each tile of COUNT_TILE pairs, the
+// exclusive sums of that table digit by digit (the largest first), and every pair to its place.  Bound: a chain of four short launches per pass,
+// two passes up to 4 M edges.  rocPRIM merges up to a million pairs, some 20 launches one behind the other, and goes digit by digit
+// beyond, in passes that last 23 us however few pairs there are: it stays where merging takes few launches and where the pairs are many (both
+// calls of the staging list, us, rocPRIM / this: 1,352 distinct ids 123 / 167, 32,506 219 / 226, 243 K 373 / 329, 817 K 410 / 333, 2.7 M 702 / 803, 10.3 M
+// 2,673 / 3,575; set-up of an eighth of 1 M nodes 709 -> 646).
+constexpr int COUNT_LEAST = 1 << 15, COUNT_MOST = 1 << 20;
+constexpr int COUNT_BITS = 11, COUNT_DIGITS = 1 << COUNT_BITS, COUNT_TILE = 2048, COUNT_STEPS = COUNT_TILE / 256;
+
+__device__ __forceinline__ int falling_digit(unsigned count, int shift) { return COUNT_DIGITS - 1 - (int)(count >> shift & (COUNT_DIGITS - 1)); }
+
+__global__ void __launch_bounds__(256) k_count_digits(const unsigned *__restrict__ cnt, int u, int shift, int tiles, int *__restrict__ table)
+{
+    __shared__ int seen[COUNT_DIGITS];
+    for (int d = threadIdx.x; d < COUNT_DIGITS; d += 256) seen[d] = 0;
+    __syncthreads();
+    const int base = (int)blockIdx.x * COUNT_TILE;
+#pragma unroll
+    for (int k = 0; k < COUNT_STEPS; ++k) {
+        const int i = base + k * 256 + (int)threadIdx.x;
+        if (i < u) atomicAdd(&seen[falling_digit(cnt[i], shift)], 1);
+    }
+    __syncthreads();
+    for (int d = threadIdx.x; d < COUNT_DIGITS; d += 256) table[(size_t)d * tiles + blockIdx.x] = seen[d];
+}
+
+// A wavefront goes over its quarter of the tile 64 pairs at a time, in order; a pair's place among those of its digit is what the wavefronts before
+// have of that digit, what this one has seen of it, and how many lanes before it hold it.
+__global__ void __launch_bounds__(256) k_place_by_digit(const unsigned *__restrict__ cnt, const int *__restrict__ ids, int u, int shift, int tiles, const int *__restrict__ table,
+                                                        unsigned *__restrict__ cnt_out, int *__restrict__ ids_out)
+{
+    __shared__ unsigned short seen[4][COUNT_DIGITS];
+    for (int d = threadIdx.x; d < 4 * COUNT_DIGITS; d += 256) (&seen[0][0])[d] = 0;
+    __syncthreads();
+    const int lane = (int)(threadIdx.x & 63u), wave = (int)(threadIdx.x >> 6);
+    const int base = (int)blockIdx.x * COUNT_TILE + wave * (COUNT_TILE / 4);
+    unsigned c[COUNT_STEPS];
+    int place[COUNT_STEPS];
+#pragma unroll
+    for (int k = 0; k < COUNT_STEPS; ++k) {
+        const int i = base + 64 * k + lane;
+        c[k] = i < u ? cnt[i] : 0;
+    }
+#pragma unroll
+    for (int k = 0; k < COUNT_STEPS; ++k) {
+        const bool on = base + 64 * k + lane < u;
+        const int d = falling_digit(c[k], shift);
+        unsigned long long same = __ballot(on);
+#pragma unroll
+        for (int b = 0; b < COUNT_BITS; ++b) {
+            const unsigned long long set = __ballot(d >> b & 1);
+            same &= d >> b & 1 ? set : ~set;
+        }
+        const int before = __popcll(same & ((1ull << lane) - 1));
+        place[k] = 0;
+        if (on) place[k] = seen[wave][d] + before;
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        if (on && before == 0) seen[wave][d] = (unsigned short)(seen[wave][d] + __popcll(same));
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+    }
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < COUNT_STEPS; ++k) {
+        const int i = base + 64 * k + lane;
+        if (i >= u) continue;
+        const int d = falling_digit(c[k], shift);
+        int to = table[(size_t)d * tiles + blockIdx.x] + place[k];
+        for (int w = 0; w < wave; ++w) to += seen[w][d];
+        cnt_out[to] = c[k];
+        ids_out[to] = ids[i];
+    }
+}
+
 struct DeviceBuffers {
     std::vector<void *> ptrs;
     ~DeviceBuffers()
@@ -246,11 +323,31 @@ MGGX_EXPORT int mggx_compact_remote_device(const int *d_remote_col, int64_t n_re
     if (!dense) mggx::k_iota<<<(u + 255) / 256, 256, 0, stream>>>(iota, u);
     const int *from = dense ? ids : iota;
     int *to = dense ? d_fetch_ids : order;
-    need = 0;
-    MGGX_HIP(rocprim::radix_sort_pairs_desc(nullptr, need, cnt, cnt_sorted, from, to, (size_t)u, 0, bits_of((long long)n), stream));
-    char *tmp2 = tmp;
-    if (need > tmp_bytes && (rc = buf.get(&tmp2, need))) return rc;
-    MGGX_HIP(rocprim::radix_sort_pairs_desc(tmp2, need, cnt, cnt_sorted, from, to, (size_t)u, 0, bits_of((long long)n), stream));
+    if (u >= mggx::COUNT_LEAST && u <= mggx::COUNT_MOST) {
+        const int passes = ((int)bits_of((long long)n) + mggx::COUNT_BITS - 1) / mggx::COUNT_BITS, tiles = (u + mggx::COUNT_TILE - 1) / mggx::COUNT_TILE;
+        const long long entries = (long long)tiles * mggx::COUNT_DIGITS;
+        int *digits = nullptr, *places = nullptr, *ids_between = nullptr;
+        char *scan_tmp = nullptr;
+        if ((rc = buf.get(&digits, (size_t)entries)) || (rc = buf.get(&places, (size_t)entries + 1)) || (rc = buf.get(&ids_between, (size_t)u)) ||
+            (rc = buf.get(&scan_tmp, mggx::scan_tmp_bytes((int)entries))))
+            return rc;
+        unsigned *cnt_from = cnt, *cnt_to = cnt_sorted;
+        const int *ids_from = from;
+        for (int p = 0; p < passes; ++p) {
+            int *ids_to = (passes - p) % 2 ? to : ids_between;  // the last pass writes `to`
+            mggx::k_count_digits<<<(unsigned)tiles, 256, 0, stream>>>(cnt_from, u, p * mggx::COUNT_BITS, tiles, digits);
+            if ((rc = mggx::exclusive_scan_i32_device(digits, places, (int)entries, scan_tmp))) return rc;
+            mggx::k_place_by_digit<<<(unsigned)tiles, 256, 0, stream>>>(cnt_from, ids_from, u, p * mggx::COUNT_BITS, tiles, places, cnt_to, ids_to);
+            std::swap(cnt_from, cnt_to);
+            ids_from = ids_to;
+        }
+    } else {
+        need = 0;
+        MGGX_HIP(rocprim::radix_sort_pairs_desc(nullptr, need, cnt, cnt_sorted, from, to, (size_t)u, 0, bits_of((long long)n), stream));
+        char *tmp2 = tmp;
+        if (need > tmp_bytes && (rc = buf.get(&tmp2, need))) return rc;
+        MGGX_HIP(rocprim::radix_sort_pairs_desc(tmp2, need, cnt, cnt_sorted, from, to, (size_t)u, 0, bits_of((long long)n), stream));
+    }
     if (dense) {
         mggx::k_places<<<(u + 255) / 256, 256, 0, stream>>>(d_fetch_ids, u, place);
         mggx::k_look_up<<<edge_blocks, 256, 0, stream>>>(d_remote_col, (long long)n, place, d_remote_col_compact);

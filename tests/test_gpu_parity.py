@@ -1138,6 +1138,20 @@ def test_compact_remote_device_dense_and_sparse_ids(gpu, n, largest):
         gpu.compact_remote_device(to_dev(col), n)
 
 
+@pytest.mark.parametrize("distinct,spread", [(32_767, 1), (32_768, 1), (34_816, 1), (34_817, 3), (50_000, 200), (1 << 20, 1), ((1 << 20) + 1, 1)])
+def test_compact_remote_device_orders_by_count(gpu, distinct, spread):
+    """The staging order where the library's own counting passes make it and on either side of their range: full and ragged tiles, counts of
+    one and of several digits (2,047, 2,048 and 5,000 on ids in different tiles), many ids of equal count, dense and sparse ids."""
+    rng = np.random.default_rng(distinct)
+    count = rng.integers(1, 4, distinct)
+    count[[1, distinct // 2, distinct - 1]] = [2_048, 5_000, 2_047]
+    count[2_040:2_060] = 2_048
+    col = rng.permutation(np.repeat(np.arange(distinct) * spread, count)).astype(np.int32)
+    want, want_ids = gpu.compact_remote(col)
+    got, got_ids = gpu.compact_remote_device(to_dev(col), len(col))
+    assert np.array_equal(got_ids.cpu().numpy(), want_ids) and np.array_equal(got.cpu().numpy(), want)
+
+
 @pytest.mark.parametrize("lens", [[64, 65, 127, 128, 129, 0, 1], [511, 512, 513, 640, 641], [20_000, 3, 700, 0, 191]])
 def test_split_csr_device_rows_of_many_chunks(gpu, lens):
     """Rows around the number of neighbors a wavefront takes at a time, and one of thousands: the device split is the host's."""
