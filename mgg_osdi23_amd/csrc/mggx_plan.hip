@@ -144,12 +144,20 @@ __global__ void __launch_bounds__(SCAN_THREADS) k_scan_apply(const F in, int *__
     }
 }
 
-// Results of a set-up call for the host: words[0] = the value at a, words[1] at b, words[2] at c (NULL: 0).
-__global__ void k_publish(const int *a, const int *b, const int *c, long long *words)
+// Results of a set-up call for the host: words[0] = the value at a, words[1] at b, words[2] at c, words[3] at d, words[4] at e (NULL: 0).
+__global__ void k_publish(const int *a, const int *b, const int *c, long long *words, const int *d = nullptr, const int *e = nullptr)
 {
     words[0] = a ? *a : 0;
     words[1] = b ? *b : 0;
     words[2] = c ? *c : 0;
+    words[3] = d ? *d : 0;
+    words[4] = e ? *e : 0;
+}
+
+__global__ void k_clear_plan(int *counter, int n, unsigned long long *chain, int workgroups)
+{
+    for (int i = threadIdx.x; i < n; i += blockDim.x) counter[i] = 0;
+    for (int i = threadIdx.x; i < workgroups; i += blockDim.x) chain[i] = 0;
 }
 
 __global__ void k_zero_words(int *w, int n)
@@ -667,28 +675,27 @@ void plan_free(Plan *p)
     delete p;
 }
 
-// Rows without partitions, and what the host needs to know of a plan, in one wait: words[0] = number of those rows,
-// words[1] = *d_a, words[2] = *d_b (NULL: 0).
-static int plan_finish(Plan *p, const int *d_a, const int *d_b, long long **words)
+// Rows without partitions, and what the host needs to know of a plan, in one wait: words[1] = number of those rows,
+// words[2] = *d_a, words[3] = *d_b (of plans by the library the most descriptors of a row), words[4] = largest of the *d_cnt_r ids in d_col_r,
+// words[5] = *d_cnt_r (NULL: 0).  Each launch here is 4 to 5 us of a plan's build, whatever it does: everything is cleared in one.
+static int plan_finish(Plan *p, const int *d_a, const int *d_b, long long **words, const int *d_col_r = nullptr, const int *d_cnt_r = nullptr)
 {
     State &s = state();
-    int *d_counter = nullptr;
+    int *d_counter = nullptr;  // rows without partitions, longest row, largest remote id
     int rc = host_words(words);
-    if (!rc) rc = dev_array(&d_counter, 2);
+    if (!rc) rc = dev_array(&d_counter, 3);
     if (!rc) rc = dev_array(&p->d_empty_rows, (size_t)p->rows);
-    const bool plain = p->blocks == 1 && !p->d_part_ptr;
-    if (!rc && plain) {  // (the caller's partition arrays may list a row's partitions apart)
-        rc = dev_array(&p->d_chain, FUSE_MAX_WORKGROUPS);
-        if (!rc) k_zero_words<<<1, 1024, 0, s.stream>>>(reinterpret_cast<int *>(p->d_chain), 2 * FUSE_MAX_WORKGROUPS);
-    }
+    const bool plain = p->blocks == 1 && !p->d_part_ptr;  // (the caller's partition arrays may list a row's partitions apart)
+    if (!rc && plain) rc = dev_array(&p->d_chain, FUSE_MAX_WORKGROUPS);
     if (rc) {
         dev_free(d_counter);
         return rc;
     }
-    long long *const w = *words + 1;  // word 0 holds the total of a scan in flight
-    k_zero_words<<<1, 64, 0, s.stream>>>(d_counter, 2);
+    k_clear_plan<<<1, 1024, 0, s.stream>>>(d_counter, 3, p->d_chain, plain ? FUSE_MAX_WORKGROUPS : 0);
+    if (d_col_r && d_cnt_r) k_max_i32<<<256, 256, 0, s.stream>>>(d_col_r, d_cnt_r, d_counter + 2);
     if (p->rows > 0) k_collect_empty<<<(p->rows + 255) / 256, 256, 0, s.stream>>>(p->d_off, p->rows, p->d_empty_rows, d_counter);
-    k_publish<<<1, 1, 0, s.stream>>>(d_counter, d_a, plain ? d_counter + 1 : d_b, w);
+    long long *const w = *words + 1;  // word 0 holds the total of a scan in flight
+    k_publish<<<1, 1, 0, s.stream>>>(d_counter, d_a, plain ? d_counter + 1 : d_b, w, d_counter + 2, d_cnt_r);
     const hipError_t el = hipGetLastError(), e = hipStreamSynchronize(s.stream);
     dev_free(d_counter);
     if (el != hipSuccess || e != hipSuccess) return fail(MGGX_EHIP, "plan: %s", hipGetErrorString(el != hipSuccess ? el : e));
@@ -794,7 +801,6 @@ int plan_get(const int *d_ptr_l, const int *d_ptr_r, const int *d_col_r, int row
     p->unit = unit_of(ps);
     const int unit = p->unit;  // neighbors per descriptor: whole partitions of one row and side, at most 16 neighbors (ps < 16)
     int rc = MGGX_OK;
-    int *d_max = nullptr;
     void *scan_tmp = nullptr;
     do {
         // One wait for everything the host needs: the number of descriptors, the edge counts, the largest remote id, the
@@ -802,20 +808,17 @@ int plan_get(const int *d_ptr_l, const int *d_ptr_r, const int *d_col_r, int row
         if ((rc = dev_array(&p->d_off, (size_t)rows + 1))) break;
         const bool remote = d_ptr_r && rows > 0;
         if (rows > 0) {
-            if ((rc = dev_alloc(&scan_tmp, scan_tmp_bytes(rows))) || (rc = dev_array(&d_max, 1))) break;
+            if ((rc = dev_alloc(&scan_tmp, scan_tmp_bytes(rows)))) break;
             long long *w = nullptr;
             if ((rc = host_words(&w))) break;
             rc = scan_launch(ScanParts{d_ptr_l, d_ptr_l + 1, d_ptr_r, d_ptr_r ? d_ptr_r + 1 : nullptr, unit}, p->d_off, rows, scan_tmp, w);
             if (rc) break;
-            k_zero_words<<<1, 64, 0, s.stream>>>(d_max, 1);
-            if (remote && d_col_r) k_max_i32<<<256, 256, 0, s.stream>>>(d_col_r, d_ptr_r + rows, d_max);
-            k_publish<<<1, 1, 0, s.stream>>>(d_max, d_ptr_r ? d_ptr_r + rows : nullptr, nullptr, w + 8);
         } else if (hipMemsetAsync(p->d_off, 0, sizeof(int), s.stream) != hipSuccess) {
             rc = fail(MGGX_EHIP, "plan: row offsets");
             break;
         }
         long long *w = nullptr;
-        if ((rc = plan_finish(p, rows > 0 ? d_ptr_l + rows : nullptr, nullptr, &w))) break;
+        if ((rc = plan_finish(p, rows > 0 ? d_ptr_l + rows : nullptr, nullptr, &w, remote ? d_col_r : nullptr, remote ? d_ptr_r + rows : nullptr))) break;
         if (rows > 0) {
             if (w[0] > 0x7fffffffLL) {
                 rc = fail(MGGX_ELIMIT, "exclusive_scan: total %lld exceeds int32", w[0]);
@@ -823,13 +826,13 @@ int plan_get(const int *d_ptr_l, const int *d_ptr_r, const int *d_col_r, int row
             }
             p->num_parts = (int)w[0];
             p->nnz_l = w[2];
-            p->nnz_r = w[9];
+            p->nnz_r = w[5];
             if (p->nnz_r > 0) {
                 if (!d_col_r) {
                     rc = fail(MGGX_EINVAL, "plan: remote edges but no remote column array");
                     break;
                 }
-                p->max_col_r = (int)w[8];
+                p->max_col_r = (int)w[4];
             }
         }
         if ((rc = dev_array(&p->d_desc, (size_t)p->num_parts))) break;
@@ -843,7 +846,6 @@ int plan_get(const int *d_ptr_l, const int *d_ptr_r, const int *d_col_r, int row
         }
     } while (0);
     dev_free(scan_tmp);
-    dev_free(d_max);
     if (rc) {
         plan_free(p);
         return rc;
