@@ -1174,7 +1174,7 @@ MGGX_EXPORT int mggx_build_part_device(const int *d_indptr, int num_nodes, int p
         own_n2p = true;
     }
     // One wait for the whole call: the arrays are laid out behind the scan, which leaves the number of partitions on the device.  (Asked
-    // for by the host first, two of a share's set-up's nine waits, 12 to 20 us each with the launch after it.)
+    // for by the host first, and waited for again behind a launch of one thread: four of the fifteen waits of a share's set-up, some 12 us each.)
     const bool layout = d_part_ptr && d_part2node;
     void *tmp = nullptr;
     long long *w = nullptr;
