@@ -307,7 +307,9 @@ int mggx_sag_np_div(float *d_out, const void *d_in_local, const void *d_in_remot
  * counting (a plan built a moment ago runs slower for its first calls) -- returns the fastest setting and its time (ms
  * per call in that last round), and
  * remembers it, so later mggx_sag_np_div calls on the same CSR arrays with the same dim and in_dtype that leave
- * wpb = dist = col_block_rows = core_rows = 0 (and ps = 0 or the winning ps) use it.  d_out holds a valid result afterwards.
+ * wpb = dist = col_block_rows = core_rows = 0 (and ps = 0 or the winning ps) use it.  Where the library's own choice of wpb and dist
+ * wins, later calls leave both to the library as the measured ones did (only then may it take whole rows per workgroup), and *best
+ * holds the numbers it chose.  d_out holds a valid result afterwards.
  * Synchronises; not for stream capture.  MGGX_AGG_ACCUMULATE is rejected (the repeated runs would add up).
  * Either out-pointer may be NULL. */
 int mggx_sag_np_div_tune(float *d_out, const void *d_in_local, const void *d_in_remote,

@@ -1850,7 +1850,10 @@ MGGX_EXPORT int mggx_sag_np_div_tune(float *d_out, const void *d_in_local, const
     rc = mggx::run_knobs(*g, bk, d_out, d_in_local, d_in_remote, d_ptr_l, d_col_l, d_ptr_r, d_col_r, lb, ub, dim, o, gate);
     if (rc) return rc;
     MGGX_HIP(hipStreamSynchronize(st.stream));
-    if (bk.wpb == 0 || bk.dist == 0) {  // the rule's setting won: report what the rule made of it for this plan
+    // Remembered as it was measured: where the rule's setting won, wpb and dist stay 0, because passed as numbers they fix the grid and
+    // with it the form of the kernel (whole rows per workgroup only where the library chooses both).  Reported is what the rule made of them.
+    const mggx::Knobs won = bk;
+    if (bk.wpb == 0 || bk.dist == 0) {
         const char *w = strstr(st.last_kernel, " wpb=");
         int rw = 0, rd = 0;
         if (w && sscanf(w, " wpb=%d dist=%d", &rw, &rd) == 2) { bk.wpb = rw; bk.dist = rd; }
@@ -1860,8 +1863,8 @@ MGGX_EXPORT int mggx_sag_np_div_tune(float *d_out, const void *d_in_local, const
                     (st.plan_build_ms + st.core_plan_build_ms - build_ms0);
     bool found = false;
     for (mggx::GraphInfo::Tuned &t : g->tuned)
-        if (t.dim == dim && t.dtype == o.in_dtype) { t.ps = bk.ps; t.wpb = bk.wpb; t.dist = bk.dist; t.block_rows = bk.block_rows; t.core_rows = bk.core_rows; t.cells = bk.cells; found = true; }
-    if (!found) g->tuned.push_back({dim, o.in_dtype, bk.ps, bk.wpb, bk.dist, bk.block_rows, bk.core_rows, bk.cells});
+        if (t.dim == dim && t.dtype == o.in_dtype) { t.ps = won.ps; t.wpb = won.wpb; t.dist = won.dist; t.block_rows = won.block_rows; t.core_rows = won.core_rows; t.cells = won.cells; found = true; }
+    if (!found) g->tuned.push_back({dim, o.in_dtype, won.ps, won.wpb, won.dist, won.block_rows, won.core_rows, won.cells});
     if (best_out) { best_out->ps = bk.ps; best_out->wpb = bk.wpb; best_out->dist = bk.dist; best_out->col_block_rows = bk.block_rows; best_out->core_rows = bk.cells ? 0 : bk.core_rows; }
     if (ms_best) *ms_best = best;
     return MGGX_OK;

@@ -159,4 +159,17 @@ FAKE hipError_t hipDeviceSynchronize() { return g_sync_fails ? result(hipErrorSt
 FAKE hipError_t hipStreamSynchronize(hipStream_t) { return hipSuccess; }
 FAKE hipError_t hipStreamWaitEvent(hipStream_t, hipEvent_t, unsigned) { return hipSuccess; }
 FAKE hipError_t hipEventRecord(hipEvent_t, hipStream_t) { return hipSuccess; }
+FAKE hipError_t hipEventCreate(hipEvent_t *e)
+{
+    *e = nullptr;
+    return hipSuccess;
+}
+FAKE hipError_t hipEventDestroy(hipEvent_t) { return hipSuccess; }
+FAKE hipError_t hipEventSynchronize(hipEvent_t) { return hipSuccess; }
+FAKE hipError_t hipEventElapsedTime(float *ms, hipEvent_t, hipEvent_t)  // every measurement is faster than the one before: the last candidate wins
+{
+    static float t = 1e6f;
+    *ms = t *= 0.99f;
+    return hipSuccess;
+}
 FAKE hipError_t hipFuncSetAttribute(const void *, hipFuncAttribute, int) { return hipSuccess; }

@@ -108,6 +108,35 @@ for rows, parts, ps, dim in sizes:
     assert sum(l.startswith("True") for l in out) > 100 and sum(l.startswith("False") for l in out) > 100
 
 
+@pytest.mark.parametrize("dim,longest,whole", [(41, 2, 1), (64, 2, 1), (64, 50, 0)])
+def test_a_search_that_the_rule_wins_leaves_the_rule_in_place(without_device, dim, longest, whole):
+    """mggx_sag_np_div_tune measures the library's own choice beside its grid.  Where that wins, later calls that leave the knobs at 0 run
+    what was measured, in the same form (whole rows per workgroup), and a call with the numbers the search reports the same grid."""
+    out = without_device(r'''
+rows, dim, parts = 4096, DIM, 6286
+ptr, col, x = malloc(4 * (rows + 1)), malloc(4), malloc(4)
+out = malloc(4 * rows * dim)
+C.memset(ptr, 0, 4 * (rows + 1))
+C.memmove(ptr + 4 * rows, C.byref(C.c_int(16 * parts)), 4)
+n = C.c_int()
+assert lib.mggx_build_part_device(at(ptr), 16, 16, 1, None, None, None, C.byref(n)) == 0  # (makes the words that set-up kernels report in)
+for word, v in ((0, parts), (1, 0), (2, 16 * parts), (3, LONGEST), (4, 0), (5, 0)):  # what the kernels of a plan's build report
+    fake.fake_word(word, C.c_longlong(v))
+args = (at(out), at(x), None, at(ptr), at(col), None, None, 0, rows, dim, rows)
+def call(ps=0, wpb=0, dist=0):
+    assert lib.mggx_sag_np_div(*args, ps, wpb, dist, None) == 0, lib.mggx_last_error()
+    return host.last_agg_kernel()
+by_rule = call()
+assert "whole=WHOLE " in by_rule, by_rule
+k, ms = host._AggKnobs(), C.c_float()
+assert lib.mggx_sag_np_div_tune(*args, 0, None, C.byref(k), C.byref(ms)) == 0, lib.mggx_last_error()
+assert host.last_agg_kernel() == by_rule and call() == by_rule, (by_rule, host.last_agg_kernel())
+grid = re.compile("parts=.* dist=.* addr")
+assert k.wpb > 0 and k.dist > 0 and grid.search(call(k.ps, k.wpb, k.dist)).group(0) == grid.search(by_rule).group(0)
+'''.replace("DIM", str(dim)).replace("LONGEST", str(longest)).replace("WHOLE", str(whole)))
+    assert out == ""
+
+
 @pytest.mark.parametrize("ask", ["malloc", "tables", "workspace", "plan"])
 def test_kept_blocks_go_where_memory_is_short(without_device, ask):
     """Set-up calls keep their device blocks for the next ones.  Every allocation of the library's that finds no memory frees
