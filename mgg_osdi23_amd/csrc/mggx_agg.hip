@@ -1573,7 +1573,7 @@ int resolve_knobs(GraphInfo &g, int dim, int dtype, int ps, int wpb, int dist, i
 }
 
 // `gate`: the call's content check of the caller's CSR arrays; every kernel launched below looks at it first.
-int run_knobs(const GraphInfo &g, const Knobs &k, float *d_out, const void *d_in_local, const void *d_in_remote, const int *d_ptr_l,
+int run_knobs(GraphInfo &g, const Knobs &k, float *d_out, const void *d_in_local, const void *d_in_remote, const int *d_ptr_l,
               const int *d_col_l, const int *d_ptr_r, const int *d_col_r, int lb, int ub, int dim, const mggx_agg_opts &o, const Gate &gate, CoreMerge *cm = nullptr)
 {
     Plan *plan = nullptr;
@@ -1581,9 +1581,8 @@ int run_knobs(const GraphInfo &g, const Knobs &k, float *d_out, const void *d_in
     const bool core_call = g.nnz_r == 0 && g.nnz_l > 0 && d_col_l && o.in_dtype == MGGX_F32 && dim >= 1 && dim <= 64 && d_out && d_in_local;
     CorePlan *cp = nullptr;
     if (k.cells > 0 && core_call) {
-        rc = cells_plan_get(d_ptr_l, d_col_l, ub - lb, lb, dim, k.cells, g.nnz_l, k.cells_share, g.serial, &cp);
+        rc = cells_plan_get(g, lb, dim, k.cells, k.cells_share, &cp);  // (none: the core from LDS, if one was asked for as well)
         if (rc) return rc;
-        if (cp->unsuitable) cp = nullptr;  // the core from LDS, if one was asked for as well
     }
     if (!cp && k.core_rows > 0 && core_call && ub - lb >= 1024) {
         rc = core_plan_get(d_ptr_l, d_col_l, ub - lb, lb, k.core_rows, core_group_rows((dim + 3) / 4, std::min(k.core_rows, ub - lb)), g.serial, &cp);
@@ -1714,10 +1713,10 @@ MGGX_EXPORT int mggx_cells_prepare(const int *d_ptr_l, const int *d_col_l, const
     if (rc) return rc;
     if (g->nnz_r > 0 || g->nnz_l < 1) return fail(MGGX_EINVAL, "cells_prepare: %lld local and %lld remote edges (local only)", (long long)g->nnz_l, (long long)g->nnz_r);
     mggx::CorePlan *p = nullptr;
-    rc = mggx::cells_plan_get(d_ptr_l, d_col_l, ub - lb, lb, dim, least_edges, g->nnz_l, 0.0, g->serial, &p);
+    rc = mggx::cells_plan_get(*g, lb, dim, least_edges, 0.0, &p);
     if (rc) return rc;
-    if (num_cells) *num_cells = p->unsuitable ? 0 : p->ncells;
-    if (num_edges) *num_edges = p->unsuitable ? 0 : p->core_nnz;
+    if (num_cells) *num_cells = p ? p->ncells : 0;
+    if (num_edges) *num_edges = p ? p->core_nnz : 0;
     for (mggx::GraphInfo::CellsAsked &c : g->cells_asked)
         if (c.dim == dim) {
             c.least = least_edges;

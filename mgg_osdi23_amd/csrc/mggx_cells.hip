@@ -563,7 +563,7 @@ int groups_of(int dim) { return (dim + 15) / 16; }
 constexpr size_t L2_SHARE = (size_t)2800 << 10;   // split features of a block of column tiles: most of an XCD's 4 MB
 int workgroups(int dim) { return 256 * (dim <= 16 ? 3 : 2); }  // as many as 256 CUs hold at once (k_cells' launch bounds)
 
-int build(CorePlan *p, int dim, long long nnz, double least_share)
+int build(CorePlan *p, int dim, long long nnz, double least_share, double *share)
 {
     State &s = state();
     const int rows = p->rows, lb = p->lb;
@@ -626,7 +626,8 @@ int build(CorePlan *p, int dim, long long nnz, double least_share)
             group_of.push_back(g);
             group_end.push_back(ncells);
         }
-    if (ncells == 0 || (double)in_cells < least_share * (double)nnz) {
+    *share = (double)in_cells / (double)nnz;
+    if (ncells == 0 || *share < least_share) {
         p->unsuitable = true;
         return MGGX_OK;
     }
@@ -741,11 +742,13 @@ int cells_sums(const CorePlan *p, const float *d_in, int dim, long long ld_in, c
 }
 
 // p->asked: least edges of a cell.  A plan whose cells hold less than least_share of the edges, one of a CSR with parallel edges, or one there
-// is no memory for is marked unsuitable.
-int cells_plan_build(CorePlan *p, int dim, long long nnz, double least_share)
+// is no memory for is marked unsuitable.  *share: what the cells hold, -1 in the last two cases.
+int cells_plan_build(CorePlan *p, int dim, long long nnz, double least_share, double *share)
 {
-    const int rc = build(p, dim, nnz, least_share);
+    *share = -1.0;
+    const int rc = build(p, dim, nnz, least_share, share);
     if (rc == MGGX_ENOMEM) {
+        *share = -1.0;
         p->unsuitable = true;
         return MGGX_OK;
     }

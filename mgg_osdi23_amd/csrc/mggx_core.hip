@@ -754,49 +754,50 @@ static int core_plan_build_device(CorePlan *p, int tc)
     return MGGX_OK;
 }
 
-static int find_or_build(const int *d_ptr_l, const int *d_col_l, int rows, int lb, int core, int group_rows, int cells, int dim, long long nnz, double least_share,
-                         int graph_serial, CorePlan **out)
+// The cached plan of this key, now the most recently used one, or NULL.
+static CorePlan *core_plan_find(const int *d_ptr_l, const int *d_col_l, int rows, int lb, int asked, int group_rows, int cells, int graph_serial)
 {
     State &s = state();
     for (size_t i = 0; i < s.cores.size(); ++i) {
         CorePlan *p = s.cores[i];
         // a plan belongs to the graph record it was built under (see drop_plans_of_record): it carries its own copy of that
         // graph's remaining CSR and index lists, and a later record of the same addresses may stand for another graph
-        if (p->d_ptr_l == d_ptr_l && p->d_col_l == d_col_l && p->rows == rows && p->lb == lb && p->asked == core && p->group_rows == group_rows &&
+        if (p->d_ptr_l == d_ptr_l && p->d_col_l == d_col_l && p->rows == rows && p->lb == lb && p->asked == asked && p->group_rows == group_rows &&
             p->cells == cells && p->graph_serial == graph_serial) {
             if (i + 1 != s.cores.size()) {  // most recently used last
                 s.cores.erase(s.cores.begin() + (long)i);
                 s.cores.push_back(p);
             }
             if (!p->pinned && capturing()) p->pinned = true;
-            *out = p;
-            return MGGX_OK;
+            return p;
         }
     }
+    return nullptr;
+}
+
+// A plan of this key, empty so far and not in the cache.
+static int core_plan_new(const int *d_ptr_l, const int *d_col_l, int rows, int lb, int asked, int group_rows, int cells, int graph_serial, CorePlan **out)
+{
     if (rows < 1 || !d_ptr_l || !d_col_l) return fail(MGGX_EINVAL, "core plan: empty or NULL CSR");
     if (capturing()) return fail(MGGX_EINVAL, "core plan: first use of this CSR and core size inside a stream capture; call once outside the capture first");
-    const auto t0 = std::chrono::steady_clock::now();
-    MGGX_HIP(hipStreamSynchronize(s.stream));
+    MGGX_HIP(hipStreamSynchronize(state().stream));
     CorePlan *p = new (std::nothrow) CorePlan;
     if (!p) return fail(MGGX_ENOMEM, "core plan");
     p->d_ptr_l = d_ptr_l;
     p->d_col_l = d_col_l;
     p->rows = rows;
     p->lb = lb;
-    p->asked = core;
+    p->asked = asked;
     p->group_rows = group_rows;
     p->cells = cells;
     p->graph_serial = graph_serial;
-    int rc = cells ? cells_plan_build(p, dim, nnz, least_share) : core_plan_build_device(p, CORE_TC);
-    if (!rc && p->unsuitable) {  // what was built on the way is not needed to remember that
-        (void)hipStreamSynchronize(s.stream);
-        core_plan_free_arrays(p);
-    }
-    if (rc) {
-        core_plan_free_arrays(p);
-        delete p;
-        return rc;
-    }
+    *out = p;
+    return MGGX_OK;
+}
+
+static void core_plan_insert(CorePlan *p)
+{
+    State &s = state();
     if (s.cores.size() >= 8)  // these plans are large (about 3 bytes per edge): keep the eight most recently used (the search compares
                               // up to six core sizes and must not rebuild one between its rounds), and any a captured graph holds
         for (size_t i = 0; i < s.cores.size(); ++i)
@@ -807,19 +808,65 @@ static int find_or_build(const int *d_ptr_l, const int *d_col_l, int rows, int l
                 break;
             }
     s.cores.push_back(p);
-    s.core_plan_build_ms += std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count();
+}
+
+static double ms_since(std::chrono::steady_clock::time_point t0) { return std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count(); }
+
+int core_plan_get(const int *d_ptr_l, const int *d_col_l, int rows, int lb, int core, int group_rows, int graph_serial, CorePlan **out)
+{
+    *out = core_plan_find(d_ptr_l, d_col_l, rows, lb, core, group_rows, 0, graph_serial);
+    if (*out) return MGGX_OK;
+    const auto t0 = std::chrono::steady_clock::now();
+    CorePlan *p = nullptr;
+    int rc = core_plan_new(d_ptr_l, d_col_l, rows, lb, core, group_rows, 0, graph_serial, &p);
+    if (rc) return rc;
+    rc = core_plan_build_device(p, CORE_TC);
+    if (rc || p->unsuitable) {  // what was built on the way is not needed to remember that
+        (void)hipStreamSynchronize(state().stream);
+        core_plan_free_arrays(p);
+    }
+    if (rc) {
+        delete p;
+        return rc;
+    }
+    core_plan_insert(p);
+    state().core_plan_build_ms += ms_since(t0);
     *out = p;
     return MGGX_OK;
 }
 
-int core_plan_get(const int *d_ptr_l, const int *d_col_l, int rows, int lb, int core, int group_rows, int graph_serial, CorePlan **out)
+// What a refusal rests on stays with the record of the CSR, not in the list of plans: it holds no memory, and refusals of a few graphs would
+// push the plans that their calls run on out of the eight places (three graphs at two widths took twelve, and rebuilt on every call).
+int cells_plan_get(GraphInfo &g, int lb, int dim, int least, double least_share, CorePlan **out)
 {
-    return find_or_build(d_ptr_l, d_col_l, rows, lb, core, group_rows, 0, 0, 0, 0.0, graph_serial, out);
-}
-
-int cells_plan_get(const int *d_ptr_l, const int *d_col_l, int rows, int lb, int dim, int least, long long nnz, double least_share, int graph_serial, CorePlan **out)
-{
-    return find_or_build(d_ptr_l, d_col_l, rows, lb, least, CORE_GROUP_ROWS, (dim + 15) / 16, dim, nnz, least_share, graph_serial, out);
+    *out = nullptr;
+    for (const GraphInfo::CellsCounted &c : g.cells_counted)
+        if (c.lb == lb && c.least == least && (c.share <= 0.0 || c.share < least_share)) return MGGX_OK;
+    const int cells = (dim + 15) / 16;
+    *out = core_plan_find(g.d_ptr_l, g.d_col_l, g.rows, lb, least, CORE_GROUP_ROWS, cells, g.serial);
+    if (*out) return MGGX_OK;
+    const auto t0 = std::chrono::steady_clock::now();
+    CorePlan *p = nullptr;
+    int rc = core_plan_new(g.d_ptr_l, g.d_col_l, g.rows, lb, least, CORE_GROUP_ROWS, cells, g.serial, &p);
+    if (rc) return rc;
+    double share = -1.0;
+    rc = cells_plan_build(p, dim, g.nnz_l, least_share, &share);
+    if (!rc) {
+        size_t i = 0;
+        while (i < g.cells_counted.size() && !(g.cells_counted[i].lb == lb && g.cells_counted[i].least == least)) ++i;
+        if (i == g.cells_counted.size()) g.cells_counted.push_back({lb, least, share});
+        else g.cells_counted[i].share = share;
+    }
+    state().core_plan_build_ms += ms_since(t0);
+    if (rc || p->unsuitable) {
+        (void)hipStreamSynchronize(state().stream);
+        core_plan_free_arrays(p);
+        delete p;
+        return rc;
+    }
+    core_plan_insert(p);
+    *out = p;
+    return MGGX_OK;
 }
 
 // The workgroups of the LDS kernel for rows of n4 16-byte pieces: every row group's tiles cut into runs of about

@@ -3,6 +3,7 @@
 // decides on the host -- which kernel a call takes, what it allocates, what it refuses -- can be read off without a GPU.
 #include <hip/hip_runtime_api.h>
 
+#include <cmath>
 #include <cstdlib>
 #include <cstring>
 #include <map>
@@ -34,6 +35,8 @@ hipError_t result(hipError_t e)
 }
 dim3 g_grid, g_block;
 size_t g_shared;
+double g_degree_first, g_degree_power;
+int g_cells, g_cell_edges, g_twice;
 hipStream_t g_stream;
 }  // namespace
 
@@ -69,9 +72,31 @@ FAKE hipError_t __hipPopCallConfiguration(dim3 *grid, dim3 *block, size_t *share
     *stream = g_stream;
     return hipSuccess;
 }
-FAKE hipError_t hipLaunchKernel(const void *f, dim3, dim3, void **, size_t, hipStream_t)
+// Two kernels whose results decide what the library does next are stood in for: the degree profile (sums of 64 degrees, falling as a
+// power of their rank) and the edges of the dense cells (the first so many hold the same number, the others none).
+FAKE void fake_degrees(double first, double power)
 {
-    launch_log() += names()[f] + "\n";
+    g_degree_first = first;
+    g_degree_power = power;
+}
+FAKE void fake_cells(int cells, int edges, int twice)
+{
+    g_cells = cells;
+    g_cell_edges = edges;
+    g_twice = twice;
+}
+FAKE hipError_t hipLaunchKernel(const void *f, dim3, dim3, void **args, size_t, hipStream_t)
+{
+    const std::string &name = names()[f];
+    launch_log() += name + "\n";
+    if (name.find("k_slice_sums") != std::string::npos) {  // (sorted, rows, slices, sums)
+        float *const sums = *static_cast<float **>(args[3]);
+        for (int s = 0; s < *static_cast<int *>(args[2]); ++s) sums[s] = (float)(g_degree_first * std::pow(s + 1.0, -g_degree_power));
+    } else if (name.find("k_cells_count") != std::string::npos) {  // (ptr, col, rank, sorted, ranked, rows, lb, ntiles, cnt, twice)
+        int *const cnt = *static_cast<int **>(args[8]);
+        for (int c = 0; c < g_cells; ++c) cnt[2 * c] = g_cell_edges;
+        **static_cast<int **>(args[9]) = g_twice;
+    }
     return hipSuccess;
 }
 FAKE hipError_t hipGetDeviceCount(int *n)
@@ -82,6 +107,17 @@ FAKE hipError_t hipGetDeviceCount(int *n)
 FAKE hipError_t hipGetDevice(int *d)
 {
     *d = 0;
+    return hipSuccess;
+}
+FAKE int hipGetStreamDeviceId(hipStream_t) { return 0; }
+FAKE hipError_t hipStreamCreateWithFlags(hipStream_t *s, unsigned)
+{
+    *s = nullptr;
+    return hipSuccess;
+}
+FAKE hipError_t hipEventCreateWithFlags(hipEvent_t *e, unsigned)
+{
+    *e = nullptr;
     return hipSuccess;
 }
 FAKE hipError_t hipSetDevice(int) { return hipSuccess; }
@@ -103,6 +139,7 @@ FAKE hipError_t hipMalloc(void **p, size_t bytes)
     if (bytes > g_budget - g_used) return result(hipErrorOutOfMemory);
     *p = aligned_alloc(256, (bytes + 255) & ~(size_t)255);
     if (!*p) return result(hipErrorOutOfMemory);
+    memset(*p, 0, bytes);  // (what no kernel writes)
     g_blocks[*p] = bytes;
     g_used += bytes;
     return hipSuccess;

@@ -137,6 +137,81 @@ assert k.wpb > 0 and k.dist > 0 and grid.search(call(k.ps, k.wpb, k.dist)).group
     assert out == ""
 
 
+CELLS = r'''
+fake.fake_degrees.argtypes = [C.c_double, C.c_double]
+n = C.c_int()
+class Graph:
+    """A CSR whose degrees promise dense cells (57 % of the edges) and a core from LDS."""
+    rows, nnz = 200_000, 14_000_000
+    def __init__(self):
+        self.ptr, self.col, self.x, self.out = malloc(4 * (self.rows + 1)), malloc(4), malloc(4), malloc(4)
+        C.memmove(self.ptr + 4 * self.rows, C.byref(C.c_int(self.nnz)), 4)
+    def args(self, dim):
+        return (at(self.out), at(self.x), None, at(self.ptr), at(self.col), None, None, 0, self.rows, dim, self.rows)
+    def call(self, dim, **kw):
+        fake.fake_clear()
+        assert lib.mggx_sag_np_div(*self.args(dim), 0, 0, 0, opts(**kw)) == 0, lib.mggx_last_error()
+        k = host.last_agg_kernel()
+        return "cells" if "cells=" in k else "LDS" if "core=" in k else "none"
+    def prepare(self, dim, least):
+        cells, edges = C.c_int64(), C.c_int64()
+        assert lib.mggx_cells_prepare(at(self.ptr), at(self.col), None, None, 0, self.rows, dim, least, C.byref(cells), C.byref(edges)) == 0, lib.mggx_last_error()
+        return cells.value, edges.value
+def builds():
+    return fake.fake_launches().count(b"_count")  # plans of cells and cores counted since the last call began
+def core_plans():
+    st = host._CacheStats()
+    lib.mggx_cache_stats(C.byref(st))
+    return st.core_plans
+g = Graph()
+assert lib.mggx_build_part_device(at(g.ptr), 16, 16, 1, None, None, None, C.byref(n)) == 0
+for word, v in ((0, 4_000), (1, 0), (2, 64_000), (3, 50), (4, 0), (5, 0)):  # what the kernels of a plan's build report
+    fake.fake_word(word, C.c_longlong(v))
+fake.fake_degrees(1_500_000., 0.78)
+'''
+
+
+def test_dense_cells_that_the_rule_refuses_can_be_asked_for(without_device):
+    """By rule a graph has dense cells where they hold 67 % of its edges; mggx_cells_prepare has them whatever the rule says.  Neither
+    answer stands in for the other, in either order, and at any width of a group of 16 columns."""
+    out = without_device(CELLS + r'''
+share = lambda s: fake.fake_cells(4_000, int(s * Graph.nnz / 4_000), 0)
+share(.6)
+assert g.call(41) == "LDS" and builds() == 2   # the cells counted, the core from LDS built
+assert g.call(41) == "LDS" and builds() == 0
+assert g.prepare(41, 1400)[0] == 4_000          # the rule's own least number of edges
+assert g.call(41) == "cells" and g.call(41) == "cells" and builds() == 0
+h = Graph()
+assert h.prepare(48, 1400)[0] == 4_000
+assert h.call(48) == "cells" and h.call(41) == "LDS" and h.call(48) == "cells"
+share(.7)
+i = Graph()
+assert i.call(41) == "cells" and i.call(41, core_rows=20480) == "LDS" and i.call(41, core_rows=-1) == "none"
+fake.fake_cells(0, 0, 0)
+j = Graph()
+assert j.prepare(41, 1400) == (0, 0) and j.call(41) == "LDS"
+fake.fake_cells(4_000, 3_000, 1)  # an edge listed twice
+k = Graph()
+assert k.prepare(41, 1) == (0, 0) and k.call(41) == "LDS"
+''')
+    assert out == ""
+
+
+def test_refused_dense_cells_leave_the_plans_in_place(without_device):
+    """Three graphs at two widths, all refused their cells: six cores from LDS, which the eight kept plans hold."""
+    out = without_device(CELLS + r'''
+fake.fake_cells(4_000, int(.6 * Graph.nnz / 4_000), 0)
+graphs = [g, Graph(), Graph()]
+for turn in range(3):
+    for dim in (41, 64):
+        for q in graphs:
+            assert q.call(dim) == "LDS"
+            assert (builds() > 0) == (turn == 0), (turn, dim, fake.fake_launches())
+assert core_plans() <= 6
+''')
+    assert out == ""
+
+
 @pytest.mark.parametrize("ask", ["malloc", "tables", "workspace", "plan"])
 def test_kept_blocks_go_where_memory_is_short(without_device, ask):
     """Set-up calls keep their device blocks for the next ones.  Every allocation of the library's that finds no memory frees
