@@ -1582,7 +1582,7 @@ int run_knobs(GraphInfo &g, const Knobs &k, float *d_out, const void *d_in_local
     CorePlan *cp = nullptr;
     if (k.cells > 0 && core_call) {
         rc = cells_plan_get(g, lb, dim, k.cells, k.cells_share, &cp);  // (none: the core from LDS, if one was asked for as well)
-        if (rc) return rc;
+        if (rc && rc != MGGX_ENOMEM) return rc;
     }
     if (!cp && k.core_rows > 0 && core_call && ub - lb >= 1024) {
         rc = core_plan_get(d_ptr_l, d_col_l, ub - lb, lb, k.core_rows, core_group_rows((dim + 3) / 4, std::min(k.core_rows, ub - lb)), g.serial, &cp);
@@ -1713,6 +1713,7 @@ MGGX_EXPORT int mggx_cells_prepare(const int *d_ptr_l, const int *d_col_l, const
     if (rc) return rc;
     if (g->nnz_r > 0 || g->nnz_l < 1) return fail(MGGX_EINVAL, "cells_prepare: %lld local and %lld remote edges (local only)", (long long)g->nnz_l, (long long)g->nnz_r);
     mggx::CorePlan *p = nullptr;
+    for (mggx::GraphInfo::CellsCounted &c : g->cells_counted) c.no_memory = false;  // asked for: tried again
     rc = mggx::cells_plan_get(*g, lb, dim, least_edges, 0.0, &p);
     if (rc) return rc;
     if (num_cells) *num_cells = p ? p->ncells : 0;

@@ -741,18 +741,12 @@ int cells_sums(const CorePlan *p, const float *d_in, int dim, long long ld_in, c
     return MGGX_OK;
 }
 
-// p->asked: least edges of a cell.  A plan whose cells hold less than least_share of the edges, one of a CSR with parallel edges, or one there
-// is no memory for is marked unsuitable.  *share: what the cells hold, -1 in the last two cases.
+// p->asked: least edges of a cell.  A plan whose cells hold less than least_share of the edges and one of a CSR with parallel edges are marked
+// unsuitable.  *share: what the cells hold, -1 with parallel edges or where the build did not get that far.
 int cells_plan_build(CorePlan *p, int dim, long long nnz, double least_share, double *share)
 {
     *share = -1.0;
-    const int rc = build(p, dim, nnz, least_share, share);
-    if (rc == MGGX_ENOMEM) {
-        *share = -1.0;
-        p->unsuitable = true;
-        return MGGX_OK;
-    }
-    return rc;
+    return build(p, dim, nnz, least_share, share);
 }
 
 }  // namespace mggx

@@ -841,7 +841,7 @@ int cells_plan_get(GraphInfo &g, int lb, int dim, int least, double least_share,
 {
     *out = nullptr;
     for (const GraphInfo::CellsCounted &c : g.cells_counted)
-        if (c.lb == lb && c.least == least && (c.share <= 0.0 || c.share < least_share)) return MGGX_OK;
+        if (c.lb == lb && c.least == least && (c.no_memory || c.share <= 0.0 || c.share < least_share)) return MGGX_OK;
     const int cells = (dim + 15) / 16;
     *out = core_plan_find(g.d_ptr_l, g.d_col_l, g.rows, lb, least, CORE_GROUP_ROWS, cells, g.serial);
     if (*out) return MGGX_OK;
@@ -851,11 +851,12 @@ int cells_plan_get(GraphInfo &g, int lb, int dim, int least, double least_share,
     if (rc) return rc;
     double share = -1.0;
     rc = cells_plan_build(p, dim, g.nnz_l, least_share, &share);
-    if (!rc) {
+    if (!rc || rc == MGGX_ENOMEM) {
         size_t i = 0;
         while (i < g.cells_counted.size() && !(g.cells_counted[i].lb == lb && g.cells_counted[i].least == least)) ++i;
-        if (i == g.cells_counted.size()) g.cells_counted.push_back({lb, least, share});
-        else g.cells_counted[i].share = share;
+        const GraphInfo::CellsCounted c{lb, least, share, rc == MGGX_ENOMEM};
+        if (i == g.cells_counted.size()) g.cells_counted.push_back(c);
+        else g.cells_counted[i] = c;
     }
     state().core_plan_build_ms += ms_since(t0);
     if (rc || p->unsuitable) {

@@ -217,9 +217,10 @@ struct GraphInfo {
     bool have_profile = false;
     struct Predicted { int dim; int block_rows; unsigned long long table_bytes; int core_rows; };
     std::vector<Predicted> predicted;  // what the cost model said for a row width (evaluated once, a millisecond of host time)
-    // Of the CSR's edges, the share that lies in cells of at least `least` edges (counted when a plan of dense cells is built); -1: there can
-    // be no such plan.  Whether that is enough is for each caller to say: what a call by rule refuses mggx_cells_prepare may want.
-    struct CellsCounted { int lb; int least; double share; };
+    // Of the CSR's edges, the share that lies in cells of at least `least` edges (counted when a plan of dense cells is built); -1: an edge is
+    // listed twice.  Whether that is enough is for each caller to say: what a call by rule refuses mggx_cells_prepare may want.
+    // no_memory: there was none for the plan; calls go on without it, and mggx_cells_prepare tries again.
+    struct CellsCounted { int lb; int least; double share; bool no_memory; };
     std::vector<CellsCounted> cells_counted;
     struct CellsAsked { int dim; int least; };
     std::vector<CellsAsked> cells_asked;  // mggx_cells_prepare
@@ -355,7 +356,7 @@ int core_row_sums(CorePlan *p, int dim, const float4 **sums);
 // Grow-only scratch of the dense-core paths (both streams of a call use it).
 int core_workspace(size_t bytes, void **p);
 // Dense cells on the matrix cores (mggx_cells.hip): the plan of a row width (found in or added to the list of core plans; NULL where its
-// cells hold less than least_share of the edges, or none), and the sums of its cells by rank, on `stream`, for run_core_finish or the
+// cells hold less than least_share of the edges, or none, or where there was no memory before; MGGX_ENOMEM where there is none now), and the sums of its cells by rank, on `stream`, for run_core_finish or the
 // finishing kernel of a column-blocked plan to add.
 int cells_plan_get(GraphInfo &g, int lb, int dim, int least, double least_share, CorePlan **out);
 int cells_plan_build(CorePlan *p, int dim, long long nnz, double least_share, double *share);

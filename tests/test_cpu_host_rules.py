@@ -212,6 +212,27 @@ assert core_plans() <= 6
     assert out == ""
 
 
+def test_dense_cells_without_memory(without_device):
+    """A plan of dense cells that finds no device memory: the call goes on without it, and later ones do not try again; who asks for it is
+    told so, and gets it once there is memory."""
+    out = without_device(CELLS + r'''
+fake.fake_cells(4_000, int(.7 * Graph.nnz / 4_000), 0)  # 64 MB of cells
+h = Graph()
+fake.fake_budget(C.c_size_t(fake.fake_used() + (48 << 20)))
+assert g.call(41) == "LDS" and builds() == 2
+assert g.call(41) == "LDS" and builds() == 0
+cells = C.c_int64(7)
+ask = lambda q: lib.mggx_cells_prepare(at(q.ptr), at(q.col), None, None, 0, q.rows, 41, 1400, C.byref(cells), None)
+assert ask(h) == ask(g) == -3 and b"device memory" in lib.mggx_last_error()
+assert g.call(41) == "LDS" and builds() == 0
+fake.fake_budget(C.c_size_t(1 << 40))
+assert g.call(41) == "LDS" and builds() == 0
+assert ask(g) == 0 and cells.value == 4_000 and g.call(41) == "cells"
+assert h.call(64) == "LDS" and ask(h) == 0 and h.call(64) == "cells" and h.call(41) == "cells"
+''')
+    assert out == ""
+
+
 @pytest.mark.parametrize("ask", ["malloc", "tables", "workspace", "plan"])
 def test_kept_blocks_go_where_memory_is_short(without_device, ask):
     """Set-up calls keep their device blocks for the next ones.  Every allocation of the library's that finds no memory frees
