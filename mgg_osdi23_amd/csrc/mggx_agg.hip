@@ -1547,7 +1547,7 @@ int resolve_knobs(GraphInfo &g, int dim, int dtype, int ps, int wpb, int dist, i
         if (e.dim == dim && e.dtype == dtype) t = &e;
     Knobs k{ps, wpb, dist, block_rows, core_rows};
     if (t && (ps == 0 || ps == t->ps) && wpb == 0 && dist == 0 && block_rows == 0 && core_rows == 0) {
-        *out = Knobs{t->ps, t->wpb, t->dist, t->block_rows, t->core_rows, t->cells, t->cells ? CELLS_SHARE : 0.0};
+        *out = Knobs{t->ps, t->wpb, t->dist, t->block_rows, t->core_rows, t->cells, t->cells_share};
         return MGGX_OK;
     }
     if (k.ps == 0) k.ps = 16;
@@ -1862,9 +1862,10 @@ MGGX_EXPORT int mggx_sag_np_div_tune(float *d_out, const void *d_in_local, const
     st.search_ms += std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - search_t0).count() -
                     (st.plan_build_ms + st.core_plan_build_ms - build_ms0);
     bool found = false;
+    const mggx::GraphInfo::Tuned record{dim, o.in_dtype, won.ps, won.wpb, won.dist, won.block_rows, won.core_rows, won.cells, won.cells_share};
     for (mggx::GraphInfo::Tuned &t : g->tuned)
-        if (t.dim == dim && t.dtype == o.in_dtype) { t.ps = won.ps; t.wpb = won.wpb; t.dist = won.dist; t.block_rows = won.block_rows; t.core_rows = won.core_rows; t.cells = won.cells; found = true; }
-    if (!found) g->tuned.push_back({dim, o.in_dtype, won.ps, won.wpb, won.dist, won.block_rows, won.core_rows, won.cells});
+        if (t.dim == dim && t.dtype == o.in_dtype) { t = record; found = true; }
+    if (!found) g->tuned.push_back(record);
     if (best_out) { best_out->ps = bk.ps; best_out->wpb = bk.wpb; best_out->dist = bk.dist; best_out->col_block_rows = bk.block_rows; best_out->core_rows = bk.cells ? 0 : bk.core_rows; }
     if (ms_best) *ms_best = best;
     return MGGX_OK;

@@ -230,7 +230,7 @@ struct GraphInfo {
     Guard guard;
     int64_t nnz_l = 0, nnz_r = 0;
     // knobs measured best by mggx_sag_np_div_tune for a row width and element type; used where a call passes 0
-    struct Tuned { int dim, dtype, ps, wpb, dist, block_rows, core_rows, cells; };
+    struct Tuned { int dim, dtype, ps, wpb, dist, block_rows, core_rows, cells; double cells_share; };
     std::vector<Tuned> tuned;
 };
 

@@ -212,6 +212,22 @@ assert core_plans() <= 6
     assert out == ""
 
 
+def test_a_search_keeps_the_dense_cells_it_measured(without_device):
+    """Cells that were asked for at a share the rule would refuse, and win a search: later calls use them, also where their plan has
+    left the cache in between and is built anew."""
+    out = without_device(CELLS + r'''
+fake.fake_cells(4_000, int(.5 * Graph.nnz / 4_000), 0)
+assert g.prepare(41, 1400)[0] == 4_000
+assert lib.mggx_sag_np_div_tune(*g.args(41), 0, None, None, None) == 0, lib.mggx_last_error()
+assert "cells=" in host.last_agg_kernel()
+for least in range(8):
+    assert Graph().prepare(41, 1000)[0] == 4_000  # eight other plans
+assert g.call(41) == "cells" and builds() == 1
+assert g.call(41) == "cells" and builds() == 0
+''')
+    assert out == ""
+
+
 def test_dense_cells_without_memory(without_device):
     """A plan of dense cells that finds no device memory: the call goes on without it, and later ones do not try again; who asks for it is
     told so, and gets it once there is memory."""
