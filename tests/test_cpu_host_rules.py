@@ -228,6 +228,22 @@ assert g.call(41) == "cells" and builds() == 0
     assert out == ""
 
 
+def test_dense_cells_asked_for_after_a_search(without_device):
+    """mggx_cells_prepare goes before the result of an earlier search on the same arrays and width, and leaves those of other widths."""
+    out = without_device(CELLS + r'''
+fake.fake_cells(4_000, int(.5 * Graph.nnz / 4_000), 0)
+for dim in (41, 40):
+    assert lib.mggx_sag_np_div_tune(*g.args(dim), 0, opts(core_rows=-1), None, None) == 0, lib.mggx_last_error()
+    assert g.call(dim) == "none"
+assert g.prepare(41, 100_000) == (0, 0) and g.call(41) == "none"
+assert g.prepare(41, 1400)[0] == 4_000
+assert g.call(41) == "cells" and g.call(40) == "none"
+assert lib.mggx_sag_np_div_tune(*g.args(41), 0, opts(core_rows=-1), None, None) == 0
+assert g.call(41) == "none"
+''')
+    assert out == ""
+
+
 def test_dense_cells_without_memory(without_device):
     """A plan of dense cells that finds no device memory: the call goes on without it, and later ones do not try again; who asks for it is
     told so, and gets it once there is memory."""
