@@ -1718,7 +1718,8 @@ MGGX_EXPORT int mggx_cells_prepare(const int *d_ptr_l, const int *d_col_l, const
     if (rc) return rc;
     if (num_cells) *num_cells = p ? p->ncells : 0;
     if (num_edges) *num_edges = p ? p->core_nnz : 0;
-    for (size_t i = 0; p && i < g->tuned.size(); ++i)  // an earlier search's result would go before it
+    if (!p) return MGGX_OK;  // nothing to use: later calls go by the rule or the search, as before
+    for (size_t i = 0; i < g->tuned.size(); ++i)  // an earlier search's result would go before it
         if (g->tuned[i].dim == dim && g->tuned[i].dtype == MGGX_F32) {
             g->tuned.erase(g->tuned.begin() + (long)i);
             break;

@@ -187,6 +187,7 @@ assert h.call(48) == "cells" and h.call(41) == "LDS" and h.call(48) == "cells"
 share(.7)
 i = Graph()
 assert i.call(41) == "cells" and i.call(41, core_rows=20480) == "LDS" and i.call(41, core_rows=-1) == "none"
+assert i.prepare(41, 100_000) == (0, 0) and i.call(41) == "cells"  # none so large: the rule's stay
 fake.fake_cells(0, 0, 0)
 j = Graph()
 assert j.prepare(41, 1400) == (0, 0) and j.call(41) == "LDS"
