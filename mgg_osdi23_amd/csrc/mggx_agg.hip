@@ -1872,7 +1872,7 @@ MGGX_EXPORT int mggx_sag_np_div_tune(float *d_out, const void *d_in_local, const
     for (mggx::GraphInfo::Tuned &t : g->tuned)
         if (t.dim == dim && t.dtype == o.in_dtype) { t = record; found = true; }
     if (!found) g->tuned.push_back(record);
-    if (best_out) { best_out->ps = bk.ps; best_out->wpb = bk.wpb; best_out->dist = bk.dist; best_out->col_block_rows = bk.block_rows; best_out->core_rows = bk.cells ? 0 : bk.core_rows; }
+    if (best_out) { best_out->ps = bk.ps; best_out->wpb = bk.wpb; best_out->dist = bk.dist; best_out->col_block_rows = bk.block_rows; best_out->core_rows = strstr(st.last_kernel, " cells=") ? 0 : bk.core_rows; }  // (refused cells: the core from LDS ran)
     if (ms_best) *ms_best = best;
     return MGGX_OK;
 }

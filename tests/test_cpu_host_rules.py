@@ -245,6 +245,21 @@ assert g.call(41) == "none"
     assert out == ""
 
 
+@pytest.mark.parametrize("share,runs", [(.6, "LDS"), (.7, "cells")])
+def test_a_search_reports_the_core_that_ran(without_device, share, runs):
+    """The rule's setting wins a search: the size of its core from LDS is reported where that is what ran, 0 where dense cells did."""
+    out = without_device(CELLS + r'''
+fake.fake_cells(4_000, int(SHARE * Graph.nnz / 4_000), 0)
+k = host._AggKnobs()
+assert lib.mggx_sag_np_div_tune(*g.args(41), 0, None, C.byref(k), None) == 0, lib.mggx_last_error()
+m = re.search(r" core=(\d+).*?( cells=|$)", host.last_agg_kernel())
+assert ("cells" if m.group(2) else "LDS") == "RUNS"
+assert k.core_rows == (int(m.group(1)) if "RUNS" == "LDS" else 0), (k.core_rows, m.group(0))
+assert g.call(41, core_rows=k.core_rows) == "RUNS"
+'''.replace("SHARE", str(share)).replace("RUNS", runs))
+    assert out == ""
+
+
 def test_dense_cells_without_memory(without_device):
     """A plan of dense cells that finds no device memory: the call goes on without it, and later ones do not try again; who asks for it is
     told so, and gets it once there is memory."""
