@@ -85,10 +85,10 @@ FAKE void fake_cells(int cells, int edges, int twice)
     g_cell_edges = edges;
     g_twice = twice;
 }
-FAKE hipError_t hipLaunchKernel(const void *f, dim3, dim3, void **args, size_t, hipStream_t)
+FAKE hipError_t hipLaunchKernel(const void *f, dim3 grid, dim3, void **args, size_t, hipStream_t)
 {
     const std::string &name = names()[f];
-    launch_log() += name + "\n";
+    launch_log() += name + " " + std::to_string(grid.x) + "\n";
     if (name.find("k_slice_sums") != std::string::npos) {  // (sorted, rows, slices, sums)
         float *const sums = *static_cast<float **>(args[3]);
         for (int s = 0; s < *static_cast<int *>(args[2]); ++s) sums[s] = (float)(g_degree_first * std::pow(s + 1.0, -g_degree_power));

@@ -137,6 +137,21 @@ assert k.wpb > 0 and k.dist > 0 and grid.search(call(k.ps, k.wpb, k.dist)).group
     assert out == ""
 
 
+def test_kernels_that_end_in_an_atomic_on_one_word_keep_to_few_workgroups(without_device):
+    """Largest remote id, rows without neighbors and longest row of a new plan: an atomic per workgroup on one address, at any number of rows."""
+    out = without_device(r'''
+rows, dim = 2_450_000, 16
+ptr, rptr, col, x = malloc(4 * (rows + 1)), malloc(4 * (rows + 1)), malloc(4), malloc(4)
+for p in (ptr, rptr): C.memmove(p + 4 * rows, C.byref(C.c_int(20_000_000)), 4)
+fake.fake_clear()
+assert lib.mggx_sag_np_div(at(x), at(x), at(x), at(ptr), at(col), at(rptr), at(col), 0, rows, dim, rows, 16, 0, 0, None) == 0, lib.mggx_last_error()
+launched = [l.split() for l in fake.fake_launches().decode().splitlines()]
+for name in ("k_max_i32", "k_collect_empty"):
+    assert [int(grid) <= 256 for k, grid in launched if name in k] == [True], launched
+''')
+    assert out == ""
+
+
 CELLS = r'''
 fake.fake_degrees.argtypes = [C.c_double, C.c_double]
 n = C.c_int()

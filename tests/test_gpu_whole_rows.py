@@ -124,3 +124,27 @@ def test_whole_rows_of_a_share_and_of_slices(gpu):
     gpu.sync()
     assert "whole=1 slices=2" in gpu.last_agg_kernel(), gpu.last_agg_kernel()
     assert_close_to_oracle(out.cpu().numpy(), want, mag, FP32_TOL, "slices")
+
+
+@pytest.mark.parametrize("V", [1, 1023, 1025, 262_145, 1_048_579])
+def test_longest_and_empty_rows_are_found_wherever_they_are(gpu, V):
+    """One row too long for the rule, or without neighbors, at the first and last places and around the strides in which a plan's build
+    goes over the rows."""
+    import torch
+    dim = 16
+    x = torch.ones(V, dim, device="cuda")
+    z, zc = torch.zeros(V + 1, dtype=torch.int32, device="cuda"), torch.zeros(1, dtype=torch.int32, device="cuda")
+    for at in sorted({r for r in (0, 63, 64, 1023, 1024, 262_143, 262_144, 786_432, V - 1) if r < V}):
+        for of_row in (2, 2000, 0):
+            deg = torch.full((V,), 2, dtype=torch.int32, device="cuda")
+            deg[at] = of_row
+            ptr = torch.zeros(V + 1, dtype=torch.int32, device="cuda")
+            ptr[1:] = deg.cumsum(0)
+            col = torch.arange(int(ptr[-1]) + 1, device="cuda", dtype=torch.int32) % V
+            out = torch.full((V, dim), 7.5, device="cuda")
+            gpu.mgg_SAG_np_div(out, x, ptr, col, z, zc, 0, V, dim, V, 0, 16, 0, 0, core_rows=-1)
+            gpu.sync()
+            k = gpu.last_agg_kernel()
+            assert V < 64 * 16 or "whole=%d" % (of_row == 2) in k, (at, of_row, k)
+            assert torch.equal(out, deg.float()[:, None].expand(V, dim)), (at, of_row)
+            gpu.forget(ptr)
