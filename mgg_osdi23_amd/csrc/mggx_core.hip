@@ -1255,9 +1255,11 @@ int predict_core_rows(GraphInfo &g, int dim, unsigned long long table_bytes, int
     return MGGX_OK;
 }
 
-double predicted_cells_share(const GraphInfo &g, int least)
+double predicted_cells_share(GraphInfo &g, int least)
 {
     if (!g.have_profile || g.nnz_l <= 0) return 0.0;
+    for (const GraphInfo::CellsByDegrees &c : g.cells_by_degrees)
+        if (c.least == least) return c.share;
     const size_t slices = std::min<size_t>(g.slice_deg.size(), 1920);
     std::vector<double> group, tile;  // degree sums of 512 rows and of 192 columns
     for (size_t s = 0; s < slices; ++s) {
@@ -1273,7 +1275,8 @@ double predicted_cells_share(const GraphInfo &g, int least)
             if (edges < least) break;  // the tiles are in falling order
             in_cells += edges;
         }
-    return in_cells / (double)g.nnz_l;
+    g.cells_by_degrees.push_back({least, in_cells / (double)g.nnz_l});
+    return g.cells_by_degrees.back().share;
 }
 
 }  // namespace mggx

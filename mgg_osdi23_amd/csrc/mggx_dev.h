@@ -222,6 +222,8 @@ struct GraphInfo {
     // no_memory: there was none for the plan; calls go on without it, and mggx_cells_prepare tries again.
     struct CellsCounted { int lb; int least; double share; bool no_memory; };
     std::vector<CellsCounted> cells_counted;
+    struct CellsByDegrees { int least; double share; };
+    std::vector<CellsByDegrees> cells_by_degrees;  // what the degrees alone say of that share (evaluated once per `least`: up to 40 us of host time)
     struct CellsAsked { int dim; int least; };
     std::vector<CellsAsked> cells_asked;  // mggx_cells_prepare
     bool internal = false;  // arrays owned by the library (the remainder CSR of a dense-core plan): no content check
@@ -363,7 +365,7 @@ int cells_plan_build(CorePlan *p, int dim, long long nnz, double least_share, do
 int cells_sums(const CorePlan *p, const float *d_in, int dim, long long ld_in, const Gate &gate, hipStream_t stream, const float4 **d_sums);
 // What the degrees alone say of the share of a CSR's edges that lies in cells of at least `least` edges (after predict_core_rows, which
 // fetches the degree profile).
-double predicted_cells_share(const GraphInfo &g, int least);
+double predicted_cells_share(GraphInfo &g, int least);
 // Second stream of the dense-core path (created on first use, default priority) and the two events that fork and join it.
 int core_side_stream(hipStream_t *stream, hipEvent_t *fork, hipEvent_t *join);
 

@@ -213,6 +213,30 @@ assert k.prepare(41, 1) == (0, 0) and k.call(41) == "LDS"
     assert out == ""
 
 
+def test_what_the_rules_need_of_the_degrees_is_worked_out_once(without_device):
+    """A call that leaves the knobs at 0 costs the host about as much as one that names what the rules choose."""
+    out = without_device(CELLS + r'''
+import time
+fake.fake_degrees(4_500_000., 0.78)  # (many cells by the degrees)
+Graph.nnz = 100_000_000
+q = Graph()
+fake.fake_cells(4_000, 0, 0)
+assert q.call(41) == "LDS"
+core = int(re.search(r" core=(\d+)", host.last_agg_kernel()).group(1))
+blk = 49152 if "blocks=1 " not in host.last_agg_kernel() else -1
+def us(ps, o):
+    best = 1e9
+    for _ in range(400):
+        t = time.perf_counter()
+        lib.mggx_sag_np_div(*q.args(41), ps, 0, 0, o)
+        best = min(best, time.perf_counter() - t)
+    return best * 1e6
+by_rule, named = us(0, opts()), us(16, opts(core_rows=core, col_block_rows=blk))
+
+assert by_rule < named + 5, (by_rule, named)  # (worked out anew: 15 us more)
+''')
+
+
 def test_refused_dense_cells_leave_the_plans_in_place(without_device):
     """Three graphs at two widths, all refused their cells: six cores from LDS, which the eight kept plans hold."""
     out = without_device(CELLS + r'''
