@@ -47,7 +47,8 @@ def test_dense_cells(gpu, V, dim, least, flags):
         want, mag = want * s[:, None], mag * s[:, None]
     if flags == "acc_relu":
         want, mag = np.maximum(want + base, 0), mag + np.abs(base)
-    for blk, ps, wpb, dist in ((-1, 16, 0, 0), (max(64, V // 5), 16, 4, 2)):  # plain order; column-blocked rest where there is enough of it
+    # the library's wpb and dist, and others (too few neighbors are left for column blocks: test_column_blocked_rest_beside_cells has those)
+    for blk, ps, wpb, dist in ((-1, 16, 0, 0), (max(64, V // 5), 16, 4, 2)):
         out = torch.full((V, ld), 7.5, device="cuda")
         if flags == "acc_relu":
             out[:, :dim] = to_dev(base)
@@ -73,6 +74,143 @@ def test_dense_cells(gpu, V, dim, least, flags):
     gpu.sync()
     assert np.array_equal(out.cpu().numpy()[:, :dim], np.repeat(np.diff(ptr).astype(np.float32)[:, None], dim, 1))
     gpu.forget(d_ptr)
+
+
+def aggregate(gpu, out, x, csr, lb, dim, flags, scale, **kw):
+    """One call with the epilogue `flags` and the knobs left to the library."""
+    V = csr[0].numel() - 1
+    args = (out, x, *csr, lb, lb + V, dim, V, 0, 16, 0, 0)
+    if flags == "gin":
+        gpu.mgg_GIN_np_div(*args, 0.5, **kw)
+    else:
+        gpu.mgg_SAG_np_div(*args, accumulate=flags == "acc_relu", relu=flags == "acc_relu", softmax=flags == "softmax",
+                           row_scale_out=scale if flags == "scale" else None, **kw)
+    gpu.sync()
+
+
+def check_epilogue(got, want, mag, base, scale, flags, what):
+    """want, mag: the oracle's sums (with the GIN term) and sums of magnitudes, before the other epilogues."""
+    if flags == "scale":
+        want, mag = want * scale[:, None], mag * scale[:, None]
+    if flags == "acc_relu":
+        want, mag = np.maximum(want + base, 0), mag + np.abs(base)
+    if flags != "softmax":
+        return assert_close_to_oracle(got, want, mag, FP32_TOL, what)
+    e = np.exp(want.astype(np.float64) - want.max(1, keepdims=True))
+    e /= e.sum(1, keepdims=True)
+    # a logit off by d moves a probability by at most a factor of exp(2 d); the quotient's own rounding and __expf add some 1e-6
+    off = 2 * FP32_TOL * mag.max(1, keepdims=True)
+    assert (np.abs(got - e) <= e * np.expm1(2 * off) + 4e-6).all(), what
+
+
+@pytest.mark.parametrize("flags", ["plain", "scale", "gin", "acc_relu", "softmax"])
+@pytest.mark.parametrize("dim", [12, 16, 17, 41, 64])
+def test_column_blocked_rest_beside_cells(gpu, dim, flags):
+    """Enough neighbors outside the cells for the rest to stay in column blocks: the kernel that finishes those adds the cells' sums (no
+    second stream to join) and applies the epilogue.  20 neighbors per row and block are asked for up to width 16, 10 beyond."""
+    import torch
+    V, least = 2000, 20_000
+    ptr, col = graph(V, 100 * V)
+    x = gpu.fill_normal((V, dim), seed=211)
+    want, mag = oracle_agg(share_of(ptr, col, V, 1, 0), x, x, dim, **(dict(flags=orc.GIN, eps=0.5) if flags == "gin" else {}))
+    csr = (to_dev(ptr), to_dev(col), *no_remote(V))
+    cells, edges = gpu.cells_prepare(*csr, 0, V, dim, least)
+    blocks = 2 if dim <= 16 else 4
+    assert 0 < cells and (len(col) - edges) >= (20 if dim <= 16 else 10) * blocks * V
+    s, base = gpu.fill_uniform((V,), 0.5, 2.0, seed=212), gpu.fill_normal((V, dim), seed=213)
+    ld = dim + 2
+    out = torch.full((V, ld), 7.5, device="cuda")
+    if flags == "acc_relu":
+        out[:, :dim] = to_dev(base)
+    aggregate(gpu, out, to_dev(x), csr, 0, dim, flags, to_dev(s), col_block_rows=V // blocks, ld_out=ld)
+    k = gpu.last_agg_kernel()
+    assert "blocks=%d " % blocks in k and "merged_finish" in k and "cells=%d" % cells in k, k
+    got = out.cpu().numpy()
+    assert np.all(got[:, dim:] == 7.5)
+    check_epilogue(got[:, :dim], want, mag, base, s, flags, k)
+    gpu.forget(csr[0])
+
+
+@pytest.mark.parametrize("flags", ["plain", "scale", "gin", "acc_relu", "softmax"])
+@pytest.mark.parametrize("dim,long_row,form", [(16, 0, "whole"), (16, 1, "fused"), (41, 0, "whole"), (41, 1, "fused"), (64, 0, "whole"), (64, 1, "fused")])
+def test_small_rest_beside_cells(gpu, dim, long_row, form, flags):
+    """The rest of a small graph in the forms of k_agg that finish their own rows: whole rows per workgroup, and counters where one row is
+    long.  The rest leaves ReLU and softmax to the kernel that adds the cells' sums."""
+    import torch
+    V, hubs = 3000, 512
+    rng = np.random.default_rng(dim)
+    rows = [set(range(hubs)) if v < hubs else set() for v in range(V)]
+    for v in range(V):
+        rows[v] |= set((hubs + rng.choice(V - hubs, rng.integers(17, 30), replace=False)).tolist())
+    if long_row:
+        rows[5] |= set(range(V))
+    ptr = np.concatenate([[0], np.cumsum([len(r) for r in rows])]).astype(np.int32)
+    col = np.concatenate([np.sort(np.fromiter(r, np.int32)) for r in rows]).astype(np.int32)
+    x = gpu.fill_normal((V, dim), seed=221)
+    want, mag = oracle_agg(share_of(ptr, col, V, 1, 0), x, x, dim, **(dict(flags=orc.GIN, eps=0.5) if flags == "gin" else {}))
+    csr = (to_dev(ptr), to_dev(col), *no_remote(V))
+    cells, edges = gpu.cells_prepare(*csr, 0, V, dim, 12_000)
+    assert 0 < cells and 0.9 * hubs * hubs < edges
+    s, base = gpu.fill_uniform((V,), 0.5, 2.0, seed=222), gpu.fill_normal((V, dim), seed=223)
+    out = to_dev(base) if flags == "acc_relu" else torch.full((V, dim), 7.5, device="cuda")
+    aggregate(gpu, out, to_dev(x), csr, 0, dim, flags, to_dev(s))
+    k = gpu.last_agg_kernel()
+    assert "fused=1 whole=%d " % (form == "whole") in k and "cells=%d" % cells in k, k
+    check_epilogue(out.cpu().numpy(), want, mag, base, s, flags, k)
+    gpu.forget(csr[0])
+
+
+@pytest.mark.parametrize("dim,block_rows", [(33, -1), (41, -1), (41, 70_000), (64, -1), (64, 70_000)])
+@pytest.mark.parametrize("flags", ["acc_relu", "softmax"])
+def test_sliced_rest_beside_cells(gpu, dim, block_rows, flags):
+    """Rows of two cache lines out of a table of 32 MB and more: the rest is gathered in two slices of columns, in plain order and in
+    column blocks."""
+    import torch
+    V, ld = 140_000, 64
+    ptr, col = graph(V, (3 if block_rows < 0 else 24) * V)
+    x = gpu.fill_normal((V, dim), seed=231)
+    want, mag = oracle_agg(share_of(ptr, col, V, 1, 0), x, x, dim)
+    csr = (to_dev(ptr), to_dev(col), *no_remote(V))
+    cells, edges = gpu.cells_prepare(*csr, 0, V, dim, 1000 if block_rows < 0 else 4000)
+    assert 0 < cells and 0 < edges < len(col)
+    base = gpu.fill_normal((V, dim), seed=233)
+    d_x = torch.full((V, ld), 1e30, device="cuda")
+    d_x[:, :dim] = to_dev(x)
+    out = to_dev(base) if flags == "acc_relu" else torch.full((V, dim), 7.5, device="cuda")
+    aggregate(gpu, out, d_x, csr, 0, dim, flags, None, ld_in=ld, col_block_rows=block_rows)
+    k = gpu.last_agg_kernel()
+    assert "slices=2" in k and "cells=%d" % cells in k and ("blocks=1 " in k) == (block_rows < 0) == ("merged_finish" not in k), k
+    check_epilogue(out.cpu().numpy(), want, mag, base, None, flags, k)
+    gpu.forget(csr[0])
+
+
+@pytest.mark.parametrize("dim", [41, 64])
+def test_dense_cells_refused_by_the_rule(gpu, dim):
+    """A graph whose degrees promise more than its cells hold (58 % of the edges in cells of 1,400 and more, the rule asks for 67): the core
+    from LDS runs, with the cells counted once; asked for, the cells run; both give the plain order's sums."""
+    import torch
+    V = 250_000
+    ptr, col = graph(V, 10_000_000, seed=7)
+    csr = (to_dev(ptr), to_dev(col), *no_remote(V))
+    x = torch.randn(V, dim, device="cuda", generator=torch.Generator(device="cuda").manual_seed(1))
+    out = torch.empty(V, dim, device="cuda")
+
+    def run(want, **kw):
+        gpu.mgg_SAG_np_div(out, kw.pop("x", x), *csr, 0, V, dim, V, 0, 0, 0, 0, **kw)
+        gpu.sync()
+        k = gpu.last_agg_kernel()
+        assert ("cells=" in k, "core=" in k) == dict(none=(False, False), LDS=(False, True), cells=(True, True))[want], k
+        return out.cpu().numpy().astype(np.float64)
+
+    plain, mag = run("none", core_rows=-1), run("none", core_rows=-1, x=x.abs())
+    refused = run("LDS")
+    built = gpu.cache_stats()["core_plan_build_ms"]
+    assert np.array_equal(run("LDS"), refused) and gpu.cache_stats()["core_plan_build_ms"] == built
+    assert gpu.cells_prepare(*csr, 0, V, dim, 1400)[0] > 0
+    asked = run("cells")
+    for got in (refused, asked):
+        assert np.all(np.abs(got - plain) <= 2 * FP32_TOL * mag)
+    gpu.forget(csr[0])
 
 
 def test_dense_cells_of_a_complete_graph(gpu):

@@ -1152,6 +1152,19 @@ def test_compact_remote_device_orders_by_count(gpu, distinct, spread):
     assert np.array_equal(got_ids.cpu().numpy(), want_ids) and np.array_equal(got.cpu().numpy(), want)
 
 
+@pytest.mark.parametrize("spread", [1, 300])
+def test_compact_remote_device_counts_of_three_digits(gpu, spread):
+    """More than 2^22 edges, so counts are ordered in three passes of 11 bits: counts that differ in the third digit, in the second and in the
+    first only, and equal ones in every tile."""
+    rng = np.random.default_rng(3)
+    count = rng.integers(1, 3, 40_000)
+    count[[7, 39_999, 20_000, 2_050, 3]] = [(1 << 22) + 5, (1 << 22) + 4, 3 << 11, 1 << 11, (1 << 11) - 1]
+    col = rng.permutation(np.repeat(np.arange(len(count)) * spread, count)).astype(np.int32)
+    want, want_ids = gpu.compact_remote(col)
+    got, got_ids = gpu.compact_remote_device(to_dev(col), len(col))
+    assert np.array_equal(got_ids.cpu().numpy(), want_ids) and np.array_equal(got.cpu().numpy(), want)
+
+
 @pytest.mark.parametrize("lens", [[64, 65, 127, 128, 129, 0, 1], [511, 512, 513, 640, 641], [20_000, 3, 700, 0, 191]])
 def test_split_csr_device_rows_of_many_chunks(gpu, lens):
     """Rows around the number of neighbors a wavefront takes at a time, and one of thousands: the device split is the host's."""
