@@ -148,13 +148,18 @@ def fail_on_parity(res, checks):
         sys.exit(4)
 
 
-def gather_ceiling(torch, host, ld_bytes, row_bytes, table_rows, edges, ms, core_edges=0, cell_edges=0):
+# A dense cell's products for 16 columns: 512 x 256 positions in 384 sparse matrix instructions, each as long as a dense bf16 one of
+# 16 x 16 x 32 (16,384 operations), at the 2.5 PFLOP/s of dense bf16.
+CELL_NS_PER_16_COLUMNS = 384 * 16384 / 2.5e15 * 1e9
+
+
+def gather_ceiling(torch, host, ld_bytes, row_bytes, table_rows, edges, ms, core_edges=0, cell_edges=0, cells=0, dim=0):
     """Where the feature table is cache resident the HBM peak does not bound the kernel; the L2 and, for the dense core,
     the LDS do.  Measured live with the library's yardsticks (random row reads of the kernel's geometry, no index
     stream, no reduction): from a 3 MB table (every load hits the L2), from a table of the kernel's size, and from an
     LDS tile.  The ceiling of a call is the longer of its two halves at those rates -- the core block's edges at the LDS
-    rate, the remaining edges at the all-hit L2 rate -- because the two kernels run side by side on different units.  Edges in
-    dense cells are not gathered at all: that kernel's own time is not part of this ceiling."""
+    rate, the remaining edges at the all-hit L2 rate -- because the two kernels run side by side on different units.  Dense
+    cells are not gathered and run before the rest: what the matrix cores need for their products at full rate is added."""
     sink = torch.empty(262144, device="cuda")
     small = max(1, (3 << 20) // ld_bytes)
     table = torch.zeros(max(small, table_rows) * ld_bytes, dtype=torch.uint8, device="cuda")
@@ -178,9 +183,12 @@ def gather_ceiling(torch, host, ld_bytes, row_bytes, table_rows, edges, ms, core
     t_lds = core_edges / (out["lds_G_rows_per_s"] * 1e9) * 1e3
     out["edges_from_lds"], out["edges_through_l2"] = int(core_edges), int(edges - core_edges - cell_edges)
     out["edges_in_dense_cells"] = int(cell_edges)
-    out["ceiling_ms"] = round(max(t_l2, t_lds), 4)
-    out["ceiling_is"] = "max(edges through the L2 / all-hit rate = %.4f ms, edges from LDS / LDS rate = %.4f ms)" % (t_l2, t_lds)
-    out["frac_of_gather_ceiling"] = round(max(t_l2, t_lds) / ms, 3)
+    t_cells = cells * ((dim + 15) // 16) * CELL_NS_PER_16_COLUMNS * 1e-6
+    ceiling = t_cells + max(t_l2, t_lds)
+    out["ceiling_ms"] = round(ceiling, 4)
+    out["ceiling_is"] = ("cells' products at the matrix cores' rate = %.4f ms + " % t_cells if cells else "") + \
+        "max(edges through the L2 / all-hit rate = %.4f ms, edges from LDS / LDS rate = %.4f ms)" % (t_l2, t_lds)
+    out["frac_of_gather_ceiling"] = round(ceiling / ms, 3)
     return out
 
 
@@ -194,6 +202,8 @@ MEASURED_TRAFFIC = {
     "gcn2_agg1_blocked": (1_746_502_963, (4, 16)),
     "gcn2_agg2_core36864_blocked": (5_892_428_288, (4, 16)),   # what the cost model picks at width 41: dense core of 36864 rows, workgroups of equal work
     "gcn2_agg1_core61440_blocked": (1_786_640_486, (4, 8)),    # ... and at width 16: 61440 rows
+    "gcn2_agg2_cells_blocked": (5_560_100_045, (4, 16)),   # dense cells instead of the core, by rule: staging, cells, their reduction, rest, finish
+    "gcn2_agg1_cells_blocked": (1_431_298_355, (4, 8)),
     "share_agg": (1_213_309_056, (4, 4)),
     "share_agg_compact": (1_028_547_520, (4, 4)),   # remote rows staged compactly (one row per distinct remote id)
     "gin_agg": (25_550_513_561, (16, 1)),
@@ -202,10 +212,12 @@ MEASURED_TRAFFIC = {
 }
 
 
-def load_traffic(kernel_key, args, blk=-1, core=-1):
+def load_traffic(kernel_key, args, blk=-1, core=-1, cells=0):
     """{"traffic": bytes or None, "traffic_measured_at": knobs} for the roofline object."""
     if core > 0:
         kernel_key += "_core%d" % core
+    if cells > 0:
+        kernel_key += "_cells"
     if blk > 0:
         if blk != 49152:
             return {"traffic": None}
@@ -215,7 +227,8 @@ def load_traffic(kernel_key, args, blk=-1, core=-1):
         return {"traffic": None}
     nbytes, (w, d) = MEASURED_TRAFFIC[kernel_key]
     return {"traffic": nbytes, "traffic_measured_at": "ps=16 wpb=%d dist=%d%s%s" % (w, d, ", column blocks of 49152 ids" if blk > 0 else "",
-                                                                                 ", dense core of %d rows" % core if core > 0 else "")}
+                                                                                 ", dense core of %d rows" % core if core > 0 else
+                                                                                 ", %d dense cells" % cells if cells else "")}
 
 
 class Knobs:
@@ -392,7 +405,7 @@ def bench_gcn2(args, torch, host):
             "avg_launch_ms": round(avg["agg2"], 4), "median_launch_ms": round(med["agg2"], 4),
             "algorithmic_bytes": b2, "algorithmic_gbps": round(b2 / (avg["agg2"] * 1e-3) / 1e9, 1),
             "algorithmic_gbps_over_hbm_peak": round(b2 / (avg["agg2"] * 1e-3) / 1e9 / HBM_PEAK_GBPS, 3),
-            **({"traffic": None} if k2.cells else load_traffic("gcn2_agg2", args, k2.blk, k2.core))}
+            **load_traffic("gcn2_agg2", args, k2.blk, k2.core, k2.cells)}
     comp = agg2_core_plan_bytes if k2.core > 0 or k2.cells else nnz * 4   # lists or cells + remaining ids, or the plain id stream
     comp += V * pitch * 4 + V * out_dim * 4 + (V + 1) * 4           # the table once, the output once, the row pointers
     agg2["compulsory_hbm_bytes"] = int(comp)
@@ -400,7 +413,7 @@ def bench_gcn2(args, torch, host):
     if agg2.get("traffic"):
         agg2["frac_traffic"] = round(agg2["traffic"] / (avg["agg2"] * 1e-3) / 1e9 / HBM_PEAK_GBPS, 4)
     agg2["gather_ceiling"] = gather_ceiling(torch, host, pitch * 4, ldo * 4, V, nnz, avg["agg2"], core_edges if k2.core > 0 else 0,
-                                            core_edges if k2.cells else 0)
+                                            core_edges if k2.cells else 0, k2.cells, out_dim)
     extra["launches_per_forward"] = ("dense 1 + aggregation %d + dense 1 + aggregation %d (softmax inside)" %
                                      ((5, 5) if (k2.core > 0 or k2.cells) and k2.blk > 0 else ((6, 6) if k2.core > 0 or k2.cells else (2, 2))))
     extra["agg2_cache_resident"] = agg2
