@@ -436,8 +436,9 @@ __global__ void __launch_bounds__(1024) MGGX_AGG_OCCUPANCY k_agg(AggArgs a)
     // at width 32: 1.59 -> 1.77 ms) and the same without it.
     constexpr bool OFF_CROSSBAR = LPR == 4 || LPR == 16 || LPR == 32;
     extern __shared__ __align__(16) float lds[];
-    // Small plans look at the gate once their first descriptors are on their way (five layers of GIN on 50 K nodes: 294 -> 281 us); not the
-    // softmax beside the counters, where it costs (GCN forward on 20 K nodes: 93.3 us, 93.8 with it, 92.4 without).
+    // Small plans look at the gate once their first descriptors are on their way: 2 - 13 % with the counters at widths 41 to 64 on power-law graphs
+    // of 4 K to 100 K nodes (us, width 41, before / behind: 38.6 / 36.4, 27.2 / 23.7, 42.8 / 40.8).  Not the softmax beside the counters, which
+    // loses 2 - 6 % on the same nine graphs (width 48: 42.2 / 44.3, 32.3 / 34.0, 49.4 / 52.2; level only at 4 K nodes).
     constexpr bool GATE_LATER = FORM == FORM_WHOLE || (FORM == FORM_FUSE && !SMX);
     const GateSeen seen = gate_read(a.gate);
     if (!GATE_LATER && gate_closed(a.gate, seen)) return;
@@ -1226,17 +1227,19 @@ int run_agg(Plan *plan, float *d_out, const void *d_in_l, const void *d_in_r, co
         return fail(MGGX_EINVAL, "aggregation: unknown input dtype %d", o.in_dtype);
     }
     // Rows of several cache lines out of a table beyond the L2s: each XCD gathers one slice of the columns, whole lines, so that its L2
-    // holds its slice of twice (four times) as many rows; every slice reads the index stream for itself.  Only where rows start on line
-    // boundaries (slices of 40, 41 or 100 packed columns share their lines: 25 to 50 % slower), fp32, without the softmax, which needs
-    // the whole row, not with a caller's own partitions (the static scratch takes what it took: its carry buffer depends on the slots), and not beside the LDS kernel, which takes the CUs the smaller hit latency would free (1 M nodes, 47 M neighbors, width
-    // 64: 950 -> 1,113 us).  Table sizes (us whole / 2 / 4 slices): 256-byte rows: 13 MB 41.0 / 42.5, 26 MB 42.7 / 44.5, 84.6 / 85.7 and 43.7 / 41.1,
-    // 44 MB 99.7 / 89.5, 77 MB 144 / 117; 512-byte rows: 15 MB 39.9 / 38.2 / 46.0, 31 MB 92 / 81 / 89, 51 MB 180 / 155 / 172, 87 MB 232 / 171 / 180 and
-    // 205 / 174 / 151, 154 MB 203 / 171 / 161 and 886 / 651 / 576, 512 MB 3,517 / 2,770 / 2,671; 1,024-byte rows: 31 MB 73 / 67 / 67, 61 MB 244 / 167 / 152,
-    // 102 MB 600 / 431 / 325, 307 MB 1,952 / 1,549 / 1,220 (eight slices: 362 at 102 MB, 1,236 at 307).  Single lines of 512-byte rows from beyond
-    // the memory-side cache cost more than pairs of them (1 M nodes, 512 MB: 813 whole, 696 in pairs, 743 in fours).  Graphs without hubs
-    // (the longest row less than 16 mean ones) re-use too little of a large slice: above 32 MB of it they stay whole (uniform
-    // neighbors, 43 MB 95 / 92, 87 MB 198 / - / 182, but 77 MB, 40 per row, 428 / 436, 256 MB 428 / 454, 512 MB 855 / - / 917); column blocks of 12 MB and
-    // more gain without hubs, too (150 K nodes, 150 per row, 256- / 512- / 1,024-byte rows: 631 -> 445, 1,435 -> 1,241, 3,153 -> 2,569).
+    // holds its slice of twice (four times) as many rows; every slice reads the index stream for itself.  fp32 rows that start on line
+    // boundaries (packed rows of 40, 41 or 100 columns share their lines: 25 to 50 % slower); not the softmax, which needs the whole
+    // row; not a caller's own partitions (the carry buffer of the static scratch depends on the slots); not beside the LDS kernel, which takes
+    // the CUs that shorter latencies would free (1 M nodes, 47 M neighbors, width 64: 950 -> 1,113 us).  us, whole / 2 / 4 slices:
+    //  - two slices: rows of two lines from tables of 32 MB (26 MB 84.6 / 85.7, 44 MB 99.7 / 89.5), longer ones from 12 MB (512-byte
+    //    rows, 15 MB: 39.9 / 38.2, 31 MB 92 / 81);
+    //  - four: rows of four lines out of 80 to 256 MB (51 MB 155 in two, 172 in four; 154 MB 171 / 161; from beyond the memory-side cache
+    //    single lines cost more than pairs of them, 512 MB 696 / 743), rows of eight from 31 MB (61 MB 167 / 152, 307 MB 1,549 / 1,220; eight
+    //    slices 1,236);
+    //  - graphs without hubs (the longest row less than 16 mean ones) re-use too little of a large slice: up to 32 MB of it (uniform
+    //    neighbors, 43 MB 95 / 92, 77 MB 428 / 436, 256 MB 428 / 454).  Column blocks gain without hubs, too (150 K nodes, 150 per row,
+    //    256- / 512- / 1,024-byte rows: 668 -> 467, 1,518 -> 1,311, 3,366 -> 2,734).
+    // The whole tables: profiles/cells_slices_whole_rows.md.
     int slices = 1, slice_cols = dim;
     {
         const auto on_line = [](const void *p) { return (reinterpret_cast<uintptr_t>(p) & 127u) == 0; };
@@ -1591,8 +1594,10 @@ int run_knobs(GraphInfo &g, const Knobs &k, float *d_out, const void *d_in_local
     }
     if (cp) {
         // Index lists: the core block is bound by the LDS, the rest of the CSR by the caches, and they run side by side, the core's
-        // sums on a second stream.  Dense cells: they hold the chip's registers, so they run first, on this stream (side by side
-        // with the rest: 405 us instead of 385 at width 16, 950 instead of 967 at width 41, 233 K nodes).
+        // sums on a second stream.  Dense cells run first, on this stream: k_cells and k_agg hold the same registers and the same fabric, and
+        // side by side they take between 3 % less and 5 % more, for a second stream and two events (us, first / beside, widths 16, 41, 64:
+        // 233 K nodes, 216 M drawn edges 368 / 385, 947 / 947, 1,006 / 1,009; 80 M 266 / 279, 634 / 633, 682 / 680; 100 K nodes, 45 M
+        // 118 / 121, 265 / 259, 320 / 310; 50 K nodes, 20 M, widths 41, 64: 114 / 117, 131 / 138).
         // Where the rest ends in the finish kernel of a column-blocked plan, the same kernel joins the side stream, adds the core's
         // sums and applies the caller's epilogue; otherwise the rest runs with the epilogue except its post-operations (ReLU,
         // softmax), and k_core_finish adds the sums (times the row scale) and applies those last.
