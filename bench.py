@@ -250,6 +250,10 @@ class Knobs:
     def tuple(self):
         return (self.ps, self.wpb, self.dist, self.blk, self.core)
 
+    def saw_cells(self, kernel):
+        m = re.search(r" cells=(\d+)", kernel)
+        self.cells = int(m.group(1)) if m else 0
+
     def observe(self, host, call):
         """Where choices were left to the library: run the call once and read back what it used."""
         call()
@@ -258,8 +262,7 @@ class Knobs:
         if self.blk == 0:
             self.blk = 49152 if m and int(m.group(1)) > 1 else -1
         if self.core == 0:
-            m = re.search(r"cells=(\d+)", k)
-            self.cells = int(m.group(1)) if m else 0
+            self.saw_cells(k)
             m = re.search(r"core=(\d+)", k)
             self.core = 0 if self.cells else int(m.group(1)) if m else -1
         m = re.search(r"wpb=(\d+) dist=(\d+)", k)
@@ -458,7 +461,10 @@ def bench_gcn2(args, torch, host):
     if not args.tune and not args.no_search:
         mark = host.cache_stats()
         t0 = time.perf_counter()
-        s1, s2 = Knobs(args, search1), Knobs(args, search2)
+        s1 = Knobs(args, search1)
+        s1.saw_cells(host.last_agg_kernel())
+        s2 = Knobs(args, search2)
+        s2.saw_cells(host.last_agg_kernel())
         torch.cuda.synchronize()
         search_wall = (time.perf_counter() - t0) * 1e3
         now = host.cache_stats()

@@ -319,10 +319,11 @@ int mggx_sag_np_div_tune(float *d_out, const void *d_in_local, const void *d_in_
 
 /* Dense cells by request (see mggx_sag_np_div): builds (or finds) the plan of dense cells of this local-only CSR for fp32 rows of dim
  * columns (1..64), of all cells with at least least_edges edges, and has later mggx_sag_np_div calls on the same arrays and dim that
- * leave core_rows = 0 use it, whatever the rule or an earlier search says (a later search decides anew).  The arrays are those of mggx_sag_np_div.  *num_cells, *num_edges (may be
- * NULL): cells kept and edges in them; 0 where there is none, or where the CSR lists an edge twice among its 122,880 rows of highest
- * degree.  Where there is no device memory for the plan the call fails with MGGX_ENOMEM (mggx_sag_np_div by rule goes on without
- * cells then, and does not try again until this call has).  Synchronises; not for a first use inside a stream capture. */
+ * leave core_rows = 0 use it, whatever the rule or an earlier search says (a later search decides anew).  The arrays are those of
+ * mggx_sag_np_div.  *num_cells, *num_edges (may be NULL): cells kept and edges in them; 0 where there is none, or where the CSR lists an
+ * edge twice among its 122,880 rows of highest degree: later calls go on as before then.  Where there is no device memory for the plan the
+ * call fails with MGGX_ENOMEM (mggx_sag_np_div by rule goes on without cells then, and does not try again until this call has).
+ * Synchronises; not for a first use inside a stream capture. */
 int mggx_cells_prepare(const int *d_ptr_l, const int *d_col_l, const int *d_ptr_r, const int *d_col_r, int lb, int ub, int dim,
                        int least_edges, int64_t *num_cells, int64_t *num_edges);
 
